@@ -561,7 +561,7 @@ def main():
                              "kernel_us": same_k, "kernel_frac": dec_bytes / same_k / 1e3 / HBM_PEAK_GBS}
     proj_us = float(np.mean(proj_replays)) if proj_replays else stages["o_proj"]["avg_us"]
     proj_bytes = hidden * hidden * 2
-    out["o_proj"] = {"kernel": "wavek_linear_kernel + linear_reduce_kernel" if proj_ws_bytes else "wavek_linear_kernel", "rows": int(bt.decoding_batches), "in_features": hidden,
+    out["o_proj"] = {"kernel": "stream_linear_kernel + linear_reduce_kernel" if proj_ws_bytes else "stream_linear_kernel", "rows": int(bt.decoding_batches), "in_features": hidden,
                      "out_features": hidden, "bound": "hbm", "weight_bytes": proj_bytes, "kernel_us": proj_us,
                      "achieved": proj_bytes / (proj_us * 1e-6) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": proj_bytes / (proj_us * 1e-6) / 1e9 / HBM_PEAK_GBS,

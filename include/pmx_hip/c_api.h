@@ -489,15 +489,15 @@ PMXHIP_API int pmxhip_rope_kv_cache_quantize(const pmxhip_rope_params* rope, con
  * one rank, an all-reduce (one GPU here, so none).  The attention output (B, Hq * D) is this call's input in
  * place.  bias may be NULL.  Strides are in halves per row.  Needs N % 16 == 0, K % 32 == 0, 16-byte aligned
  * rows of input and weight and 8-byte aligned rows of output and bias; anything else returns
- * PMXHIP_UNSUPPORTED.  The kernels of this library are written for the decode step (M up to a few hundred rows:
- * bound by streaming the K * N * 2 weight bytes); they serve any M, 128 rows at a time, allocate nothing and add
+ * PMXHIP_UNSUPPORTED.  One kernel is written for the decode step (M up to a few hundred rows: bound by streaming the
+ * K * N * 2 weight bytes), one for the query rows of prompts (compute-bound); they allocate nothing and add
  * their partial sums in a fixed order, so a call's result does not depend on timing.
- * workspace: at decode sizes there are fewer blocks of 64 output columns than CUs, so the k range is split over
+ * workspace: where the output has fewer tiles than the chip has CUs and K is long, the k range is split over
  * several workgroups whose float32 partial tiles pass through `workspace` (the role of the reference's
  * cublas_workspace argument) and are added in a fixed order by a second kernel.
  * pmxhip_row_parallel_linear_workspace_size gives the bytes that serve (M, in_features, out_features) on the
  * current device (0 = none needed); with a NULL or smaller workspace the call still computes the same function,
- * one k range per column block (slower at decode sizes).  The workspace needs 16-byte alignment and no clearing.
+ * one k range per tile (slower for a long K).  The workspace needs 16-byte alignment and no clearing.
  *
  * The _ex forms take flags.  PMXHIP_LINEAR_VENDOR_GEMM: from 384 rows on (a prefill chunk's query rows: a
  * compute-bound GEMM) the problem goes to hipBLASLt, as the reference's goes to cublasLt, if libhipblaslt.so can be

@@ -146,6 +146,36 @@ __device__ __forceinline__ void wave_lds_handoff()
     __builtin_amdgcn_wave_barrier();
 }
 
+// ---- memory -> LDS without registers ---------------------------------------------------------
+// The LDS address of a shared array.  Taking it lets the array escape, so that the compiler does not treat memory that
+// only the asm statements below write as never written.
+__device__ __forceinline__ uint32_t lds_address(const char* p)
+{
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
+}
+// 16 bytes per lane from `base` (wave-uniform) + `offset` to LDS address `lds` (wave-uniform) + 16 * lane.  Counted by
+// vmcnt, in order with the wave's other vector memory requests; the compiler knows of neither the request nor the
+// write, so waits are placed by hand (below) and "memory" keeps its own accesses on their side.  NT: non-temporal hint.
+template <bool NT>
+__device__ __forceinline__ void load_to_lds16(uint32_t lds, uint32_t offset, const void* base)
+{
+    if (NT) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(offset), "s"(base) : "memory");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
+}
+// until at most N of the wave's vector memory requests are on their way
+template <int N>
+__device__ __forceinline__ void wait_vector_memory()
+{
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N < 63 ? N : 63) : "memory");
+}
+// the same, with the wave's own LDS reads done, then the workgroup's barrier: what every wave requested up to here has
+// landed and what every wave read up to here may be overwritten
+template <int N>
+__device__ __forceinline__ void wait_and_meet()
+{
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N < 63 ? N : 63) : "memory");
+}
+
 // Index arrays (kvstarts, cachestarts) are read-only for the whole launch and are read at
 // wave-uniform addresses: viewing them through the constant address space lets the compiler use
 // scalar loads (scalar cache, no vector registers, no vector wait count) for them.

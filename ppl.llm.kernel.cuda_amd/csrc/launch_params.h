@@ -208,9 +208,8 @@ inline int ensure_dynamic_lds(const void* kernel, int bytes, hipStream_t stream,
     return set_dynamic_lds_once(kernel, bytes, ready);
 }
 
-// Rows from which the output projection is a compute-bound GEMM and, when the caller asks for it
-// (PMXHIP_LINEAR_VENDOR_GEMM), goes to the vendor library where that can be loaded (linear_library.cpp); up to here
-// this build's weight-streaming kernels are as fast or faster.
+// Rows from which the output projection goes to the vendor library when the caller asks for it
+// (PMXHIP_LINEAR_VENDOR_GEMM) and it can be loaded (linear_library.cpp).
 constexpr int64_t kLinearLibraryRows = 384;
 constexpr int64_t kLinearLibraryWorkspace = 64 << 20; // what the library is offered when the caller asks how much to bring
 bool linear_library_available();

@@ -138,3 +138,33 @@ def test_hip_linear_strided_rows_and_attention_hand_off(pkg, oracle, m):
     pkg.ops.row_parallel_linear(attn, torch.from_numpy(w).cuda(), None, out)
     torch.cuda.synchronize()
     assert_close(out.cpu().numpy(), a, w, None, "attention output in place")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [
+    # one for every tile, with rows, columns and k that are no multiples of it: 32 x 64, 64 x 64 (65 k pieces for four
+    # waves; few k on the shared ring), 128 x 64, 128 x 128, 256 x 128 in four k ranges, 256 x 256, and weights that carry the non-temporal hint
+    (37, 4112, 4096), (129, 4112, 4160), (129, 4112, 576), (333, 4112, 1056), (1000, 2576, 4128), (257, 4112, 14336), (2049, 4112, 1056),
+    (5, 8208, 4160)])
+def test_hip_linear_tile_edges(pkg, oracle, shape):
+    """float32 sums in another order than the oracle's and one rounding to half, as above."""
+    test_hip_linear_matches_oracle(pkg, oracle, shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [3, 700])
+def test_hip_linear_rows_far_apart_and_output_rows_on_8_bytes(pkg, m):
+    """Weight rows 2^23 halves apart (beyond the 32-bit row offsets of the tile kernels), and output rows that start on
+    8-byte addresses only."""
+    import torch
+    rng = np.random.default_rng(m)
+    n, k = 48, 64
+    a, w, b = draw(rng, m, n, k)
+    far = torch.zeros((n, 1 << 23), dtype=torch.float16, device="cuda")
+    far[:, :k] = torch.from_numpy(w).cuda()
+    for weight, bias in ((far[:, :k], b), (torch.from_numpy(w).cuda(), None)):
+        out = torch.full((m, n + 4), float("nan"), dtype=torch.float16, device="cuda")
+        pkg.ops.row_parallel_linear(torch.from_numpy(a).cuda(), weight, None if bias is None else torch.from_numpy(bias).cuda(), out[:, :n])
+        torch.cuda.synchronize()
+        assert_close(out[:, :n].cpu().numpy(), a, w, bias, "far rows" if bias is not None else "8-byte rows")
+        assert torch.isnan(out[:, n:]).all()
