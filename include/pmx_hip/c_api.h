@@ -285,15 +285,26 @@ typedef struct pmxhip_prefill_params {
      * prefill_query_rows proves too small (more rows than prefill sequences * max_seqlen) keeps the batch on the tile
      * kernel, which walks every row whatever the hint; otherwise the rows of a sequence beyond max_seqlen are not
      * computed and are filled with NaN, so that an understated hint shows in the output.  A layout or alignment that
-     * the decode kernels refuse also keeps the batch on the tile kernel. */
+     * the decode kernels refuse also keeps the batch on the tile kernel.
+     * Any other batch of few query tiles shares the kv tokens of a tile out over several workgroups when the workspace has
+     * pmxhip_prefill_split_workspace_size() bytes: the parts lie in it until a second launch adds them. */
     void* workspace;
     int64_t workspace_size;
 } pmxhip_prefill_params;
 
 PMXHIP_API int pmxhip_prefill_attention(const pmxhip_prefill_params* p, pmxhip_stream_t stream);
 
+/* Bytes of pmxhip_prefill_params::workspace with which a batch of few query tiles (at most one per compute unit,
+ * half of that with decode sequences in the step; at most 64 prefill sequences; walks long enough to be worth sharing) splits the kv tokens of its tiles; 0 for every other
+ * batch.  query_rows: pmxhip_prefill_params::prefill_query_rows; from_current: current_key is given; compute_units 0 =
+ * those of the current device. */
+PMXHIP_API int64_t pmxhip_prefill_split_workspace_size(int64_t batch, int64_t decoding_batches, int64_t max_seqlen,
+                                                       int64_t max_kvlen, int64_t query_rows, int64_t num_heads,
+                                                       int64_t num_kv_heads, int64_t head_dim, int32_t from_current,
+                                                       int32_t compute_units);
+
 /* Bytes of pmxhip_prefill_params::workspace with which a batch runs its short chunks on the decode step's kernel;
- * 0 when the batch is not one of short chunks (the tile kernel needs no workspace).  compute_units 0 = those of the
+ * 0 when the batch is not one of short chunks.  compute_units 0 = those of the
  * current device.  The operator class adds this to what it reports as cfg.workspace_size (the decode and the
  * prefill stage run one after the other on the stream and share the buffer). */
 PMXHIP_API int64_t pmxhip_prefill_workspace_size(int64_t batch, int64_t decoding_batches, int64_t max_seqlen,

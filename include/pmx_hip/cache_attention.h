@@ -76,6 +76,8 @@ public:
         int64_t prefill_query_rows; // not in the reference: rows of query beyond the decode rows.  A hint that lets the
                                     // prefill stage launch fewer workgroups; 0 = unknown.  A wrong value costs time only:
                                     // the stage's workgroups walk every query tile of the batch whatever the launch size.
+        int64_t prefill_workspace_offset; // not in the reference: where the prefill stage's share of the workspace starts
+                                          // (behind the decode stage's where it splits its query tiles' kv tokens, 0 otherwise)
     } cfg{};
 
     // Validates, derives strides / attn_scale / split plan and fills cfg.  Host only.

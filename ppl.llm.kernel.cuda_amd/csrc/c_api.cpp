@@ -459,19 +459,7 @@ int pmxhip_splitkv_combine(const float* partial_out, const float* partial_ml, co
 
 namespace {
 
-// Short chunks (a few query tokens per sequence: speculative decoding's candidates, the tail of a chunked prefill)
-// leave most of the tile kernel's 256 columns empty and are bound by its tile staging.  Where a kv head's (query
-// position, query head) pairs fit the 32 columns of the decode step's MFMA kernel they run there instead, over token
-// ranges with a combine kernel, which streams the cache at the decode rate.  That path has no mask, alibi or fp16-K/V
-// form and serves head_dim 64 and 128.
-constexpr int64_t kPrefillChunkColumns = 32;
-
-bool prefill_chunk_shape(int64_t max_seqlen, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim)
-{
-    if (head_dim != 64 && head_dim != 128) return false;
-    if (num_kv_heads <= 0 || num_heads % num_kv_heads != 0 || max_seqlen <= 0) return false;
-    return max_seqlen * (num_heads / num_kv_heads) <= kPrefillChunkColumns;
-}
+using pmxhip::prefill_chunk_shape;
 
 // the kernel of that path: the 16-column form where the columns fit it (head_dim 128 only), else the 32-column form
 int32_t prefill_chunk_kernel(int64_t columns, int64_t head_dim)
@@ -499,6 +487,16 @@ int64_t pmxhip_prefill_workspace_size(int64_t batch, int64_t decoding_batches, i
     if (prefill_chunk_plan(prefill_batches, max_seqlen, max_kvlen, num_heads, num_kv_heads, head_dim, compute_units, &plan) != PMXHIP_SUCCESS)
         return 0;
     return plan.workspace_size;
+}
+
+int64_t pmxhip_prefill_split_workspace_size(int64_t batch, int64_t decoding_batches, int64_t max_seqlen, int64_t max_kvlen,
+                                            int64_t query_rows, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                                            int32_t from_current, int32_t compute_units)
+{
+    if (decoding_batches < 0 || !head_dim_supported(head_dim) || num_kv_heads <= 0 || num_heads % num_kv_heads != 0) return 0;
+    return pmxhip::prefill_split_choose(batch - decoding_batches, max_seqlen, max_kvlen, query_rows, num_heads, num_kv_heads, head_dim,
+                                        from_current != 0, decoding_batches > 0, compute_units > 0 ? compute_units : current_compute_units())
+        .bytes;
 }
 
 int pmxhip_prefill_attention(const pmxhip_prefill_params* p, pmxhip_stream_t stream)
@@ -542,8 +540,9 @@ int pmxhip_prefill_attention(const pmxhip_prefill_params* p, pmxhip_stream_t str
     // sequences proves too small (more rows than sequences * max_seqlen) keeps the batch on the tile kernel, which
     // walks every row whatever the hint.
     const bool hint_covers_rows = p->prefill_query_rows <= 0 || p->prefill_query_rows <= prefill_batches * p->max_seqlen;
-    if (!from_current && !p->attn_mask && !p->alibi_slopes && p->workspace && aligned16(p->workspace) && hint_covers_rows &&
-        prefill_chunk_shape(p->max_seqlen, p->num_heads, p->num_kv_heads, p->head_dim)) {
+    const bool short_chunks = !from_current && !p->attn_mask && !p->alibi_slopes &&
+                              prefill_chunk_shape(p->max_seqlen, p->num_heads, p->num_kv_heads, p->head_dim);
+    if (short_chunks && p->workspace && aligned16(p->workspace) && hint_covers_rows) {
         pmxhip_decode_plan plan;
         if (prefill_chunk_plan(prefill_batches, p->max_seqlen, p->max_kvlen, p->num_heads, p->num_kv_heads, p->head_dim, 0, &plan) ==
                 PMXHIP_SUCCESS &&
@@ -629,6 +628,18 @@ int pmxhip_prefill_attention(const pmxhip_prefill_params* p, pmxhip_stream_t str
     a.cache_stride_h = p->cache_stride_h;
     a.cache_stride_kv = p->cache_stride_kv;
     a.cachestarts_stride_b = p->cachestarts_stride_b;
+    if (!short_chunks && p->workspace && aligned16(p->workspace)) {
+        // few query tiles: their kv tokens shared out over the chip, the parts in the caller's workspace
+        const pmxhip::PrefillSplit split =
+            pmxhip::prefill_split_choose(prefill_batches, p->max_seqlen, p->max_kvlen, a.query_rows, p->num_heads, p->num_kv_heads,
+                                         p->head_dim, from_current, p->decoding_batches > 0, current_compute_units());
+        if (split.ranges > 0 && split.bytes <= p->workspace_size) {
+            a.split_ranges = split.ranges;
+            a.split_gain = split.gain;
+            a.split_out = (float*)p->workspace;
+            a.split_ml = (float*)((char*)p->workspace + split.out_bytes);
+        }
+    }
     return launch_result("prefill_attention", pmxhip::launch_prefill(a, stream));
 }
 

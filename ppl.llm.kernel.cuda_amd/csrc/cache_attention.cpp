@@ -18,6 +18,8 @@
 #include "pmx_hip/rotary_position_embedding.h"
 #include "pmx_hip/row_parallel_linear.h"
 
+#include "launch_params.h"
+
 namespace ppl { namespace kernel { namespace llm { namespace cuda { namespace pmx {
 
 namespace {
@@ -218,10 +220,22 @@ ppl::common::RetCode dynamic_batching_multi_head_cache_attention::heuristic_prep
     cfg.workspace_size = plan.workspace_size;
     // short prefill chunks run on the decode step's kernel and keep their split-KV pieces in the same workspace (the
     // two stages follow each other on the stream)
-    if (enable_cache_prefill && prefill_batches > 0 && !attn_mask && !alibi_slopes) {
+    cfg.prefill_workspace_offset = 0;
+    if (prefill_batches > 0 && enable_cache_prefill && !attn_mask && !alibi_slopes &&
+        pmxhip::prefill_chunk_shape(max_seqlen, num_heads, num_kv_heads, head_dim)) {
         const int64_t chunk_ws = pmxhip_prefill_workspace_size(batch, decoding_batches, max_seqlen, max_kvlen, num_heads,
                                                                num_kv_heads, head_dim, device_prop.multiProcessorCount);
         if (chunk_ws > cfg.workspace_size) cfg.workspace_size = chunk_ws;
+    } else if (prefill_batches > 0 && specify_decoding_multi_block != 0) {
+        // a batch of few query tiles shares out their kv tokens and keeps the parts behind the decode stage's pieces
+        // (disjoint, so that the stages may still run side by side); 0 asks for no split and no workspace
+        const pmxhip::PrefillSplit split =
+            pmxhip::prefill_split_choose(prefill_batches, max_seqlen, max_kvlen, cfg.prefill_query_rows, num_heads, num_kv_heads,
+                                         head_dim, !enable_cache_prefill, decoding_batches > 0, device_prop.multiProcessorCount);
+        if (split.ranges > 0) {
+            cfg.prefill_workspace_offset = (cfg.workspace_size + 255) / 256 * 256;
+            cfg.workspace_size = cfg.prefill_workspace_offset + split.bytes;
+        }
     }
     cfg.enable_cache_prefill = enable_cache_prefill;
     return ppl::common::RC_SUCCESS;
@@ -339,8 +353,12 @@ ppl::common::RetCode dynamic_batching_multi_head_cache_attention::forward_prefil
     p.mask_stride_h = cfg.mask_stride_h;
     p.alibi_slopes = static_cast<const float*>(cfg.alibi_slopes);
     p.prefill_query_rows = cfg.prefill_query_rows;
-    p.workspace = cfg.workspace;
-    p.workspace_size = cfg.workspace_size;
+    if (cfg.workspace &&
+        (cfg.prefill_workspace_offset > 0 ||
+         pmxhip::prefill_chunk_shape(cfg.max_seqlen, cfg.num_heads, cfg.num_kv_heads, cfg.head_dim))) {
+        p.workspace = static_cast<char*>(cfg.workspace) + cfg.prefill_workspace_offset;
+        p.workspace_size = cfg.workspace_size - cfg.prefill_workspace_offset;
+    }
     if (!cfg.enable_cache_prefill) { // kernel.cu:2181-2212: the step's own fp16 K/V only, no cache read
         p.current_key = cfg.current_key;
         p.current_value = cfg.current_value;
@@ -374,8 +392,7 @@ ppl::common::RetCode dynamic_batching_multi_head_cache_attention::forward(const 
     // the prefill stage on the short-chunk route writes its pieces into the workspace that the decode stage is using
     const bool shared_workspace =
         cfg.workspace != nullptr && cfg.decoding_multi_block_size > 1 && cfg.enable_cache_prefill && !cfg.attn_mask && !cfg.alibi_slopes &&
-        pmxhip_prefill_workspace_size(cfg.batch, cfg.decoding_batches, cfg.max_seqlen, cfg.max_kvlen, cfg.num_heads, cfg.num_kv_heads,
-                                      cfg.head_dim, cfg.device_prop ? cfg.device_prop->multiProcessorCount : 0) > 0;
+        pmxhip::prefill_chunk_shape(cfg.max_seqlen, cfg.num_heads, cfg.num_kv_heads, cfg.head_dim);
     if (cfg.decoding_batches <= 0 || cfg.prefill_batches <= 0 || side_stream == stream || shared_workspace) return forward(stream);
     if (!fork_event || !join_event) {
         PMX_LOG_ERROR("forward on two streams needs a fork and a join event");

@@ -180,4 +180,17 @@ bool decode_quad_launch_ok(const DecodeLaunch& a)
     return true;
 }
 
+// Short chunks (a few query tokens per sequence: speculative decoding's candidates, the tail of a chunked prefill)
+// leave most of the tile kernel's 256 columns empty and are bound by its tile staging.  Where a kv head's (query
+// position, query head) pairs fit the 32 columns of the decode step's MFMA kernel they run there instead, over token
+// ranges with a combine kernel, which streams the cache at the decode rate.  That path has no mask, alibi or fp16-K/V
+// form and serves head_dim 64 and 128.
+bool prefill_chunk_shape(int64_t max_seqlen, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim)
+{
+    constexpr int64_t kPrefillChunkColumns = 32;
+    if (head_dim != 64 && head_dim != 128) return false;
+    if (num_kv_heads <= 0 || num_heads % num_kv_heads != 0 || max_seqlen <= 0) return false;
+    return max_seqlen * (num_heads / num_kv_heads) <= kPrefillChunkColumns;
+}
+
 } // namespace pmxhip

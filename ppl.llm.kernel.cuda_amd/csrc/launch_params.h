@@ -111,7 +111,30 @@ struct PrefillLaunch {
     const void* current_value;
     int64_t key_stride_s;
     int64_t value_stride_s;
+    // the kv tokens of a tile shared out over workgroups (prefill_split_choose): ranges per kv head, 0 = whole tiles
+    int32_t split_ranges;
+    int32_t split_gain;         // weight a split has to take off the call before the kernels go by it
+    float* split_out;           // [kv head][range][first / last part] accumulators of a tile
+    float* split_ml;            // ... and (maximum, exp-sum) of its columns
 };
+
+// A range of a split prefill holds at least this many kv tokens.
+constexpr int kPrefillSplitMinTokens = 192;
+// What a split costs -- the parts written, read again and added by a second launch, about 20 us -- in kv tokens of a tile's
+// walk (a tile of 64 takes 3.4 us, from half rows 2 us).  16 q / 4 kv heads of 128, one prompt of 594 rows over 1575 (44 tiles):
+// layer call 160 -> 82 us; 5 / 5 heads, three prompts of 1737 rows (105 tiles): 127 -> 77 us; 14 / 2 heads of 64, 126 tiles of 7 kv
+// tiles, where 320 tokens are saved: level.
+constexpr int kPrefillSplitGain = 512, kPrefillSplitGain16 = 640;
+// Whether a batch of at most `rows` query rows (0 = unknown) in `sequences` sequences has too few query tiles for the chip,
+// so that their kv tokens are worth sharing out; the ranges per kv head and the workspace that takes.  `kv16`: K/V
+// are the step's own half rows; `mixed`: the step has decode sequences too.
+struct PrefillSplit {
+    int32_t ranges = 0; // 0 = whole tiles
+    int32_t gain = 0;
+    int64_t out_bytes = 0, bytes = 0;
+};
+PrefillSplit prefill_split_choose(int64_t sequences, int64_t max_seqlen, int64_t max_kvlen, int64_t rows, int64_t num_heads,
+                                  int64_t num_kv_heads, int64_t head_dim, bool kv16, bool mixed, int compute_units);
 
 // One strided copy of whole pages (cache bytes or scale bytes) between the cache and the outer buffer.
 struct PageCopyLaunch {
@@ -280,6 +303,8 @@ void launch_splitkv_combine_rows(const float* partial_out, const float* partial_
                                  const int64_t* piece_end, int64_t rows, int64_t head_dim, void* output,
                                  hipStream_t stream);
 int launch_prefill(const PrefillLaunch& a, hipStream_t stream);
+// decode_select.cpp: whether a prefill batch of this shape runs on the decode step's kernels when it has a workspace
+bool prefill_chunk_shape(int64_t max_seqlen, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim);
 
 } // namespace pmxhip
 

@@ -154,6 +154,90 @@ __device__ __forceinline__ bool pick_query_tile(const PrefillLaunch& a, int ppw,
     return false;
 }
 
+// ---- a batch of few query tiles: the kv tokens of a tile are shared out over several workgroups ----
+// A workgroup fills a CU, so a batch with fewer (tile, kv head) items than CUs leaves the others idle while each item walks
+// its whole context.  Then the tiles of the batch are laid end to end as one stream per kv head -- a tile weighs the
+// kv tokens it walks plus kSplitStart for its start -- and the stream is cut into `split_ranges` equal ranges, one per
+// workgroup: a range holds parts of at most two tiles (its first and its last) and whole tiles between them.  The
+// parts leave unnormalised sums with their (maximum, exp-sum) pairs in the workspace and prefill_combine_kernel adds
+// them.  Both kernels derive the same cuts from seqstarts and kvstarts.
+// Weights are closed forms of (prior tokens, tile number): tile t of a sequence weighs start + base + step (t + 1).
+constexpr int64_t kSplitStart = 64;
+struct SplitStream {
+    // this lane's sequence
+    int64_t end = 0, cost = 0; // end of its tiles in the stream, and their weight
+    int64_t base = 0;          // kv tokens ahead of its first tile
+    int tiles = 0;
+    // of the whole batch
+    int64_t total = 0, step = 0;
+    int64_t per = 0;           // weight of a range; 0: the batch is not split
+};
+__device__ __forceinline__ int64_t uniform64(int64_t v)
+{
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uint64_t)v);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)v >> 32));
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ int64_t wave_max64(int64_t v)
+{
+    for (int sh = 32; sh >= 1; sh >>= 1) {
+        const int64_t o = __shfl_xor(v, sh);
+        v = o > v ? o : v;
+    }
+    return v;
+}
+__device__ __forceinline__ int64_t split_tile_start(int64_t base, int64_t step, int64_t t)
+{
+    return t * (kSplitStart + base) + step * (t * (t + 1) / 2);
+}
+__device__ __forceinline__ SplitStream split_stream(const PrefillLaunch& a, int ppw, int lane)
+{
+    SplitStream r;
+    r.step = a.is_causal ? ppw : 0;
+    if (lane < (int)a.prefill_batches) {
+        const int64_t qlen = a.seqstarts[lane + 1] - a.seqstarts[lane], kvlen = a.kvstarts[lane + 1] - a.kvstarts[lane];
+        r.base = a.is_causal ? kvlen - qlen : kvlen;
+        r.base = r.base > 0 ? r.base : 0;
+        r.tiles = qlen > 0 ? (int)((qlen + ppw - 1) / ppw) : 0;
+        r.cost = split_tile_start(r.base, r.step, r.tiles);
+    }
+    r.end = r.cost;
+    for (int sh = 1; sh < kWave; sh <<= 1) { // prefix sum over the sequences
+        const int64_t below = __shfl_up(r.end, sh);
+        if (lane >= sh) r.end += below;
+    }
+    r.total = uniform64(__shfl(r.end, kWave - 1));
+    const int64_t longest = uniform64(wave_max64(r.tiles > 0 ? kSplitStart + r.base + r.step * r.tiles : 0));
+    const int64_t ranges = a.split_ranges;
+    int64_t per = uniform64((r.total + ranges - 1) / ranges);
+    if (per < kPrefillSplitMinTokens) per = kPrefillSplitMinTokens;
+    r.per = longest - per >= a.split_gain ? per : 0; // (the call takes as long as its longest tile otherwise)
+    return r;
+}
+// the tile of the stream that holds position u < total (wave-uniform)
+__device__ __forceinline__ void split_locate(const SplitStream& st, int64_t u, int& b, int& t, int64_t& begin, int64_t& weight)
+{
+    b = __builtin_popcountll(__builtin_amdgcn_ballot_w64(st.end <= u));
+    const int64_t base = uniform64(__shfl(st.base, b)), first = uniform64(__shfl(st.end - st.cost, b));
+    int lo = 0, hi = __builtin_amdgcn_readfirstlane(__shfl(st.tiles, b)); // split_tile_start(lo) <= u - first < split_tile_start(hi)
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (first + split_tile_start(base, st.step, mid) <= u) lo = mid;
+        else hi = mid;
+    }
+    t = lo;
+    begin = first + split_tile_start(base, st.step, lo);
+    weight = kSplitStart + base + st.step * (lo + 1);
+}
+// the kv tile of `bn` tokens at which a cut v positions behind the start of a tile of that weight falls
+__device__ __forceinline__ int split_cut(int64_t v, int64_t weight, int n_tiles, int bn)
+{
+    if (v <= 0) return 0;
+    if (v >= weight) return n_tiles;
+    const int64_t k = v <= kSplitStart ? 0 : (v - kSplitStart + bn / 2) / bn;
+    return k < n_tiles ? (int)k : n_tiles;
+}
+
 } // namespace
 
 // SRC: where K/V come from: 0 = int8 cache in 128-token pages, 1 = int8 cache in contiguous runs,
@@ -177,7 +261,9 @@ __device__ __forceinline__ bool pick_query_tile(const PrefillLaunch& a, int ppw,
 // fragment reads alone take what the LDS port allows (512 KB per tile and CU at 256 bytes per clock).  A form with
 // four waves of 64 columns (half the fragment reads per product, fragments requested two steps ahead, the whole
 // register file per wave) took 1094 us: one wave per SIMD exposes every wait that a second wave covers.
-template <int D, int SRC, bool EXTRA>
+//
+// SPLIT: the launch has one workgroup per range of the split stream (above) instead of one per tile.
+template <int D, int SRC, bool EXTRA, bool SPLIT>
 __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_attention_kernel(const PrefillLaunch a)
 {
     constexpr bool PAGED = SRC == 0;
@@ -249,9 +335,35 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_attention_kernel(c
     // The workgroups of the launch share the batch's query tiles: workgroup (item, kv head) takes the items
     // item, item + item_stride, ... in the order of falling cost, so that a launch that was sized from a hint that
     // understates the batch still covers every tile (it only takes longer).
+    int64_t u_next = -1; // SPLIT: where in the stream the range's next part starts (-1: not yet known)
     for (int item = blockIdx.x / (int)a.num_kv_heads;; item += item_stride) {
     int b_pick = 0, tile_pick = 0;
-    if (!pick_query_tile(a, ppw, item, lane, b_pick, tile_pick)) return;
+    // The look-up below depends on nothing that changes from item to item but `item`; its lane masks and addresses, computed
+    // once ahead of the loop, would sit in registers that the tile loop does not have.
+    int pick_lane = lane;
+    asm volatile("" : "+v"(pick_lane));
+    int64_t cut_from = 0, cut_to = 0, weight = 0; // SPLIT: the part of the tile, in stream positions behind its start
+    int slot = 0;                                 // SPLIT: the range's first part or a later one
+    bool split = false;
+    if (SPLIT) {
+        // (looked up again for every part: nothing of it stays in vector registers through the tile loop)
+        const SplitStream stream = split_stream(a, ppw, pick_lane);
+        split = stream.per > 0;
+        if (split) {
+            const int range = blockIdx.x / (unsigned)a.num_kv_heads;
+            const int64_t u0 = range * stream.per;
+            const int64_t u_end = u0 + stream.per < stream.total ? u0 + stream.per : stream.total;
+            if (u_next < 0) u_next = u0;
+            if (u_next >= u_end) return;
+            int64_t begin = 0;
+            split_locate(stream, u_next, b_pick, tile_pick, begin, weight);
+            slot = 2 * range + (u_next == u0 ? 0 : 1);
+            cut_from = u_next - begin;
+            u_next = begin + weight < u_end ? begin + weight : u_end;
+            cut_to = u_next - begin;
+        }
+    }
+    if (!split && !pick_query_tile(a, ppw, item, pick_lane, b_pick, tile_pick)) return;
     const int b = __builtin_amdgcn_readfirstlane(b_pick);
     const int64_t q_row0 = a.seqstarts[b];
     const int qlen = (int)(a.seqstarts[b + 1] - q_row0);
@@ -280,7 +392,16 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_attention_kernel(c
         wg_lim = last_pos + 1 + kvlen - qlen;
         wg_lim = wg_lim < 0 ? 0 : (wg_lim > kvlen ? kvlen : wg_lim);
     }
-    const int n_tiles = (wg_lim + kBN - 1) / kBN;
+    const int all_tiles = (wg_lim + kBN - 1) / kBN;
+    // the kv tiles [first_tile, n_tiles) are walked: all of them, or this workgroup's part
+    int first_tile = 0, n_tiles = all_tiles;
+    bool whole = true;
+    if (SPLIT && split) {
+        first_tile = __builtin_amdgcn_readfirstlane(split_cut(cut_from, weight, all_tiles, kBN));
+        n_tiles = __builtin_amdgcn_readfirstlane(split_cut(cut_to, weight, all_tiles, kBN));
+        whole = first_tile == 0 && n_tiles == all_tiles;
+        if (!whole && first_tile >= n_tiles) continue; // the cut left nothing of the tile on this side
+    }
 
     // ---- Q fragments: B operand of S^T = K Q^T; lane holds Q[col][16 s + 8 hh .. +8] ----
     f16x8 qf[KSTEPS];
@@ -400,12 +521,12 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_attention_kernel(c
 
     // Prologue: tile 0 dequantised into buffer 0, raw bytes of tile 1 in registers.
     int64_t row_next = 0;
-    if (n_tiles > 0) {
-        load_tile(0, tile_row(0));
+    if (n_tiles > first_tile) {
+        load_tile(first_tile, tile_row(first_tile));
 #pragma unroll
         for (int k = 0; k < N_SLICES; ++k) store_slice(0, k);
-        if (n_tiles > 1) load_tile(1, tile_row(1));
-        row_next = tile_row(2);
+        if (n_tiles > first_tile + 1) load_tile(first_tile + 1, tile_row(first_tile + 1));
+        row_next = tile_row(first_tile + 2);
         __syncthreads();
     }
     // tokens this wave's columns attend to: beyond the largest limit (a tile past its columns' limits, or a wave
@@ -423,7 +544,7 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_attention_kernel(c
 
     // ---- one tile, for a wave that has columns in it.  limit: some element may lie beyond its column's limit ----
     auto tile_body = [&](int tile, const bool limit) {
-        const int buf = tile & 1;
+        const int buf = (tile - first_tile) & 1;
         const half_t* const sK = smem + buf * TILE_HALVES;
         const half_t* const sKlo = sK + K_HALVES;
         const half_t* const sV = KV16 ? sKlo : sKlo + K_HALVES;
@@ -646,12 +767,12 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_attention_kernel(c
 #undef PMX_FENCE
     };
 
-    for (int tile = 0; tile < n_tiles; ++tile) {
+    for (int tile = first_tile; tile < n_tiles; ++tile) {
         if (tile * kBN < wave_lim) {
             tile_body(tile, (tile + 1) * kBN > wave_lim_min);
         } else {
 #pragma unroll
-            for (int k = 0; k < N_SLICES; ++k) store_slice((tile & 1) ^ 1, k);
+            for (int k = 0; k < N_SLICES; ++k) store_slice(((tile - first_tile) & 1) ^ 1, k);
             if (tile + 2 < n_tiles) {
                 load_tile(tile + 2, row_next);
                 row_next = tile_row(tile + 3);
@@ -669,6 +790,21 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_attention_kernel(c
     // kernel, and lines left dirty in the memory-side cache are written back during whatever runs next (a decode launch
     // after 89 MB of such rows took 12 us longer).
     const float l_tot = l_run + __shfl_xor(l_run, 32);
+    if (SPLIT && !whole) {
+        // a part: the accumulators as they lie, 1 KB per store, and the columns' (maximum, exp-sum)
+        if (__builtin_amdgcn_ballot_w64(col_on) != 0) {
+            const int64_t piece = (int64_t)kvh * 2 * a.split_ranges + slot;
+            float* const out = a.split_out + ((piece * 8 + wave) * (D / 8) * kWave + lane) * 4;
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    *(f32x4*)(out + (4 * cb + r) * (kWave * 4)) =
+                        f32x4{o_acc[cb][4 * r], o_acc[cb][4 * r + 1], o_acc[cb][4 * r + 2], o_acc[cb][4 * r + 3]};
+            if (hh == 0) *(float2*)(a.split_ml + (piece * kCols + col) * 2) = float2{m_run, l_tot};
+        }
+        continue;
+    }
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     {
         constexpr int EP_STRIDE = D + 8;                  // halves per staged row (rows stay 16-byte aligned)
@@ -734,7 +870,7 @@ struct PrefillTile16 {
 static_assert((PrefillTile16<256>::V_STRIDE * 2) % 128 == 64, "V row stride");
 } // namespace
 
-template <int D, int SRC, bool EXTRA>
+template <int D, int SRC, bool EXTRA, bool SPLIT>
 __global__ __launch_bounds__(kPrefillThreads, D <= 128 ? 4 : 2) void prefill_attention16_kernel(const PrefillLaunch a)
 {
     constexpr bool PAGED = SRC == 0;
@@ -788,9 +924,35 @@ __global__ __launch_bounds__(kPrefillThreads, D <= 128 ? 4 : 2) void prefill_att
         u_g[u] = u_on[u] ? idx % GPT : 0;
     }
 
+    int64_t u_next = -1; // SPLIT: where in the stream the range's next part starts (-1: not yet known)
     for (int item = blockIdx.x / (int)a.num_kv_heads;; item += item_stride) {
     int b_pick = 0, tile_pick = 0;
-    if (!pick_query_tile(a, ppw, item, lane, b_pick, tile_pick)) return;
+    // The look-up below depends on nothing that changes from item to item but `item`; its lane masks and addresses, computed
+    // once ahead of the loop, would sit in registers that the tile loop does not have.
+    int pick_lane = lane;
+    asm volatile("" : "+v"(pick_lane));
+    int64_t cut_from = 0, cut_to = 0, weight = 0; // SPLIT: the part of the tile, in stream positions behind its start
+    int slot = 0;                                 // SPLIT: the range's first part or a later one
+    bool split = false;
+    if (SPLIT) {
+        // (looked up again for every part: nothing of it stays in vector registers through the tile loop)
+        const SplitStream stream = split_stream(a, ppw, pick_lane);
+        split = stream.per > 0;
+        if (split) {
+            const int range = blockIdx.x / (unsigned)a.num_kv_heads;
+            const int64_t u0 = range * stream.per;
+            const int64_t u_end = u0 + stream.per < stream.total ? u0 + stream.per : stream.total;
+            if (u_next < 0) u_next = u0;
+            if (u_next >= u_end) return;
+            int64_t begin = 0;
+            split_locate(stream, u_next, b_pick, tile_pick, begin, weight);
+            slot = 2 * range + (u_next == u0 ? 0 : 1);
+            cut_from = u_next - begin;
+            u_next = begin + weight < u_end ? begin + weight : u_end;
+            cut_to = u_next - begin;
+        }
+    }
+    if (!split && !pick_query_tile(a, ppw, item, pick_lane, b_pick, tile_pick)) return;
     const int b = __builtin_amdgcn_readfirstlane(b_pick);
     const int64_t q_row0 = a.seqstarts[b];
     const int qlen = (int)(a.seqstarts[b + 1] - q_row0);
@@ -818,7 +980,16 @@ __global__ __launch_bounds__(kPrefillThreads, D <= 128 ? 4 : 2) void prefill_att
         wg_lim = last_pos + 1 + kvlen - qlen;
         wg_lim = wg_lim < 0 ? 0 : (wg_lim > kvlen ? kvlen : wg_lim);
     }
-    const int n_tiles = (wg_lim + kBN16 - 1) / kBN16;
+    const int all_tiles = (wg_lim + kBN16 - 1) / kBN16;
+    // the kv tiles [first_tile, n_tiles) are walked: all of them, or this workgroup's part
+    int first_tile = 0, n_tiles = all_tiles;
+    bool whole = true;
+    if (SPLIT && split) {
+        first_tile = __builtin_amdgcn_readfirstlane(split_cut(cut_from, weight, all_tiles, kBN16));
+        n_tiles = __builtin_amdgcn_readfirstlane(split_cut(cut_to, weight, all_tiles, kBN16));
+        whole = first_tile == 0 && n_tiles == all_tiles;
+        if (!whole && first_tile >= n_tiles) continue; // the cut left nothing of the tile on this side
+    }
     int wave_lim = lim;
 #pragma unroll
     for (int sh = 32; sh >= 1; sh >>= 1) {
@@ -921,15 +1092,15 @@ __global__ __launch_bounds__(kPrefillThreads, D <= 128 ? 4 : 2) void prefill_att
     };
 
     __syncthreads(); // the previous item's last tile has been read by every wave
-    if (n_tiles > 0) {
-        load_tile(0);
+    if (n_tiles > first_tile) {
+        load_tile(first_tile);
         store_tile(0);
-        if (n_tiles > 1) load_tile(1);
+        if (n_tiles > first_tile + 1) load_tile(first_tile + 1);
         __syncthreads();
     }
 
-    for (int tile = 0; tile < n_tiles; ++tile) {
-        const int buf = tile & 1;
+    for (int tile = first_tile; tile < n_tiles; ++tile) {
+        const int buf = (tile - first_tile) & 1;
         // the next tile into the other buffer (every wave is past its reads of it since the barrier that ended the
         // previous iteration), and the raw bytes of the tile after next into the freed registers
         if (tile + 1 < n_tiles) store_tile(buf ^ 1);
@@ -1035,6 +1206,16 @@ __global__ __launch_bounds__(kPrefillThreads, D <= 128 ? 4 : 2) void prefill_att
     // ---- normalise and store: element j of tile ct <-> channel 16 ct + 4 kq + j ----
     float l_tot = l_run + __shfl_xor(l_run, 16);
     l_tot += __shfl_xor(l_tot, 32);
+    if (SPLIT && !whole) {
+        if (__builtin_amdgcn_ballot_w64(col_on) != 0) {
+            const int64_t piece = (int64_t)kvh * 2 * a.split_ranges + slot;
+            float* const out = a.split_out + ((piece * 8 + wave) * CT * kWave + lane) * 4;
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) *(f32x4*)(out + ct * (kWave * 4)) = o_acc[ct];
+            if (kq == 0) *(float2*)(a.split_ml + (piece * kCols16 + col) * 2) = float2{m_run, l_tot};
+        }
+        continue;
+    }
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     if (col_on) {
         half_t* op = (half_t*)a.output + (q_row0 + pos) * a.output_stride_s + (int64_t)h * D + 4 * kq;
@@ -1047,6 +1228,118 @@ __global__ __launch_bounds__(kPrefillThreads, D <= 128 ? 4 : 2) void prefill_att
         }
     }
     } // items
+}
+
+// Adds the parts that a split launch left of a tile: out = sum_i o_i 2^(m_i - M) / sum_i l_i 2^(m_i - M).  One workgroup per
+// (tile, kv head, wave of columns); its four waves share the wave's fragments, which lie as the accumulators lay (1 KB
+// per load).  A tile that one range holds entirely was written by that range.
+template <int D, int CPW>
+__global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillLaunch a)
+{
+    constexpr int COLS = 8 * CPW;                 // columns of a tile
+    constexpr int BN = CPW == 32 ? kBN : kBN16;
+    constexpr int FRAGS = D * CPW / 256;          // 16-byte fragments per lane of a wave of columns
+    constexpr int FW = FRAGS / 4;                 // ... per wave of this workgroup
+    static_assert(FRAGS % 4 == 0, "fragments per wave");
+    const int lane = threadIdx.x & 63;
+    const int part = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int G = (int)(a.num_heads / a.num_kv_heads);
+    const int ppw = COLS / G > 0 ? COLS / G : 1;
+    const int kvh = blockIdx.x % (unsigned)a.num_kv_heads;
+    const int cwave = blockIdx.y;
+
+    const SplitStream st = split_stream(a, ppw, lane);
+    if (st.per == 0) return;
+    // the item-th tile of the stream
+    int tiles_end = st.tiles;
+    for (int sh = 1; sh < kWave; sh <<= 1) {
+        const int below = __shfl_up(tiles_end, sh);
+        if (lane >= sh) tiles_end += below;
+    }
+    // (a launch sized from a hint that understates the batch still covers every tile)
+    for (int item = blockIdx.x / (unsigned)a.num_kv_heads;; item += gridDim.x / (unsigned)a.num_kv_heads) {
+    const int b = __builtin_popcountll(__builtin_amdgcn_ballot_w64(tiles_end <= item));
+    if (b >= kWave) return;
+    const int t = item - __builtin_amdgcn_readfirstlane(__shfl(tiles_end - st.tiles, b));
+    const int64_t base = uniform64(__shfl(st.base, b));
+    const int64_t begin = uniform64(__shfl(st.end - st.cost, b)) + split_tile_start(base, st.step, t);
+    const int64_t weight = kSplitStart + base + st.step * (t + 1);
+
+    const int64_t q_row0 = a.seqstarts[b];
+    const int qlen = (int)(a.seqstarts[b + 1] - q_row0);
+    const int kvlen = (int)(a.kvstarts[b + 1] - a.kvstarts[b]);
+    const int p0 = t * ppw;
+    int wg_lim = kvlen;
+    if (a.is_causal) {
+        const int last_pos = p0 + ppw - 1 < qlen - 1 ? p0 + ppw - 1 : qlen - 1;
+        wg_lim = last_pos + 1 + kvlen - qlen;
+        wg_lim = wg_lim < 0 ? 0 : (wg_lim > kvlen ? kvlen : wg_lim);
+    }
+    const int all_tiles = (wg_lim + BN - 1) / BN;
+    const int col = cwave * CPW + lane % CPW;
+    const int pos = p0 + col / G;
+    const bool col_on = col < ppw * G && pos < qlen;
+    if (__builtin_amdgcn_ballot_w64(col_on) == 0) continue;
+
+    // a range that starts in front of the tile holds it as its last part, the others as their first
+    const int64_t r_first = uniform64(begin / st.per), r_last = uniform64((begin + weight - 1) / st.per);
+    const int64_t piece0 = (int64_t)kvh * 2 * a.split_ranges;
+    auto holds = [&](int64_t r) { // wave-uniform
+        return split_cut(r * st.per - begin, weight, all_tiles, BN) < split_cut((r + 1) * st.per - begin, weight, all_tiles, BN);
+    };
+    auto piece_of = [&](int64_t r) { return piece0 + 2 * r + (r * st.per < begin ? 1 : 0); };
+    int parts = 0;
+    for (int64_t r = r_first; r <= r_last; ++r) parts += holds(r) ? 1 : 0;
+    if (parts <= 1) continue;
+    // U parts at a time, all their loads in flight together; the running maximum rescales what has been added before
+    constexpr int U = 4;
+    float M = kNegBig, den = 0.f;
+    f32x4 o[FW];
+#pragma unroll
+    for (int f = 0; f < FW; ++f) o[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int64_t r = r_first; r <= r_last; r += U) {
+        f32x4 row[U][FW];
+        float2 ml[U];
+        bool on[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            on[u] = r + u <= r_last && holds(r + u);
+            ml[u] = float2{kNegBig, 0.f};
+            if (on[u]) { // wave-uniform
+                const int64_t piece = piece_of(r + u);
+                ml[u] = *(const float2*)(a.split_ml + (piece * COLS + col) * 2);
+                const float* src = a.split_out + (((piece * 8 + cwave) * FRAGS + part * FW) * kWave + lane) * 4;
+#pragma unroll
+                for (int f = 0; f < FW; ++f) row[u][f] = *(const f32x4*)(src + f * (kWave * 4));
+            }
+        }
+        float m_new = M;
+#pragma unroll
+        for (int u = 0; u < U; ++u) m_new = fmaxf(m_new, ml[u].x);
+        const float alpha = __builtin_amdgcn_exp2f(M - m_new);
+        M = m_new;
+        den *= alpha;
+#pragma unroll
+        for (int f = 0; f < FW; ++f) o[f] *= alpha;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (on[u]) {
+                const float w = __builtin_amdgcn_exp2f(ml[u].x - M);
+                den = __builtin_fmaf(ml[u].y, w, den);
+#pragma unroll
+                for (int f = 0; f < FW; ++f) o[f] += row[u][f] * w;
+            }
+    }
+    if (!col_on) continue;
+    const float inv = den > 0.f ? 1.f / den : 0.f;
+    half_t* const out = (half_t*)a.output + (q_row0 + pos) * a.output_stride_s + (int64_t)(kvh * G + col % G) * D + 4 * (lane / CPW);
+#pragma unroll
+    for (int f = 0; f < FW; ++f) {
+        const f32x4 v = o[f] * inv;
+        // fragment i: channels (256 / CPW) i + 4 (lane / CPW) ..
+        *(f16x4*)(out + (part * FW + f) * (256 / CPW)) = f16x4{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+    }
+    }
 }
 
 template <int D, int SRC>
@@ -1067,14 +1360,121 @@ static DeviceMask& prefill_variant_ready()
     return ready;
 }
 
+// the one-time attribute call of a variant covers its split form too: a process that has run either may capture both
+template <int D, int SRC, bool EXTRA>
+static int ready_prefill_variant(hipStream_t stream, bool may_capture)
+{
+    constexpr int lds_bytes = (int)prefill_lds_bytes<D, SRC>();
+    DeviceMask& ready = prefill_variant_ready<D, SRC, EXTRA>();
+    const uint64_t bit = current_device_bit();
+    if (bit != 0 && (ready.load(std::memory_order_acquire) & bit)) return kLaunchOk;
+    DeviceMask none{0}; // (the mask of the variant is set when both attributes are)
+    if (may_capture) {
+        if (int rc = ensure_dynamic_lds((const void*)prefill_attention_kernel<D, SRC, EXTRA, true>, lds_bytes, stream, none)) return rc;
+    } else if (int rc = set_dynamic_lds_once((const void*)prefill_attention_kernel<D, SRC, EXTRA, true>, lds_bytes, none)) {
+        return rc;
+    }
+    return set_dynamic_lds_once((const void*)prefill_attention_kernel<D, SRC, EXTRA, false>, lds_bytes, ready);
+}
 template <int D, int SRC, bool EXTRA>
 static int launch_prefill_variant(const PrefillLaunch& a, dim3 grid, hipStream_t stream)
 {
     constexpr size_t lds_bytes = prefill_lds_bytes<D, SRC>();
-    if (int rc = ensure_dynamic_lds((const void*)prefill_attention_kernel<D, SRC, EXTRA>, (int)lds_bytes, stream,
-                                    prefill_variant_ready<D, SRC, EXTRA>()))
+    if (int rc = ready_prefill_variant<D, SRC, EXTRA>(stream, true)) return rc;
+    if (a.split_ranges > 0)
+        hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, true>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
+    else
+        hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, false>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
+    return kLaunchOk;
+}
+
+template <int D>
+static int launch_prefill_src(const PrefillLaunch& a, dim3 grid, hipStream_t stream)
+{
+    const bool extra = a.attn_mask != nullptr || a.alibi_slopes != nullptr;
+    const int src = a.current_key ? 2 : (a.cache_mode == 1 ? 0 : 1);
+    if (extra) {
+        if (src == 0) return launch_prefill_variant<D, 0, true>(a, grid, stream);
+        if (src == 1) return launch_prefill_variant<D, 1, true>(a, grid, stream);
+        return launch_prefill_variant<D, 2, true>(a, grid, stream);
+    }
+    if (src == 0) return launch_prefill_variant<D, 0, false>(a, grid, stream);
+    if (src == 1) return launch_prefill_variant<D, 1, false>(a, grid, stream);
+    return launch_prefill_variant<D, 2, false>(a, grid, stream);
+}
+
+
+template <int D, int SRC>
+constexpr size_t prefill16_lds_bytes()
+{
+    return 2 * (SRC == 2 ? 1 : 2) * kBN16 * (PrefillTile16<D>::K_STRIDE + PrefillTile16<D>::V_STRIDE) * sizeof(half_t);
+}
+
+template <int D, int SRC, bool EXTRA>
+static DeviceMask& prefill16_variant_ready()
+{
+    static DeviceMask ready{0};
+    return ready;
+}
+
+// the one-time attribute call of a variant covers its split form too: a process that has run either may capture both
+template <int D, int SRC, bool EXTRA>
+static int ready_prefill16_variant(hipStream_t stream, bool may_capture)
+{
+    constexpr int lds_bytes = (int)prefill16_lds_bytes<D, SRC>();
+    DeviceMask& ready = prefill16_variant_ready<D, SRC, EXTRA>();
+    const uint64_t bit = current_device_bit();
+    if (bit != 0 && (ready.load(std::memory_order_acquire) & bit)) return kLaunchOk;
+    DeviceMask none{0}; // (the mask of the variant is set when both attributes are)
+    if (may_capture) {
+        if (int rc = ensure_dynamic_lds((const void*)prefill_attention16_kernel<D, SRC, EXTRA, true>, lds_bytes, stream, none)) return rc;
+    } else if (int rc = set_dynamic_lds_once((const void*)prefill_attention16_kernel<D, SRC, EXTRA, true>, lds_bytes, none)) {
         return rc;
-    hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
+    }
+    return set_dynamic_lds_once((const void*)prefill_attention16_kernel<D, SRC, EXTRA, false>, lds_bytes, ready);
+}
+template <int D, int SRC, bool EXTRA>
+static int launch_prefill16_variant(const PrefillLaunch& a, dim3 grid, hipStream_t stream)
+{
+    constexpr size_t lds_bytes = prefill16_lds_bytes<D, SRC>();
+    if (int rc = ready_prefill16_variant<D, SRC, EXTRA>(stream, true)) return rc;
+    if (a.split_ranges > 0)
+        hipLaunchKernelGGL((prefill_attention16_kernel<D, SRC, EXTRA, true>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
+    else
+        hipLaunchKernelGGL((prefill_attention16_kernel<D, SRC, EXTRA, false>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
+    return kLaunchOk;
+}
+
+template <int D>
+static int launch_prefill16_src(const PrefillLaunch& a, dim3 grid, hipStream_t stream)
+{
+    const bool extra = a.attn_mask != nullptr || a.alibi_slopes != nullptr;
+    const int src = a.current_key ? 2 : (a.cache_mode == 1 ? 0 : 1);
+    if (extra) {
+        if (src == 0) return launch_prefill16_variant<D, 0, true>(a, grid, stream);
+        if (src == 1) return launch_prefill16_variant<D, 1, true>(a, grid, stream);
+        return launch_prefill16_variant<D, 2, true>(a, grid, stream);
+    }
+    if (src == 0) return launch_prefill16_variant<D, 0, false>(a, grid, stream);
+    if (src == 1) return launch_prefill16_variant<D, 1, false>(a, grid, stream);
+    return launch_prefill16_variant<D, 2, false>(a, grid, stream);
+}
+
+// the launch of `items` (tile, kv head) workgroups, or of the ranges of the split stream and their combine
+template <int D, int CPW>
+static int launch_prefill_items(const PrefillLaunch& a, int64_t items, hipStream_t stream)
+{
+    if (a.split_ranges <= 0) {
+        const dim3 grid((unsigned)(items * a.num_kv_heads), 1, 1);
+        if constexpr (CPW == 32) return launch_prefill_src<D>(a, grid, stream);
+        else return launch_prefill16_src<D>(a, grid, stream);
+    }
+    const dim3 grid((unsigned)(a.split_ranges * a.num_kv_heads), 1, 1);
+    int rc;
+    if constexpr (CPW == 32) rc = launch_prefill_src<D>(a, grid, stream);
+    else rc = launch_prefill16_src<D>(a, grid, stream);
+    if (rc != kLaunchOk) return rc;
+    hipLaunchKernelGGL((prefill_combine_kernel<D, CPW>), dim3((unsigned)(items * a.num_kv_heads), 8), dim3(256), 0, stream, a);
     return kLaunchOk;
 }
 
@@ -1090,41 +1490,7 @@ static int launch_prefill_d(const PrefillLaunch& a, hipStream_t stream)
         const int64_t by_rows = a.query_rows / ppw + a.prefill_batches;
         if (by_rows < items) items = by_rows;
     }
-    const dim3 grid((unsigned)(items * a.num_kv_heads), 1, 1);
-    const bool extra = a.attn_mask != nullptr || a.alibi_slopes != nullptr;
-    const int src = a.current_key ? 2 : (a.cache_mode == 1 ? 0 : 1);
-    if (extra) {
-        if (src == 0) return launch_prefill_variant<D, 0, true>(a, grid, stream);
-        if (src == 1) return launch_prefill_variant<D, 1, true>(a, grid, stream);
-        return launch_prefill_variant<D, 2, true>(a, grid, stream);
-    }
-    if (src == 0) return launch_prefill_variant<D, 0, false>(a, grid, stream);
-    if (src == 1) return launch_prefill_variant<D, 1, false>(a, grid, stream);
-    return launch_prefill_variant<D, 2, false>(a, grid, stream);
-}
-
-template <int D, int SRC>
-constexpr size_t prefill16_lds_bytes()
-{
-    return 2 * (SRC == 2 ? 1 : 2) * kBN16 * (PrefillTile16<D>::K_STRIDE + PrefillTile16<D>::V_STRIDE) * sizeof(half_t);
-}
-
-template <int D, int SRC, bool EXTRA>
-static DeviceMask& prefill16_variant_ready()
-{
-    static DeviceMask ready{0};
-    return ready;
-}
-
-template <int D, int SRC, bool EXTRA>
-static int launch_prefill16_variant(const PrefillLaunch& a, dim3 grid, hipStream_t stream)
-{
-    constexpr size_t lds_bytes = prefill16_lds_bytes<D, SRC>();
-    if (int rc = ensure_dynamic_lds((const void*)prefill_attention16_kernel<D, SRC, EXTRA>, (int)lds_bytes, stream,
-                                    prefill16_variant_ready<D, SRC, EXTRA>()))
-        return rc;
-    hipLaunchKernelGGL((prefill_attention16_kernel<D, SRC, EXTRA>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
-    return kLaunchOk;
+    return launch_prefill_items<D, 32>(a, items, stream);
 }
 
 template <int D>
@@ -1139,17 +1505,37 @@ static int launch_prefill16_d(const PrefillLaunch& a, hipStream_t stream)
         if (by_rows < items) items = by_rows;
     }
     if (items * a.num_kv_heads > 0x7fffffff) return kLaunchNoKernel;
-    const dim3 grid((unsigned)(items * a.num_kv_heads), 1, 1);
-    const bool extra = a.attn_mask != nullptr || a.alibi_slopes != nullptr;
-    const int src = a.current_key ? 2 : (a.cache_mode == 1 ? 0 : 1);
-    if (extra) {
-        if (src == 0) return launch_prefill16_variant<D, 0, true>(a, grid, stream);
-        if (src == 1) return launch_prefill16_variant<D, 1, true>(a, grid, stream);
-        return launch_prefill16_variant<D, 2, true>(a, grid, stream);
-    }
-    if (src == 0) return launch_prefill16_variant<D, 0, false>(a, grid, stream);
-    if (src == 1) return launch_prefill16_variant<D, 1, false>(a, grid, stream);
-    return launch_prefill16_variant<D, 2, false>(a, grid, stream);
+    return launch_prefill_items<D, 16>(a, items, stream);
+}
+
+PrefillSplit prefill_split_choose(int64_t sequences, int64_t max_seqlen, int64_t max_kvlen, int64_t rows, int64_t num_heads,
+                                  int64_t num_kv_heads, int64_t head_dim, bool kv16, bool mixed, int compute_units)
+{
+    PrefillSplit r;
+    const int64_t cols = head_dim == 256 ? kCols16 : kCols;
+    if (kv16) max_kvlen = max_seqlen;
+    if (sequences <= 0 || sequences > kWave || max_seqlen <= 0 || max_kvlen <= 0 || num_kv_heads <= 0 || num_heads < num_kv_heads ||
+        compute_units <= 0)
+        return r;
+    const int64_t g = num_heads / num_kv_heads;
+    if (g > cols) return r;
+    const int64_t ppw = cols / g, ranges = compute_units / num_kv_heads;
+    int64_t tiles = sequences * ((max_seqlen + ppw - 1) / ppw);
+    if (rows > 0 && rows / ppw + sequences < tiles) tiles = rows / ppw + sequences;
+    // (with more tiles than workgroups the order of the tiles, the dear ones first, balances the call well enough)
+    // In a step with decode sequences max_kvlen may be theirs, and the kernels may then find walks too short to share:
+    // that costs a launch (5 us), which half of the chip idle has to be worth.
+    if (ranges < 2 || tiles > (mixed && !kv16 ? ranges / 2 : ranges)) return r;
+    const int64_t prior = max_kvlen > max_seqlen ? max_kvlen - max_seqlen : 0;
+    const int64_t longest = kSplitStart + max_kvlen, mean = kSplitStart + prior + (max_kvlen - prior) / 2;
+    int64_t per = tiles * mean / ranges;
+    if (per < kPrefillSplitMinTokens) per = kPrefillSplitMinTokens;
+    r.gain = kv16 ? kPrefillSplitGain16 : kPrefillSplitGain;
+    if (longest - per < r.gain) return r;
+    r.ranges = (int32_t)ranges;
+    r.out_bytes = num_kv_heads * 2 * ranges * cols * head_dim * (int64_t)sizeof(float);
+    r.bytes = r.out_bytes + num_kv_heads * 2 * ranges * cols * 2 * (int64_t)sizeof(float);
+    return r;
 }
 
 int launch_prefill(const PrefillLaunch& a, hipStream_t stream)
@@ -1166,8 +1552,7 @@ int launch_prefill(const PrefillLaunch& a, hipStream_t stream)
 template <int D, int SRC, bool EXTRA>
 static int init_prefill_variant()
 {
-    return set_dynamic_lds_once((const void*)prefill_attention_kernel<D, SRC, EXTRA>, (int)prefill_lds_bytes<D, SRC>(),
-                                prefill_variant_ready<D, SRC, EXTRA>());
+    return ready_prefill_variant<D, SRC, EXTRA>(nullptr, false);
 }
 template <int D>
 static int init_prefill_d()
@@ -1182,8 +1567,7 @@ static int init_prefill_d()
 template <int D, int SRC, bool EXTRA>
 static int init_prefill16_variant()
 {
-    return set_dynamic_lds_once((const void*)prefill_attention16_kernel<D, SRC, EXTRA>, (int)prefill16_lds_bytes<D, SRC>(),
-                                prefill16_variant_ready<D, SRC, EXTRA>());
+    return ready_prefill16_variant<D, SRC, EXTRA>(nullptr, false);
 }
 template <int D>
 static int init_prefill16_d()

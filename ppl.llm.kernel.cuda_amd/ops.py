@@ -173,7 +173,8 @@ def prefill_attention(query, output, cache, scale, seqstarts, kvstarts, cachesta
     """Multi-query-token attention of the prefill sequences.  Optional: additive half `attn_mask` with its
     strides, float32 `alibi_slopes` [Hq], `current_key`/`current_value` [rows, KVH, D] to attend over
     the step's own fp16 rows instead of the cache, and a `workspace` of prefill_workspace_size() bytes with which a
-    batch of short chunks runs on the decode step's kernel."""
+    batch of short chunks runs on the decode step's kernel, or of prefill_split_workspace_size() bytes with which a batch
+    of few query tiles is split over its kv tokens."""
     p = PrefillParams()
     p.query = _ptr(query)
     p.output = _ptr(output)
@@ -226,6 +227,14 @@ def prefill_workspace_size(batch, decoding_batches, max_seqlen, max_kvlen, num_h
     other batch (cus = 0: the compute units of the current device)."""
     return int(_lib.lib().pmxhip_prefill_workspace_size(batch, decoding_batches, max_seqlen, max_kvlen, num_heads,
                                                         num_kv_heads, head_dim, cus))
+
+
+def prefill_split_workspace_size(batch, decoding_batches, max_seqlen, max_kvlen, query_rows, num_heads, num_kv_heads, head_dim,
+                                 from_current=False, cus=0):
+    """Bytes of the workspace with which a batch of few query tiles shares their kv tokens out over the chip; 0 for every
+    other batch."""
+    return int(_lib.lib().pmxhip_prefill_split_workspace_size(batch, decoding_batches, max_seqlen, max_kvlen, query_rows, num_heads,
+                                                              num_kv_heads, head_dim, 1 if from_current else 0, cus))
 
 
 def _rope_params(query, key, start_pos, seqstarts, rotated_query, rotated_key, *, theta, rotary_dim, batch, max_seqlen,

@@ -305,3 +305,68 @@ def test_prefill_output_rows_aligned_to_8_bytes_only(pkg, oracle):
         dev.output = keep
     np.testing.assert_array_equal(got8, got)
     assert torch.isnan(buf[:4]).all() and torch.isnan(buf[4 + n:]).all()
+
+
+@pytest.mark.parametrize("shape,q_lens,prior", [
+    ((32, 8, 128), [65, 300, 17, 129], [700, 0, 2000, 130]),  # a tile is a block of kv tokens long: 64 positions
+    ((8, 8, 128), [257, 1, 64], [1500, 900, 3000]),           # one query head per kv head: 256 positions per tile
+    ((5, 5, 128), [600], [1111]),                             # kv heads that do not divide the compute units
+    ((48, 1, 128), [33, 500, 2], [640, 0, 1200]),             # five positions per tile, a single kv head: the most ranges
+    ((8, 2, 64), [200, 90, 33], [0, 1000, 2500]),
+    ((12, 4, 96), [129, 64, 300], [1000, 63, 0]),
+    ((16, 8, 256), [100, 33, 17], [900, 0, 1500]),            # the 16-column kernel
+    ((8, 1, 256), [70, 300], [2000, 0]),
+])
+@pytest.mark.parametrize("form", ["paged", "contiguous", "not_causal", "alibi_mask"])
+def test_prefill_tiles_split_over_their_kv_tokens(pkg, oracle, shape, q_lens, prior, form):
+    """With the workspace of prefill_split_workspace_size() the kv tokens of a few query tiles are shared out over the chip:
+    same results as the oracle and as whole tiles, also where the hints understate the batch."""
+    hq, hkv, d = shape
+    bt, dev, q, cache, scale = make_case(pkg, oracle, 410 + hq + d, num_heads=hq, num_kv_heads=hkv, head_dim=d,
+                                         cache_mode=0 if form == "contiguous" else 1, dec_kv_lens=[33],
+                                         prefill_q_lens=q_lens, prefill_prior=prior, outliers=True)
+    bt.is_causal = form != "not_causal"
+    extra = {}
+    if form == "alibi_mask":
+        mask, ms, mh = make_prefill_mask(bt, np.random.default_rng(12), False)
+        slopes = (2.0 ** (-8.0 * np.arange(1, hq + 1) / hq)).astype(np.float32)
+        ref = oracle_prefill_ex(oracle, bt, q, cache, scale, attn_mask=mask, mask_stride_s=ms, mask_stride_h=mh, alibi_slopes=slopes)
+        extra = dict(attn_mask=torch.from_numpy(mask).cuda(), mask_stride_s=ms, mask_stride_h=mh,
+                     alibi_slopes=torch.from_numpy(slopes).cuda())
+    else:
+        ref = oracle_prefill(oracle, bt, q, cache, scale)
+    rows = sum(q_lens)
+    ws_bytes = pkg.ops.prefill_split_workspace_size(bt.batch, 1, bt.max_seqlen, bt.max_kvlen, rows, hq, hkv, d)
+    assert ws_bytes > 0
+    ws = torch.full((ws_bytes // 4,), float("nan"), dtype=torch.float32, device="cuda")
+    whole = run_prefill(pkg, dev, **extra)
+    got = run_prefill(pkg, dev, workspace=ws, **extra)
+    assert not torch.isnan(ws).all()  # parts were written
+    assert np.isnan(got[:1]).all()
+    assert_attention_close(got[1:], ref[1:], "split %s %s" % (shape, form))
+    # The two differ by the order of float32 sums: three units in the last place of a half, at the row's largest value
+    assert np.abs(got[1:] - whole[1:]).max() <= 3 * 2.0 ** -11 * np.abs(whole[1:]).max()
+    hinted = run_prefill(pkg, dev, workspace=ws, prefill_query_rows=1, **extra)  # understates the batch: only time
+    np.testing.assert_array_equal(hinted, got)
+
+
+@pytest.mark.parametrize("shape", [(32, 8, 128), (8, 2, 64), (8, 4, 96), (8, 2, 256)])
+def test_prefill_tiles_split_from_current_key_value(pkg, oracle, shape):
+    """The split form over the step's own half K/V rows, through the operator class, whose workspace holds the decode
+    stage's pieces and, behind them, the parts of the query tiles."""
+    hq, hkv, d = shape
+    bt, rng = pkg.workloads.custom_batch(820 + d, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=0,
+                                         dec_kv_lens=[5, 900], prefill_q_lens=[1000, 90], prefill_prior=[0, 0], outliers=True)
+    dev = pkg.harness.DeviceBatch(bt)
+    q, k, v = pkg.workloads.step_inputs(bt, rng)
+    dev.set_step_inputs(q, k, v)
+    cache, scale = host_cache(bt)
+    ref = oracle_prefill_ex(oracle, bt, q, cache, scale, current_key=k, current_value=v)
+    assert pkg.ops.prefill_split_workspace_size(bt.batch, 2, bt.max_seqlen, bt.max_kvlen, 1090, hq, hkv, d, True) > 0
+    op = dev.make_operator(enable_cache_prefill=False)
+    op.workspace.view(torch.float32)[:].fill_(float("nan"))
+    dev.output.fill_(float("nan"))
+    assert op.forward_prefill() == 0
+    torch.cuda.synchronize()
+    assert not torch.isnan(op.workspace.view(torch.float32)).all()
+    assert_attention_close(dev.output.float().cpu().numpy()[2:], ref[2:], "split, half K/V %s" % (shape,))
