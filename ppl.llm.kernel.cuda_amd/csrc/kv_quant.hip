@@ -220,64 +220,64 @@ __global__ __launch_bounds__(kQuantThreads) void rope_append_kernel(const RopeLa
     const int tokens_per_wg = a.tokens_per_wg; // at most kQuantThreads / pairs; pairs <= 128
     const int64_t first = a.seqstarts[0];
     const int64_t n_tokens = a.seqstarts[a.batch] - first;
-    const int64_t tok0 = (int64_t)blockIdx.x * tokens_per_wg;
-    if (tok0 >= n_tokens) return;
     const bool append = a.cache != nullptr;
+    for (int64_t tok0 = (int64_t)blockIdx.x * tokens_per_wg; tok0 < n_tokens; tok0 += (int64_t)gridDim.x * tokens_per_wg) {
+    int thread = threadIdx.x;
+    asm volatile("" : "+v"(thread));
 
-    // the rows of this workgroup's tokens, as units of 8 channels: the query heads' groups, then the key heads' (a
-    // key unit also carries the same group of V when the step appends)
+    // the rows of this workgroup's tokens, as units of 8 channels: the query heads' groups, and the key heads' (a key unit
+    // also carries the same group of V when the step appends)
     const int gph = a.head_dim >> 3; // groups of 8 channels per head
     const int q_units = (int)a.num_heads * gph;
     const int k_units = (int)a.num_key_heads * gph;
-    const int units = q_units + k_units;
     int n_here = tokens_per_wg;
     if (tok0 + n_here > n_tokens) n_here = (int)(n_tokens - tok0);
-    const int work = n_here * units;
+    const int q_work = n_here * q_units, k_work = n_here * k_units;
+    const half_t* const value = (const half_t*)(append ? a.value : a.key); // (read for nothing where nothing is appended)
+    const int64_t value_stride = append ? a.value_stride_s : a.key_stride_s;
 
     struct Unit {
         int tl, h, d0;
-        bool is_query;
         int64_t in_tok, idx;
     };
-    auto unit_of = [&](int w) -> Unit {
+    // (the quotient by a multiplication where the launcher found it exact for every unit of a workgroup)
+    auto unit_of = [&](int w, int per_token, uint32_t magic) -> Unit {
         Unit r;
-        r.tl = w / units;
-        int u = w - r.tl * units;
-        r.is_query = u < q_units;
-        if (!r.is_query) u -= q_units;
-        r.h = u / gph;
+        r.tl = magic ? (int)__umulhi((uint32_t)w, magic) : w / per_token;
+        const int u = w - r.tl * per_token;
+        r.h = magic ? (int)__umulhi((uint32_t)u, a.gph_magic) : u / gph;
         r.d0 = (u - r.h * gph) << 3;
         r.in_tok = first + tok0 + r.tl;
-        r.idx = (int64_t)r.h * a.head_dim + r.d0;
+        r.idx = (int64_t)u << 3;
         return r;
     };
-    auto load_row = [&](const Unit& r) -> u32x4 {
-        return r.is_query ? *(const u32x4*)((const half_t*)a.query + r.in_tok * a.query_stride_s + r.idx)
-                          : *(const u32x4*)((const half_t*)a.key + r.in_tok * a.key_stride_s + r.idx);
+    // Units beyond the work load the last unit's rows: every load of a batch is issued whatever the remainder, so that
+    // the wait for a batch leaves the next one in flight.
+    constexpr int kQueries = 3; // query units per thread and batch; key units one
+    auto load_queries = [&](int w0, u32x4 (&rows)[kQueries]) {
+#pragma unroll
+        for (int j = 0; j < kQueries; ++j) {
+            const int w = w0 + (int)thread + j * kQuantThreads;
+            const Unit r = unit_of(w < q_work ? w : q_work - 1, q_units, a.q_magic);
+            rows[j] = *(const u32x4*)((const half_t*)a.query + r.in_tok * a.query_stride_s + r.idx);
+        }
     };
-    auto load_value = [&](const Unit& r) -> u32x4 {
-        return *(const u32x4*)((const half_t*)a.value + r.in_tok * a.value_stride_s + r.idx);
+    auto load_key = [&](int w0, u32x4& k, u32x4& v) {
+        const int w = w0 + (int)thread;
+        const Unit r = unit_of(w < k_work ? w : k_work - 1, k_units, a.k_magic);
+        k = *(const u32x4*)((const half_t*)a.key + r.in_tok * a.key_stride_s + r.idx);
+        v = *(const u32x4*)(value + r.in_tok * value_stride + r.idx);
     };
 
     // The rows depend on nothing that follows (index arrays -> sequence -> cos/sin and cache row), so a thread's
     // first units are requested before all that and travel meanwhile; a decode step, with a token per workgroup
     // and a few units per thread, has no others.
-    constexpr int kEarly = 3;
-    u32x4 early_row[kEarly], early_value[kEarly];
-#pragma unroll
-    for (int j = 0; j < kEarly; ++j) {
-        const int w = threadIdx.x + j * kQuantThreads;
-        early_row[j] = u32x4{0, 0, 0, 0};
-        early_value[j] = u32x4{0, 0, 0, 0};
-        if (w < work) {
-            const Unit r = unit_of(w);
-            early_row[j] = load_row(r);
-            if (append && !r.is_query) early_value[j] = load_value(r);
-        }
-    }
+    u32x4 q_row[kQueries], k_row = {0, 0, 0, 0}, v_row = {0, 0, 0, 0};
+    if (k_units > 0) load_key(0, k_row, v_row);
+    load_queries(0, q_row);
 
     {
-        const int tl = threadIdx.x / pairs, i = threadIdx.x - tl * pairs;
+        const int tl = thread / pairs, i = thread - tl * pairs;
         const int64_t tok = tok0 + tl;
         const bool active = tl < tokens_per_wg && tok < n_tokens;
         const int64_t in_tok = first + tok;
@@ -297,13 +297,13 @@ __global__ __launch_bounds__(kQuantThreads) void rope_append_kernel(const RopeLa
             }
         }
         if (count_search) { // every lane of the wave is here
-            const int wave0 = threadIdx.x & ~(kWave - 1);
+            const int wave0 = thread & ~(kWave - 1);
             const int tl_hi = (wave0 + kWave - 1) / pairs;
             for (int t = wave0 / pairs; t <= tl_hi; ++t) {
                 const int64_t tk = tok0 + t;
                 if (t >= tokens_per_wg || tk >= n_tokens) break;
                 if (__builtin_amdgcn_ballot_w64(tl == t && b < 0) == 0) continue;
-                const int bt = sequence_by_count(a.seqstarts, (int)a.batch, first + tk, threadIdx.x & (kWave - 1));
+                const int bt = sequence_by_count(a.seqstarts, (int)a.batch, first + tk, thread & (kWave - 1));
                 if (tl == t && b < 0) {
                     b = bt;
                     pos = a.start_pos[bt] + (first + tk - a.seqstarts[bt]);
@@ -335,8 +335,8 @@ __global__ __launch_bounds__(kQuantThreads) void rope_append_kernel(const RopeLa
                 c = (float)cd;
                 s = (float)sd;
             }
-            s_cos[threadIdx.x] = c;
-            s_sin[threadIdx.x] = s;
+            s_cos[thread] = c;
+            s_sin[thread] = s;
             if (i == 0 && append)
                 s_row[tl] = token_row<PAGED>(a.cachestarts, PAGED ? (int64_t)b * a.cachestarts_stride_b : (int64_t)b, pos);
         }
@@ -360,11 +360,12 @@ __global__ __launch_bounds__(kQuantThreads) void rope_append_kernel(const RopeLa
         return out;
     };
 
-    auto finish = [&](const Unit& r, u32x4 raw, const u32x4 vraw) {
-        if (r.is_query) {
-            *(u32x4*)((half_t*)a.rotated_query + r.in_tok * a.rotated_query_stride_s + r.idx) = rotate(raw, r.d0, r.tl);
-            return;
-        }
+    auto finish_query = [&](int w, const u32x4 raw) {
+        const Unit r = unit_of(w, q_units, a.q_magic);
+        *(u32x4*)((half_t*)a.rotated_query + r.in_tok * a.rotated_query_stride_s + r.idx) = rotate(raw, r.d0, r.tl);
+    };
+    auto finish_key = [&](int w, u32x4 raw, const u32x4 vraw) {
+        const Unit r = unit_of(w, k_units, a.k_magic);
         if (!a.bypass_key) raw = rotate(raw, r.d0, r.tl);
         if (a.rotated_key) *(u32x4*)((half_t*)a.rotated_key + r.in_tok * a.rotated_key_stride_s + r.idx) = raw;
         if (append) {
@@ -378,18 +379,31 @@ __global__ __launch_bounds__(kQuantThreads) void rope_append_kernel(const RopeLa
             __builtin_nontemporal_store(vq.scale, &((half_t*)a.scale)[v_out >> 3]);
         }
     };
-
-#pragma unroll
-    for (int j = 0; j < kEarly; ++j) {
-        const int w = threadIdx.x + j * kQuantThreads;
-        if (w < work) finish(unit_of(w), early_row[j], early_value[j]);
+    // The next units travel while these are rotated and stored: one after the other, each waiting for its own rows, a
+    // workgroup of four tokens of 32 query / 8 kv heads of 128 spent seven memory latencies in a row.
+    int w0 = 0;
+    for (; w0 + kQuantThreads <= k_work; w0 += kQuantThreads) {
+        u32x4 k_next, v_next;
+        load_key(w0 + kQuantThreads, k_next, v_next);
+        finish_key(w0 + (int)thread, k_row, v_row);
+        k_row = k_next;
+        v_row = v_next;
     }
-    for (int w = threadIdx.x + kEarly * kQuantThreads; w < work; w += kQuantThreads) {
-        const Unit r = unit_of(w);
-        const u32x4 raw = load_row(r);
-        u32x4 vraw = {0, 0, 0, 0};
-        if (append && !r.is_query) vraw = load_value(r);
-        finish(r, raw, vraw);
+    if (w0 + (int)thread < k_work) finish_key(w0 + (int)thread, k_row, v_row);
+    for (w0 = 0; w0 + kQueries * kQuantThreads <= q_work; w0 += kQueries * kQuantThreads) {
+        u32x4 next[kQueries];
+        load_queries(w0 + kQueries * kQuantThreads, next);
+#pragma unroll
+        for (int j = 0; j < kQueries; ++j) finish_query(w0 + (int)thread + j * kQuantThreads, q_row[j]);
+#pragma unroll
+        for (int j = 0; j < kQueries; ++j) q_row[j] = next[j];
+    }
+#pragma unroll
+    for (int j = 0; j < kQueries; ++j) {
+        const int w = w0 + (int)thread + j * kQuantThreads;
+        if (w < q_work) finish_query(w, q_row[j]);
+    }
+    __syncthreads(); // the next tokens' coefficients overwrite these
     }
 }
 
@@ -411,9 +425,22 @@ int launch_rope(const RopeLaunch& a_in, int compute_units, hipStream_t stream)
     const int64_t spread = a.max_tokens / (2 * (int64_t)(compute_units > 0 ? compute_units : 256));
     if (tokens_per_wg > spread) tokens_per_wg = spread > 1 ? (int)spread : 1;
     a.tokens_per_wg = tokens_per_wg;
-    const unsigned blocks = (unsigned)((a.max_tokens + tokens_per_wg - 1) / tokens_per_wg);
-    if (a.cache_mode == 1) hipLaunchKernelGGL(rope_append_kernel<true>, dim3(blocks), dim3(kQuantThreads), 0, stream, a);
-    else hipLaunchKernelGGL(rope_append_kernel<false>, dim3(blocks), dim3(kQuantThreads), 0, stream, a);
+    // n / d = mulhi(n, floor(2^32 / d) + 1) for n d < 2^32 and d >= 2
+    const uint64_t gph = (uint64_t)(a.head_dim >> 3);
+    auto magic = [&](uint64_t per_token) -> uint32_t {
+        const bool exact = gph >= 2 && per_token > 0 && per_token < (1u << 16) && (uint64_t)tokens_per_wg * per_token * per_token < (1ull << 32);
+        return exact ? (uint32_t)((1ull << 32) / per_token + 1) : 0;
+    };
+    a.q_magic = magic((uint64_t)a.num_heads * gph);
+    a.k_magic = magic((uint64_t)a.num_key_heads * gph);
+    a.gph_magic = gph >= 2 ? (uint32_t)((1ull << 32) / gph + 1) : 0;
+    // max_tokens is batch * max_seqlen, in a mixed step many times the rows there are: as many workgroups as the chip holds at
+    // once, which walk the tokens in turn
+    int64_t blocks = (a.max_tokens + tokens_per_wg - 1) / tokens_per_wg;
+    const int64_t resident = 8 * (int64_t)(compute_units > 0 ? compute_units : 256);
+    if (blocks > resident) blocks = resident;
+    if (a.cache_mode == 1) hipLaunchKernelGGL(rope_append_kernel<true>, dim3((unsigned)blocks), dim3(kQuantThreads), 0, stream, a);
+    else hipLaunchKernelGGL(rope_append_kernel<false>, dim3((unsigned)blocks), dim3(kQuantThreads), 0, stream, a);
     return kLaunchOk;
 }
 

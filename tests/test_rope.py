@@ -150,3 +150,29 @@ def test_gpu_rope_many_sequences(pkg, oracle, shape, n_dec, n_prefill):
     np.testing.assert_array_equal(d_rk.cpu().numpy().view(np.uint16), rk_ref.view(np.uint16))
     np.testing.assert_array_equal(dev.cache.cpu().numpy(), cache_ref)
     np.testing.assert_array_equal(dev.scale.cpu().numpy().view(np.uint16), scale_ref.view(np.uint16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(71, 1, 64), (48, 1, 128), (3, 3, 96), (16, 8, 256), (5, 2, 8)])
+def test_gpu_rope_several_tokens_per_workgroup(pkg, oracle, shape):
+    """Steps whose workgroups take several tokens, and several such groups in turn, with units that fill no whole number of
+    batches: in place and with the append, bit for bit against the oracle."""
+    import torch
+    hq, hk, d = shape
+    bt, rng = pkg.workloads.custom_batch(91 + d, num_heads=hq, num_kv_heads=hk, head_dim=d, cache_mode=1, dec_kv_lens=[7, 300],
+                                         prefill_q_lens=[4100, 3, 2700], prefill_prior=[0, 129, 1000])
+    dev = pkg.harness.DeviceBatch(bt)
+    q, k, v = pkg.workloads.step_inputs(bt, rng)
+    dev.set_step_inputs(q, k, v)
+    kw = dict(theta=10000.0, rotary_dim=d, batch=bt.batch, max_seqlen=bt.max_seqlen)
+    rq_ref, rk_ref = oracle.rotary_position_embedding(q, k, bt.start_pos, bt.seqstarts, 10000.0, d)
+    cache_ref, scale_ref = host_cache(bt)
+    oracle.kv_cache_quantize(rk_ref, v, bt.seqstarts, bt.cachestarts, bt.start_pos, bt.layer_idx, bt.num_kv_heads,
+                             bt.head_dim, bt.page_size, cache=cache_ref, scale=scale_ref, **oracle_layout_kwargs(bt))
+    pkg.ops.rope_key_value_cache(dev.query, dev.new_key, dev.new_value, dev.start_pos, dev.seqstarts, dev.cachestarts,
+                                 dev.query, None, dev.cache, dev.scale, num_layer=bt.num_layer, layer_idx=bt.layer_idx,
+                                 **dev.layout_kwargs(), **kw)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(dev.query.cpu().numpy().view(np.uint16), rq_ref.view(np.uint16))
+    np.testing.assert_array_equal(dev.cache.cpu().numpy(), cache_ref)
+    np.testing.assert_array_equal(dev.scale.cpu().numpy().view(np.uint16), scale_ref.view(np.uint16))
