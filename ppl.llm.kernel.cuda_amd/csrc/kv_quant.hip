@@ -18,6 +18,7 @@
 // token is found by bisection over seqstarts, so no workgroup is launched per
 // (position, sequence) pair that does not exist.
 #include <cmath>
+#include <cstring>
 
 #include "device_common.h"
 #include "launch_params.h"
@@ -407,6 +408,13 @@ __global__ __launch_bounds__(kQuantThreads) void rope_append_kernel(const RopeLa
     }
 }
 
+static uint32_t bitcast_host(float v)
+{
+    uint32_t u;
+    memcpy(&u, &v, sizeof(u));
+    return u;
+}
+
 int launch_rope(const RopeLaunch& a_in, int compute_units, hipStream_t stream)
 {
     if (a_in.max_tokens <= 0) return kLaunchOk;
@@ -415,7 +423,14 @@ int launch_rope(const RopeLaunch& a_in, int compute_units, hipStream_t stream)
     const int pairs = a.head_dim / 2, rd2 = a.rotary_dim / 2;
     a.has_inv_freq = 0;
     if (a.scaling_type != 2 && rd2 <= 128) {
-        for (int i = 0; i < rd2; ++i) a.inv_freq[i] = 1.0f / (float)pow((double)a.theta, (double)((float)i / (float)rd2));
+        // a model has one such table: the thread's last one is kept (64 powers cost as much as the launch)
+        static thread_local struct { float theta; int rd2; float table[128]; } last = {0.f, -1, {}};
+        if (last.rd2 != rd2 || bitcast_host(last.theta) != bitcast_host(a.theta)) {
+            for (int i = 0; i < rd2; ++i) last.table[i] = 1.0f / (float)pow((double)a.theta, (double)((float)i / (float)rd2));
+            last.theta = a.theta;
+            last.rd2 = rd2;
+        }
+        memcpy(a.inv_freq, last.table, sizeof(float) * rd2);
         a.has_inv_freq = 1;
     }
     // A workgroup computes the coefficients of its tokens once and shares them through LDS: as many tokens as its

@@ -41,9 +41,9 @@ def _ptr(t):
 
 
 def _stream(stream=None):
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    if stream is None: # torch.cuda.current_stream() without the Stream object around the handle (a microsecond per call)
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    return stream.cuda_stream
 
 
 def compute_units(device=None):
@@ -239,19 +239,12 @@ def prefill_split_workspace_size(batch, decoding_batches, max_seqlen, max_kvlen,
 
 def _rope_params(query, key, start_pos, seqstarts, rotated_query, rotated_key, *, theta, rotary_dim, batch, max_seqlen,
                  bypass_key=False, max_position_embeddings=2048, scaling_type=0, scaling_factor=1.0):
-    p = _lib.RopeParams()
-    hq, d = int(query.shape[1]), int(query.shape[2])
-    hk = int(key.shape[1])
-    p.query, p.key = _ptr(query), _ptr(key)
-    p.start_pos, p.seqstarts = _ptr(start_pos), _ptr(seqstarts)
-    p.theta, p.bypass_key, p.rotary_dim, p.batch = theta, 1 if bypass_key else 0, rotary_dim, batch
-    p.num_heads, p.num_key_heads, p.head_dim, p.max_seqlen = hq, hk, d, max_seqlen
-    p.max_position_embeddings, p.scaling_type, p.scaling_factor = max_position_embeddings, scaling_type, scaling_factor
-    p.query_stride_s = p.rotated_query_stride_s = hq * d
-    p.key_stride_s = p.rotated_key_stride_s = hk * d
-    p.rotated_query = _ptr(rotated_query)
-    p.rotated_key = _ptr(rotated_key) if rotated_key is not None else None
-    return p
+    _, hq, d = query.shape
+    hk = key.shape[1]
+    # in the order of the structure's fields (one call: field by field costs as much as the launch)
+    return _lib.RopeParams(_ptr(query), _ptr(key), _ptr(start_pos), _ptr(seqstarts), theta, 1 if bypass_key else 0, rotary_dim,
+                           batch, hq, hk, d, max_seqlen, max_position_embeddings, scaling_type, scaling_factor,
+                           hq * d, hk * d, hq * d, hk * d, _ptr(rotated_query), _ptr(rotated_key))
 
 
 def rotary_position_embedding(query, key, start_pos, seqstarts, rotated_query, rotated_key, *, stream=None, check=True, **kw):
@@ -269,16 +262,10 @@ def rope_key_value_cache(query, key, value, start_pos, seqstarts, cachestarts, r
     """The rotation and, in the same kernel, the quantise/append of the rotated key and of `value`;
     `rotated_key` may be None."""
     p = _rope_params(query, key, start_pos, seqstarts, rotated_query, rotated_key, **kw)
-    st = KvstoreParams()
-    st.current_key, st.current_value = _ptr(key), _ptr(value)
-    st.seqstarts, st.cachestarts, st.start_pos = _ptr(seqstarts), _ptr(cachestarts), _ptr(start_pos)
-    st.num_layer, st.layer_idx = num_layer, layer_idx
-    st.num_kv_heads, st.head_dim, st.page_size = p.num_key_heads, p.head_dim, page_size
-    st.current_key_stride_s = st.current_value_stride_s = p.key_stride_s
-    st.cache_stride_s, st.cache_stride_l, st.cache_stride_h = cache_stride_s, cache_stride_l, cache_stride_h
-    st.cache_stride_kv, st.cachestarts_stride_b = cache_stride_kv, cachestarts_stride_b
-    st.cache, st.scale = _ptr(cache), _ptr(scale)
-    st.batch, st.max_seqlen, st.cache_mode = p.batch, p.max_seqlen, cache_mode
+    # in the order of the structure's fields
+    st = KvstoreParams(p.key, _ptr(value), p.seqstarts, _ptr(cachestarts), p.start_pos, num_layer, layer_idx, p.num_key_heads,
+                       p.head_dim, page_size, p.key_stride_s, p.key_stride_s, cache_stride_s, cache_stride_l, cache_stride_h,
+                       cache_stride_kv, cachestarts_stride_b, _ptr(cache), _ptr(scale), p.batch, p.max_seqlen, cache_mode)
     rc = _lib.lib().pmxhip_rope_kv_cache_quantize(ctypes.byref(p), ctypes.byref(st), _stream(stream))
     if check and rc != RC_SUCCESS:
         raise PmxError(rc, "rope_kv_cache_quantize")
@@ -330,7 +317,7 @@ def row_parallel_linear(input, weight, bias, output, *, workspace=None, stream=N
     last dimension (row strides may exceed the row).  The single-rank case of the reference's row_parallel_linear.
     `workspace`: a uint8 tensor of row_parallel_linear_workspace_size bytes, or None (slower at decode sizes).
     `vendor_gemm`: from 384 rows on, hand the GEMM to hipBLASLt where it loads (off: this library's kernels)."""
-    n, k = int(weight.shape[0]), int(weight.shape[1])
+    n, k = weight.shape
     m = input.numel() // k  # a contiguous (B, Hq, D) attention output is the (B, Hq * D) input in place
 
     def row_stride(t, width):
