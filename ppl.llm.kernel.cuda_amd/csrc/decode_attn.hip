@@ -492,6 +492,8 @@ __global__ __launch_bounds__(64 * NW) void decode_combine_kernel(const DecodeLau
     constexpr int PPW = 64 / LPR; // piece rows per wave and request (D = 96: two, the last 16 lanes idle)
     constexpr int SLOTS = NW * PPW;
     constexpr int U = 4;
+    constexpr int kPairBlocks = 8; // blocks of 64 ranges whose (max, sum) pairs the lanes hold together
+    static_assert(64 % SLOTS == 0, "a batch step within a block of 64 ranges");
     __shared__ float s_part[SLOTS][D];
     const int b = blockIdx.y;
     const int h = blockIdx.x;
@@ -584,6 +586,72 @@ __global__ __launch_bounds__(64 * NW) void decode_combine_kernel(const DecodeLau
             for (int u = 0; u < U; ++u) {
                 const float wk = __shfl(wt, src[u] < 0 ? 0 : src[u]);
                 if (src[u] >= 0 && wk != 0.f) o += row[u] * wk;
+            }
+        }
+    } else if (NW == 8 && w1 - w0 < 64 * kPairBlocks) {
+        // (eight waves only: the other forms' registers would limit how many of their rows a CU holds)
+        // Up to 512 ranges, kPairBlocks per lane: every (max, sum) pair of the row is requested at once, together with the
+        // first rows, and the rows follow in batches of up to eight per lane.  Block by block, each with its pairs in
+        // front of its rows, a row of 340 pieces waited for memory 18 times.
+        const int n = (int)(w1 - w0) + 1;
+        constexpr int PB = 128 / SLOTS < 8 ? 128 / SLOTS : 8; // rows per slot and batch; 128 ranges are 1 / PB batches
+        auto load_rows = [&](int k0, f32x4 (&row)[PB]) {
+#pragma unroll
+            for (int u = 0; u < PB; ++u) {
+                const int k = k0 + u * SLOTS + slot;
+                row[u] = *(const f32x4*)(a.partial_out + ((w0 + (k < n && sub < PPW ? k : n - 1) + b) * a.num_heads + h) * D + c4 * 4);
+            }
+        };
+        f32x4 row[PB];
+        load_rows(0, row);
+        float m[kPairBlocks], l[kPairBlocks];
+        bool live[kPairBlocks];
+#pragma unroll
+        for (int r = 0; r < kPairBlocks; ++r) {
+            m[r] = kNegBig;
+            l[r] = 0.f;
+            live[r] = false;
+            if (64 * r + lane < n) {
+                const int64_t w = w0 + 64 * r + lane;
+                int64_t pa, pe;
+                const int64_t r0 = w * per;
+                piece_bounds(r0, (r0 + per < total) ? r0 + per : total, s_beg, s_end - s_beg, a.wg_tokens, pa, pe);
+                live[r] = pe > pa;
+                if (live[r]) {
+                    const float2 ml = *(const float2*)(a.partial_ml + ((w + b) * a.num_heads + h) * 2);
+                    m[r] = ml.x;
+                    l[r] = ml.y;
+                }
+            }
+        }
+        int pieces = 0;
+        float M = kNegBig;
+#pragma unroll
+        for (int r = 0; r < kPairBlocks; ++r) {
+            pieces += __builtin_popcountll(__builtin_amdgcn_ballot_w64(live[r]));
+            M = fmaxf(M, m[r]);
+        }
+        if (pieces <= 1) return; // the cuts moved onto one boundary: the decode kernel wrote the final output
+#pragma unroll
+        for (int s = 32; s >= 1; s >>= 1) M = fmaxf(M, __shfl_xor(M, s));
+        float wt[kPairBlocks];
+#pragma unroll
+        for (int r = 0; r < kPairBlocks; ++r) {
+            wt[r] = live[r] ? l[r] * __builtin_amdgcn_exp2f(m[r] - M) : 0.f; // an empty piece's row may be stale: weight zero
+            den += wt[r];
+        }
+#pragma unroll
+        for (int r = 0; r < kPairBlocks; r += 2) {
+            if (64 * r >= n) break;
+            for (int k0 = 64 * r; k0 < 64 * r + 128 && k0 < n; k0 += PB * SLOTS) {
+                if (k0 > 0) load_rows(k0, row);
+#pragma unroll
+                for (int u = 0; u < PB; ++u) {
+                    const int kb = k0 + u * SLOTS; // (SLOTS divides 64: a batch step lies in one block of 64 ranges)
+                    const int k = kb + slot;
+                    const float wk = __shfl((kb & 64) != 0 ? wt[r + 1] : wt[r], k & 63);
+                    if (k < n && sub < PPW && wk != 0.f) o += row[u] * wk;
+                }
             }
         }
     } else {
@@ -749,11 +817,13 @@ static int launch_decode_d(const DecodeLaunch& a, int stage, hipStream_t stream)
     {
         // waves per (sequence, head) row by the mean number of pieces per sequence: with many rows of a few
         // pieces each, extra waves only add dispatch work (measured: 8 / 9 / 13 us for 1 / 2 / 4 waves on 128
-        // sequences of about five pieces, 17 / 12 / 9 us on one sequence of 256 pieces)
+        // sequences of about five pieces, 17 / 12 / 9 us on one sequence of 256 pieces); more than 64 pieces go to
+        // eight waves (one sequence of 4096 tokens, 128 pieces: layer call 19.2 -> 17.8 us; three of 14 000: 31.4 -> 28.8)
         const dim3 cgrid((unsigned)a.num_heads, (unsigned)a.decoding_batches);
         if (a.ranges <= 16 * a.decoding_batches) hipLaunchKernelGGL((decode_combine_kernel<D, 1>), cgrid, dim3(64), 0, stream, a);
         else if (a.ranges <= 48 * a.decoding_batches) hipLaunchKernelGGL((decode_combine_kernel<D, 2>), cgrid, dim3(128), 0, stream, a);
-        else hipLaunchKernelGGL((decode_combine_kernel<D, 4>), cgrid, dim3(256), 0, stream, a);
+        else if (a.ranges <= 64 * a.decoding_batches) hipLaunchKernelGGL((decode_combine_kernel<D, 4>), cgrid, dim3(256), 0, stream, a);
+        else hipLaunchKernelGGL((decode_combine_kernel<D, 8>), cgrid, dim3(512), 0, stream, a);
     }
     return kLaunchOk;
 }

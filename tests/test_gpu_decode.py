@@ -305,3 +305,16 @@ def test_decode_full_size_properties(pkg, oracle, name):
                                             bt.num_heads, bt.num_kv_heads, bt.head_dim, bt.attn_scale, 0,
                                             bt.page_size, **kw)
             assert_attention_close(got_many[b, h], o, "%s b=%d h=%d" % (name, b, h))
+
+
+@pytest.mark.parametrize("shape", [(8, 8, 64), (6, 2, 96), (8, 2, 128), (4, 2, 256)])
+def test_decode_more_pieces_than_lanes(pkg, oracle, shape):
+    """One long sequence: more than 64 pieces per row run eight waves, up to 512 of them with every (max, sum) pair held by
+    the lanes, beyond that block by block."""
+    hq, hkv, d = shape
+    bt, dev, q, cache, scale = make_case(pkg, oracle, 320 + d, num_heads=hq, num_kv_heads=hkv, head_dim=d,
+                                         cache_mode=1, dec_kv_lens=[19000], outliers=True)
+    ref = oracle_decode(oracle, bt, q, cache, scale)
+    for ranges in (65, 128, 129, 200, 511, 590):
+        got, plan = run_decode(dev, ranges)
+        assert_attention_close(got, ref, "shape %s ranges %d" % (shape, ranges))
