@@ -628,11 +628,12 @@ int pmxhip_prefill_attention(const pmxhip_prefill_params* p, pmxhip_stream_t str
     a.cache_stride_h = p->cache_stride_h;
     a.cache_stride_kv = p->cache_stride_kv;
     a.cachestarts_stride_b = p->cachestarts_stride_b;
+    a.compute_units = current_compute_units();
     if (!short_chunks && p->workspace && aligned16(p->workspace)) {
         // few query tiles: their kv tokens shared out over the chip, the parts in the caller's workspace
         const pmxhip::PrefillSplit split =
             pmxhip::prefill_split_choose(prefill_batches, p->max_seqlen, p->max_kvlen, a.query_rows, p->num_heads, p->num_kv_heads,
-                                         p->head_dim, from_current, p->decoding_batches > 0, current_compute_units());
+                                         p->head_dim, from_current, p->decoding_batches > 0, a.compute_units);
         if (split.ranges > 0 && split.bytes <= p->workspace_size) {
             a.split_ranges = split.ranges;
             a.split_gain = split.gain;

@@ -111,6 +111,7 @@ struct PrefillLaunch {
     const void* current_value;
     int64_t key_stride_s;
     int64_t value_stride_s;
+    int32_t compute_units;
     // the kv tokens of a tile shared out over workgroups (prefill_split_choose): ranges per kv head, 0 = whole tiles
     int32_t split_ranges;
     int32_t split_gain;         // weight a split has to take off the call before the kernels go by it

@@ -263,8 +263,10 @@ __device__ __forceinline__ int split_cut(int64_t v, int64_t weight, int n_tiles,
 // register file per wave) took 1094 us: one wave per SIMD exposes every wait that a second wave covers.
 //
 // SPLIT: the launch has one workgroup per range of the split stream (above) instead of one per tile.
-template <int D, int SRC, bool EXTRA, bool SPLIT>
-__global__ __launch_bounds__(kPrefillThreads, 2) void prefill_attention_kernel(const PrefillLaunch a)
+// WPS: waves per SIMD the registers are cut for.  4 (two workgroups per CU) fits head_dim 64 over half K/V rows, whose tiles
+// need no low parts (60 KB of LDS) and whose waves hold half the accumulators; see launch_prefill_variant.
+template <int D, int SRC, bool EXTRA, bool SPLIT, int WPS = 2>
+__global__ __launch_bounds__(kPrefillThreads, WPS) void prefill_attention_kernel(const PrefillLaunch a)
 {
     constexpr bool PAGED = SRC == 0;
     constexpr bool KV16 = SRC == 2;
@@ -1353,6 +1355,8 @@ constexpr size_t prefill_lds_bytes()
     return tiles > with_epilogue ? tiles : with_epilogue;
 }
 
+static_assert(prefill_lds_bytes<64, 2>() <= 64 * 1024, "two workgroups per CU, and no attribute call for that variant");
+
 template <int D, int SRC, bool EXTRA>
 static DeviceMask& prefill_variant_ready()
 {
@@ -1383,7 +1387,13 @@ static int launch_prefill_variant(const PrefillLaunch& a, dim3 grid, hipStream_t
     if (int rc = ready_prefill_variant<D, SRC, EXTRA>(stream, true)) return rc;
     if (a.split_ranges > 0)
         hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, true>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
-    else
+    else if (D == 64 && SRC == 2 && !EXTRA && grid.x > (unsigned)a.compute_units) {
+        // More workgroups than CUs: two per CU cover each other's waits although a few registers spill (32 q / 8 kv heads, 12
+        // prompts of 300-3000 rows: layer call 356 -> 282 us).  With a workgroup per CU or fewer only the spills are left
+        // (8 / 8 heads, six prompts of 300-1500 rows: 46.9 against 48.7 us).
+        if constexpr (D == 64 && SRC == 2 && !EXTRA)
+            hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, false, 4>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
+    } else
         hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, false>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
     return kLaunchOk;
 }

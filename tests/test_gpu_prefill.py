@@ -370,3 +370,20 @@ def test_prefill_tiles_split_from_current_key_value(pkg, oracle, shape):
     torch.cuda.synchronize()
     assert not torch.isnan(op.workspace.view(torch.float32)).all()
     assert_attention_close(dev.output.float().cpu().numpy()[2:], ref[2:], "split, half K/V %s" % (shape,))
+
+
+@pytest.mark.parametrize("shape,q_lens", [((32, 8, 64), [1, 63, 64, 65, 200, 700, 333, 900]), ((8, 8, 64), [1100, 257] * 6)])
+def test_prefill_from_current_key_value_more_tiles_than_compute_units(pkg, oracle, shape, q_lens):
+    """head_dim 64 over the step's half K/V rows with more (tile, kv head) items than compute units: two workgroups per CU."""
+    hq, hkv, d = shape
+    ppw = 256 * hkv // hq
+    assert sum((n + ppw - 1) // ppw for n in q_lens) * hkv > pkg.ops.compute_units()
+    bt, rng = pkg.workloads.custom_batch(860 + hq, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=0, dec_kv_lens=[],
+                                         prefill_q_lens=q_lens, prefill_prior=[0] * len(q_lens), outliers=True)
+    dev = pkg.harness.DeviceBatch(bt)
+    q, k, v = pkg.workloads.step_inputs(bt, rng)
+    dev.set_step_inputs(q, k, v)
+    cache, scale = host_cache(bt)
+    ref = oracle_prefill_ex(oracle, bt, q, cache, scale, current_key=k, current_value=v)
+    got = run_prefill(pkg, dev, current_key=dev.new_key, current_value=dev.new_value)
+    assert_attention_close(got, ref, "two workgroups per CU %s" % (shape,))
