@@ -77,7 +77,8 @@ public:
                                     // prefill stage launch fewer workgroups; 0 = unknown.  A wrong value costs time only:
                                     // the stage's workgroups walk every query tile of the batch whatever the launch size.
         int64_t prefill_workspace_offset; // not in the reference: where the prefill stage's share of the workspace starts
-                                          // (behind the decode stage's where it splits its query tiles' kv tokens, 0 otherwise)
+                                          // (0: short chunks, shared with the decode stage; behind its pieces where query
+                                          // tiles are split over their kv tokens; -1: the stage uses none)
     } cfg{};
 
     // Validates, derives strides / attn_scale / split plan and fills cfg.  Host only.

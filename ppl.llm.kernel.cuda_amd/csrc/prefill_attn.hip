@@ -255,7 +255,8 @@ __device__ __forceinline__ int split_cut(int64_t v, int64_t weight, int n_tiles,
 // issued (the rescale then waits for them, being a reader of their accumulators).
 //
 // Measured on the mixed workload (16 sequences of 256-1024 query rows over up to 2048 prior tokens, 32 query / 8 kv
-// heads of 128): the kernel takes 655 us; built without its products 442 us, without the LDS fragment reads 543 us,
+// heads of 128), before the tile look-up left the registers (2 % less since): the kernel takes 655 us; built
+// without its products 442 us, without the LDS fragment reads 543 us,
 // without dequantisation and global loads 531 us, without exp and the split of p 673 us, without the tile barrier
 // 662 us, with none of these 131 us: the parts add up to the whole, so little of them runs concurrently.  The
 // fragment reads alone take what the LDS port allows (512 KB per tile and CU at 256 bytes per clock).  A form with

@@ -350,26 +350,28 @@ def test_prefill_tiles_split_over_their_kv_tokens(pkg, oracle, shape, q_lens, pr
     np.testing.assert_array_equal(hinted, got)
 
 
+@pytest.mark.parametrize("decodes", [[5, 900], []])
 @pytest.mark.parametrize("shape", [(32, 8, 128), (8, 2, 64), (8, 4, 96), (8, 2, 256)])
-def test_prefill_tiles_split_from_current_key_value(pkg, oracle, shape):
+def test_prefill_tiles_split_from_current_key_value(pkg, oracle, shape, decodes):
     """The split form over the step's own half K/V rows, through the operator class, whose workspace holds the decode
     stage's pieces and, behind them, the parts of the query tiles."""
     hq, hkv, d = shape
     bt, rng = pkg.workloads.custom_batch(820 + d, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=0,
-                                         dec_kv_lens=[5, 900], prefill_q_lens=[1000, 90], prefill_prior=[0, 0], outliers=True)
+                                         dec_kv_lens=decodes, prefill_q_lens=[1000, 90], prefill_prior=[0, 0], outliers=True)
     dev = pkg.harness.DeviceBatch(bt)
     q, k, v = pkg.workloads.step_inputs(bt, rng)
     dev.set_step_inputs(q, k, v)
     cache, scale = host_cache(bt)
     ref = oracle_prefill_ex(oracle, bt, q, cache, scale, current_key=k, current_value=v)
-    assert pkg.ops.prefill_split_workspace_size(bt.batch, 2, bt.max_seqlen, bt.max_kvlen, 1090, hq, hkv, d, True) > 0
+    n_dec = len(decodes)
+    assert pkg.ops.prefill_split_workspace_size(bt.batch, n_dec, bt.max_seqlen, bt.max_kvlen, 1090, hq, hkv, d, True) > 0
     op = dev.make_operator(enable_cache_prefill=False)
     op.workspace.view(torch.float32)[:].fill_(float("nan"))
     dev.output.fill_(float("nan"))
     assert op.forward_prefill() == 0
     torch.cuda.synchronize()
     assert not torch.isnan(op.workspace.view(torch.float32)).all()
-    assert_attention_close(dev.output.float().cpu().numpy()[2:], ref[2:], "split, half K/V %s" % (shape,))
+    assert_attention_close(dev.output.float().cpu().numpy()[n_dec:], ref[n_dec:], "split, half K/V %s" % (shape,))
 
 
 @pytest.mark.parametrize("shape,q_lens", [((32, 8, 64), [1, 63, 64, 65, 200, 700, 333, 900]), ((8, 8, 64), [1100, 257] * 6)])
