@@ -285,19 +285,27 @@ typedef struct pmxhip_prefill_params {
      * prefill_query_rows proves too small (more rows than prefill sequences * max_seqlen) keeps the batch on the tile
      * kernel, which walks every row whatever the hint; otherwise the rows of a sequence beyond max_seqlen are not
      * computed and are filled with NaN, so that an understated hint shows in the output.  A layout or alignment that
-     * the decode kernels refuse also keeps the batch on the tile kernel.
-     * Any other batch of few query tiles shares the kv tokens of a tile out over several workgroups when the workspace has
-     * pmxhip_prefill_split_workspace_size() bytes: the parts lie in it until a second launch adds them. */
+     * the decode kernels refuse also keeps the batch on the tile kernel.  A batch that is not one of short chunks leaves
+     * the buffer alone (pmxhip_prefill_attention_split has one of its own). */
     void* workspace;
     int64_t workspace_size;
 } pmxhip_prefill_params;
 
 PMXHIP_API int pmxhip_prefill_attention(const pmxhip_prefill_params* p, pmxhip_stream_t stream);
 
-/* Bytes of pmxhip_prefill_params::workspace with which a batch of few query tiles (at most one per compute unit,
- * half of that with decode sequences in the step; at most 64 prefill sequences; walks long enough to be worth sharing) splits the kv tokens of its tiles; 0 for every other
- * batch.  query_rows: pmxhip_prefill_params::prefill_query_rows; from_current: current_key is given; compute_units 0 =
- * those of the current device. */
+/* pmxhip_prefill_attention with a second workspace (16-byte aligned; NULL = none): where it has the bytes of
+ * pmxhip_prefill_split_workspace_size(), a batch of few query tiles that does not run as short chunks shares the kv
+ * tokens of a tile out over several workgroups.  Their parts lie in split_workspace until a second launch of this call
+ * adds them, so between the two nothing else may write there: it must not overlap params::workspace, nor the workspace
+ * of a decode stage that may run on another stream meanwhile. */
+PMXHIP_API int pmxhip_prefill_attention_split(const pmxhip_prefill_params* p, void* split_workspace,
+                                              int64_t split_workspace_size, pmxhip_stream_t stream);
+
+/* Bytes of the split workspace with which a batch of few query tiles (at most one per compute unit, half of that with
+ * decode sequences in the step unless current_key is given; at most 64 prefill sequences; walks long enough to be
+ * worth sharing) splits the kv tokens of its tiles; 0 for every other batch.  query_rows:
+ * pmxhip_prefill_params::prefill_query_rows; from_current: current_key is given; compute_units 0 = those of the
+ * current device. */
 PMXHIP_API int64_t pmxhip_prefill_split_workspace_size(int64_t batch, int64_t decoding_batches, int64_t max_seqlen,
                                                        int64_t max_kvlen, int64_t query_rows, int64_t num_heads,
                                                        int64_t num_kv_heads, int64_t head_dim, int32_t from_current,

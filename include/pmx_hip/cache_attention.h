@@ -76,9 +76,9 @@ public:
         int64_t prefill_query_rows; // not in the reference: rows of query beyond the decode rows.  A hint that lets the
                                     // prefill stage launch fewer workgroups; 0 = unknown.  A wrong value costs time only:
                                     // the stage's workgroups walk every query tile of the batch whatever the launch size.
-        int64_t prefill_workspace_offset; // not in the reference: where the prefill stage's share of the workspace starts
-                                          // (0: short chunks, shared with the decode stage; behind its pieces where query
-                                          // tiles are split over their kv tokens; -1: the stage uses none)
+        // not in the reference: where the prefill stage splits its query tiles over their kv tokens, the parts' share of the
+        // workspace, behind the decode stage's pieces; size 0 = no split
+        int64_t prefill_workspace_offset, prefill_split_size;
     } cfg{};
 
     // Validates, derives strides / attn_scale / split plan and fills cfg.  Host only.

@@ -501,6 +501,12 @@ int64_t pmxhip_prefill_split_workspace_size(int64_t batch, int64_t decoding_batc
 
 int pmxhip_prefill_attention(const pmxhip_prefill_params* p, pmxhip_stream_t stream)
 {
+    return pmxhip_prefill_attention_split(p, nullptr, 0, stream);
+}
+
+int pmxhip_prefill_attention_split(const pmxhip_prefill_params* p, void* split_workspace, int64_t split_workspace_size,
+                                   pmxhip_stream_t stream)
+{
     if (!p) return fail(PMXHIP_INVALID_VALUE, "prefill_attention: null params");
     const int64_t prefill_batches = p->batch - p->decoding_batches;
     if (prefill_batches < 0 || p->decoding_batches < 0)
@@ -629,16 +635,16 @@ int pmxhip_prefill_attention(const pmxhip_prefill_params* p, pmxhip_stream_t str
     a.cache_stride_kv = p->cache_stride_kv;
     a.cachestarts_stride_b = p->cachestarts_stride_b;
     a.compute_units = current_compute_units();
-    if (!short_chunks && p->workspace && aligned16(p->workspace)) {
+    if (!short_chunks && split_workspace && aligned16(split_workspace)) {
         // few query tiles: their kv tokens shared out over the chip, the parts in the caller's workspace
         const pmxhip::PrefillSplit split =
             pmxhip::prefill_split_choose(prefill_batches, p->max_seqlen, p->max_kvlen, a.query_rows, p->num_heads, p->num_kv_heads,
                                          p->head_dim, from_current, p->decoding_batches > 0, a.compute_units);
-        if (split.ranges > 0 && split.bytes <= p->workspace_size) {
+        if (split.ranges > 0 && split.bytes <= split_workspace_size) {
             a.split_ranges = split.ranges;
             a.split_gain = split.gain;
-            a.split_out = (float*)p->workspace;
-            a.split_ml = (float*)((char*)p->workspace + split.out_bytes);
+            a.split_out = (float*)split_workspace;
+            a.split_ml = (float*)((char*)split_workspace + split.out_bytes);
         }
     }
     return launch_result("prefill_attention", pmxhip::launch_prefill(a, stream));

@@ -220,13 +220,13 @@ ppl::common::RetCode dynamic_batching_multi_head_cache_attention::heuristic_prep
     cfg.workspace_size = plan.workspace_size;
     // short prefill chunks run on the decode step's kernel and keep their split-KV pieces in the same workspace (the
     // two stages follow each other on the stream)
-    cfg.prefill_workspace_offset = -1;
+    cfg.prefill_workspace_offset = 0;
+    cfg.prefill_split_size = 0;
     if (prefill_batches > 0 && enable_cache_prefill && !attn_mask && !alibi_slopes &&
         pmxhip::prefill_chunk_shape(max_seqlen, num_heads, num_kv_heads, head_dim)) {
         const int64_t chunk_ws = pmxhip_prefill_workspace_size(batch, decoding_batches, max_seqlen, max_kvlen, num_heads,
                                                                num_kv_heads, head_dim, device_prop.multiProcessorCount);
         if (chunk_ws > cfg.workspace_size) cfg.workspace_size = chunk_ws;
-        cfg.prefill_workspace_offset = 0;
     } else if (prefill_batches > 0 && specify_decoding_multi_block != 0) {
         // a batch of few query tiles shares out their kv tokens and keeps the parts behind the decode stage's pieces
         // (disjoint, so that the stages may still run side by side); 0 asks for no split and no workspace
@@ -235,6 +235,7 @@ ppl::common::RetCode dynamic_batching_multi_head_cache_attention::heuristic_prep
                                          head_dim, !enable_cache_prefill, decoding_batches > 0, device_prop.multiProcessorCount);
         if (split.ranges > 0) {
             cfg.prefill_workspace_offset = (cfg.workspace_size + 255) / 256 * 256;
+            cfg.prefill_split_size = split.bytes;
             cfg.workspace_size = cfg.prefill_workspace_offset + split.bytes;
         }
     }
@@ -354,17 +355,17 @@ ppl::common::RetCode dynamic_batching_multi_head_cache_attention::forward_prefil
     p.mask_stride_h = cfg.mask_stride_h;
     p.alibi_slopes = static_cast<const float*>(cfg.alibi_slopes);
     p.prefill_query_rows = cfg.prefill_query_rows;
-    if (cfg.workspace && cfg.prefill_workspace_offset >= 0) {
-        p.workspace = static_cast<char*>(cfg.workspace) + cfg.prefill_workspace_offset;
-        p.workspace_size = cfg.workspace_size - cfg.prefill_workspace_offset;
-    }
+    p.workspace = cfg.workspace;
+    p.workspace_size = cfg.workspace_size;
+    void* split_workspace = nullptr;
+    if (cfg.workspace && cfg.prefill_split_size > 0) split_workspace = static_cast<char*>(cfg.workspace) + cfg.prefill_workspace_offset;
     if (!cfg.enable_cache_prefill) { // kernel.cu:2181-2212: the step's own fp16 K/V only, no cache read
         p.current_key = cfg.current_key;
         p.current_value = cfg.current_value;
         p.key_stride_s = cfg.k_stride_s;
         p.value_stride_s = cfg.v_stride_s;
     }
-    return to_retcode(pmxhip_prefill_attention(&p, stream));
+    return to_retcode(pmxhip_prefill_attention_split(&p, split_workspace, split_workspace ? cfg.prefill_split_size : 0, stream));
 }
 
 ppl::common::RetCode dynamic_batching_multi_head_cache_attention::forward(const hipStream_t stream)

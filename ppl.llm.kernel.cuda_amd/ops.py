@@ -174,7 +174,7 @@ def prefill_attention(query, output, cache, scale, seqstarts, kvstarts, cachesta
     strides, float32 `alibi_slopes` [Hq], `current_key`/`current_value` [rows, KVH, D] to attend over
     the step's own fp16 rows instead of the cache, and a `workspace` of prefill_workspace_size() bytes with which a
     batch of short chunks runs on the decode step's kernel, or of prefill_split_workspace_size() bytes with which a batch
-    of few query tiles is split over its kv tokens."""
+    of few query tiles is split over its kv tokens (no other call may use the workspace while this one runs)."""
     p = PrefillParams()
     p.query = _ptr(query)
     p.output = _ptr(output)
@@ -216,7 +216,7 @@ def prefill_attention(query, output, cache, scale, seqstarts, kvstarts, cachesta
     if workspace is not None:
         p.workspace = _ptr(workspace)
         p.workspace_size = int(workspace.numel() * workspace.element_size())
-    rc = _lib.lib().pmxhip_prefill_attention(ctypes.byref(p), _stream(stream))
+    rc = _lib.lib().pmxhip_prefill_attention_split(ctypes.byref(p), p.workspace, p.workspace_size, _stream(stream))
     if check and rc != RC_SUCCESS:
         raise PmxError(rc, "prefill_attention")
     return rc

@@ -350,6 +350,32 @@ def test_prefill_tiles_split_over_their_kv_tokens(pkg, oracle, shape, q_lens, pr
     np.testing.assert_array_equal(hinted, got)
 
 
+def test_plain_entry_leaves_the_workspace_of_other_batches_alone(pkg, oracle, monkeypatch):
+    """pmxhip_prefill_attention writes its workspace for short chunks only: a caller may have a decode stage's pieces there,
+    on another stream.  Parts of query tiles go to the second workspace of pmxhip_prefill_attention_split."""
+    hq, hkv, d = 32, 8, 128
+    bt, dev, q, cache, scale = make_case(pkg, oracle, 440, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=1, dec_kv_lens=[],
+                                         prefill_q_lens=[300], prefill_prior=[2000], outliers=True)
+    split_bytes = pkg.ops.prefill_split_workspace_size(1, 0, 300, 2300, 300, hq, hkv, d)
+    assert split_bytes > 0
+    lib = pkg._lib.lib()
+
+    class PlainEntry:
+        pmxhip_prefill_attention = staticmethod(lib.pmxhip_prefill_attention)
+
+        @staticmethod
+        def pmxhip_prefill_attention_split(p, split_workspace, split_workspace_size, stream):
+            return lib.pmxhip_prefill_attention(p, stream)
+
+    ws = torch.full((split_bytes // 4,), float("nan"), dtype=torch.float32, device="cuda")
+    with monkeypatch.context() as m:
+        m.setattr(pkg._lib, "lib", PlainEntry)
+        got = run_prefill(pkg, dev, workspace=ws)
+    assert torch.isnan(ws).all()
+    np.testing.assert_array_equal(got, run_prefill(pkg, dev))
+    assert_attention_close(got, oracle_prefill(oracle, bt, q, cache, scale), "plain entry")
+
+
 @pytest.mark.parametrize("decodes", [[5, 900], []])
 @pytest.mark.parametrize("shape", [(32, 8, 128), (8, 2, 64), (8, 4, 96), (8, 2, 256)])
 def test_prefill_tiles_split_from_current_key_value(pkg, oracle, shape, decodes):

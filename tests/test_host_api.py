@@ -228,6 +228,21 @@ def test_c_entry_points_reject_bad_arguments_without_launching(pkg, hip_lib):
     assert hip_lib.pmxhip_prefill_attention(ctypes.byref(f), None) == 2
 
 
+def test_prefill_parts_lie_behind_the_decode_pieces(pkg, hip_lib):
+    """The operator's workspace: the decode stage's pieces, then -- where the query tiles are split over their kv tokens -- the
+    parts, so that the two stages may run side by side."""
+    rows, kvlen = 1200, 1900
+    over = dict(batch=4, decoding_batches=3, max_seqlen=rows, max_kvlen=kvlen, query_shape=(rows + 3, 8, 128), num_heads=8,
+                current_key_shape=(rows + 3, 8, 128), current_value_shape=(rows + 3, 8, 128), output_shape=(rows + 3, 8, 128))
+    plan = pkg.ops.decode_plan(3, 8, 8, 128, kvlen, cus=256)
+    split = pkg.ops.prefill_split_workspace_size(4, 3, rows, kvlen, rows, 8, 8, 128, cus=256)
+    assert plan.workspace_size > 0 and split > 0
+    op, rc = prepare(pkg, **over)
+    assert rc == 0 and op.cfg.workspace_size == (plan.workspace_size + 255) // 256 * 256 + split
+    op, rc = prepare(pkg, specify_decoding_multi_block=0, **over)
+    assert rc == 0 and op.cfg.workspace_size == 0
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py measures one GPU; asking for more ends with a message that says so, before any device work."""
     import os
