@@ -303,7 +303,9 @@ PMXHIP_API int pmxhip_prefill_attention_split(const pmxhip_prefill_params* p, vo
 
 /* Bytes of the split workspace with which a batch of few query tiles (at most one per compute unit, half of that with
  * decode sequences in the step unless current_key is given; at most 64 prefill sequences; walks long enough to be
- * worth sharing) splits the kv tokens of its tiles; 0 for every other batch.  query_rows:
+ * worth sharing) splits the kv tokens of its tiles; 0 for every other batch.  max_kvlen: the longest kv length of the
+ * PREFILL sequences -- a decode sequence's longer one makes the call pay a second launch and the memory for nothing --
+ * 0 = unknown (then only the tiles' own rows count); pmxhip_prefill_params::max_kvlen in the same sense.  query_rows:
  * pmxhip_prefill_params::prefill_query_rows; from_current: current_key is given; compute_units 0 = those of the
  * current device. */
 PMXHIP_API int64_t pmxhip_prefill_split_workspace_size(int64_t batch, int64_t decoding_batches, int64_t max_seqlen,
@@ -396,6 +398,9 @@ typedef struct pmxhip_mhca* pmxhip_mhca_t;
 PMXHIP_API pmxhip_mhca_t pmxhip_mhca_create(void);
 PMXHIP_API void pmxhip_mhca_destroy(pmxhip_mhca_t op);
 PMXHIP_API int pmxhip_mhca_heuristic_prepare(pmxhip_mhca_t op, const pmxhip_mhca_prepare_args* args);
+/* with the longest kv length of the prefill sequences, which the batch-wide max_kvlen does not tell beside decode
+ * sequences (0 = unknown, as above) */
+PMXHIP_API int pmxhip_mhca_heuristic_prepare_ex(pmxhip_mhca_t op, const pmxhip_mhca_prepare_args* args, int64_t prefill_max_kvlen);
 PMXHIP_API int pmxhip_mhca_get_derived(pmxhip_mhca_t op, pmxhip_mhca_derived* out);
 PMXHIP_API int pmxhip_mhca_set_workspace(pmxhip_mhca_t op, void* workspace);
 PMXHIP_API int pmxhip_mhca_forward_kvstore(pmxhip_mhca_t op, pmxhip_stream_t stream);

@@ -76,6 +76,7 @@ public:
         int64_t prefill_query_rows; // not in the reference: rows of query beyond the decode rows.  A hint that lets the
                                     // prefill stage launch fewer workgroups; 0 = unknown.  A wrong value costs time only:
                                     // the stage's workgroups walk every query tile of the batch whatever the launch size.
+        int64_t prefill_max_kvlen; // not in the reference: the longest kv length of the prefill sequences, 0 = unknown
         // not in the reference: where the prefill stage splits its query tiles over their kv tokens, the parts' share of the
         // workspace, behind the decode stage's pieces; size 0 = no split
         int64_t prefill_workspace_offset, prefill_split_size;
@@ -106,6 +107,35 @@ public:
         const int32_t specify_decoding_tpb,         // 0, 256 or 512
         void* cache, void* scale, // int8 cache and float16 group-of-8 scales, same strides (/8)
         const ppl::common::TensorShape* output_shape, void* output); // (Sq, Hq, D)
+
+    // The same with what the batch-wide max_kvlen does not tell beside decode sequences: the longest kv length of the prefill
+    // sequences (0 = unknown, as above).  Given, a step with a few query tiles over a long history splits them over
+    // their kv tokens; unknown, it does so only where the tiles' own rows are worth it.  A wrong value costs time only.
+    ppl::common::RetCode heuristic_prepare(
+        const hipDeviceProp_t& device_prop,
+        const ppl::common::TensorShape* query_shape, const void* query,
+        const ppl::common::TensorShape* current_key_shape, const void* current_key,
+        const ppl::common::TensorShape* current_value_shape, const void* current_value,
+        const ppl::common::TensorShape* attn_mask_shape, const void* attn_mask,
+        const void* seqstarts, const void* kvstarts,
+        const void* cachestarts, const void* start_pos,
+        const void* alibi_slopes,
+        const bool is_causal,
+        const int64_t batch, const int64_t decoding_batches,
+        const int64_t max_seqlen, const int64_t max_kvlen,
+        const int64_t layer_idx, const int64_t num_layer,
+        const int64_t num_heads, const int64_t num_kv_heads, const int64_t head_dim,
+        const int32_t cache_mode, const int64_t page_size,
+        const int64_t cache_stride_s, const int64_t cache_stride_l,
+        const int64_t cache_stride_h, const int64_t cache_stride_kv,
+        const int64_t cachestarts_stride_b,
+        const bool enable_cache_prefill,
+        const bool enable_sharemem_mhca, const bool enable_infinity_mhca, const bool enable_infinity_gqca,
+        const int32_t specify_decoding_multi_block,
+        const int32_t specify_decoding_tpb,
+        void* cache, void* scale,
+        const ppl::common::TensorShape* output_shape, void* output,
+        const int64_t prefill_max_kvlen);
 
     // Stages, all asynchronous on `stream`; kvstore first.
     ppl::common::RetCode forward_kvstore(const hipStream_t stream);

@@ -28,7 +28,7 @@ EXPORTED_SYMBOLS = (
     "pmxhip_decode_attention_stage", "pmxhip_decode_attention_static", "pmxhip_decode_kernel_name",
     "pmxhip_splitkv_combine",
     "pmxhip_prefill_attention", "pmxhip_prefill_attention_split", "pmxhip_prefill_workspace_size", "pmxhip_prefill_split_workspace_size",
-    "pmxhip_mhca_create", "pmxhip_mhca_destroy", "pmxhip_mhca_heuristic_prepare",
+    "pmxhip_mhca_create", "pmxhip_mhca_destroy", "pmxhip_mhca_heuristic_prepare", "pmxhip_mhca_heuristic_prepare_ex",
     "pmxhip_mhca_get_derived", "pmxhip_mhca_set_workspace",
     "pmxhip_mhca_forward_kvstore", "pmxhip_mhca_forward_decode", "pmxhip_mhca_forward_prefill",
     "pmxhip_mhca_forward", "pmxhip_mhca_forward_streams",
@@ -250,6 +250,8 @@ def lib():
     L.pmxhip_mhca_destroy.argtypes = [c_vp]
     L.pmxhip_mhca_heuristic_prepare.restype = ctypes.c_int
     L.pmxhip_mhca_heuristic_prepare.argtypes = [c_vp, ctypes.POINTER(MhcaPrepareArgs)]
+    L.pmxhip_mhca_heuristic_prepare_ex.restype = ctypes.c_int
+    L.pmxhip_mhca_heuristic_prepare_ex.argtypes = [c_vp, ctypes.POINTER(MhcaPrepareArgs), c_i64]
     L.pmxhip_mhca_get_derived.restype = ctypes.c_int
     L.pmxhip_mhca_get_derived.argtypes = [c_vp, ctypes.POINTER(MhcaDerived)]
     L.pmxhip_mhca_set_workspace.restype = ctypes.c_int

@@ -70,6 +70,41 @@ ppl::common::RetCode dynamic_batching_multi_head_cache_attention::heuristic_prep
     void* cache, void* scale,
     const ppl::common::TensorShape* output_shape, void* output)
 {
+    return heuristic_prepare(device_prop, query_shape, query, current_key_shape, current_key, current_value_shape, current_value,
+                             attn_mask_shape, attn_mask, seqstarts, kvstarts, cachestarts, start_pos, alibi_slopes, is_causal, batch,
+                             decoding_batches, max_seqlen, max_kvlen, layer_idx, num_layer, num_heads, num_kv_heads, head_dim,
+                             cache_mode, page_size, cache_stride_s, cache_stride_l, cache_stride_h, cache_stride_kv,
+                             cachestarts_stride_b, enable_cache_prefill, enable_sharemem_mhca, enable_infinity_mhca,
+                             enable_infinity_gqca, specify_decoding_multi_block, specify_decoding_tpb, cache, scale, output_shape,
+                             output, 0);
+}
+
+ppl::common::RetCode dynamic_batching_multi_head_cache_attention::heuristic_prepare(
+    const hipDeviceProp_t& device_prop,
+    const ppl::common::TensorShape* query_shape, const void* query,
+    const ppl::common::TensorShape* current_key_shape, const void* current_key,
+    const ppl::common::TensorShape* current_value_shape, const void* current_value,
+    const ppl::common::TensorShape* attn_mask_shape, const void* attn_mask,
+    const void* seqstarts, const void* kvstarts,
+    const void* cachestarts, const void* start_pos,
+    const void* alibi_slopes,
+    const bool is_causal,
+    const int64_t batch, const int64_t decoding_batches,
+    const int64_t max_seqlen, const int64_t max_kvlen,
+    const int64_t layer_idx, const int64_t num_layer,
+    const int64_t num_heads, const int64_t num_kv_heads, const int64_t head_dim,
+    const int32_t cache_mode, const int64_t page_size,
+    const int64_t cache_stride_s, const int64_t cache_stride_l,
+    const int64_t cache_stride_h, const int64_t cache_stride_kv,
+    const int64_t cachestarts_stride_b,
+    const bool enable_cache_prefill,
+    const bool enable_sharemem_mhca, const bool enable_infinity_mhca, const bool enable_infinity_gqca,
+    const int32_t specify_decoding_multi_block,
+    const int32_t specify_decoding_tpb,
+    void* cache, void* scale,
+    const ppl::common::TensorShape* output_shape, void* output,
+    const int64_t prefill_max_kvlen)
+{
     // ---- shape checks, in the reference's order (utils.cu:68-95) ----
     if (query_shape->GetDim(1) != num_heads) {
         PMX_LOG_ERROR("currently do not support leading dim on query's num_heads");
@@ -222,6 +257,8 @@ ppl::common::RetCode dynamic_batching_multi_head_cache_attention::heuristic_prep
     // two stages follow each other on the stream)
     cfg.prefill_workspace_offset = 0;
     cfg.prefill_split_size = 0;
+    // without decode sequences max_kvlen is the prompts'; beside them it may be theirs
+    cfg.prefill_max_kvlen = prefill_max_kvlen > 0 ? prefill_max_kvlen : (decoding_batches > 0 ? 0 : max_kvlen);
     if (prefill_batches > 0 && enable_cache_prefill && !attn_mask && !alibi_slopes &&
         pmxhip::prefill_chunk_shape(max_seqlen, num_heads, num_kv_heads, head_dim)) {
         const int64_t chunk_ws = pmxhip_prefill_workspace_size(batch, decoding_batches, max_seqlen, max_kvlen, num_heads,
@@ -231,7 +268,7 @@ ppl::common::RetCode dynamic_batching_multi_head_cache_attention::heuristic_prep
         // a batch of few query tiles shares out their kv tokens and keeps the parts behind the decode stage's pieces
         // (disjoint, so that the stages may still run side by side); 0 asks for no split and no workspace
         const pmxhip::PrefillSplit split =
-            pmxhip::prefill_split_choose(prefill_batches, max_seqlen, max_kvlen, cfg.prefill_query_rows, num_heads, num_kv_heads,
+            pmxhip::prefill_split_choose(prefill_batches, max_seqlen, cfg.prefill_max_kvlen, cfg.prefill_query_rows, num_heads, num_kv_heads,
                                          head_dim, !enable_cache_prefill, decoding_batches > 0, device_prop.multiProcessorCount);
         if (split.ranges > 0) {
             cfg.prefill_workspace_offset = (cfg.workspace_size + 255) / 256 * 256;
@@ -358,7 +395,10 @@ ppl::common::RetCode dynamic_batching_multi_head_cache_attention::forward_prefil
     p.workspace = cfg.workspace;
     p.workspace_size = cfg.workspace_size;
     void* split_workspace = nullptr;
-    if (cfg.workspace && cfg.prefill_split_size > 0) split_workspace = static_cast<char*>(cfg.workspace) + cfg.prefill_workspace_offset;
+    if (cfg.workspace && cfg.prefill_split_size > 0) {
+        split_workspace = static_cast<char*>(cfg.workspace) + cfg.prefill_workspace_offset;
+        p.max_kvlen = cfg.prefill_max_kvlen;
+    }
     if (!cfg.enable_cache_prefill) { // kernel.cu:2181-2212: the step's own fp16 K/V only, no cache read
         p.current_key = cfg.current_key;
         p.current_value = cfg.current_value;
@@ -711,6 +751,11 @@ void pmxhip_mhca_destroy(pmxhip_mhca_t op) { delete op; }
 
 int pmxhip_mhca_heuristic_prepare(pmxhip_mhca_t h, const pmxhip_mhca_prepare_args* a)
 {
+    return pmxhip_mhca_heuristic_prepare_ex(h, a, 0);
+}
+
+int pmxhip_mhca_heuristic_prepare_ex(pmxhip_mhca_t h, const pmxhip_mhca_prepare_args* a, int64_t prefill_max_kvlen)
+{
     if (!h || !a) return PMXHIP_INVALID_VALUE;
     h->prop.multiProcessorCount = a->compute_units;
     h->prop.sharedMemPerBlockOptin = (size_t)a->shared_mem_per_block_optin;
@@ -724,7 +769,7 @@ int pmxhip_mhca_heuristic_prepare(pmxhip_mhca_t h, const pmxhip_mhca_prepare_arg
         a->cache_stride_s, a->cache_stride_l, a->cache_stride_h, a->cache_stride_kv, a->cachestarts_stride_b,
         a->enable_cache_prefill != 0, a->enable_sharemem_mhca != 0, a->enable_infinity_mhca != 0,
         a->enable_infinity_gqca != 0, a->specify_decoding_multi_block, a->specify_decoding_tpb, a->cache, a->scale, &os,
-        a->output);
+        a->output, prefill_max_kvlen);
     h->prepared = rc == ppl::common::RC_SUCCESS;
     return (int)rc;
 }

@@ -128,13 +128,14 @@ constexpr int kPrefillSplitMinTokens = 192;
 constexpr int kPrefillSplitGain = 512, kPrefillSplitGain16 = 640;
 // Whether a batch of at most `rows` query rows (0 = unknown) in `sequences` sequences has too few query tiles for the chip,
 // so that their kv tokens are worth sharing out; the ranges per kv head and the workspace that takes.  `kv16`: K/V
-// are the step's own half rows; `mixed`: the step has decode sequences too.
+// are the step's own half rows; `mixed`: the step has decode sequences too; `prefill_max_kvlen`: the longest kv length of the
+// prefill sequences (0 = unknown).
 struct PrefillSplit {
     int32_t ranges = 0; // 0 = whole tiles
     int32_t gain = 0;
     int64_t out_bytes = 0, bytes = 0;
 };
-PrefillSplit prefill_split_choose(int64_t sequences, int64_t max_seqlen, int64_t max_kvlen, int64_t rows, int64_t num_heads,
+PrefillSplit prefill_split_choose(int64_t sequences, int64_t max_seqlen, int64_t prefill_max_kvlen, int64_t rows, int64_t num_heads,
                                   int64_t num_kv_heads, int64_t head_dim, bool kv16, bool mixed, int compute_units);
 
 // One strided copy of whole pages (cache bytes or scale bytes) between the cache and the outer buffer.

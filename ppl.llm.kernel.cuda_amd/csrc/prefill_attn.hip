@@ -1519,13 +1519,14 @@ static int launch_prefill16_d(const PrefillLaunch& a, hipStream_t stream)
     return launch_prefill_items<D, 16>(a, items, stream);
 }
 
-PrefillSplit prefill_split_choose(int64_t sequences, int64_t max_seqlen, int64_t max_kvlen, int64_t rows, int64_t num_heads,
+PrefillSplit prefill_split_choose(int64_t sequences, int64_t max_seqlen, int64_t prefill_max_kvlen, int64_t rows, int64_t num_heads,
                                   int64_t num_kv_heads, int64_t head_dim, bool kv16, bool mixed, int compute_units)
 {
     PrefillSplit r;
     const int64_t cols = head_dim == 256 ? kCols16 : kCols;
-    if (kv16) max_kvlen = max_seqlen;
-    if (sequences <= 0 || sequences > kWave || max_seqlen <= 0 || max_kvlen <= 0 || num_kv_heads <= 0 || num_heads < num_kv_heads ||
+    const bool known = kv16 || prefill_max_kvlen > 0;
+    const int64_t max_kvlen = kv16 || !known ? max_seqlen : prefill_max_kvlen; // (a sequence has its own rows at least)
+    if (sequences <= 0 || sequences > kWave || max_seqlen <= 0 || num_kv_heads <= 0 || num_heads < num_kv_heads ||
         compute_units <= 0)
         return r;
     const int64_t g = num_heads / num_kv_heads;
@@ -1534,12 +1535,14 @@ PrefillSplit prefill_split_choose(int64_t sequences, int64_t max_seqlen, int64_t
     int64_t tiles = sequences * ((max_seqlen + ppw - 1) / ppw);
     if (rows > 0 && rows / ppw + sequences < tiles) tiles = rows / ppw + sequences;
     // (with more tiles than workgroups the order of the tiles, the dear ones first, balances the call well enough)
-    // In a step with decode sequences max_kvlen may be theirs, and the kernels may then find walks too short to share:
-    // that costs a launch (5 us), which half of the chip idle has to be worth.
+    // Beside decode sequences, which fill the chip in their turn, half of it has to be idle.
     if (ranges < 2 || tiles > (mixed && !kv16 ? ranges / 2 : ranges)) return r;
     const int64_t prior = max_kvlen > max_seqlen ? max_kvlen - max_seqlen : 0;
-    const int64_t longest = kSplitStart + max_kvlen, mean = kSplitStart + prior + (max_kvlen - prior) / 2;
-    int64_t per = tiles * mean / ranges;
+    // With the prompts' history unknown the split has to be worth its second launch whatever it is: every tile is taken to weigh as
+    // much as the longest, and as each token of history adds more to the longest than to a range, the kernels (split_stream) then
+    // agree.  A decode sequence's kv length in its place made short prompts pay that launch for nothing.
+    const int64_t longest = kSplitStart + max_kvlen, mean = known ? kSplitStart + prior + (max_kvlen - prior) / 2 : longest;
+    int64_t per = known ? tiles * mean / ranges : (tiles * mean + ranges - 1) / ranges;
     if (per < kPrefillSplitMinTokens) per = kPrefillSplitMinTokens;
     r.gain = kv16 ? kPrefillSplitGain16 : kPrefillSplitGain;
     if (longest - per < r.gain) return r;

@@ -104,7 +104,7 @@ class DeviceBatch:
             num_heads=bt.num_heads, num_kv_heads=bt.num_kv_heads, head_dim=bt.head_dim,
             specify_decoding_multi_block=specify_decoding_multi_block,
             cache=self.cache, scale=self.scale, output=self.output,
-            output_shape=(n_rows, bt.num_heads, bt.head_dim))
+            output_shape=(n_rows, bt.num_heads, bt.head_dim), prefill_max_kvlen=bt.prefill_max_kvlen)
         kw.update(self.layout_kwargs())
         kw.update(overrides)
         rc = op.heuristic_prepare(**kw)

@@ -232,7 +232,7 @@ def prefill_workspace_size(batch, decoding_batches, max_seqlen, max_kvlen, num_h
 def prefill_split_workspace_size(batch, decoding_batches, max_seqlen, max_kvlen, query_rows, num_heads, num_kv_heads, head_dim,
                                  from_current=False, cus=0):
     """Bytes of the workspace with which a batch of few query tiles shares their kv tokens out over the chip; 0 for every
-    other batch."""
+    other batch.  `max_kvlen`: of the prefill sequences (0 = unknown)."""
     return int(_lib.lib().pmxhip_prefill_split_workspace_size(batch, decoding_batches, max_seqlen, max_kvlen, query_rows, num_heads,
                                                               num_kv_heads, head_dim, 1 if from_current else 0, cus))
 
@@ -359,10 +359,10 @@ class DynamicBatchingMultiHeadCacheAttention:
                           enable_cache_prefill=True, enable_sharemem_mhca=True, enable_infinity_mhca=True,
                           enable_infinity_gqca=True, specify_decoding_multi_block=1, specify_decoding_tpb=0,
                           cache=None, scale=None, output=None, output_shape, datatype=DATATYPE_FLOAT16,
-                          compute_units_override=None, shared_mem_per_block_optin=65536):
+                          compute_units_override=None, shared_mem_per_block_optin=65536, prefill_max_kvlen=0):
         """Same arguments, in the same order of meaning, as the reference's heuristic_prepare
-        (multi_head_cache_attention.h:107-148).  Returns the status code; pointers may be None
-        for host-only validation runs."""
+        (multi_head_cache_attention.h:107-148), and the longest kv length of the prefill sequences (0 = unknown).
+        Returns the status code; pointers may be None for host-only validation runs."""
         a = MhcaPrepareArgs()
         a.compute_units = compute_units_override if compute_units_override is not None else compute_units()
         a.shared_mem_per_block_optin = shared_mem_per_block_optin
@@ -409,7 +409,7 @@ class DynamicBatchingMultiHeadCacheAttention:
         # keep the tensors alive for as long as the operator may launch on them
         self._keep = (query, current_key, current_value, attn_mask, seqstarts, kvstarts, cachestarts, start_pos,
                       alibi_slopes, cache, scale, output)
-        return _lib.lib().pmxhip_mhca_heuristic_prepare(self._h, ctypes.byref(a))
+        return _lib.lib().pmxhip_mhca_heuristic_prepare_ex(self._h, ctypes.byref(a), prefill_max_kvlen)
 
     @property
     def cfg(self):

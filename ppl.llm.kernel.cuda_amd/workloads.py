@@ -122,6 +122,11 @@ class Batch:
         return int(self.kv_lens.max()) if len(self.kv_lens) else 0
 
     @property
+    def prefill_max_kvlen(self):
+        """Longest kv length of the prefill sequences (0 = there are none)."""
+        return int(self.kv_lens[self.decoding_batches:].max(initial=0))
+
+    @property
     def attn_scale(self):
         return float(np.float32(1.0 / np.sqrt(np.float32(self.head_dim))))
 

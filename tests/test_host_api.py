@@ -243,6 +243,53 @@ def test_prefill_parts_lie_behind_the_decode_pieces(pkg, hip_lib):
     assert rc == 0 and op.cfg.workspace_size == 0
 
 
+def mixed_args(q_lens, max_kvlen, hq=32, hkv=8, d=128, decodes=3):
+    rows = int(sum(q_lens)) + decodes
+    return dict(batch=len(q_lens) + decodes, decoding_batches=decodes, max_seqlen=int(max(q_lens)), max_kvlen=max_kvlen, num_heads=hq,
+                num_kv_heads=hkv, head_dim=d, query_shape=(rows, hq, d), current_key_shape=(rows, hkv, d),
+                current_value_shape=(rows, hkv, d), output_shape=(rows, hq, d))
+
+
+def test_short_prompts_beside_long_decode_sequences_are_not_split(pkg, hip_lib):
+    """max_kvlen may be a decode sequence's: alone it asks for no workspace (and no second launch) for the prompts.  Their own
+    length, where the caller gives it, does."""
+    args = mixed_args([70], 4096)
+    pieces = pkg.ops.decode_plan(3, 32, 8, 128, 4096, cus=256).workspace_size
+    op, rc = prepare(pkg, **args)
+    assert rc == 0 and op.cfg.workspace_size == pieces
+    op, rc = prepare(pkg, prefill_max_kvlen=70, **args)
+    assert rc == 0 and op.cfg.workspace_size == pieces
+    op, rc = prepare(pkg, prefill_max_kvlen=3000, **args)
+    assert rc == 0 and op.cfg.workspace_size > pieces + (1 << 20)
+
+
+def test_unknown_history_is_split_only_where_the_kernels_agree(pkg, hip_lib):
+    """The rule of split_stream in csrc/prefill_attn.hip, in numpy: whatever the prompts' history, a batch that the host splits
+    beside decode sequences without knowing it is split by the kernels (else the second launch is for nothing)."""
+    import numpy as np
+    rng = np.random.default_rng(21)
+    split = 0
+    for _ in range(4000):
+        hkv = int(rng.choice([1, 2, 4, 8, 16]))
+        hq = hkv * int(rng.choice([1, 2, 4, 8]))
+        d = int(rng.choice([64, 96, 128, 256]))
+        cols = 128 if d == 256 else 256
+        ppw, ranges = cols // (hq // hkv), 256 // hkv
+        q = rng.integers(1, int(rng.choice([100, 1000, 4000])), size=int(rng.integers(1, 12)))
+        prior = rng.integers(0, int(rng.choice([1, 300, 8000])) + 1, size=len(q))
+        size = pkg.ops.prefill_split_workspace_size(len(q) + 1, 1, int(q.max()), 0, int(q.sum()), hq, hkv, d, cus=256)
+        if size == 0:
+            continue
+        split += 1
+        for causal in (True, False):
+            step, base = (ppw, prior) if causal else (0, prior + q)
+            tiles = -(-q // ppw)
+            total = int((tiles * (64 + base) + step * (tiles * (tiles + 1) // 2)).sum())
+            per = max(-(-total // ranges), 192)
+            assert int((64 + base + step * tiles).max()) - per >= 512, (q, prior, hq, hkv, d, causal)
+    assert split > 100
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py measures one GPU; asking for more ends with a message that says so, before any device work."""
     import os
