@@ -516,11 +516,11 @@ PMXHIP_API int pmxhip_rope_kv_cache_quantize(const pmxhip_rope_params* rope, con
  * PMXHIP_UNSUPPORTED.  One kernel is written for the decode step (M up to a few hundred rows: bound by streaming the
  * K * N * 2 weight bytes), one for the query rows of prompts (compute-bound); they allocate nothing and add
  * their partial sums in a fixed order, so a call's result does not depend on timing.
- * workspace: where the output has fewer tiles than the chip has CUs and K is long, the k range is split over
- * several workgroups whose float32 partial tiles pass through `workspace` (the role of the reference's
- * cublas_workspace argument) and are added in a fixed order by a second kernel.
+ * workspace: where that is estimated to be 5 % faster (a long K, and tiles that fill the CUs badly: too few of them, or a last
+ * round with few), the k range is split over 2 or 4 workgroups whose float32 partial tiles pass through `workspace`
+ * (the role of the reference's cublas_workspace argument) and are added in a fixed order by a second kernel.
  * pmxhip_row_parallel_linear_workspace_size gives the bytes that serve (M, in_features, out_features) on the
- * current device (0 = none needed); with a NULL or smaller workspace the call still computes the same function,
+ * current device: 0 = none needed, at most 256 MiB; with a NULL or smaller workspace the call still computes the same function,
  * one k range per tile (slower for a long K).  The workspace needs 16-byte alignment and no clearing.
  *
  * The _ex forms take flags.  PMXHIP_LINEAR_VENDOR_GEMM: from 384 rows on (a prefill chunk's query rows: a
@@ -542,6 +542,22 @@ PMXHIP_API int pmxhip_row_parallel_linear_ex(pmxhip_stream_t stream, const void*
                                              int64_t m, int64_t in_features, int64_t out_features, int64_t input_stride,
                                              int64_t weight_stride, int64_t output_stride, int64_t workspace_size,
                                              void* workspace, void* output, int32_t flags);
+/* Which kernel a call of this library's own kernels launches for these sizes, for tests and sizing; host only.
+ * workspace_size: what the call would be given (INT64_MAX: the best); compute_units 0 = those of the current device.  Row
+ * strides of 2^23 halves and more take the ROWS kernel whatever the plan says. */
+typedef enum pmxhip_linear_kernel_t {
+    PMXHIP_LINEAR_KERNEL_ROWS = 0,   /* 16 columns x 128 rows per workgroup, any row stride */
+    PMXHIP_LINEAR_KERNEL_STREAM = 1, /* decode-sized M */
+    PMXHIP_LINEAR_KERNEL_TILE = 2    /* from a few hundred rows */
+} pmxhip_linear_kernel_t;
+typedef struct pmxhip_linear_plan {
+    int32_t kernel;          /* pmxhip_linear_kernel_t */
+    int32_t tile_n, tile_m;  /* output columns and rows of a workgroup */
+    int32_t k_ranges;
+    int64_t workspace_size;  /* of the partial tiles; 0 with one k range */
+} pmxhip_linear_plan;
+PMXHIP_API int pmxhip_row_parallel_linear_plan(int64_t m, int64_t in_features, int64_t out_features, int64_t workspace_size,
+                                               int32_t compute_units, pmxhip_linear_plan* out);
 /* Loads hipBLASLt and creates its handle on the current device (PMXHIP_LINEAR_VENDOR_GEMM); PMXHIP_UNSUPPORTED when
  * the library cannot be loaded.  Host only; allocates. */
 PMXHIP_API int pmxhip_init_vendor_gemm(void);

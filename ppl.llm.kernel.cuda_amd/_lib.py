@@ -35,7 +35,8 @@ EXPORTED_SYMBOLS = (
     "pmxhip_kv_cache_reorder", "pmxhip_kv_cache_invert_reorder",
     "pmxhip_rotary_position_embedding", "pmxhip_rope_kv_cache_quantize",
     "pmxhip_row_parallel_linear", "pmxhip_row_parallel_linear_workspace_size",
-    "pmxhip_row_parallel_linear_ex", "pmxhip_row_parallel_linear_workspace_size_ex", "pmxhip_init_vendor_gemm",
+    "pmxhip_row_parallel_linear_ex", "pmxhip_row_parallel_linear_workspace_size_ex", "pmxhip_row_parallel_linear_plan",
+    "pmxhip_init_vendor_gemm",
 )
 
 
@@ -130,6 +131,16 @@ class ReorderStride(ctypes.Structure):
         return s
 
 
+class LinearPlan(ctypes.Structure):
+    _fields_ = [("kernel", c_i32), ("tile_n", c_i32), ("tile_m", c_i32), ("k_ranges", c_i32), ("workspace_size", c_i64)]
+
+
+# pmxhip_linear_kernel_t
+LINEAR_KERNEL_ROWS = 0
+LINEAR_KERNEL_STREAM = 1
+LINEAR_KERNEL_TILE = 2
+
+
 class TensorShape(ctypes.Structure):
     _fields_ = [("dim_count", c_i32), ("data_type", c_i32), ("dims", c_i64 * 4)]
 
@@ -220,6 +231,8 @@ def lib():
     L.pmxhip_row_parallel_linear_ex.argtypes = [c_vp] * 4 + [c_i64] * 7 + [c_vp, c_vp, ctypes.c_int32]
     L.pmxhip_row_parallel_linear_workspace_size_ex.restype = c_i64
     L.pmxhip_row_parallel_linear_workspace_size_ex.argtypes = [c_i64] * 3 + [ctypes.c_int32]
+    L.pmxhip_row_parallel_linear_plan.restype = ctypes.c_int
+    L.pmxhip_row_parallel_linear_plan.argtypes = [c_i64] * 4 + [c_i32, ctypes.POINTER(LinearPlan)]
     L.pmxhip_init_vendor_gemm.restype = ctypes.c_int
     L.pmxhip_init_vendor_gemm.argtypes = []
     L.pmxhip_init.restype = ctypes.c_int

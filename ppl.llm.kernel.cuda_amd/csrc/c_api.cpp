@@ -805,11 +805,26 @@ int64_t pmxhip_row_parallel_linear_workspace_size(int64_t m, int64_t in_features
 int64_t pmxhip_row_parallel_linear_workspace_size_ex(int64_t m, int64_t in_features, int64_t out_features, int32_t flags)
 {
     if (m <= 0 || in_features <= 0 || out_features <= 0) return 0;
-    const int64_t own = pmxhip::linear_workspace_bytes(m, out_features, in_features, current_compute_units());
+    const int64_t own = pmxhip::linear_plan(m, out_features, in_features, current_compute_units(), INT64_MAX).workspace_bytes;
     if ((flags & PMXHIP_LINEAR_VENDOR_GEMM) && m >= pmxhip::kLinearLibraryRows && pmxhip::linear_library_available() &&
         own < pmxhip::kLinearLibraryWorkspace)
         return pmxhip::kLinearLibraryWorkspace;
     return own;
+}
+
+int pmxhip_row_parallel_linear_plan(int64_t m, int64_t in_features, int64_t out_features, int64_t workspace_size, int32_t compute_units,
+                                    pmxhip_linear_plan* out)
+{
+    if (!out || m <= 0 || in_features <= 0 || out_features <= 0) return fail(PMXHIP_INVALID_VALUE, "row_parallel_linear_plan: bad sizes");
+    const pmxhip::LinearPlan plan =
+        pmxhip::linear_plan(m, out_features, in_features, compute_units > 0 ? compute_units : current_compute_units(), workspace_size);
+    static_assert((int)pmxhip::kLinStream == PMXHIP_LINEAR_KERNEL_STREAM && (int)pmxhip::kLinTile == PMXHIP_LINEAR_KERNEL_TILE, "kernel numbers");
+    out->kernel = plan.kernel;
+    out->tile_n = plan.tile_n;
+    out->tile_m = plan.tile_m;
+    out->k_ranges = plan.splits;
+    out->workspace_size = plan.workspace_bytes;
+    return PMXHIP_SUCCESS;
 }
 
 int pmxhip_row_parallel_linear(pmxhip_stream_t stream, const void* input, const void* weight, const void* bias, int64_t m,

@@ -197,9 +197,17 @@ struct LinearLaunch {
     int64_t m, n, k;
     int64_t input_stride, weight_stride, output_stride;
 };
-// workspace: float32 partial tiles of the k ranges (linear_workspace_bytes; may be null: then one k range)
+// workspace: float32 partial tiles of the k ranges (LinearPlan::workspace_bytes; may be null: then one k range)
 int launch_linear(const LinearLaunch& a, int compute_units, void* workspace, int64_t workspace_bytes, hipStream_t stream);
-int64_t linear_workspace_bytes(int64_t m, int64_t n, int64_t k, int compute_units);
+// what launch_linear takes for a problem of ordinary row strides when it has that much workspace (INT64_MAX: the best)
+enum LinearKernel { kLinFarRows, kLinStream, kLinTile }; // pmxhip_linear_kernel_t
+struct LinearPlan {
+    LinearKernel kernel = kLinFarRows;
+    int tile_n = 16, tile_m = 128;
+    int splits = 1;
+    int64_t workspace_bytes = 0;
+};
+LinearPlan linear_plan(int64_t m, int64_t n, int64_t k, int compute_units, int64_t workspace_bytes);
 
 // The one-time hipFuncSetAttribute of a kernel whose dynamic LDS exceeds the default limit: once per kernel and
 // device (`ready` holds a bit per device; devices 0-63, like the other per-device caches of the library -- a

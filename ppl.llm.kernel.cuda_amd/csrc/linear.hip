@@ -481,8 +481,13 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(const LinearLaunch a
 // beats its weights at 5.7 TB/s.  The constants are a fit to 1800 timings (nine tiles x 1, 2 and 4 ranges x M = 1 .. 6000 on
 // seven weight shapes from 2048 x 2048 to 4096 x 14336): the tile that the estimate picks takes 1.01 times what the best one
 // takes in the mean, 1.15 at worst.
+// More than one k range costs the caller a workspace, so it has to be worth it: its estimate beats the best one-range tile's by 5 %
+// (over those shapes that gives up gains below the model's own error), and the partial tiles take at most 256 MiB, what the
+// memory-side cache holds between the launch that writes them and the one that adds them.  (Without the two bounds prompts asked for
+// up to 700 MB, (3472, 14336, 14336) for 398 MB of them at an estimate of 1360.2 against 1360.6 us.)
 namespace {
-enum LinearKernel { kLinStream, kLinTile };
+constexpr float kLinearSplitGain = 0.05f;
+constexpr int64_t kLinearSplitBytes = (int64_t)256 << 20;
 struct LinearTile {
     LinearKernel kernel;
     int tn, tm;
@@ -497,16 +502,17 @@ constexpr int kLinearTileCount = (int)(sizeof(kLinearTiles) / sizeof(kLinearTile
 // rows of a tile are addressed as a 64-bit base plus a 32-bit byte offset: up to 256 rows of less than 2^23 halves
 constexpr int64_t kLinearMaxStride = (int64_t)1 << 23;
 
-struct LinearPlan {
+struct LinearChoice {
     int tile = -1; // index into kLinearTiles
     int splits = 1;
+    float us = 0.f;
 };
 
-LinearPlan linear_choose(int64_t m, int64_t n, int64_t k, int compute_units, int64_t workspace_bytes)
+LinearChoice linear_choose(int64_t m, int64_t n, int64_t k, int compute_units, int64_t workspace_bytes)
 {
     const int64_t cus = compute_units > 0 ? compute_units : 256;
-    LinearPlan best;
-    float best_us = 0.f;
+    if (workspace_bytes > kLinearSplitBytes) workspace_bytes = kLinearSplitBytes;
+    LinearChoice one, split;
     const float stream_us = 2.f + (float)n * (float)k * 2.f / 5.7e6f;
     for (int i = 0; i < kLinearTileCount; ++i) {
         const LinearTile& c = kLinearTiles[i];
@@ -522,22 +528,30 @@ LinearPlan linear_choose(int64_t m, int64_t n, int64_t k, int compute_units, int
             float us = (float)rounds * (c.start_us + (float)(per * unit) * c.ns_per_k * 1e-3f);
             if (s > 1) us += 4.f + (float)s * (float)m * (float)n * 8.f / 5.5e6f;
             us = fmaxf(us, stream_us) + 0.1f * fminf(us, stream_us); // what overlaps the stream still shows a little
-            if (best.tile < 0 || us < best_us) {
+            LinearChoice& best = s > 1 ? split : one;
+            if (best.tile < 0 || us < best.us) {
                 best.tile = i;
                 best.splits = s;
-                best_us = us;
+                best.us = us;
             }
         }
     }
-    return best;
+    return split.tile >= 0 && split.us < one.us * (1.f - kLinearSplitGain) ? split : one;
 }
 } // namespace
 
-int64_t linear_workspace_bytes(int64_t m, int64_t n, int64_t k, int compute_units)
+LinearPlan linear_plan(int64_t m, int64_t n, int64_t k, int compute_units, int64_t workspace_bytes)
 {
-    if (m <= 0 || n <= 0 || k <= 0) return 0;
-    const LinearPlan plan = linear_choose(m, n, k, compute_units, INT64_MAX);
-    return plan.splits > 1 ? (int64_t)plan.splits * m * n * (int64_t)sizeof(float) : 0;
+    LinearPlan plan;
+    if (m <= 0 || n <= 0 || k <= 0) return plan;
+    const LinearChoice c = linear_choose(m, n, k, compute_units, workspace_bytes);
+    if (c.tile < 0) return plan;
+    plan.kernel = kLinearTiles[c.tile].kernel;
+    plan.tile_n = kLinearTiles[c.tile].tn;
+    plan.tile_m = kLinearTiles[c.tile].tm;
+    plan.splits = c.splits;
+    if (c.splits > 1) plan.workspace_bytes = (int64_t)c.splits * m * n * (int64_t)sizeof(float);
+    return plan;
 }
 
 int launch_linear(const LinearLaunch& a, int compute_units, void* workspace, int64_t workspace_bytes, hipStream_t stream)
@@ -546,7 +560,7 @@ int launch_linear(const LinearLaunch& a, int compute_units, void* workspace, int
     if (a.n % kLinCols != 0 || a.k % kLinKStep != 0 || a.k <= 0) return kLaunchNoKernel;
     // as many k ranges as the workspace holds partial tiles for; none: one k range
     if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 15u)) workspace_bytes = 0;
-    const LinearPlan plan = linear_choose(a.m, a.n, a.k, compute_units, workspace_bytes);
+    const LinearChoice plan = linear_choose(a.m, a.n, a.k, compute_units, workspace_bytes);
     if (plan.tile < 0 || a.weight_stride >= kLinearMaxStride || a.input_stride >= kLinearMaxStride) {
         const int64_t mblocks = (a.m + kLinRows - 1) / kLinRows;
         if (a.n / kLinCols > 0x7fffffff || mblocks > 65535) return kLaunchNoKernel;

@@ -307,6 +307,15 @@ def row_parallel_linear_workspace_size(m, in_features, out_features, vendor_gemm
                                                                         LINEAR_VENDOR_GEMM if vendor_gemm else 0))
 
 
+def row_parallel_linear_plan(m, in_features, out_features, workspace_size=(1 << 63) - 1, cus=0):
+    """Kernel, tile and k ranges of a row_parallel_linear call that is given `workspace_size` bytes (default: the best)."""
+    plan = _lib.LinearPlan()
+    rc = _lib.lib().pmxhip_row_parallel_linear_plan(m, in_features, out_features, workspace_size, cus, ctypes.byref(plan))
+    if rc != RC_SUCCESS:
+        raise PmxError(rc, "row_parallel_linear_plan")
+    return plan
+
+
 def vendor_gemm_available():
     """True when hipBLASLt could be loaded and gave a handle on the current device (allocates; never under capture)."""
     return _lib.lib().pmxhip_init_vendor_gemm() == RC_SUCCESS
