@@ -78,3 +78,20 @@ def test_the_command_fails_on_a_hazard_and_on_nothing_to_check(lint, tmp_path, m
     assert run(asm_load("v[10:13]") + ["v_mov_b32 v40, v11"] + asm_wait(0)) == 1
     assert run(["v_mov_b32 v1, v2"]) == 1  # no hand-scheduled kernel found: the check itself went wrong
     assert "0 hand-scheduled kernels checked" in capsys.readouterr().out
+
+
+def test_asm_that_writes_m0_says_so():
+    """The compiler keeps values of its own in m0 (register indexing, its direct-to-LDS loads): an asm statement that writes it
+    has to name it as clobbered."""
+    import re
+    csrc = os.path.join(ROOT, "ppl.llm.kernel.cuda_amd", "csrc")
+    found = 0
+    for name in sorted(os.listdir(csrc)):
+        if not name.endswith((".h", ".hip", ".cpp")):
+            continue
+        for stmt in re.findall(r"\basm\b[^;]*?\(.*?\)\s*;", open(os.path.join(csrc, name)).read(), flags=re.S):
+            template, _, operands = stmt.partition("::") if "::" in stmt else stmt.partition('" :')
+            if re.search(r"\bs_\w+ m0\b", template):
+                found += 1
+                assert '"m0"' in operands, "%s: %s" % (name, stmt)
+    assert found >= 2
