@@ -239,8 +239,7 @@ def prefill_split_workspace_size(batch, decoding_batches, max_seqlen, max_kvlen,
 
 def _rope_params(query, key, start_pos, seqstarts, rotated_query, rotated_key, *, theta, rotary_dim, batch, max_seqlen,
                  bypass_key=False, max_position_embeddings=2048, scaling_type=0, scaling_factor=1.0):
-    _, hq, d = query.shape
-    hk = key.shape[1]
+    hq, d, hk = query.shape[1], query.shape[2], key.shape[1]
     # in the order of the structure's fields (one call: field by field costs as much as the launch)
     return _lib.RopeParams(_ptr(query), _ptr(key), _ptr(start_pos), _ptr(seqstarts), theta, 1 if bypass_key else 0, rotary_dim,
                            batch, hq, hk, d, max_seqlen, max_position_embeddings, scaling_type, scaling_factor,
@@ -326,7 +325,7 @@ def row_parallel_linear(input, weight, bias, output, *, workspace=None, stream=N
     last dimension (row strides may exceed the row).  The single-rank case of the reference's row_parallel_linear.
     `workspace`: a uint8 tensor of row_parallel_linear_workspace_size bytes, or None (slower at decode sizes).
     `vendor_gemm`: from 384 rows on, hand the GEMM to hipBLASLt where it loads (off: this library's kernels)."""
-    n, k = weight.shape
+    n, k = weight.shape[0], weight.shape[1]
     m = input.numel() // k  # a contiguous (B, Hq, D) attention output is the (B, Hq * D) input in place
 
     def row_stride(t, width):

@@ -290,6 +290,19 @@ def test_unknown_history_is_split_only_where_the_kernels_agree(pkg, hip_lib):
     assert split > 100
 
 
+def test_calls_take_tensors_with_dimensions_of_one_behind_the_row(pkg, hip_lib, monkeypatch):
+    """A query of (rows, heads, head_dim, 1) and a weight of (out, in, 1) are the same rows."""
+    import torch
+    monkeypatch.setattr(pkg.ops, "_ptr", lambda t: 16 if t is not None else None)
+    monkeypatch.setattr(pkg.ops, "_stream", lambda stream=None: None)
+    rows = torch.empty((0, 4, 64, 1), dtype=torch.float16)
+    pkg.ops.rotary_position_embedding(rows, rows, rows, rows, rows, rows, theta=1e4, rotary_dim=64, batch=0, max_seqlen=0)
+    p = pkg.ops._rope_params(rows, rows[:, :2], rows, rows, rows, rows, theta=1e4, rotary_dim=64, batch=0, max_seqlen=0)
+    assert (p.num_heads, p.num_key_heads, p.head_dim, p.query_stride_s, p.rotated_key_stride_s) == (4, 2, 64, 256, 128)
+    pkg.ops.row_parallel_linear(torch.empty((0, 64), dtype=torch.float16), torch.empty((32, 64, 1), dtype=torch.float16), None,
+                                torch.empty((0, 32), dtype=torch.float16))
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py measures one GPU; asking for more ends with a message that says so, before any device work."""
     import os
