@@ -40,9 +40,15 @@ def _ptr(t):
     return t.data_ptr()
 
 
+# torch.cuda.current_stream() without the Stream object around the handle (a microsecond per call), where torch has it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(stream=None):
-    if stream is None: # torch.cuda.current_stream() without the Stream object around the handle (a microsecond per call)
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if stream is None:
+        if _raw_stream is None:
+            return torch.cuda.current_stream().cuda_stream
+        return _raw_stream(torch.cuda.current_device())
     return stream.cuda_stream
 
 

@@ -303,6 +303,21 @@ def test_calls_take_tensors_with_dimensions_of_one_behind_the_row(pkg, hip_lib, 
                                 torch.empty((0, 32), dtype=torch.float16))
 
 
+def test_current_stream_without_the_private_call(pkg, monkeypatch):
+    """A torch without the private raw-stream call serves the public one."""
+    import importlib.util
+    import types
+    import torch
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    spec = importlib.util.spec_from_file_location(pkg.__name__ + ".ops_again", pkg.ops.__file__)
+    ops = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(ops)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=4711))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    assert ops._stream() == 4711
+    assert ops._stream(types.SimpleNamespace(cuda_stream=12)) == 12
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py measures one GPU; asking for more ends with a message that says so, before any device work."""
     import os
