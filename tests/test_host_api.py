@@ -25,6 +25,33 @@ def test_library_exports_every_declared_symbol(pkg, hip_lib):
     assert b"gfx950" in hip_lib.pmxhip_version()
 
 
+def test_python_structures_follow_the_header(pkg):
+    """Every ctypes structure has the header's fields in the header's order and types (some are filled by position)."""
+    L = pkg._lib
+    text = open(os.path.join(ROOT, "include", "pmx_hip", "c_api.h")).read()
+    text = re.sub(r"/\*.*?\*/", "", text, flags=re.S)
+    kinds = {"int64_t": L.c_i64, "int32_t": L.c_i32, "float": L.c_f32, "pmxhip_tensor_shape": L.TensorShape}
+    classes = dict(kvstore_params=L.KvstoreParams, decode_params=L.DecodeParams, decode_plan=L.DecodePlan, prefill_params=L.PrefillParams,
+                   tensor_shape=L.TensorShape, mhca_prepare_args=L.MhcaPrepareArgs, mhca_derived=L.MhcaDerived,
+                   reorder_stride=L.ReorderStride, rope_params=L.RopeParams, linear_plan=L.LinearPlan)
+    bodies = dict(re.findall(r"typedef struct pmxhip_(\w+) \{(.*?)\} pmxhip_\1;", text, flags=re.S))
+    assert sorted(bodies) == sorted(classes)
+    for name, cls in classes.items():
+        want = []
+        for decl in filter(None, (d.strip() for d in bodies[name].split(";"))):
+            kind, rest = re.match(r"(?:const )?(\w+)\s*(.*)", decl, flags=re.S).groups()
+            for field in rest.split(","):
+                field = field.strip()
+                array = re.match(r"(\w+)\[(\d+)\]$", field)
+                if field.startswith("*"):
+                    want.append((field.lstrip("* "), L.c_vp))
+                elif array:
+                    want.append((array.group(1), kinds[kind] * int(array.group(2))))
+                else:
+                    want.append((field, kinds[kind]))
+        assert [tuple(f) for f in cls._fields_] == want, name
+
+
 def base_args(**over):
     kw = dict(query_shape=(6, 32, 128), current_key_shape=(6, 8, 128), current_value_shape=(6, 8, 128),
               output_shape=(6, 32, 128), batch=6, decoding_batches=6, max_seqlen=1, max_kvlen=4096, layer_idx=0,
