@@ -216,3 +216,93 @@ def test_unsupported_configurations_report_not_crash(pkg):
     assert op.forward_prefill() == pkg.ops.RC_UNSUPPORTED
     assert op.forward() == pkg.ops.RC_UNSUPPORTED       # first failure wins
     torch.cuda.synchronize()
+
+
+def split_case(pkg, oracle, seed):
+    """Decode sequences of several ranges beside one prompt whose query tiles the kernels do split: its longest walk is
+    2500 + 300 tokens, a range about a sixth of that, and a split asks for 512 between the two."""
+    bt, rng = pkg.workloads.custom_batch(seed, num_heads=32, num_kv_heads=8, head_dim=128, cache_mode=1,
+                                         dec_kv_lens=[700, 2, 1900, 130, 1, 2000], prefill_q_lens=[300], prefill_prior=[2500],
+                                         outliers=True)
+    cache, scale = host_cache(bt)
+    dev = pkg.harness.DeviceBatch(bt)
+    for b, pos, k_rows, v_rows in oracle_fill_history(oracle, pkg, bt, rng, cache, scale):
+        dev.append_rows(b, pos, k_rows, v_rows)
+    q, k, v = pkg.workloads.step_inputs(bt, rng)
+    dev.set_step_inputs(q, k, v)
+    op = dev.make_operator(specify_decoding_multi_block=1)
+    pieces = pkg.ops.decode_plan(6, 32, 8, 128, bt.max_kvlen).workspace_size
+    parts = (pieces + 255) // 256 * 256
+    assert pieces > 0 and op.cfg.workspace_size > parts
+    oracle_append_step(oracle, bt, k, v, cache, scale)
+    ref = oracle_prefill(oracle, bt, q, cache, scale)
+    ref[:bt.decoding_batches] = oracle_decode(oracle, bt, q, cache, scale)
+    return dev, op, pieces, parts, ref
+
+
+def test_split_prefill_beside_the_decode_stage(pkg, oracle):
+    """Parts of query tiles behind the decode stage's pieces: neither stage writes the other's share of the workspace, and
+    with the two on two streams -- from the host and replayed from a graph -- the rows are those of one stream, bit for bit."""
+    dev, op, pieces, parts, ref = split_case(pkg, oracle, 407)
+    ws = op.workspace[:op.workspace.numel() // 4 * 4].view(torch.float32)
+    main, side = torch.cuda.Stream(), torch.cuda.Stream()
+    fork, join = torch.cuda.Event(), torch.cuda.Event()
+    fork.record(main)
+    join.record(main)
+    main.synchronize()
+    with torch.cuda.stream(main):
+        assert op.forward_kvstore(main) == 0
+        ws.fill_(float("nan"))
+        assert op.forward_prefill(main) == 0
+        main.synchronize()
+        assert torch.isnan(ws[:parts // 4]).all() and not torch.isnan(ws[parts // 4:]).all()
+        ws.fill_(float("nan"))
+        assert op.forward_decode(main) == 0
+        main.synchronize()
+        assert not torch.isnan(ws[:pieces // 4]).all() and torch.isnan(ws[pieces // 4:]).all()
+        one_stream = dev.output.clone()
+        for rep in range(3):
+            dev.output.fill_(float("nan"))
+            assert op.forward_streams(main, side, fork, join) == 0
+            after = dev.output.clone()
+            main.synchronize()
+            assert torch.equal(after.view(torch.int16), one_stream.view(torch.int16)), "call %d" % rep
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=main):
+            assert op.forward_streams(main, side, fork, join) == 0
+            assert op.forward_streams(main, side, fork, join) == 0
+        for rep in range(3):
+            dev.output.fill_(float("nan"))
+            ws.fill_(float("nan"))
+            graph.replay()
+            main.synchronize()
+            assert torch.equal(dev.output.view(torch.int16), one_stream.view(torch.int16)), "replay %d" % rep
+            assert op.forward(main) == 0
+            main.synchronize()
+            assert torch.equal(dev.output.view(torch.int16), one_stream.view(torch.int16)), "eager after replay %d" % rep
+    assert_attention_close(one_stream.float().cpu().numpy(), ref, "rows")
+
+
+def test_split_prefill_in_a_hip_graph(pkg, oracle):
+    """A captured step whose query tiles are split: every replay writes the parts anew and gives the eager rows."""
+    dev, op, pieces, parts, ref = split_case(pkg, oracle, 408)
+    ws = op.workspace[:op.workspace.numel() // 4 * 4].view(torch.float32)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert op.forward(side) == 0
+        side.synchronize()
+        eager = dev.output.clone()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            assert op.forward(side) == 0
+            assert op.forward(side) == 0
+        for rep in range(3):
+            dev.output.fill_(float("nan"))
+            ws.fill_(float("nan"))
+            graph.replay()
+            side.synchronize()
+            assert not torch.isnan(ws[parts // 4:]).all()
+            assert torch.equal(dev.output.view(torch.int16), eager.view(torch.int16)), "replay %d" % rep
+            assert op.forward(side) == 0
+            side.synchronize()
+    assert_attention_close(eager.float().cpu().numpy(), ref, "eager rows")

@@ -162,15 +162,49 @@ def test_hip_linear_strided_rows_and_attention_hand_off(pkg, oracle, m):
     assert_close(out.cpu().numpy(), a, w, None, "attention output in place")
 
 
+# (M, N, K) and the kernel (1 = stream, 2 = tile), tile (columns, rows) and k ranges that serve it with a workspace on 256 CUs: one
+# for every tile, with rows, columns and k that are no multiples of it; every tile that takes several k ranges, with a
+# number of pipeline stages that the ranges do not divide; weights that carry the non-temporal hint
+PLANS = [
+    ((5, 8208, 4160), (1, 16, 16, 1)), ((33, 2064, 4160), (1, 32, 32, 1)), ((37, 4112, 4096), (1, 32, 64, 1)),
+    ((129, 4112, 4160), (1, 64, 64, 1)),                                     # 65 k pieces for four waves
+    ((129, 4112, 576), (2, 64, 64, 1)), ((333, 4112, 1056), (2, 128, 64, 1)), ((1000, 2576, 4128), (2, 128, 128, 1)),
+    ((640, 4112, 14368), (2, 256, 256, 4)), ((2049, 4112, 1056), (2, 256, 256, 1)),
+    ((16, 1024, 8256), (1, 16, 16, 4)), ((20, 4096, 14400), (1, 32, 32, 2)), ((40, 4096, 14400), (1, 64, 64, 4)),
+    ((80, 4096, 14400), (1, 64, 64, 2)), ((129, 32, 4064), (2, 64, 64, 4)), ((70, 2064, 8224), (2, 128, 64, 4)),
+    ((600, 2064, 8224), (2, 128, 128, 2)), ((257, 4112, 14336), (2, 256, 128, 4)),
+]
+
+
+@pytest.mark.parametrize("shape,want", PLANS)
+def test_plan_of_the_tile_edges(pkg, hip_lib, shape, want):
+    """Changed constants would move these shapes to other kernels, and the test below with them."""
+    m, n, k = shape
+    p = pkg.ops.row_parallel_linear_plan(m, k, n, cus=256)
+    assert (p.kernel, p.tile_n, p.tile_m, p.k_ranges) == want
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("shape", [
-    # one for every tile, with rows, columns and k that are no multiples of it: 32 x 64, 64 x 64 (65 k pieces for four
-    # waves; few k on the shared ring), 128 x 64, 128 x 128, 256 x 128 in four k ranges, 256 x 256, and weights that carry the non-temporal hint
-    (37, 4112, 4096), (129, 4112, 4160), (129, 4112, 576), (333, 4112, 1056), (1000, 2576, 4128), (257, 4112, 14336), (2049, 4112, 1056),
-    (5, 8208, 4160)])
-def test_hip_linear_tile_edges(pkg, oracle, shape):
-    """float32 sums in another order than the oracle's and one rounding to half, as above."""
+@pytest.mark.parametrize("shape,want", PLANS)
+def test_hip_linear_tile_edges(pkg, oracle, shape, want):
+    """float32 sums in another order than the oracle's and one rounding to half, as above; and the partial tiles of several k
+    ranges are added in a fixed order: the same call twice gives the same bits."""
+    import torch
+    m, n, k = shape
+    p = pkg.ops.row_parallel_linear_plan(m, k, n)
+    assert (p.kernel, p.tile_n, p.tile_m, p.k_ranges) == want
     test_hip_linear_matches_oracle(pkg, oracle, shape)
+    if p.k_ranges > 1:
+        rng = np.random.default_rng(m)
+        a, w, b = (torch.from_numpy(x).cuda() for x in draw(rng, m, n, k))
+        outs = []
+        for fill in (float("nan"), 1.0):
+            ws = torch.full((p.workspace_size // 4,), fill, dtype=torch.float32, device="cuda")
+            outs.append(torch.empty((m, n), dtype=torch.float16, device="cuda"))
+            pkg.ops.row_parallel_linear(a, w, b, outs[-1], workspace=ws)
+            torch.cuda.synchronize()
+            assert not (ws == 1.0).all() and not torch.isnan(ws).all()  # the partial tiles went through it
+        assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
 
 
 @pytest.mark.gpu
