@@ -481,13 +481,16 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(const LinearLaunch a
 // beats its weights at 5.7 TB/s.  The constants are a fit to 1800 timings (nine tiles x 1, 2 and 4 ranges x M = 1 .. 6000 on
 // seven weight shapes from 2048 x 2048 to 4096 x 14336): the tile that the estimate picks takes 1.01 times what the best one
 // takes in the mean, 1.15 at worst.
-// More than one k range costs the caller a workspace, so it has to be worth it: its estimate beats the best one-range tile's by 5 %
-// (over those shapes that gives up gains below the model's own error), and the partial tiles take at most 256 MiB, what the
-// memory-side cache holds between the launch that writes them and the one that adds them.  (Without the two bounds prompts asked for
-// up to 700 MB, (3472, 14336, 14336) for 398 MB of them at an estimate of 1360.2 against 1360.6 us.)
+// More than one k range costs the caller a workspace.  Up to 16 MiB of partial tiles, a decode step's, are taken for any gain in
+// the estimate; more have to be worth it by 5 %, and they take at most 256 MiB, what the memory-side cache holds between the
+// launch that writes them and the one that adds them.  (Without these bounds prompts asked for up to 700 MB, (3472, 14336, 14336)
+// for 398 MB of them at an estimate of 1360.2 against 1360.6 us.)  Measured with the split against without, estimates less than
+// 5 % apart: (2187, 4096, 14336) 143 MB 358 against 298 us, (343, 8192, 8192) 45 MB 79 against 68, (925, 5120, 5120) 38 MB
+// 76 against 73; below 16 MiB it goes either way: (33, 8192, 8192) 24.8 against 28.5, (231, 6144, 4096) 25.8 against 27.3,
+// (91, 8192, 8192) 36.5 against 27.7.
 namespace {
 constexpr float kLinearSplitGain = 0.05f;
-constexpr int64_t kLinearSplitBytes = (int64_t)256 << 20;
+constexpr int64_t kLinearSplitFreeBytes = (int64_t)16 << 20, kLinearSplitBytes = (int64_t)256 << 20;
 struct LinearTile {
     LinearKernel kernel;
     int tn, tm;
@@ -512,7 +515,7 @@ LinearChoice linear_choose(int64_t m, int64_t n, int64_t k, int compute_units, i
 {
     const int64_t cus = compute_units > 0 ? compute_units : 256;
     if (workspace_bytes > kLinearSplitBytes) workspace_bytes = kLinearSplitBytes;
-    LinearChoice one, split;
+    LinearChoice one, split; // the best of one k range or a small workspace; the best of the others
     const float stream_us = 2.f + (float)n * (float)k * 2.f / 5.7e6f;
     for (int i = 0; i < kLinearTileCount; ++i) {
         const LinearTile& c = kLinearTiles[i];
@@ -528,7 +531,8 @@ LinearChoice linear_choose(int64_t m, int64_t n, int64_t k, int compute_units, i
             float us = (float)rounds * (c.start_us + (float)(per * unit) * c.ns_per_k * 1e-3f);
             if (s > 1) us += 4.f + (float)s * (float)m * (float)n * 8.f / 5.5e6f;
             us = fmaxf(us, stream_us) + 0.1f * fminf(us, stream_us); // what overlaps the stream still shows a little
-            LinearChoice& best = s > 1 ? split : one;
+            const bool large = s > 1 && s * m * n * (int64_t)sizeof(float) > kLinearSplitFreeBytes;
+            LinearChoice& best = large ? split : one;
             if (best.tile < 0 || us < best.us) {
                 best.tile = i;
                 best.splits = s;
