@@ -25,6 +25,7 @@ so nothing of a layer's cache is left in the 256 MB memory-side cache when its t
 the figure of the regime in which every call re-reads one layer, for comparison.
 """
 import argparse
+import itertools
 import json
 import os
 import sys
@@ -471,18 +472,24 @@ def main():
         stages["prefill"] = time_stage(lambda: layer_ops[next_layer()].forward_prefill(stream), n_ev)
 
     # the projection behind the attention (single-rank row_parallel_linear) on this step's decode rows: a square
-    # weight of (heads * head_dim)^2 halves, streamed once per call
+    # weight of (heads * head_dim)^2 halves, streamed once per call.  As with the cache, call i takes matrix i mod n: in a model the
+    # other layers' weights pass between two calls on one matrix, and 512 MB of them leave nothing of it in the memory-side cache
     hidden = bt.num_heads * bt.head_dim
-    w_proj = (torch.randn((hidden, hidden), device="cuda") * hidden ** -0.5).to(torch.float16)
+    w_projs = [(torch.randn((hidden, hidden), device="cuda") * hidden ** -0.5).to(torch.float16)
+               for _ in range(min(256, -(-(512 << 20) // (2 * hidden * hidden))))]
+    proj_turn = itertools.cycle(w_projs)
     proj_in = dev.output[:bt.decoding_batches]
     proj_out = torch.empty((bt.decoding_batches, hidden), dtype=torch.float16, device="cuda")
     proj_ws_bytes = ops.row_parallel_linear_workspace_size(bt.decoding_batches, hidden, hidden)
     proj_ws = torch.empty(proj_ws_bytes, dtype=torch.uint8, device="cuda") if proj_ws_bytes else None
-    stages["o_proj"] = time_stage(lambda: ops.row_parallel_linear(proj_in, w_proj, None, proj_out, workspace=proj_ws), n_ev)
-    proj_replays = None
+    stages["o_proj"] = time_stage(lambda: ops.row_parallel_linear(proj_in, next(proj_turn), None, proj_out, workspace=proj_ws), n_ev)
+    proj_replays = proj_same_replays = None
     if not args.eager:
         try:
-            proj_replays = replay_times(lambda st: ops.row_parallel_linear(proj_in, w_proj, None, proj_out, workspace=proj_ws, stream=st))
+            proj_replays = replay_times(lambda st: ops.row_parallel_linear(proj_in, next(proj_turn), None, proj_out,
+                                                                           workspace=proj_ws, stream=st))
+            proj_same_replays = replay_times(lambda st: ops.row_parallel_linear(proj_in, w_projs[0], None, proj_out,
+                                                                                workspace=proj_ws, stream=st))
         except Exception:
             torch.cuda.synchronize()
 
@@ -561,11 +568,16 @@ def main():
                              "kernel_us": same_k, "kernel_frac": dec_bytes / same_k / 1e3 / HBM_PEAK_GBS}
     proj_us = float(np.mean(proj_replays)) if proj_replays else stages["o_proj"]["avg_us"]
     proj_bytes = hidden * hidden * 2
-    out["o_proj"] = {"kernel": "stream_linear_kernel + linear_reduce_kernel" if proj_ws_bytes else "stream_linear_kernel", "rows": int(bt.decoding_batches), "in_features": hidden,
-                     "out_features": hidden, "bound": "hbm", "weight_bytes": proj_bytes, "kernel_us": proj_us,
+    proj_plan = ops.row_parallel_linear_plan(bt.decoding_batches, hidden, hidden)
+    out["o_proj"] = {"kernel": ["skinny_linear_kernel", "stream_linear_kernel", "tile_linear_kernel"][proj_plan.kernel] +
+                               (" + linear_reduce_kernel" if proj_plan.k_ranges > 1 else ""),
+                     "rows": int(bt.decoding_batches), "in_features": hidden, "out_features": hidden, "bound": "hbm",
+                     "weights": "call i on matrix i mod %d" % len(w_projs), "weight_bytes": proj_bytes, "kernel_us": proj_us,
                      "achieved": proj_bytes / (proj_us * 1e-6) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": proj_bytes / (proj_us * 1e-6) / 1e9 / HBM_PEAK_GBS,
                      "kernel_us_launch_loop": stages["o_proj"]["avg_us"],
+                     "kernel_us_same_weights": float(np.mean(proj_same_replays)) if proj_same_replays else None,
+                     "note_same_weights": "every call on one matrix, which then stays in the memory-side cache: bound by filling LDS",
                      "note": "not part of `value`: the step after the layer call, timed on its own"}
     if "prefill" in stages:
         fl = bt.prefill_flops()
