@@ -342,9 +342,11 @@ __global__ __launch_bounds__(kPrefillThreads, WPS) void prefill_attention_kernel
     for (int item = blockIdx.x / (int)a.num_kv_heads;; item += item_stride) {
     int b_pick = 0, tile_pick = 0;
     // The look-up below depends on nothing that changes from item to item but `item`; its lane masks and addresses, computed
-    // once ahead of the loop, would sit in registers that the tile loop does not have.
+    // once ahead of the loop, would sit in registers that the tile loop does not have (12 prompts of 512 rows over 1500, 32 q / 8 kv
+    // heads of 128: 424 -> 418 us, one of 300 over 200: 40.2 -> 39.0).  With mask or alibi over pages of the narrow heads the
+    // schedule that follows is the worse one (64: 408 against 413 us, 96: 469.7 against 472.5).
     int pick_lane = lane;
-    asm volatile("" : "+v"(pick_lane));
+    if constexpr (SPLIT || !(PAGED && EXTRA && D < 128)) asm volatile("" : "+v"(pick_lane));
     int64_t cut_from = 0, cut_to = 0, weight = 0; // SPLIT: the part of the tile, in stream positions behind its start
     int slot = 0;                                 // SPLIT: the range's first part or a later one
     bool split = false;
@@ -930,10 +932,10 @@ __global__ __launch_bounds__(kPrefillThreads, D <= 128 ? 4 : 2) void prefill_att
     int64_t u_next = -1; // SPLIT: where in the stream the range's next part starts (-1: not yet known)
     for (int item = blockIdx.x / (int)a.num_kv_heads;; item += item_stride) {
     int b_pick = 0, tile_pick = 0;
-    // The look-up below depends on nothing that changes from item to item but `item`; its lane masks and addresses, computed
-    // once ahead of the loop, would sit in registers that the tile loop does not have.
+    // (as in the kernel above: 12 prompts of 512 rows over 1500, 16 q / 8 kv heads of 256, alibi: 626 -> 621 us; over the step's half
+    // rows 97 -> 91; without extra terms from the cache the tile loop is the slower one with it: 525 against 535)
     int pick_lane = lane;
-    asm volatile("" : "+v"(pick_lane));
+    if constexpr (SPLIT || EXTRA || KV16) asm volatile("" : "+v"(pick_lane));
     int64_t cut_from = 0, cut_to = 0, weight = 0; // SPLIT: the part of the tile, in stream positions behind its start
     int slot = 0;                                 // SPLIT: the range's first part or a later one
     bool split = false;
