@@ -211,7 +211,13 @@ __global__ __launch_bounds__(kQuantThreads) void kv_quantize_kernel(const QuantL
 // angle = inv * float(pos) (linear scaling: inv * (float(pos) / factor)); cos and sin are those of the
 // binary32 angle, correctly rounded to binary32 (evaluated in binary64).  The reference evaluates the
 // same formula with the approximate __powf / __sincosf intrinsics.
-template <bool PAGED>
+//
+// LOOP: the launch has fewer workgroups than the step may have tokens (launch_rope) and they walk the tokens in turn; without it
+// every token has its workgroup and the code of a turn stands alone.  DIVIDE: a unit's token and head by integer divisions,
+// where the reciprocals are not exact.  Neither is decided in the kernel: at decode sizes what it waits for is
+// its own instructions on their way from memory, and with both in one kernel a step of few heads took a fifth longer (8 / 8 heads of 64,
+// 128 decode sequences, fused 5.2 us in a replayed graph, 4.3 apart; 32 / 8 of 128 5.5 and 5.0; the mixed step 39.1 and 38.6).
+template <bool PAGED, bool LOOP, bool DIVIDE>
 __global__ __launch_bounds__(kQuantThreads) void rope_append_kernel(const RopeLaunch a)
 {
     // a workgroup takes as many consecutive tokens as its threads can compute coefficients for in one go
@@ -224,7 +230,7 @@ __global__ __launch_bounds__(kQuantThreads) void rope_append_kernel(const RopeLa
     const bool append = a.cache != nullptr;
     for (int64_t tok0 = (int64_t)blockIdx.x * tokens_per_wg; tok0 < n_tokens; tok0 += (int64_t)gridDim.x * tokens_per_wg) {
     int thread = threadIdx.x;
-    asm volatile("" : "+v"(thread));
+    if constexpr (LOOP) asm volatile("" : "+v"(thread)); // (nothing that depends on it is held from turn to turn)
 
     // the rows of this workgroup's tokens, as units of 8 channels: the query heads' groups, and the key heads' (a key unit
     // also carries the same group of V when the step appends)
@@ -241,12 +247,11 @@ __global__ __launch_bounds__(kQuantThreads) void rope_append_kernel(const RopeLa
         int tl, h, d0;
         int64_t in_tok, idx;
     };
-    // (the quotient by a multiplication where the launcher found it exact for every unit of a workgroup)
     auto unit_of = [&](int w, int per_token, uint32_t magic) -> Unit {
         Unit r;
-        r.tl = magic ? (int)__umulhi((uint32_t)w, magic) : w / per_token;
+        r.tl = DIVIDE ? w / per_token : (int)__umulhi((uint32_t)w, magic);
         const int u = w - r.tl * per_token;
-        r.h = magic ? (int)__umulhi((uint32_t)u, a.gph_magic) : u / gph;
+        r.h = DIVIDE ? u / gph : (int)__umulhi((uint32_t)u, a.gph_magic);
         r.d0 = (u - r.h * gph) << 3;
         r.in_tok = first + tok0 + r.tl;
         r.idx = (int64_t)u << 3;
@@ -255,10 +260,13 @@ __global__ __launch_bounds__(kQuantThreads) void rope_append_kernel(const RopeLa
     // Units beyond the work load the last unit's rows: every load of a batch is issued whatever the remainder, so that
     // the wait for a batch leaves the next one in flight.
     constexpr int kQueries = 3; // query units per thread and batch; key units one
+    // The query units start at the wave behind the last key unit's: a token of few heads has its query and key units in different
+    // waves (8 / 1 heads of 128, 128 decode sequences, fused: 4.7 us where they share one, 4.4 so).
+    const int q_thread = (thread - ((k_work + kWave - 1) & ~(kWave - 1))) & (kQuantThreads - 1);
     auto load_queries = [&](int w0, u32x4 (&rows)[kQueries]) {
 #pragma unroll
         for (int j = 0; j < kQueries; ++j) {
-            const int w = w0 + (int)thread + j * kQuantThreads;
+            const int w = w0 + q_thread + j * kQuantThreads;
             const Unit r = unit_of(w < q_work ? w : q_work - 1, q_units, a.q_magic);
             rows[j] = *(const u32x4*)((const half_t*)a.query + r.in_tok * a.query_stride_s + r.idx);
         }
@@ -395,15 +403,16 @@ __global__ __launch_bounds__(kQuantThreads) void rope_append_kernel(const RopeLa
         u32x4 next[kQueries];
         load_queries(w0 + kQueries * kQuantThreads, next);
 #pragma unroll
-        for (int j = 0; j < kQueries; ++j) finish_query(w0 + (int)thread + j * kQuantThreads, q_row[j]);
+        for (int j = 0; j < kQueries; ++j) finish_query(w0 + q_thread + j * kQuantThreads, q_row[j]);
 #pragma unroll
         for (int j = 0; j < kQueries; ++j) q_row[j] = next[j];
     }
 #pragma unroll
     for (int j = 0; j < kQueries; ++j) {
-        const int w = w0 + (int)thread + j * kQuantThreads;
+        const int w = w0 + q_thread + j * kQuantThreads;
         if (w < q_work) finish_query(w, q_row[j]);
     }
+    if constexpr (!LOOP) return;
     __syncthreads(); // the next tokens' coefficients overwrite these
     }
 }
@@ -440,22 +449,34 @@ int launch_rope(const RopeLaunch& a_in, int compute_units, hipStream_t stream)
     const int64_t spread = a.max_tokens / (2 * (int64_t)(compute_units > 0 ? compute_units : 256));
     if (tokens_per_wg > spread) tokens_per_wg = spread > 1 ? (int)spread : 1;
     a.tokens_per_wg = tokens_per_wg;
-    // n / d = mulhi(n, floor(2^32 / d) + 1) for n d < 2^32 and d >= 2
+    // n / d = mulhi(n, floor(2^32 / d) + 1) for n d < 2^32 and d >= 2: exact for every unit of a workgroup, or divide
     const uint64_t gph = (uint64_t)(a.head_dim >> 3);
+    bool exact = gph >= 2;
     auto magic = [&](uint64_t per_token) -> uint32_t {
-        const bool exact = gph >= 2 && per_token > 0 && per_token < (1u << 16) && (uint64_t)tokens_per_wg * per_token * per_token < (1ull << 32);
-        return exact ? (uint32_t)((1ull << 32) / per_token + 1) : 0;
+        if (per_token == 0) return 0; // (no such unit)
+        if (per_token >= (1u << 16) || (uint64_t)tokens_per_wg * per_token * per_token >= (1ull << 32)) exact = false;
+        return (uint32_t)((1ull << 32) / per_token + 1);
     };
     a.q_magic = magic((uint64_t)a.num_heads * gph);
     a.k_magic = magic((uint64_t)a.num_key_heads * gph);
-    a.gph_magic = gph >= 2 ? (uint32_t)((1ull << 32) / gph + 1) : 0;
-    // max_tokens is batch * max_seqlen, in a mixed step many times the rows there are: as many workgroups as the chip holds at
-    // once, which walk the tokens in turn
+    a.gph_magic = magic(gph);
+    // max_tokens is batch * max_seqlen, in a mixed step many times the rows there are: about as many workgroups as the chip holds
+    // at once (67 vector registers: seven per CU) walk the tokens in turn.  Seven, eight or fourteen per CU measure the same
+    // (mixed step 43.1 us over one set of rows).
     int64_t blocks = (a.max_tokens + tokens_per_wg - 1) / tokens_per_wg;
     const int64_t resident = 8 * (int64_t)(compute_units > 0 ? compute_units : 256);
-    if (blocks > resident) blocks = resident;
-    if (a.cache_mode == 1) hipLaunchKernelGGL(rope_append_kernel<true>, dim3((unsigned)blocks), dim3(kQuantThreads), 0, stream, a);
-    else hipLaunchKernelGGL(rope_append_kernel<false>, dim3((unsigned)blocks), dim3(kQuantThreads), 0, stream, a);
+    const bool loop = blocks > resident;
+    if (loop) blocks = resident;
+    const dim3 grid((unsigned)blocks);
+#define PMX_ROPE(LOOP, DIVIDE) \
+    do { \
+        if (a.cache_mode == 1) hipLaunchKernelGGL((rope_append_kernel<true, LOOP, DIVIDE>), grid, dim3(kQuantThreads), 0, stream, a); \
+        else hipLaunchKernelGGL((rope_append_kernel<false, LOOP, DIVIDE>), grid, dim3(kQuantThreads), 0, stream, a); \
+    } while (0)
+    if (!exact) PMX_ROPE(true, true);
+    else if (loop) PMX_ROPE(true, false);
+    else PMX_ROPE(false, false);
+#undef PMX_ROPE
     return kLaunchOk;
 }
 

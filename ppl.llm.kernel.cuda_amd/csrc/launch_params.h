@@ -173,7 +173,7 @@ struct RopeLaunch {
     float inv_freq[128];
     int32_t has_inv_freq;
     int32_t tokens_per_wg;      // consecutive tokens one workgroup takes, at most 256 / (head_dim / 2)
-    uint32_t q_magic, k_magic, gph_magic; // reciprocals of a token's query and key units and of a head's groups; 0 = divide
+    uint32_t q_magic, k_magic, gph_magic; // reciprocals of a token's query and key units and of a head's groups
     // append part (same meaning as QuantLaunch)
     int8_t* cache;
     void* scale;

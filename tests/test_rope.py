@@ -153,6 +153,15 @@ def test_gpu_rope_many_sequences(pkg, oracle, shape, n_dec, n_prefill):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(8, 1, 128), (1, 1, 64), (14, 2, 64), (3, 1, 96), (5, 2, 16), (40, 40, 128), (64, 8, 128), (2100, 2, 256)])
+@pytest.mark.parametrize("n_dec,n_prefill", [(5, 3), (30, 0)])
+def test_gpu_rope_units_of_few_and_many_heads(pkg, oracle, shape, n_dec, n_prefill):
+    """Key units that fill part of a wave, one wave and several, with the query units in the waves behind them; the last shape
+    has more units per token than the reciprocals serve."""
+    test_gpu_rope_many_sequences(pkg, oracle, shape, n_dec, n_prefill)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shape", [(71, 1, 64), (48, 1, 128), (3, 3, 96), (16, 8, 256), (5, 2, 8)])
 def test_gpu_rope_several_tokens_per_workgroup(pkg, oracle, shape):
     """Steps whose workgroups take several tokens, and several such groups in turn, with units that fill no whole number of
