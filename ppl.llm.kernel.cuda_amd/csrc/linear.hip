@@ -61,7 +61,7 @@ __device__ __forceinline__ f16x4 finish4(const f32x4 v, const void* bias, int64_
 // ---- any row stride: a workgroup owns 16 output columns and up to 128 rows, fragments straight from memory --------------
 // Eight waves take the 32-wide k steps in turn (adjacent 64-byte pieces of a weight row), keep the weight requests four
 // steps ahead and the input requests two, and add their partial tiles through LDS at the end, in a fixed order.
-// It runs only where the rows of an operand lie 2^23 halves or more apart; with ordinary strides the input that every
+// It runs where the rows of an operand lie 2^23 halves or more apart, and on few long rows without workspace (linear_choose); with ordinary strides the input that every
 // workgroup re-reads (M * K * 2 bytes) makes it 42 us on (128, 4096, 4096), where stream_linear_kernel takes 11.6.
 __global__ __launch_bounds__(kLinThreads) void skinny_linear_kernel(const LinearLaunch a)
 {
@@ -540,7 +540,12 @@ LinearChoice linear_choose(int64_t m, int64_t n, int64_t k, int compute_units, i
             }
         }
     }
-    return split.tile >= 0 && split.us < one.us * (1.f - kLinearSplitGain) ? split : one;
+    const LinearChoice best = split.tile >= 0 && split.us < one.us * (1.f - kLinearSplitGain) ? split : one;
+    // Long rows of an odd number of 32 k have no tile of the streaming kernel; where a caller without workspace leaves a few of the large
+    // tiles to walk them alone, the 16-column form has more workgroups: (1, 2064, 4128) 16.3 against 17.3 us, (8, 512, 8224) 25.9 against
+    // 30.7, (16, 2560, 14368) 49.1 against 51.7.  With 32 rows, 3072 columns or 2080 k it is level or behind.
+    if (best.splits == 1 && k % 64 != 0 && k >= 4096 && m <= 16 && n / kLinCols * 8 <= 5 * cus) return LinearChoice();
+    return best;
 }
 } // namespace
 

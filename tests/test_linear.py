@@ -187,6 +187,23 @@ def test_plan_of_the_tile_edges(pkg, hip_lib, shape, want):
     assert (p.kernel, p.tile_n, p.tile_m, p.k_ranges) == want
 
 
+@pytest.mark.parametrize("shape,kernel", [((1, 2064, 4128), 0), ((16, 2560, 14368), 0), ((17, 2560, 14368), 2), ((16, 2576, 14368), 2),
+                                          ((8, 512, 4064), 2), ((8, 512, 8192), 1)])
+def test_plan_without_workspace(pkg, hip_lib, shape, kernel):
+    """Few long rows of an odd number of 32 k: the 16-column form, at the edges of its rule; with a workspace the k range is split."""
+    m, n, k = shape
+    assert pkg.ops.row_parallel_linear_plan(m, k, n, workspace_size=0, cus=256).kernel == kernel
+    if kernel == 0:
+        assert pkg.ops.row_parallel_linear_plan(m, k, n, cus=256).k_ranges > 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 2064, 4128), (16, 2560, 14368), (7, 16, 4128)])
+def test_hip_linear_few_long_rows(pkg, oracle, shape):
+    """... whose sums are the oracle's within the same tolerance, with the workspace and without."""
+    test_hip_linear_matches_oracle(pkg, oracle, shape)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape,want", PLANS)
 def test_hip_linear_tile_edges(pkg, oracle, shape, want):
