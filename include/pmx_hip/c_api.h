@@ -517,7 +517,7 @@ PMXHIP_API int pmxhip_rope_kv_cache_quantize(const pmxhip_rope_params* rope, con
  * K * N * 2 weight bytes), one for the query rows of prompts (compute-bound); they allocate nothing and add
  * their partial sums in a fixed order, so a call's result does not depend on timing.
  * workspace: where that is estimated to be faster (a long K, and tiles that fill the CUs badly: too few of them, or a last
- * round with few; by at least 5 % if it takes more than 16 MiB), the k range is split over 2 or 4 workgroups whose float32 partial tiles pass through `workspace`
+ * round with few; by at least 5 % if it takes more than 32 MiB), the k range is split over 2 or 4 workgroups whose float32 partial tiles pass through `workspace`
  * (the role of the reference's cublas_workspace argument) and are added in a fixed order by a second kernel.
  * pmxhip_row_parallel_linear_workspace_size gives the bytes that serve (M, in_features, out_features) on the
  * current device: 0 = none needed, at most 256 MiB; with a NULL or smaller workspace the call still computes the same function,

@@ -481,16 +481,15 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(const LinearLaunch a
 // beats its weights at 5.7 TB/s.  The constants are a fit to 1800 timings (nine tiles x 1, 2 and 4 ranges x M = 1 .. 6000 on
 // seven weight shapes from 2048 x 2048 to 4096 x 14336): the tile that the estimate picks takes 1.01 times what the best one
 // takes in the mean, 1.15 at worst.
-// More than one k range costs the caller a workspace.  Up to 16 MiB of partial tiles, a decode step's, are taken for any gain in
-// the estimate; more have to be worth it by 5 %, and they take at most 256 MiB, what the memory-side cache holds between the
-// launch that writes them and the one that adds them.  (Without these bounds prompts asked for up to 700 MB, (3472, 14336, 14336)
-// for 398 MB of them at an estimate of 1360.2 against 1360.6 us.)  Measured with the split against without, estimates less than
-// 5 % apart: (2187, 4096, 14336) 143 MB 358 against 298 us, (343, 8192, 8192) 45 MB 79 against 68, (925, 5120, 5120) 38 MB
-// 76 against 73; below 16 MiB it goes either way: (33, 8192, 8192) 24.8 against 28.5, (231, 6144, 4096) 25.8 against 27.3,
+// More than one k range costs the caller a workspace.  Up to 32 MiB of partial tiles are taken for any gain in the estimate; more
+// have to be worth it by 5 %, and they take at most 256 MiB, what the memory-side cache holds between the launch that writes
+// them and the one that adds them.  (Without these bounds prompts asked for up to 700 MB, (3472, 14336, 14336) for 398 MB of
+// them at an estimate of 1360.2 against 1360.6 us.)  Measured with the split against without, estimates less than 5 % apart: (2187, 4096, 14336) 143 MB 358 against 298 us, (343, 8192, 8192) 45 MB 79 against 68, (925, 5120, 5120) 38 MB
+// 76 against 73; below 32 MiB it goes either way: (33, 8192, 8192) 24.8 against 28.5, (300, 4096, 14336) 58.4 against 63.5,
 // (91, 8192, 8192) 36.5 against 27.7.
 namespace {
 constexpr float kLinearSplitGain = 0.05f;
-constexpr int64_t kLinearSplitFreeBytes = (int64_t)16 << 20, kLinearSplitBytes = (int64_t)256 << 20;
+constexpr int64_t kLinearSplitFreeBytes = (int64_t)32 << 20, kLinearSplitBytes = (int64_t)256 << 20;
 struct LinearTile {
     LinearKernel kernel;
     int tn, tm;

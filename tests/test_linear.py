@@ -72,11 +72,11 @@ def test_c_entry_point_rejects_bad_arguments_without_launching(pkg, hip_lib):
 
 def test_k_ranges_are_worth_their_workspace(pkg, hip_lib):
     """Whatever the shape, a call asks for at most 256 MiB of partial tiles, and prompts whose tiles fill the chip for none: more
-    than 16 MiB have to be estimated 5 % faster.  With less workspace the plan has fewer ranges, never more than fit."""
+    than 32 MiB have to be estimated 5 % faster.  With less workspace the plan has fewer ranges, never more than fit."""
     plan = pkg.ops.row_parallel_linear_plan
     assert plan(3472, 14336, 14336, cus=256).workspace_size == 0  # 784 tiles of 256 x 256: 1360.2 against 1360.6 us
     assert plan(2187, 14336, 4096, cus=256).workspace_size == 0
-    assert 0 < plan(33, 8192, 8192, cus=256).workspace_size <= 16 << 20
+    assert 0 < plan(33, 8192, 8192, cus=256).workspace_size <= 32 << 20
     splits = 0
     for k, n in [(2048, 2048), (4096, 4096), (8192, 8192), (14336, 4096), (4096, 14336), (14336, 14336), (28672, 8192), (8192, 28672),
                  (1024, 8192), (4128, 4112)]:
@@ -175,7 +175,7 @@ PLANS = [
     ((16, 1024, 8256), (1, 16, 16, 4)), ((20, 4096, 14400), (1, 32, 32, 2)), ((40, 4096, 14400), (1, 64, 64, 4)),
     ((80, 4096, 14400), (1, 64, 64, 2)), ((129, 32, 4064), (2, 64, 64, 4)), ((70, 2064, 8224), (2, 128, 64, 4)),
     ((600, 2064, 8224), (2, 128, 128, 2)), ((200, 4112, 8224), (2, 256, 128, 4)),
-    ((257, 4112, 14336), (2, 128, 128, 2)),
+    ((257, 4112, 14336), (2, 256, 128, 4)),
 ]
 
 
