@@ -203,7 +203,7 @@ __global__ __launch_bounds__(kQuantThreads) void kv_quantize_kernel(const QuantL
 
 // Rotary position embedding of Q and K (interleaved pairs, reference:
 // src/ppl/kernel/llm/cuda/pmx/rotary_position_embedding.cu:35-91, 268-343), optionally fused with the
-// quantise/append above: one workgroup per new token; the cos/sin of the token's position are computed
+// quantise/append above: a workgroup takes a few consecutive tokens; the cos/sin of a token's position are computed
 // once per pair (not once per head) and shared through LDS; a lane then rotates one group of 8 channels
 // of a query head, or rotates and quantises the same group of K and quantises that of V.
 //

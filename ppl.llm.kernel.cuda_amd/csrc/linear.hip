@@ -161,8 +161,11 @@ __global__ __launch_bounds__(kLinThreads) void skinny_linear_kernel(const Linear
 // own ring of NS stages and waits for nothing but its own requests.  LDS rows are 128 bytes without padding (the DMA
 // writes lane i at 16 i); the 16-byte chunk c of row r lies in slot c ^ ((r >> 1) & 7), so that the fragment reads of
 // sixteen rows cover all 64 banks.  The four partial tiles meet in LDS and are added in wave order.
-// NT: the weights carry the non-temporal hint (one row tile, so every weight byte is used once; worth it only where the
-// weights do not stay in the 256 MB memory-side cache: 134 MB 25.6 against 29 us, 33 MB 7.4 against 7.0).
+// NT: the weights carry the non-temporal hint (one row tile, so every weight byte is used once).  It pays where the weights come
+// from memory, and costs where they wait in the 256 MB memory-side cache.  One row, microseconds with the hint / without,
+// calls that take 600 MB of matrices in turn (a model's layers) and calls on one matrix: 134 MB 25.2 / 28.9 and 23.5 / 22.0,
+// 117 MB 22.1 / 25.3 and 20.8 / 19.3, 52 MB 14.0 / 14.5 and 14.1 / 10.6, 50 MB 12.2 / 12.9 and 11.2 / 10.3, 33 MB 7.7 / 7.7 and
+// 5.5 / 5.2, with 32 rows 13.2 / 12.2 and 10.2 / 9.1: on from 64 MB.
 // Against the form with fragments loaded into registers that this replaces: (1, 4096, 4096) 10.3 -> 7.0 us, (16, 4096,
 // 4096) 10.9 -> 7.9, (128, 4096, 4096) 22.2 -> 11.6, (32, 8192, 8192) 36.7 -> 24.5, (32, 5120, 5120) 25.6 -> 11.0.
 constexpr int kStreamWaves = 4;
@@ -298,10 +301,11 @@ __global__ __launch_bounds__(64 * kStreamWaves) void stream_linear_kernel(const 
 // so neither the LDS reads nor the barrier stand between products.  Requests are NS - 1 stages ahead.
 // LDS rows are 64 bytes: chunk c of row r lies in slot c ^ ((r >> 2) & 3) (sixteen rows cover all banks).
 // With 256 x 256 tiles and eight waves a wave has 4 x 2 tiles of 32 x 32: 12 fragment reads per 16 products.
-// Bound by the matrix pipes at the clock the chip holds under them: (4000, 4096, 4096), 256 tiles for 256 CUs, 122 us =
-// 1097 TFLOP/s, the same with 3, 4 or 5 stages, either wave shape and with or without raised wave priority; 8192 in
-// all three 1170 (a large library product reaches 1150-1180 here).  (11104, 4096, 4096), 704 tiles in three rounds: 349 us =
-// 1067 TFLOP/s; the weight-streaming kernel that took these sizes before: 1064 us.
+// (4000, 4096, 4096), 256 tiles for 256 CUs, 122 us = 1097 TFLOP/s, the same with 3, 4 or 5 stages, either wave shape and with
+// or without raised wave priority; 8192 in all three 1170 (a large library product reaches 1150-1180 here).  (11104, 4096, 4096),
+// 704 tiles in three rounds of 256: 355-370 us by box = 1010-1050 TFLOP/s; the weight-streaming kernel that took these sizes before:
+// 1067.  Counters of that call: the matrix pipes are busy for 58 % of the shader cycles (63 % of those in which tiles run), at a
+// clock that falls to 1.75 GHz under them; waves stand at a wait or barrier for 31 % of their time.
 template <int TN, int TM, int WN, int WM, int NS>
 __global__ __launch_bounds__(64 * WN * WM, 2) void tile_linear_kernel(const LinearLaunch a, const int splits, float* __restrict__ partial)
 {
@@ -479,13 +483,13 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(const LinearLaunch a
 // A round of workgroups over the CUs takes a start (prologue and epilogue) plus its k length times a cost per k; a split adds
 // the partial tiles' way through memory and a second launch (4 us + 8 bytes per element and range at 5.5 TB/s); no call
 // beats its weights at 5.7 TB/s.  The constants are a fit to 1800 timings (nine tiles x 1, 2 and 4 ranges x M = 1 .. 6000 on
-// seven weight shapes from 2048 x 2048 to 4096 x 14336): the tile that the estimate picks takes 1.01 times what the best one
-// takes in the mean, 1.15 at worst.
+// seven weight shapes from 2048 x 2048 to 4096 x 14336, repeated calls on one matrix, which the memory-side cache held): the tile
+// that the estimate picks takes 1.01 times what the best one takes in the mean, 1.15 at worst.
 // More than one k range costs the caller a workspace.  Up to 32 MiB of partial tiles are taken for any gain in the estimate; more
 // have to be worth it by 5 %, and they take at most 256 MiB, what the memory-side cache holds between the launch that writes
 // them and the one that adds them.  (Without these bounds prompts asked for up to 700 MB, (3472, 14336, 14336) for 398 MB of
-// them at an estimate of 1360.2 against 1360.6 us.)  Measured with the split against without, estimates less than 5 % apart: (2187, 4096, 14336) 143 MB 358 against 298 us, (343, 8192, 8192) 45 MB 79 against 68, (925, 5120, 5120) 38 MB
-// 76 against 73; below 32 MiB it goes either way: (33, 8192, 8192) 24.8 against 28.5, (300, 4096, 14336) 58.4 against 63.5,
+// them at an estimate of 1360.2 against 1360.6 us.)  Measured with the split against without, estimates less than 5 % apart:
+// (2187, 4096, 14336) 143 MB 358 against 298 us, (343, 8192, 8192) 45 MB 79 against 68, (925, 5120, 5120) 38 MB 76 against 73; below 32 MiB it goes either way: (33, 8192, 8192) 24.8 against 28.5, (300, 4096, 14336) 58.4 against 63.5,
 // (91, 8192, 8192) 36.5 against 27.7.
 namespace {
 constexpr float kLinearSplitGain = 0.05f;
@@ -579,7 +583,7 @@ int launch_linear(const LinearLaunch& a, int compute_units, void* workspace, int
     const int splits = plan.splits;
     float* const part = (float*)workspace;
     const dim3 grid((unsigned)(((a.n + c.tn - 1) / c.tn) * ((a.m + c.tm - 1) / c.tm) * splits));
-    // one row tile: every weight byte is used once; 64 MB and more of them do not wait in the memory-side cache
+    // one row tile: every weight byte is used once; from 64 MB on the hint pays more than it costs (stream_linear_kernel)
     const bool nt = a.m <= c.tm && a.n * a.k >= ((int64_t)32 << 20);
 #define PMX_STREAM(TN, TM, NS) \
     do { \

@@ -2,7 +2,7 @@
 // reference makes this choice for every call (one cublasLt GEMM,
 // src/ppl/kernel/llm/cuda/pmx/row_parallel_linear.cu:57-81).  hipBLASLt is loaded on first use with dlopen, so the
 // library has no link-time dependency on it; where it is absent (or refuses the shape) the caller runs this
-// build's own kernels (linear.hip: 349 us on 11104 rows of 4096 x 4096, where the library takes 403).
+// build's own kernels (linear.hip: 355-370 us on 11104 rows of 4096 x 4096, where the library takes 403).
 // Host only.
 #include <dlfcn.h>
 

@@ -1392,7 +1392,7 @@ static int launch_prefill_variant(const PrefillLaunch& a, dim3 grid, hipStream_t
         hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, true>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
     else if (D == 64 && SRC == 2 && !EXTRA && grid.x > (unsigned)a.compute_units) {
         // More workgroups than CUs: two per CU cover each other's waits although a few registers spill (32 q / 8 kv heads, 12
-        // prompts of 300-3000 rows: layer call 356 -> 282 us).  With a workgroup per CU or fewer only the spills are left
+        // prompts of 300-3000 rows: layer call 356 -> 287 us).  With a workgroup per CU or fewer only the spills are left
         // (8 / 8 heads, six prompts of 300-1500 rows: 46.9 against 48.7 us).
         if constexpr (D == 64 && SRC == 2 && !EXTRA)
             hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, false, 4>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
