@@ -10,7 +10,7 @@
 //   stream_linear_kernel  decode-sized M: a workgroup owns a small tile of the output over the whole of K, its four waves
 //                         split K between them, each with a ring of its own and no barrier before the end
 //   tile_linear_kernel    from a few hundred rows: a workgroup owns a large tile, its waves share every stage of a common ring
-//   skinny_linear_kernel  rows that lie too far apart for the 32-bit row offsets of the other two
+//   skinny_linear_kernel  rows that lie too far apart for the 32-bit row offsets of the other two, and a few long rows without workspace
 // linear_choose() picks kernel, tile and number of k ranges from a cost per workgroup that was measured for each.
 #include "device_common.h"
 #include "launch_params.h"

@@ -99,7 +99,7 @@ def test_k_ranges_are_worth_their_workspace(pkg, hip_lib):
                                    (128, 14336 // 8, 4096), (3, 4096, 32), (129, 32, 4064), (17, 64, 64), (128, 128, 3136),
                                    (300, 8192, 1024), (5, 64, 2240), (1, 64, 512), (16, 128, 1024), (17, 64, 1536), (33, 192, 2048),
                                    (65, 64, 512), (130, 192, 2048), (240, 4096, 4096),
-                                   # many rows (a prefill chunk's): this library's kernels, 128 rows at a time
+                                   # many rows (a prefill chunk's)
                                    (384, 256, 512), (1000, 512, 1024), (2500, 1024, 2048), (640, 4096, 4096)])
 def test_hip_linear_matches_oracle(pkg, oracle, shape, vendor_gemm=False):
     import torch
