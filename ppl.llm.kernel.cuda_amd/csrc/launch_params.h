@@ -112,6 +112,7 @@ struct PrefillLaunch {
     int64_t key_stride_s;
     int64_t value_stride_s;
     int32_t compute_units;
+    int32_t cols_per_wg;        // (position, head) columns of a workgroup of the 32-column kernel
     // the kv tokens of a tile shared out over workgroups (prefill_split_choose): ranges per kv head, 0 = whole tiles
     int32_t split_ranges;
     int32_t split_gain;         // weight a split has to take off the call before the kernels go by it

@@ -266,8 +266,9 @@ __device__ __forceinline__ int split_cut(int64_t v, int64_t weight, int n_tiles,
 // SPLIT: the launch has one workgroup per range of the split stream (above) instead of one per tile.
 // WPS: waves per SIMD the registers are cut for.  4 (two workgroups per CU) fits head_dim 64 over half K/V rows, whose tiles
 // need no low parts (60 KB of LDS) and whose waves hold half the accumulators; see launch_prefill_variant.
-template <int D, int SRC, bool EXTRA, bool SPLIT, int WPS = 2>
-__global__ __launch_bounds__(kPrefillThreads, WPS) void prefill_attention_kernel(const PrefillLaunch a)
+// NWV: waves of a workgroup, 32 (position, head) columns each; four of them over half K/V rows, see prefill_columns.
+template <int D, int SRC, bool EXTRA, bool SPLIT, int WPS = 2, int NWV = 8>
+__global__ __launch_bounds__(NWV * kWave, WPS) void prefill_attention_kernel(const PrefillLaunch a)
 {
     constexpr bool PAGED = SRC == 0;
     constexpr bool KV16 = SRC == 2;
@@ -278,10 +279,12 @@ __global__ __launch_bounds__(kPrefillThreads, WPS) void prefill_attention_kernel
     constexpr int V_STRIDE = PrefillTile<D>::V_STRIDE; // halves per V row in LDS (row-major, like K)
     // Staging: thread t takes group t % GPT of the tokens t / GPT, t / GPT + K_TSTEP, ...  With 12 groups per row
     // (head_dim 96) the first 384 threads stage 32 tokens per pass and the last two waves stage nothing.
-    constexpr int K_TSTEP = GPT == 12 ? 32 : kPrefillThreads / GPT; // tokens between a thread's units
+    constexpr int THREADS = NWV * kWave;
+    constexpr int COLS = NWV * 32;
+    constexpr int K_TSTEP = GPT == 12 ? THREADS / 16 : THREADS / GPT; // tokens between a thread's units
     constexpr int STAGERS = K_TSTEP * GPT;                           // threads that stage (whole waves)
     constexpr int UNITS = kBN / K_TSTEP;                             // (token, group) units per staging thread, of K and of V each
-    static_assert(STAGERS <= kPrefillThreads && STAGERS % 64 == 0 && UNITS * K_TSTEP == kBN, "staging units");
+    static_assert(STAGERS <= THREADS && STAGERS % 64 == 0 && UNITS * K_TSTEP == kBN, "staging units");
 
     // K is kept as an unevaluated sum hi + lo of two halves: hi = fp16(int8 * scale) and
     // lo = the rounding error of that product (exact, from one fused multiply-add), so that
@@ -311,7 +314,7 @@ __global__ __launch_bounds__(kPrefillThreads, WPS) void prefill_attention_kernel
     const int v_frag_off = (4 * hh + ((lane & 15) >> 2)) * V_STRIDE + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
 
     const int G = (int)(a.num_heads / a.num_kv_heads);
-    const int ppw = kCols / G > 0 ? kCols / G : 1; // query positions per workgroup
+    const int ppw = COLS / G > 0 ? COLS / G : 1; // query positions per workgroup
     const int kvh = blockIdx.x % (int)a.num_kv_heads;
     const int item_stride = gridDim.x / (int)a.num_kv_heads;
 
@@ -1347,14 +1350,14 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillLaunc
     }
 }
 
-template <int D, int SRC>
+template <int D, int SRC, int NWV = 8>
 constexpr size_t prefill_lds_bytes()
 {
     // int8 source: K hi/lo tiles + V hi/lo tiles (above the 64 KB static limit for D = 128, hence dynamic);
-    // fp16 source: one K tile and one V tile; two buffers of each.  The epilogue's staging (eight waves x 32 rows and
+    // fp16 source: one K tile and one V tile; two buffers of each.  The epilogue's staging (NWV waves x 32 rows and
     // their offsets) starts where the second buffer starts and may reach beyond it.
     constexpr size_t tiles = 2 * (SRC == 2 ? 1 : 2) * kBN * (PrefillTile<D>::K_STRIDE + PrefillTile<D>::V_STRIDE) * sizeof(half_t);
-    constexpr size_t with_epilogue = (kEpilogueBase<D, SRC>() + 8 * (32 * (D + 8) + 32 * 4)) * sizeof(half_t);
+    constexpr size_t with_epilogue = (kEpilogueBase<D, SRC>() + NWV * (32 * (D + 8) + 32 * 4)) * sizeof(half_t);
     return tiles > with_epilogue ? tiles : with_epilogue;
 }
 
@@ -1381,6 +1384,11 @@ static int ready_prefill_variant(hipStream_t stream, bool may_capture)
     } else if (int rc = set_dynamic_lds_once((const void*)prefill_attention_kernel<D, SRC, EXTRA, true>, lds_bytes, none)) {
         return rc;
     }
+    if constexpr (SRC == 2) {
+        DeviceMask half{0}; // (a kernel of its own: `none` may have been marked by the call above)
+        if (int rc = set_dynamic_lds_once((const void*)prefill_attention_kernel<D, SRC, EXTRA, false, 2, 4>, (int)prefill_lds_bytes<D, SRC, 4>(), half))
+            return rc;
+    }
     return set_dynamic_lds_once((const void*)prefill_attention_kernel<D, SRC, EXTRA, false>, lds_bytes, ready);
 }
 template <int D, int SRC, bool EXTRA>
@@ -1390,7 +1398,10 @@ static int launch_prefill_variant(const PrefillLaunch& a, dim3 grid, hipStream_t
     if (int rc = ready_prefill_variant<D, SRC, EXTRA>(stream, true)) return rc;
     if (a.split_ranges > 0)
         hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, true>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
-    else if (D == 64 && SRC == 2 && !EXTRA && grid.x > (unsigned)a.compute_units) {
+    else if (SRC == 2 && a.cols_per_wg == 128) {
+        if constexpr (SRC == 2)
+            hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, false, 2, 4>), grid, dim3(256), (prefill_lds_bytes<D, SRC, 4>()), stream, a);
+    } else if (D == 64 && SRC == 2 && !EXTRA && grid.x > (unsigned)a.compute_units) {
         // More workgroups than CUs: two per CU cover each other's waits although a few registers spill (32 q / 8 kv heads, 12
         // prompts of 300-3000 rows: layer call 356 -> 287 us).  With a workgroup per CU or fewer only the spills are left
         // (8 / 8 heads, six prompts of 300-1500 rows: 46.9 against 48.7 us).
@@ -1495,7 +1506,7 @@ template <int D>
 static int launch_prefill_d(const PrefillLaunch& a, hipStream_t stream)
 {
     const int G = (int)(a.num_heads / a.num_kv_heads);
-    const int ppw = kCols / G > 0 ? kCols / G : 1;
+    const int ppw = a.cols_per_wg / G > 0 ? a.cols_per_wg / G : 1;
     // one workgroup per (query tile, kv head) that the batch can have at most; the kernel numbers the real ones first.
     // Every sequence has at most the tiles of max_seqlen; all together at most one per ppw rows plus a partial one each.
     int64_t items = a.prefill_batches * ((a.max_seqlen + ppw - 1) / ppw);
@@ -1554,8 +1565,24 @@ PrefillSplit prefill_split_choose(int64_t sequences, int64_t max_seqlen, int64_t
     return r;
 }
 
-int launch_prefill(const PrefillLaunch& a, hipStream_t stream)
+// Columns of a workgroup of the 32-column kernel.  Over half K/V rows (no dequantisation, so little shared work to lose) four waves
+// of 128 columns do better than eight of 256: two workgroups fit a CU (at most 68 KB of LDS each) and one computes while the other
+// waits at its tile's barriers, and the last tiles of a batch are half as long: 32 q / 8 kv heads of 128, 12 prompts
+// of 300-3000 rows 509 -> 497 us, 64 prompts of 30-150 rows 59 -> 54, with alibi slopes four prompts of
+// 300-2500 rows 239 -> 218; 32 / 32 heads, 26 prompts of 270-336 rows 158 -> 128; one prompt of 1000 rows is level.
+// The int8 cache keeps 256: its tiles, dequantised once per workgroup, take all of a CU's LDS.  So does a group whose heads fill
+// 128 columns worse (48 heads per kv head: 96 of 128, 240 of 256).
+static int prefill_columns(const PrefillLaunch& a)
 {
+    const int64_t g = a.num_heads / a.num_kv_heads;
+    const bool half_rows = a.current_key && a.split_ranges <= 0 && a.head_dim != 256;
+    return half_rows && 2 * (128 / g * g) * 25 >= (kCols / g * g) * 24 ? 128 : kCols;
+}
+
+int launch_prefill(const PrefillLaunch& in, hipStream_t stream)
+{
+    PrefillLaunch a = in;
+    a.cols_per_wg = prefill_columns(a);
     switch (a.head_dim) {
         case 64: return a.num_heads / a.num_kv_heads > kCols ? kLaunchNoKernel : launch_prefill_d<64>(a, stream);
         case 128: return a.num_heads / a.num_kv_heads > kCols ? kLaunchNoKernel : launch_prefill_d<128>(a, stream);

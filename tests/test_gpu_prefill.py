@@ -416,3 +416,28 @@ def test_prefill_from_current_key_value_more_tiles_than_compute_units(pkg, oracl
     ref = oracle_prefill_ex(oracle, bt, q, cache, scale, current_key=k, current_value=v)
     got = run_prefill(pkg, dev, current_key=dev.new_key, current_value=dev.new_value)
     assert_attention_close(got, ref, "two workgroups per CU %s" % (shape,))
+
+
+@pytest.mark.parametrize("shape", [(32, 8, 128), (28, 4, 64), (6, 3, 96), (10, 1, 128), (48, 1, 64), (128, 1, 128), (130, 1, 64)])
+def test_prefill_from_current_key_value_at_the_edges_of_half_workgroups(pkg, oracle, shape):
+    """Half K/V rows run in workgroups of 128 columns (or 256, where the heads of a group fill those better): prompts that end
+    at, before and behind such a tile, with and without the extra terms."""
+    hq, hkv, d = shape
+    ppw = max(128 * hkv // hq, 1)
+    q_lens = [1, ppw, max(ppw - 1, 1), ppw + 1, 2 * ppw, 2 * ppw + 1, 4 * ppw - 1]
+    bt, rng = pkg.workloads.custom_batch(880 + hq, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=0, dec_kv_lens=[5],
+                                         prefill_q_lens=q_lens, prefill_prior=[0] * len(q_lens), outliers=True)
+    dev = pkg.harness.DeviceBatch(bt)
+    q, k, v = pkg.workloads.step_inputs(bt, rng)
+    dev.set_step_inputs(q, k, v)
+    cache, scale = host_cache(bt)
+    mask, ms, mh = make_prefill_mask(bt, rng, False)
+    slopes = (2.0 ** (-8.0 * np.arange(1, hq + 1) / hq)).astype(np.float32)
+    for host, device in (({}, {}),
+                         (dict(attn_mask=mask, mask_stride_s=ms, mask_stride_h=mh, alibi_slopes=slopes),
+                          dict(attn_mask=torch.from_numpy(mask).cuda(), mask_stride_s=ms, mask_stride_h=mh,
+                               alibi_slopes=torch.from_numpy(slopes).cuda()))):
+        ref = oracle_prefill_ex(oracle, bt, q, cache, scale, current_key=k, current_value=v, **host)
+        got = run_prefill(pkg, dev, current_key=dev.new_key, current_value=dev.new_value, **device)
+        assert_attention_close(got[1:], ref[1:], "half workgroups %s %s" % (shape, sorted(host)))
+        assert np.isnan(got[:1]).all()
