@@ -91,7 +91,9 @@ PMXHIP_API int pmxhip_kv_cache_quantize(const pmxhip_kvstore_params* p, pmxhip_s
  * split-KV partials and their combine (kernel.cu:600-678).  The split is not a
  * fixed block count: the kv tokens of all decode sequences form one stream that
  * is cut into `num_token_ranges` equal ranges, one workgroup each, and a second
- * kernel merges the pieces of every sequence that spans more than one range.
+ * kernel merges the pieces of every sequence that spans more than one range.  With a
+ * single range (short sequences, or no workspace) the kernels that can take every
+ * sequence whole, by workgroups of its own, and nothing is merged.
  * Zero the struct before filling it in (memset, `= {0}`): fields added behind the
  * reference's, such as kernel_request, mean "as before" only when they are zero.
  *
@@ -162,7 +164,8 @@ typedef struct pmxhip_decode_plan {
     int64_t partial_out_size;   /* bytes: float32 partial outputs */
     int64_t partial_ml_size;    /* bytes: float32 (running max, exp-sum) pairs */
     int64_t workspace_size;     /* total bytes */
-    int32_t kernel;             /* pmxhip_decode_kernel_t the plan was made for.  The launch falls back to the
+    int32_t kernel;             /* pmxhip_decode_kernel_t the plan was made for: the shape's over long streams.  A launch without
+                                   a request takes a few, or whole, sequences to the column kernels, and falls back to the
                                    general kernel when the quad kernel's needs of the buffers (16-byte aligned
                                    output rows) are not met; pmxhip_decode_kernel_name tells what a call runs. */
 } pmxhip_decode_plan;
@@ -182,7 +185,7 @@ PMXHIP_API int pmxhip_decode_attention(const pmxhip_decode_params* p, pmxhip_str
 
 /* Name of the token-range kernel that pmxhip_decode_attention(p) launches ("" if the call would be rejected):
  * one of decode_attention_kernel, decode_attention_quad_kernel, decode_attention_mfma16_kernel,
- * decode_attention_mfma_kernel -- the names a profiler's kernel trace shows.  Host only, launches nothing. */
+ * decode_attention_mfma_kernel, decode_attention_mfma32_kernel (32 columns, whole sequences) -- the names a profiler's kernel trace shows.  Host only, launches nothing. */
 PMXHIP_API const char* pmxhip_decode_kernel_name(const pmxhip_decode_params* p);
 
 /* pmxhip_decode_attention for callers that cannot allocate: it has no counterpart in the reference, whose caller

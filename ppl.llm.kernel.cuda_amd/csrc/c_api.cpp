@@ -241,39 +241,12 @@ int pmxhip_decode_plan_make_kernel(int64_t decoding_batches, int64_t num_heads, 
         return fail(PMXHIP_UNSUPPORTED, "decode_plan: kernel %d (%s) does not serve %lld query / %lld kv heads of %lld channels",
                     kernel_request, pmxhip::decode_kernel_name(kernel_request), (long long)num_heads, (long long)num_kv_heads,
                     (long long)head_dim);
-    const int min_tokens = pmxhip::decode_min_tokens_per_range(c.wg_tokens);
-
     int64_t ranges = num_token_ranges_hint;
     if (ranges == 0) {
-        const int64_t groups = ((num_kv_heads + c.kv_heads_per_group - 1) / c.kv_heads_per_group) * c.num_passes;
-        int cus = compute_units > 0 ? compute_units : current_compute_units();
+        const int cus = compute_units > 0 ? compute_units : current_compute_units();
         if (cus <= 0) return fail(PMXHIP_INVALID_VALUE, "decode_plan: compute_units not given and no current device");
-        // as many ranges as the kernel wants workgroups per CU for a long stream (decode_select.cpp: the quad kernel
-        // one wave per SIMD, the others two; more, smaller workgroups where a wave serves one or two kv heads)
-        const int64_t long_slots = (int64_t)cus * c.wgs_per_cu;
-        const int64_t slots = (int64_t)cus * c.wgs_per_cu_short; // what the rules for short batches below count with
-        ranges = (long_slots + groups - 1) / groups;
-        // A short batch: ranges of about 128 tokens (twice the smallest) where those still fill half of the slots,
-        // shorter ones -- down to the smallest -- only to get that far: a piece has a fixed cost, and an idle CU costs more.
-        const int64_t max_tokens = decoding_batches * (max_kvlen > 0 ? max_kvlen : 1);
-        const int64_t comfortable = 2 * (int64_t)min_tokens;
-        const int64_t useful = (max_tokens + comfortable - 1) / comfortable;
-        if (ranges > useful) {
-            ranges = useful;
-            const int64_t half = slots / 2 / groups > 1 ? slots / 2 / groups : 1;
-            if (ranges < half) {
-                const int64_t finer = (max_tokens + min_tokens - 1) / min_tokens;
-                ranges = half < finer ? half : finer;
-            }
-            // a step of a few sequences: below a workgroup per two CUs the ranges go down to the kernel's floor
-            const int64_t sparse = cus / 2 / groups > 1 ? cus / 2 / groups : 1;
-            if (ranges < sparse) {
-                const int floor_tokens = pmxhip::decode_floor_tokens_per_range(c.wg_tokens);
-                const int64_t finest = (max_tokens + floor_tokens - 1) / floor_tokens;
-                ranges = sparse < finest ? sparse : finest;
-            }
-        }
-        if (ranges < 1) ranges = 1;
+        ranges = pmxhip::decode_choose_ranges(c, decoding_batches, max_kvlen, head_dim, num_heads, num_kv_heads, cus,
+                                              kernel_request == PMXHIP_DECODE_KERNEL_AUTO);
     }
     plan->num_token_ranges = (int32_t)ranges;
     plan->kv_heads_per_group = c.kv_heads_per_group;
@@ -350,6 +323,9 @@ int decode_prepare(const char* who, const pmxhip_decode_params* p, void* workspa
     if (!pmxhip::decode_choose(p->head_dim, p->num_heads, p->num_kv_heads, p->kernel_request, &c))
         return fail(PMXHIP_UNSUPPORTED, "%s: kernel %d (%s) does not serve this shape", who, p->kernel_request,
                     pmxhip::decode_kernel_name(p->kernel_request));
+    const int cus = current_compute_units();
+    if (p->kernel_request == PMXHIP_DECODE_KERNEL_AUTO)
+        pmxhip::decode_choose_launch(p->decoding_batches, p->num_token_ranges, p->head_dim, p->num_heads, p->num_kv_heads, cus, &c);
     if (c.kernel == pmxhip::kDecodeKernelQuad && !pmxhip::decode_quad_launch_ok(a)) {
         if (p->kernel_request == PMXHIP_DECODE_KERNEL_QUAD)
             return fail(PMXHIP_UNSUPPORTED, "%s: the quad kernel needs 16-byte aligned output rows and, with attn_mask, at "
@@ -369,6 +345,7 @@ int decode_prepare(const char* who, const pmxhip_decode_params* p, void* workspa
     a.num_passes = c.num_passes;
     a.wg_tokens = c.wg_tokens;
     a.min_tokens_per_range = pmxhip::decode_floor_tokens_per_range(c.wg_tokens);
+    pmxhip::decode_choose_form(&a, cus);
 
     if (a.ranges > 1) {
         const int64_t pieces = (int64_t)a.ranges + p->decoding_batches;
@@ -442,7 +419,7 @@ const char* pmxhip_decode_kernel_name(const pmxhip_decode_params* p)
     // the workspace plays no part in the choice; a dummy satisfies the size check
     alignas(16) static char dummy[16];
     if (decode_prepare_quiet("decode_kernel_name", p, p->workspace ? p->workspace : dummy, INT64_MAX, &a) != PMXHIP_SUCCESS) return "";
-    return pmxhip::decode_kernel_name(a.kernel);
+    return pmxhip::decode_kernel_name(a);
 }
 
 int pmxhip_splitkv_combine(const float* partial_out, const float* partial_ml, const int64_t* piece_begin,
@@ -472,8 +449,8 @@ int prefill_chunk_plan(int64_t prefill_batches, int64_t max_seqlen, int64_t max_
                        int64_t head_dim, int32_t compute_units, pmxhip_decode_plan* plan)
 {
     const int64_t columns = max_seqlen * (num_heads / num_kv_heads);
-    return pmxhip_decode_plan_make_kernel(prefill_batches, num_kv_heads * columns, num_kv_heads, head_dim, max_kvlen,
-                                          compute_units, 0, prefill_chunk_kernel(columns, head_dim), plan);
+    return pmxhip_decode_plan_make_kernel(prefill_batches, num_kv_heads * columns, num_kv_heads, head_dim, max_kvlen, compute_units, 0,
+                                          prefill_chunk_kernel(columns, head_dim), plan);
 }
 
 } // namespace
@@ -591,6 +568,8 @@ int pmxhip_prefill_attention_split(const pmxhip_prefill_params* p, void* split_w
                 c.seqstarts = p->seqstarts + p->decoding_batches;
                 c.chunk_q_heads = (int32_t)g;
                 c.chunk_causal = p->is_causal ? 1 : 0;
+                c.by_sequence = 0;
+                c.shared_pieces = 1; // (the plan's ranges are a wave's)
                 return launch_result("prefill_attention", pmxhip::launch_decode(c, 0, stream));
             }
         }

@@ -788,9 +788,13 @@ static int launch_decode_d(const DecodeLaunch& a, int stage, hipStream_t stream)
     if (stage != 2) {
         switch (a.kernel) {
             case kDecodeKernelMfma16:
+                if (D != 64 && D != 128 && !a.by_sequence) return kLaunchNoKernel;
+                launch_decode_columns(a, stream);
+                break;
             case kDecodeKernelMfma32:
-                if (D != 128 && !(D == 64 && a.kernel == kDecodeKernelMfma32)) return kLaunchNoKernel;
-                launch_decode_mfma(a, stream);
+                if (D == 256 || (D == 96 && !a.by_sequence)) return kLaunchNoKernel;
+                if (a.by_sequence) launch_decode_columns(a, stream);
+                else launch_decode_mfma(a, stream);
                 break;
             case kDecodeKernelQuad:
                 if (D != 64 && D != 128 && D != 256) return kLaunchNoKernel;
@@ -812,7 +816,7 @@ static int launch_decode_d(const DecodeLaunch& a, int stage, hipStream_t stream)
             default: return kLaunchNoKernel;
         }
     }
-    if (stage == 1) return kLaunchOk;
+    if (stage == 1 || a.by_sequence) return kLaunchOk; // (whole sequences: nothing to merge)
     // always run: it also writes the zero rows of empty sequences
     {
         // waves per (sequence, head) row by the mean number of pieces per sequence: with many rows of a few

@@ -105,7 +105,8 @@ __device__ __forceinline__ float quad_lane(float v)
 // NS: head slots a lane accumulates: 4, or 1 when every kv head has ONE query head (MHA): the lanes that hold the
 // complete logits of the three absent heads then take head 0's probabilities (one swizzle per value instead of the
 // all-gather) and a single set of 16 accumulators -- a quarter of the PV arithmetic.
-template <bool PAGED, int GP, int WP, bool MASK, int HD, int NS = 4>
+// SEQ: the launch has a single range and workgroup x takes sequence x whole (nothing is left to merge).
+template <bool PAGED, int GP, int WP, bool MASK, int HD, int NS = 4, bool SEQ = false>
 __global__ __launch_bounds__(kWave * WP * GP, 2) void decode_attention_quad_kernel(const DecodeLaunch a)
 {
     constexpr int D = HD;
@@ -138,12 +139,28 @@ __global__ __launch_bounds__(kWave * WP * GP, 2) void decode_attention_quad_kern
 
     const const_i64_ptr kvstarts = as_constant(a.kvstarts);
     const const_i64_ptr cachestarts = as_constant(a.cachestarts);
-    const int64_t kv_base = kvstarts[0];
-    const int64_t total = stream_length(kvstarts[a.decoding_batches] - kv_base, a.decoding_batches);
-    const int64_t per = tokens_per_range(total, a.ranges, BLK, a.min_tokens_per_range);
-    const int64_t r0 = (int64_t)blockIdx.x * per;
-    if (r0 >= total) return;
-    const int64_t r1 = (r0 + per < total) ? r0 + per : total;
+    int64_t kv_base = 0, r0 = 0, r1 = 0;
+    int64_t seq_start = 0, seq_end = 0;
+    int b = blockIdx.x;
+    if constexpr (SEQ) { // the workgroup's range is sequence blockIdx.x
+        seq_start = kvstarts[b];
+        seq_end = kvstarts[b + 1];
+        r0 = sequence_origin(seq_start, b);
+        r1 = r0 + (seq_end - seq_start);
+        if (seq_end <= seq_start) { // the reference yields 0/(0+1e-6) = 0 (kernel.cu:516)
+            const int first = blockIdx.y * (KPW * WP), count = (int)a.num_kv_heads - first < KPW * WP ? (int)a.num_kv_heads - first : KPW * WP;
+            half_t* const out = (half_t*)a.output + (int64_t)b * a.output_stride_s + (int64_t)first * G * D;
+            for (int c = tid; c < count * G * D; c += (int)blockDim.x) out[c] = (half_t)0.f;
+            return;
+        }
+    } else {
+        kv_base = kvstarts[0];
+        const int64_t total = stream_length(kvstarts[a.decoding_batches] - kv_base, a.decoding_batches);
+        const int64_t per = tokens_per_range(total, a.ranges, BLK, a.min_tokens_per_range);
+        r0 = (int64_t)blockIdx.x * per;
+        if (r0 >= total) return;
+        r1 = (r0 + per < total) ? r0 + per : total;
+    }
 
     // Addressing: a 64-bit base per wave (scalar registers) that carries the layer and the wave's first kv head, and
     // a 32-bit offset per lane: (token in block) * stride_s + (second kv head of the wave ? stride_h : 0) + channel.
@@ -162,9 +179,9 @@ __global__ __launch_bounds__(kWave * WP * GP, 2) void decode_attention_quad_kern
     // that follows another in the range starts at its sequence's first token, so kvstarts and the first page table
     // entry (contiguous cache: the sequence's first row) are known when the piece before it begins, and its first
     // cache rows are requested without a dependent load in front of them.
-    int64_t seq_start, seq_end, ahead_end = 0, ahead_row = 0, first_row = 0;
+    int64_t ahead_end = 0, ahead_row = 0, first_row = 0;
     bool have_first_row = false;
-    int b = find_sequence(kvstarts, a.kvstarts, (int)a.decoding_batches, r0, (int)(threadIdx.x & 63), seq_start, seq_end);
+    if constexpr (!SEQ) b = find_sequence(kvstarts, a.kvstarts, (int)a.decoding_batches, r0, (int)(threadIdx.x & 63), seq_start, seq_end);
     for (; b < a.decoding_batches; ++b, seq_start = seq_end, seq_end = ahead_end, first_row = ahead_row, have_first_row = true) {
         const int64_t first_token = seq_start - kv_base;
         if (stream_length(first_token, b) >= r1) break; // the sequence's interval starts beyond the range
@@ -676,8 +693,44 @@ static void launch_decode_quad_two_sets(const DecodeLaunch& a, hipStream_t strea
     else hipLaunchKernelGGL((decode_attention_quad_kernel<false, 2, WP, false, HD>), grid, dim3(2 * WP * kWave), 0, stream, a);
 }
 
+template <int WP, int HD>
+static void launch_decode_quad_seq(const DecodeLaunch& a, hipStream_t stream)
+{
+    constexpr int KPW = HD == 256 ? 1 : 2;
+    const dim3 grid((unsigned)a.decoding_batches, (unsigned)((a.num_kv_heads + KPW * WP - 1) / (KPW * WP)), 1);
+    const bool paged = a.cache_mode == 1;
+    if constexpr (HD != 64) {
+        if (a.num_kv_repeats == 1) {
+            if (paged) hipLaunchKernelGGL((decode_attention_quad_kernel<true, 1, WP, false, HD, 1, true>), grid, dim3(kWave * WP), 0, stream, a);
+            else hipLaunchKernelGGL((decode_attention_quad_kernel<false, 1, WP, false, HD, 1, true>), grid, dim3(kWave * WP), 0, stream, a);
+            return;
+        }
+    }
+    if (paged) hipLaunchKernelGGL((decode_attention_quad_kernel<true, 1, WP, false, HD, 4, true>), grid, dim3(kWave * WP), 0, stream, a);
+    else hipLaunchKernelGGL((decode_attention_quad_kernel<false, 1, WP, false, HD, 4, true>), grid, dim3(kWave * WP), 0, stream, a);
+}
+
+template <int HD>
+static void launch_decode_quad_seq_d(const DecodeLaunch& a, int waves, hipStream_t stream)
+{
+    switch (waves) {
+    case 4: launch_decode_quad_seq<4, HD>(a, stream); break;
+    case 2: launch_decode_quad_seq<2, HD>(a, stream); break;
+    default: launch_decode_quad_seq<1, HD>(a, stream); break;
+    }
+}
+
 void launch_decode_quad(const DecodeLaunch& a, hipStream_t stream)
 {
+    if (a.by_sequence) { // (no mask, up to four query heads per kv head: decode_choose_form)
+        const int seq_waves = a.kv_heads_per_group / (a.head_dim == 256 ? 1 : 2);
+        switch (a.head_dim) {
+        case 64: launch_decode_quad_seq_d<64>(a, seq_waves, stream); break;
+        case 128: launch_decode_quad_seq_d<128>(a, seq_waves, stream); break;
+        default: launch_decode_quad_seq_d<256>(a, seq_waves, stream); break;
+        }
+        return;
+    }
     const int waves = a.kv_heads_per_group / (a.head_dim == 256 ? 1 : 2);
     if (a.num_kv_repeats > 4) { // two sets of waves: the second takes query heads 4-7 of the same kv heads
         if (a.head_dim == 256) { // a wave per kv head

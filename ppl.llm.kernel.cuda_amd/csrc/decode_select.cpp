@@ -26,16 +26,20 @@ bool quad_serves(int64_t head_dim, int64_t g, int64_t num_kv_heads)
 
 } // namespace
 
-const char* decode_kernel_name(int32_t kernel)
+namespace {
+const char* kernel_name(int32_t kernel, bool by_sequence)
 {
     switch (kernel) {
         case kDecodeKernelGeneral: return "decode_attention_kernel";
         case kDecodeKernelQuad: return "decode_attention_quad_kernel";
         case kDecodeKernelMfma16: return "decode_attention_mfma16_kernel";
-        case kDecodeKernelMfma32: return "decode_attention_mfma_kernel";
+        case kDecodeKernelMfma32: return by_sequence ? "decode_attention_mfma32_kernel" : "decode_attention_mfma_kernel";
         default: return "";
     }
 }
+} // namespace
+const char* decode_kernel_name(const DecodeLaunch& a) { return kernel_name(a.kernel, a.by_sequence != 0); }
+const char* decode_kernel_name(int32_t kernel) { return kernel_name(kernel, false); }
 
 bool decode_choose(int64_t head_dim, int64_t num_heads, int64_t num_kv_heads, int32_t requested, DecodeChoice* out)
 {
@@ -167,6 +171,184 @@ bool decode_fit_cache_strides(int64_t head_dim, int64_t num_heads, int64_t num_k
         return decode_fit_cache_strides(head_dim, num_heads, num_kv_heads, other, stride_s, stride_h, c);
     }
     return false;
+}
+
+bool decode_choose_columns(int64_t head_dim, int64_t columns, int64_t num_kv_heads, DecodeChoice* out)
+{
+    if ((head_dim != 64 && head_dim != 96 && head_dim != 128 && head_dim != 256) || columns <= 0 || num_kv_heads <= 0) return false;
+    DecodeChoice c{};
+    c.kernel = columns <= kDecodeMfma16Columns || head_dim == 256 ? kDecodeKernelMfma16 : kDecodeKernelMfma32;
+    const int cols = c.kernel == kDecodeKernelMfma16 ? kDecodeMfma16Columns : kDecodeMfmaColumns;
+    c.kv_heads_per_group = num_kv_heads % 4 == 0 ? 4 : (num_kv_heads % 2 == 0 ? 2 : 1); // a wave per kv head
+    c.q_heads_per_pass = cols;
+    c.num_passes = (int32_t)((columns + cols - 1) / cols);
+    c.wg_tokens = kDecodeMfmaTokens;
+    c.wgs_per_cu = kDecodeMfmaWavesPerCu / c.kv_heads_per_group;
+    c.wgs_per_cu_short = c.wgs_per_cu;
+    *out = c;
+    return true;
+}
+
+namespace {
+
+// (kv head, pass) workgroups of one sequence or range on the column kernels
+int64_t column_groups(int64_t head_dim, int64_t columns, int64_t num_kv_heads)
+{
+    DecodeChoice c;
+    return decode_choose_columns(head_dim, columns, num_kv_heads, &c) ? num_kv_heads * c.num_passes : 0;
+}
+
+// Workgroups of eight waves that a CU holds: their rings are all of its LDS, half of it at head_dim 64.
+int64_t eight_wave_groups_per_cu(int64_t head_dim) { return head_dim == 64 ? 2 : 1; }
+
+// Waves that share a sequence's tokens when every workgroup has a sequence (and kv head, and pass) of its own: eight while
+// that leaves no workgroup waiting for a CU, four up to two rounds of workgroups, beyond that there are waves enough (a
+// wave per kv head).  32 q / 8 kv heads of 128, lengths L/3 to L: 16 sequences of 512 tokens 11.1 / 11.6 us with eight / four
+// waves, 64 of 256 14.9 / 11.6 and 19.3 with one, 64 of 1024 35.3 / 30.8 / 64.0.
+int decode_share(int64_t workgroups, int64_t head_dim, int compute_units)
+{
+    if (compute_units <= 0) return 1;
+    if (workgroups <= eight_wave_groups_per_cu(head_dim) * compute_units) return 8;
+    return workgroups <= (head_dim == 256 ? 4 : 5) * (int64_t)compute_units ? 4 : 1;
+}
+
+// The quad kernel takes its shapes sequence by sequence where every one of its waves (two kv heads, eight to a CU) has a sequence to
+// begin with: 32 q / 8 kv heads of 128, 512 sequences of 100-300 tokens 57 us, 61 on the column kernel, 68 cut into ranges.
+bool quad_by_sequence(int64_t sequences, int64_t num_kv_heads, int64_t g, int compute_units)
+{
+    return g <= 4 && compute_units > 0 && sequences * num_kv_heads >= 16 * (int64_t)compute_units;
+}
+
+// What a batch costs (us) sequence by sequence, and cut into ranges with a combine launch behind it: fits to timings of 11
+// head shapes x 1-256 sequences x 256-16384 tokens (lengths L/3 to L), within 20 % of nearly all of them.  Only their
+// order is used.
+constexpr double kSequenceMargin = 0.8; // (estimates: a batch goes sequence by sequence where that is clearly the cheaper one)
+// A wave's block of 32 tokens takes `alone` with a wave per SIMD and `shared` with two; a workgroup starts in 3.5.
+// `quad`: the rate of the quad kernel, where that is the one for the shape (0: the column kernels).
+double sequence_cost(int64_t sequences, int64_t max_kvlen, int64_t head_dim, int64_t columns, int64_t num_kv_heads, int cus, double quad = 0)
+{
+    const int64_t wgs = sequences * column_groups(head_dim, columns, num_kv_heads);
+    const double wide = columns > kDecodeMfma16Columns && head_dim != 256 ? 1.15 : 1.0;
+    const double shared = wide * (head_dim == 64 ? 1.6 : head_dim == 96 ? 2.6 : head_dim == 128 ? 3.0 : 4.6);
+    const double alone = wide * (head_dim == 64 ? 1.24 : head_dim == 96 ? 1.55 : head_dim == 128 ? 1.75 : 2.8);
+    const int share = decode_share(wgs, head_dim, cus);
+    const double blocks = (double)((max_kvlen + 32 * share - 1) / (32 * share));
+    if (share == 8) return 4.4 + shared * blocks * (wgs > cus ? 2 : 1);
+    if (share == 4 && wgs <= cus) return 4.4 + alone * blocks;
+    if (share == 4 && wgs <= 2 * cus) return 4.6 + shared * blocks;
+    if (quad > 0 && quad_by_sequence(sequences, num_kv_heads, 1, cus)) { // its waves have two kv heads, or one of 256 channels
+        const double rounds = sequences * num_kv_heads / (16.0 * cus);
+        return 1 + rounds * (4.5 + 0.7 * quad * 2 * blocks);
+    }
+    const double rounds = share == 4 ? wgs / (2.0 * cus) : wgs / (8.0 * cus);
+    if (rounds <= 1) return 4.5 + (wgs <= 4 * cus ? alone : shared) * blocks;
+    return 1 + rounds * (3.5 + 0.8 * shared * blocks);
+}
+double quad_rate(int64_t head_dim, int64_t g) { return head_dim == 64 ? 2.2 : (head_dim == 128 ? (g == 1 ? 2.4 : 3.5) : (g == 1 ? 4.8 : (g <= 4 ? 5.7 : 12.0))); }
+double ranges_cost(const DecodeChoice& c, int64_t sequences, int64_t max_kvlen, int64_t head_dim, int64_t g, int64_t num_kv_heads, int cus)
+{
+    // waves' blocks of 32 tokens and one kv head, two more for the start and the end of a sequence
+    const double blocks = (double)(sequences * num_kv_heads * (c.kernel == kDecodeKernelQuad ? 1 : c.num_passes)) *
+                          (0.67 * (double)max_kvlen / 32 + 2);
+    double each = 0; // us for eight of them on every CU
+    switch (c.kernel) {
+        case kDecodeKernelQuad:
+            each = quad_rate(head_dim, g);
+            break;
+        case kDecodeKernelMfma16: each = 3.6; break;
+        case kDecodeKernelMfma32: each = head_dim == 64 ? 2.3 : 4.7; break;
+        default: each = 2.7 * (double)head_dim / 96; break;
+    }
+    return 12 + each * blocks / (8.0 * cus);
+}
+
+// One to four sequences cut into ranges run on the column kernels where those are the faster ones: 32 q / 8 kv heads of 128, one
+// sequence of 1024 / 4096 / 16384 tokens 14.1 / 15.3 / 21.4 us on the quad kernel, 11.3 / 12.8 / 19.5 here; four of 1024 / 2048 /
+// 4096 14.0 / 16.7 / 19.1 and 11.6 / 13.3 / 16.9.  Not with one query head per kv head at head_dim 128 (the quad kernel has a
+// quarter of the arithmetic to do there: one of 4096 15.5 against 18.8) and not at head_dim 256.  Sixteen are level.
+constexpr int64_t kFewSequences = 4;
+bool few_sequences_on_columns(int64_t sequences, int64_t head_dim, int64_t g)
+{
+    return sequences <= kFewSequences && (head_dim == 64 || (head_dim == 128 && g >= 2));
+}
+
+} // namespace
+
+bool decode_choose_launch(int64_t sequences, int64_t ranges, int64_t head_dim, int64_t num_heads, int64_t num_kv_heads, int compute_units,
+                          DecodeChoice* c)
+{
+    const int64_t g = num_heads / num_kv_heads;
+    if (ranges == 1) {
+        if (c->kernel == kDecodeKernelQuad && quad_by_sequence(sequences, num_kv_heads, g, compute_units)) return true;
+        return decode_choose_columns(head_dim, g, num_kv_heads, c);
+    }
+    if (c->kernel == kDecodeKernelQuad && few_sequences_on_columns(sequences, head_dim, g)) return decode_choose_columns(head_dim, g, num_kv_heads, c);
+    return true;
+}
+
+int64_t decode_choose_ranges(const DecodeChoice& by_shape, int64_t sequences, int64_t max_kvlen, int64_t head_dim, int64_t num_heads,
+                             int64_t num_kv_heads, int compute_units, bool automatic)
+{
+    const int64_t g = num_heads / num_kv_heads;
+    const int64_t max_tokens = sequences * (max_kvlen > 0 ? max_kvlen : 1);
+    DecodeChoice c = by_shape;
+    if (automatic && compute_units > 0) {
+        const double quad = by_shape.kernel == kDecodeKernelQuad && g <= 4 ? quad_rate(head_dim, g) : 0;
+        if (sequence_cost(sequences, max_kvlen > 0 ? max_kvlen : 1, head_dim, g, num_kv_heads, compute_units, quad) <
+            kSequenceMargin * ranges_cost(by_shape, sequences, max_kvlen > 0 ? max_kvlen : 1, head_dim, g, num_kv_heads, compute_units))
+            return 1;
+        decode_choose_launch(sequences, 2, head_dim, num_heads, num_kv_heads, compute_units, &c);
+    }
+    const bool columns = c.kernel == kDecodeKernelMfma16 || c.kernel == kDecodeKernelMfma32;
+    const int min_tokens = decode_min_tokens_per_range(c.wg_tokens);
+    const int64_t groups = ((num_kv_heads + c.kv_heads_per_group - 1) / c.kv_heads_per_group) * c.num_passes;
+    if (automatic && c.kernel == kDecodeKernelMfma16 && sequences == 1 && max_tokens <= kSharedStreamTokens) {
+        // a single sequence: ranges of 128 tokens or more that four waves share, one workgroup per CU
+        const int64_t most = compute_units / column_groups(head_dim, g, num_kv_heads);
+        const int64_t useful = (max_tokens + 127) / 128;
+        return useful < most ? useful : (most > 1 ? most : 2);
+    }
+    // as many ranges as the kernel wants workgroups per CU for a long stream (the quad kernel one wave per SIMD, the
+    // others two; more, smaller workgroups where a wave serves one or two kv heads)
+    const int64_t long_slots = (int64_t)compute_units * c.wgs_per_cu;
+    const int64_t slots = (int64_t)compute_units * c.wgs_per_cu_short; // what the rules for short batches below count with
+    int64_t ranges = (long_slots + groups - 1) / groups;
+    // A short batch: ranges of about 128 tokens (twice the smallest) where those still fill half of the slots,
+    // shorter ones -- down to the smallest -- only to get that far: a piece has a fixed cost, and an idle CU costs more.
+    const int64_t comfortable = 2 * (int64_t)min_tokens;
+    const int64_t useful = (max_tokens + comfortable - 1) / comfortable;
+    if (ranges > useful) {
+        ranges = useful;
+        const int64_t half = slots / 2 / groups > 1 ? slots / 2 / groups : 1;
+        if (ranges < half) {
+            // (the column kernels' smallest is a block: 64 q / 8 kv heads of 128, one sequence of 4096 tokens 15.1 us with ranges of 64
+            // tokens and 13.8 with 32, four of 1024 15.5 and 12.8; 14 / 2 heads of 64, 16 of 1024 13.0 and 10.5)
+            const int64_t smallest = automatic && columns ? kDecodeMfmaTokens : min_tokens;
+            const int64_t finer = (max_tokens + smallest - 1) / smallest;
+            ranges = half < finer ? half : finer;
+        }
+        // a step of a few sequences: below a workgroup per two CUs the ranges go down to the kernel's floor
+        const int64_t sparse = compute_units / 2 / groups > 1 ? compute_units / 2 / groups : 1;
+        if (ranges < sparse) {
+            const int floor_tokens = decode_floor_tokens_per_range(c.wg_tokens);
+            const int64_t finest = (max_tokens + floor_tokens - 1) / floor_tokens;
+            ranges = sparse < finest ? sparse : finest;
+        }
+    }
+    return ranges > 1 ? ranges : 1;
+}
+
+void decode_choose_form(DecodeLaunch* a, int compute_units)
+{
+    a->by_sequence = 0;
+    a->shared_pieces = 1;
+    const bool columns = a->kernel == kDecodeKernelMfma16 || a->kernel == kDecodeKernelMfma32;
+    if (!columns && a->kernel != kDecodeKernelQuad) return;
+    a->by_sequence = a->ranges == 1 && (columns || (a->attn_mask == nullptr && a->num_kv_repeats <= 4));
+    if (!columns) return;
+    const int64_t wgs = (a->by_sequence ? a->decoding_batches : a->ranges) * a->num_kv_heads * a->num_passes;
+    if (a->by_sequence) a->shared_pieces = decode_share(wgs, a->head_dim, compute_units);
+    else if (a->kernel == kDecodeKernelMfma16 && a->decoding_batches == 1 && wgs <= compute_units) a->shared_pieces = 4;
 }
 
 bool decode_quad_launch_ok(const DecodeLaunch& a)

@@ -67,6 +67,8 @@ struct DecodeLaunch {
     int32_t wg_tokens;            // tokens one workgroup iteration covers: the unit of the range cuts, a property
                                   // of the kernel named by `kernel` (the combine kernel derives the same cuts from it)
     int32_t min_tokens_per_range;
+    int32_t by_sequence;          // one range, quad and column kernels: workgroup x takes sequence x whole (and writes the rows of an empty one)
+    int32_t shared_pieces;        // column kernels: waves per kv head that share the tokens of a piece (1, 4 or 8)
     int32_t kernel;               // DecodeKernel that runs the token ranges; never kDecodeKernelAuto at launch
     // Chunks of a few query tokens per sequence on the 32-column kernel (nullptr = one query token per sequence, row =
     // sequence index): rows of sequence b are seqstarts[b] .. seqstarts[b + 1]; num_kv_repeats and num_heads then count
@@ -261,7 +263,7 @@ enum DecodeKernel : int32_t {
     kDecodeKernelAuto = 0,    // as a request: by shape
     kDecodeKernelGeneral = 1, // decode_attn.hip: VALU, every head_dim and head count, up to 8 query heads per pass
     kDecodeKernelQuad = 2,    // decode_attn_quad.hip: 4x4x4 MFMA per quad; head_dim 64 or 128 (two or more kv heads) or 256
-    kDecodeKernelMfma16 = 3,  // decode_attn_mfma.hip: 16 query-head columns, head_dim 128
+    kDecodeKernelMfma16 = 3,  // decode_attn_columns.hip: 16 query-head columns (as a request: head_dim 128)
     kDecodeKernelMfma32 = 4,  // decode_attn_mfma.hip: 32 query-head columns per pass, head_dim 128 or 64
 };
 // Fewest tokens a range is given: with fewer, the start of a piece (lookups, query rows, first rows of the cache) and
@@ -299,7 +301,22 @@ bool decode_fit_cache_strides(int64_t head_dim, int64_t num_heads, int64_t num_k
 // What the quad kernel needs of a launch beyond the C ABI's own checks: 16-byte aligned output rows and,
 // with attn_mask, one set of waves and mask offsets within 32 bits.
 bool decode_quad_launch_ok(const DecodeLaunch& a);
-const char* decode_kernel_name(int32_t kernel);
+// The column kernels (decode_attn_columns.hip, decode_attn_mfma.hip) for any head_dim and number of columns per kv head: what short chunks and
+// batches taken sequence by sequence run on (as requests of the C ABI they serve fewer shapes, decode_choose).
+bool decode_choose_columns(int64_t head_dim, int64_t columns, int64_t num_kv_heads, DecodeChoice* out);
+// The kernel of a launch without a request, from the choice by shape (`c`, replaced) and the number of ranges: a single
+// range means that every sequence is taken whole by workgroups of its own.
+bool decode_choose_launch(int64_t sequences, int64_t ranges, int64_t head_dim, int64_t num_heads, int64_t num_kv_heads, int compute_units,
+                          DecodeChoice* c);
+// The number of ranges of a plan.  `automatic`: no kernel was requested.
+int64_t decode_choose_ranges(const DecodeChoice& by_shape, int64_t sequences, int64_t max_kvlen, int64_t head_dim, int64_t num_heads,
+                             int64_t num_kv_heads, int compute_units, bool automatic);
+// A single sequence of more tokens is cut as any other stream.
+constexpr int64_t kSharedStreamTokens = 32768;
+// How the kernel takes the launch: by_sequence and shared_pieces.
+void decode_choose_form(DecodeLaunch* a, int compute_units);
+const char* decode_kernel_name(const DecodeLaunch& a);
+const char* decode_kernel_name(int32_t kernel); // over token ranges
 int decode_wg_tokens(int head_dim, int kv_heads_per_group); // of the general kernel
 constexpr int kDecodeQuadTokens = 16;
 constexpr int kDecodeMfmaWavesPerCu = 8; // 20 KB of LDS per wave
@@ -307,7 +324,8 @@ constexpr int kDecodeMfmaTokens = 32;
 constexpr int kDecodeMfma16Columns = 16;
 constexpr int kDecodeMfmaColumns = 32;
 void launch_decode_quad(const DecodeLaunch& a, hipStream_t stream);
-void launch_decode_mfma(const DecodeLaunch& a, hipStream_t stream);
+void launch_decode_mfma(const DecodeLaunch& a, hipStream_t stream);    // 32 columns over token ranges
+void launch_decode_columns(const DecodeLaunch& a, hipStream_t stream); // 16 columns, and 32 on whole sequences
 // One-time attribute calls of the kernels whose dynamic LDS exceeds the default limit, all variants at once.
 int init_decode_kernels();
 int init_prefill_kernels();

@@ -318,3 +318,46 @@ def test_decode_more_pieces_than_lanes(pkg, oracle, shape):
     for ranges in (65, 128, 129, 200, 511, 590):
         got, plan = run_decode(dev, ranges)
         assert_attention_close(got, ref, "shape %s ranges %d" % (shape, ranges))
+
+
+EDGES = [1, 31, 32, 33, 64, 65, 17, 96, 97, 127, 2, 128, 129]
+
+
+@pytest.mark.parametrize("cache_mode", [0, 1])
+@pytest.mark.parametrize("shape,sequences,name", [
+    # (kv heads x passes x sequences) workgroups: eight waves share a sequence's tokens, then four, then one
+    ((32, 8, 128), 13, "mfma16"), ((32, 8, 128), 60, "mfma16"), ((32, 8, 128), 170, "mfma16"), ((14, 2, 64), 300, "mfma16"),
+    ((14, 2, 64), 650, "mfma16"), ((6, 6, 96), 13, "mfma16"), ((6, 6, 96), 60, "mfma16"), ((3, 3, 96), 430, "mfma16"),
+    ((3, 1, 256), 13, "mfma16"), ((8, 2, 256), 200, "mfma16"), ((24, 1, 256), 600, "mfma16"), ((20, 1, 128), 13, "mfma32"),
+    ((40, 2, 64), 260, "mfma32"), ((40, 1, 96), 150, "mfma32"), ((20, 1, 128), 1300, "mfma32"),
+    # more sequences yet: the quad kernel, where it serves the shape
+    ((8, 8, 64), 512, "quad"), ((9, 9, 64), 456, "quad"), ((12, 12, 128), 342, "quad"), ((16, 8, 128), 512, "quad"), ((18, 9, 256), 456, "quad")])
+def test_decode_sequence_by_sequence(pkg, oracle, shape, sequences, name, cache_mode):
+    """A plan of one range: every sequence is taken whole, by its own workgroups; no workspace, no pieces to merge."""
+    hq, hkv, d = shape
+    bt, dev, q, cache, scale = make_case(pkg, oracle, 610 + hq + d, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=cache_mode,
+                                         dec_kv_lens=[EDGES[i % 13] + 160 * (i % 7 == 3) for i in range(sequences)], outliers=True)
+    empty = [0, 6, sequences - 1]
+    bt.kv_lens[empty] = 0
+    bt.kvstarts = np.concatenate([[0], np.cumsum(bt.kv_lens)]).astype(np.int64)
+    dev.kvstarts.copy_(torch.from_numpy(bt.kvstarts))
+    ref = oracle_decode(oracle, bt, q, cache, scale)
+    assert dev.decode_only(1, name_only=True) == "decode_attention_%s_kernel" % name
+    got, plan = run_decode(dev, 1)
+    assert plan.workspace_size == 0
+    assert_attention_close(got, ref, "by sequence %s x %d" % (shape, sequences))
+    assert (got[empty] == 0).all()
+
+
+@pytest.mark.parametrize("cache_mode", [0, 1])
+@pytest.mark.parametrize("lens", [[1], [33], [1000], [4097], [1, 4095], [31, 2000, 32, 700]])
+@pytest.mark.parametrize("shape", [(32, 8, 128), (14, 2, 64), (8, 8, 64), (12, 6, 128), (40, 8, 128)])
+def test_decode_of_a_few_sequences(pkg, oracle, shape, lens, cache_mode):
+    """Up to four sequences run on the 16-column kernel over ranges, a single one's ranges shared by four waves."""
+    hq, hkv, d = shape
+    bt, dev, q, cache, scale = make_case(pkg, oracle, 650 + hq + d, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=cache_mode,
+                                         dec_kv_lens=lens, outliers=True)
+    ref = oracle_decode(oracle, bt, q, cache, scale)
+    for ranges in (0, 2, 9, 40):
+        got, plan = run_decode(dev, ranges)
+        assert_attention_close(got, ref, "%s %s ranges %d" % (shape, lens, plan.num_token_ranges))

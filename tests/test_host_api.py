@@ -206,6 +206,22 @@ def test_decode_plan_names_its_kernel(pkg, hip_lib):
             pkg.ops.decode_plan(16, hq, hkv, d, 4096, cus=256, kernel=k)
 
 
+def test_decode_plan_takes_short_sequences_whole(pkg, hip_lib):
+    """Batches of short sequences need no ranges (and so no workspace); long ones, and requested kernels, are cut as before."""
+    L = pkg._lib
+    for n, hq, hkv, d, kv in [(32, 32, 8, 128, 256), (4, 32, 8, 128, 256), (64, 14, 2, 64, 256), (448, 8, 1, 256, 148), (12, 32, 8, 64, 553)]:
+        plan = pkg.ops.decode_plan(n, hq, hkv, d, kv, cus=256)
+        assert plan.num_token_ranges == 1 and plan.workspace_size == 0, (n, hq, hkv, d, kv)
+        assert pkg.ops.decode_plan(n, hq, hkv, d, kv, cus=256, ranges_hint=5).num_token_ranges == 5
+    for n, hq, hkv, d, kv in [(64, 32, 8, 128, 4096), (1, 32, 8, 128, 4096), (16, 64, 8, 128, 8192), (8, 16, 8, 256, 8192)]:
+        plan = pkg.ops.decode_plan(n, hq, hkv, d, kv, cus=256)
+        assert plan.num_token_ranges > 1 and plan.workspace_size > 0, (n, hq, hkv, d, kv)
+    assert pkg.ops.decode_plan(32, 32, 8, 128, 256, cus=256, kernel=L.DECODE_KERNEL_QUAD).num_token_ranges > 1
+    # a single sequence: at most a workgroup per (range, kv head) on every compute unit
+    plan = pkg.ops.decode_plan(1, 32, 8, 128, 32768, cus=256)
+    assert plan.num_token_ranges == 32
+
+
 def test_c_entry_points_reject_bad_arguments_without_launching(pkg, hip_lib):
     """Argument checks run before any device work, so they can be exercised on the host."""
     import ctypes
