@@ -283,6 +283,7 @@ typedef struct pmxhip_prefill_params {
      * <= 32, head_dim 64 or 128, no attn_mask, alibi or current_key -- runs on the decode step's MFMA kernels over
      * token ranges, with (query position, query head) pairs as its columns and the split-KV pieces in this
      * workspace; without it, or for any other batch, the tile kernel runs.  Results are the same within the tolerance.
+     * (Chunks of that size over short histories run there sequence by sequence, at every head_dim, and use no workspace.)
      * On that path max_seqlen must bound the query rows of every prefill sequence, as it does in the reference's
      * call (kernel.cu:2143), because the step has max_seqlen query positions per sequence.  A max_seqlen that
      * prefill_query_rows proves too small (more rows than prefill sequences * max_seqlen) keeps the batch on the tile

@@ -266,8 +266,9 @@ namespace {
 
 // Checks of a decode call and the launch block it becomes.  `workspace` / `workspace_size` are the caller's
 // (pmxhip_decode_attention) or the library's static array (pmxhip_decode_attention_static).
+// `columns`: the column kernels whatever the shape (short chunks).
 int decode_prepare(const char* who, const pmxhip_decode_params* p, void* workspace, int64_t workspace_size,
-                   pmxhip::DecodeLaunch* out)
+                   pmxhip::DecodeLaunch* out, bool columns = false)
 {
     if (!head_dim_supported(p->head_dim))
         return fail(PMXHIP_UNSUPPORTED, "cache flash decoding attention do not support head dim %lld", (long long)p->head_dim);
@@ -320,11 +321,12 @@ int decode_prepare(const char* who, const pmxhip_decode_params* p, void* workspa
     // needs of the buffers beyond this entry point's own checks.  Everything that depends on the kernel (the unit
     // of the range cuts above all, which the combine kernel must share) follows from this one choice.
     pmxhip::DecodeChoice c;
-    if (!pmxhip::decode_choose(p->head_dim, p->num_heads, p->num_kv_heads, p->kernel_request, &c))
+    if (columns ? !pmxhip::decode_choose_columns(p->head_dim, p->num_kv_repeats, p->num_kv_heads, &c)
+                : !pmxhip::decode_choose(p->head_dim, p->num_heads, p->num_kv_heads, p->kernel_request, &c))
         return fail(PMXHIP_UNSUPPORTED, "%s: kernel %d (%s) does not serve this shape", who, p->kernel_request,
                     pmxhip::decode_kernel_name(p->kernel_request));
     const int cus = current_compute_units();
-    if (p->kernel_request == PMXHIP_DECODE_KERNEL_AUTO)
+    if (!columns && p->kernel_request == PMXHIP_DECODE_KERNEL_AUTO)
         pmxhip::decode_choose_launch(p->decoding_batches, p->num_token_ranges, p->head_dim, p->num_heads, p->num_kv_heads, cus, &c);
     if (c.kernel == pmxhip::kDecodeKernelQuad && !pmxhip::decode_quad_launch_ok(a)) {
         if (p->kernel_request == PMXHIP_DECODE_KERNEL_QUAD)
@@ -364,10 +366,10 @@ int decode_prepare(const char* who, const pmxhip_decode_params* p, void* workspa
 }
 
 int decode_prepare_quiet(const char* who, const pmxhip_decode_params* p, void* workspace, int64_t workspace_size,
-                         pmxhip::DecodeLaunch* out)
+                         pmxhip::DecodeLaunch* out, bool columns = false)
 {
     g_quiet = true;
-    const int rc = decode_prepare(who, p, workspace, workspace_size, out);
+    const int rc = decode_prepare(who, p, workspace, workspace_size, out, columns);
     g_quiet = false;
     return rc;
 }
@@ -525,53 +527,60 @@ int pmxhip_prefill_attention_split(const pmxhip_prefill_params* p, void* split_w
     const bool hint_covers_rows = p->prefill_query_rows <= 0 || p->prefill_query_rows <= prefill_batches * p->max_seqlen;
     const bool short_chunks = !from_current && !p->attn_mask && !p->alibi_slopes &&
                               prefill_chunk_shape(p->max_seqlen, p->num_heads, p->num_kv_heads, p->head_dim);
-    if (short_chunks && p->workspace && aligned16(p->workspace) && hint_covers_rows) {
-        pmxhip_decode_plan plan;
-        if (prefill_chunk_plan(prefill_batches, p->max_seqlen, p->max_kvlen, p->num_heads, p->num_kv_heads, p->head_dim, 0, &plan) ==
-                PMXHIP_SUCCESS &&
-            plan.workspace_size <= p->workspace_size && aligned16(p->cache) && !(reinterpret_cast<uintptr_t>(p->scale) & 3u) &&
-            // what the decode kernels ask of the layout beyond this stage's own checks (else: the tile kernel)
-            p->cache_stride_s % 16 == 0 && p->cache_stride_l % 16 == 0 && p->cache_stride_h % 16 == 0 && p->cache_stride_kv % 16 == 0 &&
-            p->cache_stride_h >= 0 && p->cache_stride_s >= 0 && 32.0 * (double)p->cache_stride_s + 256.0 < 2147483648.0) {
-            const int64_t g = p->num_heads / p->num_kv_heads;
-            pmxhip_decode_params d;
-            memset(&d, 0, sizeof(d));
-            d.query = p->query;
-            d.output = p->output;
-            d.cache = p->cache;
-            d.scale = p->scale;
-            d.cachestarts = p->cachestarts + p->decoding_batches * p->cachestarts_stride_b;
-            d.kvstarts = p->kvstarts + p->decoding_batches;
-            d.attn_scale = p->attn_scale;
-            d.layer_idx = p->layer_idx;
-            d.num_kv_repeats = p->max_seqlen * g; // columns per kv head
-            d.page_size = p->page_size;
-            d.query_stride_s = p->query_stride_s;
-            d.output_stride_s = p->output_stride_s;
-            d.cache_stride_s = p->cache_stride_s;
-            d.cache_stride_l = p->cache_stride_l;
-            d.cache_stride_h = p->cache_stride_h;
-            d.cache_stride_kv = p->cache_stride_kv;
-            d.cachestarts_stride_b = p->cachestarts_stride_b;
-            d.decoding_batches = prefill_batches;
-            d.num_heads = p->num_kv_heads * d.num_kv_repeats;
-            d.num_kv_heads = p->num_kv_heads;
-            d.head_dim = p->head_dim;
-            d.cache_mode = p->cache_mode;
-            d.num_token_ranges = plan.num_token_ranges;
-            d.workspace = p->workspace;
-            d.workspace_size = p->workspace_size;
-            d.kernel_request = prefill_chunk_kernel(d.num_kv_repeats, p->head_dim);
-            pmxhip::DecodeLaunch c;
-            // what the decode kernels refuse (an alignment, a stride) the tile kernel may still serve
-            if (decode_prepare_quiet("prefill_attention", &d, d.workspace, d.workspace_size, &c) == PMXHIP_SUCCESS) {
-                c.seqstarts = p->seqstarts + p->decoding_batches;
-                c.chunk_q_heads = (int32_t)g;
-                c.chunk_causal = p->is_causal ? 1 : 0;
-                c.by_sequence = 0;
-                c.shared_pieces = 1; // (the plan's ranges are a wave's)
-                return launch_result("prefill_attention", pmxhip::launch_decode(c, 0, stream));
-            }
+    const int64_t g = p->num_heads / p->num_kv_heads;
+    const int64_t columns = p->max_seqlen * g; // per kv head
+    // what the decode kernels ask of the layout beyond this stage's own checks (else: the tile kernel)
+    const bool column_layout = !from_current && !p->attn_mask && !p->alibi_slopes && aligned16(p->cache) &&
+                               !(reinterpret_cast<uintptr_t>(p->scale) & 3u) && p->cache_stride_s % 16 == 0 && p->cache_stride_l % 16 == 0 &&
+                               p->cache_stride_h % 16 == 0 && p->cache_stride_kv % 16 == 0 && p->cache_stride_h >= 0 &&
+                               p->cache_stride_s >= 0 && 32.0 * (double)p->cache_stride_s + 256.0 < 2147483648.0;
+    pmxhip_decode_plan plan;
+    const bool ranges_served = short_chunks && column_layout && p->workspace && aligned16(p->workspace) && hint_covers_rows &&
+                               prefill_chunk_plan(prefill_batches, p->max_seqlen, p->max_kvlen, p->num_heads, p->num_kv_heads,
+                                                  p->head_dim, 0, &plan) == PMXHIP_SUCCESS &&
+                               plan.workspace_size <= p->workspace_size;
+    const int cus = current_compute_units();
+    // sequence by sequence they need no workspace, and the kernel walks every row of a sequence whatever max_seqlen says
+    const bool by_sequence = column_layout && pmxhip::prefill_by_sequence(prefill_batches, p->max_seqlen, p->max_kvlen, p->num_heads,
+                                                                          p->num_kv_heads, p->head_dim, ranges_served, cus);
+    if (ranges_served || by_sequence) {
+        pmxhip_decode_params d;
+        memset(&d, 0, sizeof(d));
+        d.query = p->query;
+        d.output = p->output;
+        d.cache = p->cache;
+        d.scale = p->scale;
+        d.cachestarts = p->cachestarts + p->decoding_batches * p->cachestarts_stride_b;
+        d.kvstarts = p->kvstarts + p->decoding_batches;
+        d.attn_scale = p->attn_scale;
+        d.layer_idx = p->layer_idx;
+        d.num_kv_repeats = columns;
+        d.page_size = p->page_size;
+        d.query_stride_s = p->query_stride_s;
+        d.output_stride_s = p->output_stride_s;
+        d.cache_stride_s = p->cache_stride_s;
+        d.cache_stride_l = p->cache_stride_l;
+        d.cache_stride_h = p->cache_stride_h;
+        d.cache_stride_kv = p->cache_stride_kv;
+        d.cachestarts_stride_b = p->cachestarts_stride_b;
+        d.decoding_batches = prefill_batches;
+        d.num_heads = p->num_kv_heads * d.num_kv_repeats;
+        d.num_kv_heads = p->num_kv_heads;
+        d.head_dim = p->head_dim;
+        d.cache_mode = p->cache_mode;
+        d.num_token_ranges = by_sequence ? 1 : plan.num_token_ranges;
+        d.kernel_request = prefill_chunk_kernel(columns, p->head_dim); // (over ranges)
+        d.workspace = p->workspace;
+        d.workspace_size = p->workspace_size;
+        pmxhip::DecodeLaunch c;
+        // what the decode kernels refuse (an alignment, a stride) the tile kernel may still serve
+        if (decode_prepare_quiet("prefill_attention", &d, d.workspace, d.workspace_size, &c, by_sequence) == PMXHIP_SUCCESS) {
+            c.seqstarts = p->seqstarts + p->decoding_batches;
+            c.chunk_q_heads = (int32_t)g;
+            c.chunk_causal = p->is_causal ? 1 : 0;
+            c.by_sequence = by_sequence;
+            if (!by_sequence) c.shared_pieces = 1; // (the plan's ranges are a wave's)
+            return launch_result("prefill_attention", pmxhip::launch_decode(c, 0, stream));
         }
     }
 

@@ -375,4 +375,26 @@ bool prefill_chunk_shape(int64_t max_seqlen, int64_t num_heads, int64_t num_kv_h
     return max_seqlen * (num_heads / num_kv_heads) <= kPrefillChunkColumns;
 }
 
+// Chunks of up to 32 columns go sequence by sequence where the estimates say so: against ranges (equal work, the estimates differ by
+// the combine launch and the pieces; 12 % is what they err by) 64 q / 8 kv heads of 128, 147 chunks of 2-4 rows over up to 391 tokens
+// 63 -> 52 us, 16 / 4 heads, 15 of 2 over 433 17.1 -> 14.0; against the tile kernel, whose workgroups have 256 columns for them and which
+// is what serves head_dim 96 and 256 and calls without a workspace: 16 / 16 heads of 256, 30 of 2-18 over 3208 429 -> 192 us, 8 / 1 heads
+// of 256, 178 of 1-2 over 591 59 -> 24, 32 / 32 heads of 96, four of 2 over 6971 114 -> 97.
+bool prefill_by_sequence(int64_t sequences, int64_t max_seqlen, int64_t max_kvlen, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                         bool ranges_served, int compute_units)
+{
+    constexpr int64_t kMostColumns = 32; // (a pass of the 32-column form, two of the 16-column form at head_dim 256)
+    if (num_kv_heads <= 0 || num_heads % num_kv_heads != 0 || max_seqlen <= 0 || sequences <= 0 || max_kvlen <= 0 || compute_units <= 0) return false;
+    const int64_t columns = max_seqlen * (num_heads / num_kv_heads);
+    DecodeChoice c;
+    if (columns > kMostColumns || !decode_choose_columns(head_dim, columns, num_kv_heads, &c)) return false;
+    const double cost = sequence_cost(sequences, max_kvlen, head_dim, columns, num_kv_heads, compute_units);
+    if (ranges_served) return cost < 0.88 * ranges_cost(c, sequences, max_kvlen, head_dim, columns, num_kv_heads, compute_units);
+    // the tile kernel: a workgroup per (sequence, kv head) and CU, 3.4 us for 64 kv tokens, or the tokens of few of them shared out
+    const double tile = (head_dim == 256 ? 7.0 : head_dim == 64 ? 2.4 : 3.4) / 64 * (double)max_kvlen;
+    const double rounds = (double)(sequences * num_kv_heads) / compute_units;
+    const double alone = rounds < 1 ? 8 + tile : 4 + rounds * (4 + 0.75 * tile), shared = 30 + rounds * tile;
+    return cost < kSequenceMargin * (rounds < 1 && shared < alone ? shared : alone);
+}
+
 } // namespace pmxhip

@@ -441,3 +441,22 @@ def test_prefill_from_current_key_value_at_the_edges_of_half_workgroups(pkg, ora
         got = run_prefill(pkg, dev, current_key=dev.new_key, current_value=dev.new_value, **device)
         assert_attention_close(got[1:], ref[1:], "half workgroups %s %s" % (shape, sorted(host)))
         assert np.isnan(got[:1]).all()
+
+
+@pytest.mark.parametrize("is_causal", [True, False])
+@pytest.mark.parametrize("cache_mode", [0, 1])
+@pytest.mark.parametrize("shape,sequences,q_max", [((8, 1, 256), 9, 4), ((4, 4, 96), 12, 9), ((12, 3, 96), 100, 4), ((4, 2, 256), 150, 8),
+                                                   ((8, 8, 64), 70, 4), ((6, 6, 128), 240, 5), ((4, 2, 64), 700, 3), ((14, 2, 128), 60, 3)])
+def test_prefill_short_chunks_sequence_by_sequence(pkg, oracle, shape, sequences, q_max, cache_mode, is_causal):
+    """A few query rows per sequence over short histories, no workspace: a sequence is the work of eight, four or one waves
+    (fewer with more sequences).  Histories at the edges of a block of 32 tokens and of a wave's share of them."""
+    hq, hkv, d = shape
+    q_lens = [1 + i % q_max for i in range(sequences)]
+    prior = [(0, 31, 32, 95, 128, 200, 1, 63)[i % 8] for i in range(sequences)]
+    bt, dev, q, cache, scale = make_case(pkg, oracle, 380 + hq + d, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=cache_mode,
+                                         dec_kv_lens=[33], prefill_q_lens=q_lens, prefill_prior=prior, outliers=True)
+    bt.is_causal = is_causal
+    ref = oracle_prefill(oracle, bt, q, cache, scale)
+    got = run_prefill(pkg, dev, is_causal=is_causal)
+    assert_attention_close(got[1:], ref[1:], "chunks by sequence %s" % (shape,))
+    assert np.isnan(got[:1]).all()
