@@ -16,6 +16,8 @@
 //
 // Exactness follows the prefill kernel: K^ = int8 * scale, V^ and p are kept as hi + lo pairs of halves
 // (2 MFMAs per QK step, 3 per PV step), so no fp16 rounding of the dequantised cache enters the result.
+// Against float64 the outputs' error is that of rounding them to half, as with the kernels that served these batches before (32 q /
+// 8 kv heads of 128, 16 sequences of 30-200: rms 7.43e-5, maximum 9.60e-4 for either, and for the rounding alone; ten shapes).
 //
 // The cache rows travel from memory into a wave-private LDS ring without registers (global_load_lds), two blocks
 // ahead of the arithmetic, and across sequences: the blocks of a range are one stream to the requests, so the first
