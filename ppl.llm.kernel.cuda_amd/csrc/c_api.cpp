@@ -317,37 +317,24 @@ int decode_prepare(const char* who, const pmxhip_decode_params* p, void* workspa
     a.head_dim = (int32_t)p->head_dim;
     a.ranges = p->num_token_ranges;
 
-    // The kernel that will run, decided once and here: by shape (or by request), then by what the quad kernel
-    // needs of the buffers beyond this entry point's own checks.  Everything that depends on the kernel (the unit
-    // of the range cuts above all, which the combine kernel must share) follows from this one choice.
+    // The kernel that will run, decided once and here: by shape (or by request), by the number of ranges and by what the
+    // kernels need of the buffers and the cache layout beyond this entry point's own checks.  Everything that depends on
+    // the kernel (the unit of the range cuts above all, which the combine kernel must share) follows from this one choice.
     pmxhip::DecodeChoice c;
-    if (columns ? !pmxhip::decode_choose_columns(p->head_dim, p->num_kv_repeats, p->num_kv_heads, &c)
-                : !pmxhip::decode_choose(p->head_dim, p->num_heads, p->num_kv_heads, p->kernel_request, &c))
+    switch (pmxhip::decode_select(&a, p->kernel_request, columns, current_compute_units(), &c)) {
+    case pmxhip::DecodeSelect::kSelected: break;
+    case pmxhip::DecodeSelect::kNoKernel:
         return fail(PMXHIP_UNSUPPORTED, "%s: kernel %d (%s) does not serve this shape", who, p->kernel_request,
                     pmxhip::decode_kernel_name(p->kernel_request));
-    const int cus = current_compute_units();
-    if (!columns && p->kernel_request == PMXHIP_DECODE_KERNEL_AUTO)
-        pmxhip::decode_choose_launch(p->decoding_batches, p->num_token_ranges, p->head_dim, p->num_heads, p->num_kv_heads, cus, &c);
-    if (c.kernel == pmxhip::kDecodeKernelQuad && !pmxhip::decode_quad_launch_ok(a)) {
-        if (p->kernel_request == PMXHIP_DECODE_KERNEL_QUAD)
-            return fail(PMXHIP_UNSUPPORTED, "%s: the quad kernel needs 16-byte aligned output rows and, with attn_mask, at "
-                                            "most four query heads per kv head", who);
-        pmxhip::decode_choose(p->head_dim, p->num_heads, p->num_kv_heads, pmxhip::kDecodeKernelGeneral, &c);
-    }
-    // ... and by the cache layout: 32-bit lane offsets against a 64-bit base per wave (decode_fit_cache_strides)
-    if (!pmxhip::decode_fit_cache_strides(p->head_dim, p->num_heads, p->num_kv_heads, p->kernel_request, p->cache_stride_s,
-                                          p->cache_stride_h, &c))
+    case pmxhip::DecodeSelect::kQuadBuffers:
+        return fail(PMXHIP_UNSUPPORTED, "%s: the quad kernel needs 16-byte aligned output rows and, with attn_mask, at "
+                                        "most four query heads per kv head", who);
+    case pmxhip::DecodeSelect::kCacheStrides: // 32-bit lane offsets against a 64-bit base per wave
         return fail(PMXHIP_UNSUPPORTED,
                     "%s: cache_stride_s %lld / cache_stride_h %lld: the rows of one block of %d tokens%s must lie within 2 GiB",
                     who, (long long)p->cache_stride_s, (long long)p->cache_stride_h, c.wg_tokens,
                     c.kernel == pmxhip::kDecodeKernelQuad ? " of the two kv heads of a wave (requested quad kernel)" : "");
-    a.kernel = c.kernel;
-    a.kv_heads_per_group = c.kv_heads_per_group;
-    a.q_heads_per_pass = c.q_heads_per_pass;
-    a.num_passes = c.num_passes;
-    a.wg_tokens = c.wg_tokens;
-    a.min_tokens_per_range = pmxhip::decode_floor_tokens_per_range(c.wg_tokens);
-    pmxhip::decode_choose_form(&a, cus);
+    }
 
     if (a.ranges > 1) {
         const int64_t pieces = (int64_t)a.ranges + p->decoding_batches;

@@ -95,9 +95,13 @@ __global__ __launch_bounds__(kDecodeThreads, (GT <= 4 ? 2 : 1)) void decode_atte
     const int64_t kv_base = kvstarts[0];
     const int64_t total = stream_length(kvstarts[a.decoding_batches] - kv_base, a.decoding_batches);
     const int64_t per = tokens_per_range(total, a.ranges, wg_tokens, a.min_tokens_per_range);
-    const int64_t r0 = (int64_t)blockIdx.x * per;
+    int64_t r0 = (int64_t)blockIdx.x * per;
+    int64_t r1 = (r0 + per < total) ? r0 + per : total;
+    if (a.by_sequence) { // the workgroup's range is sequence blockIdx.x
+        r0 = sequence_origin(kvstarts[blockIdx.x] - kv_base, blockIdx.x);
+        r1 = r0 + (kvstarts[blockIdx.x + 1] - kvstarts[blockIdx.x]);
+    }
     if (r0 >= total) return;
-    const int64_t r1 = (r0 + per < total) ? r0 + per : total;
 
     // Addressing: a wave-uniform 64-bit base per block (scalar registers) plus a 32-bit per-lane
     // offset: (token in block) * stride_s + (head in group) * stride_h + channel.
@@ -801,7 +805,8 @@ static int launch_decode_d(const DecodeLaunch& a, int stage, hipStream_t stream)
                 launch_decode_quad(a, stream);
                 break;
             case kDecodeKernelGeneral: {
-                const dim3 grid((unsigned)a.ranges, (unsigned)(a.num_kv_heads / a.kv_heads_per_group), (unsigned)a.num_passes);
+                const dim3 grid((unsigned)(a.by_sequence ? a.decoding_batches : a.ranges), (unsigned)(a.num_kv_heads / a.kv_heads_per_group),
+                                (unsigned)a.num_passes);
                 int rc = kLaunchNoKernel;
                 switch (a.q_heads_per_pass) {
                     case 1: rc = launch_decode_dgt<D, 1>(a, grid, stream); break;
@@ -816,7 +821,8 @@ static int launch_decode_d(const DecodeLaunch& a, int stage, hipStream_t stream)
             default: return kLaunchNoKernel;
         }
     }
-    if (stage == 1 || a.by_sequence) return kLaunchOk; // (whole sequences: nothing to merge)
+    // (whole sequences: nothing to merge; the general kernel leaves the zero rows of empty ones to the combine kernel)
+    if (stage == 1 || (a.by_sequence && a.kernel != kDecodeKernelGeneral)) return kLaunchOk;
     // always run: it also writes the zero rows of empty sequences
     {
         // waves per (sequence, head) row by the mean number of pieces per sequence: with many rows of a few
@@ -871,13 +877,6 @@ int launch_decode(const DecodeLaunch& a, int stage, hipStream_t stream)
         case 256: return launch_decode_d<256>(a, stage, stream);
         default: return kLaunchNoKernel;
     }
-}
-
-int decode_wg_tokens(int head_dim, int kv_heads_per_group)
-{
-    const int lps = head_dim == 64 ? 4 : (head_dim == 256 ? 16 : 8);
-    const int spw = kWave / lps;
-    return kTB * (spw / kv_heads_per_group) * kDecodeWaves;
 }
 
 void launch_splitkv_combine_rows(const float* partial_out, const float* partial_ml, const int64_t* piece_begin,

@@ -700,6 +700,11 @@ static void launch_decode_quad_seq(const DecodeLaunch& a, hipStream_t stream)
     const dim3 grid((unsigned)a.decoding_batches, (unsigned)((a.num_kv_heads + KPW * WP - 1) / (KPW * WP)), 1);
     const bool paged = a.cache_mode == 1;
     if constexpr (HD != 64) {
+        if (a.attn_mask != nullptr) {
+            if (paged) hipLaunchKernelGGL((decode_attention_quad_kernel<true, 1, WP, true, HD, 4, true>), grid, dim3(kWave * WP), 0, stream, a);
+            else hipLaunchKernelGGL((decode_attention_quad_kernel<false, 1, WP, true, HD, 4, true>), grid, dim3(kWave * WP), 0, stream, a);
+            return;
+        }
         if (a.num_kv_repeats == 1) {
             if (paged) hipLaunchKernelGGL((decode_attention_quad_kernel<true, 1, WP, false, HD, 1, true>), grid, dim3(kWave * WP), 0, stream, a);
             else hipLaunchKernelGGL((decode_attention_quad_kernel<false, 1, WP, false, HD, 1, true>), grid, dim3(kWave * WP), 0, stream, a);
@@ -722,7 +727,7 @@ static void launch_decode_quad_seq_d(const DecodeLaunch& a, int waves, hipStream
 
 void launch_decode_quad(const DecodeLaunch& a, hipStream_t stream)
 {
-    if (a.by_sequence) { // (no mask, up to four query heads per kv head: decode_choose_form)
+    if (a.by_sequence) { // (up to four query heads per kv head, no mask at head_dim 64: decode_select)
         const int seq_waves = a.kv_heads_per_group / (a.head_dim == 256 ? 1 : 2);
         switch (a.head_dim) {
         case 64: launch_decode_quad_seq_d<64>(a, seq_waves, stream); break;
@@ -744,7 +749,7 @@ void launch_decode_quad(const DecodeLaunch& a, hipStream_t stream)
         }
         return;
     }
-    if (a.head_dim == 64) { // no mask form: decode_quad_launch_ok sends masked steps to the general kernel
+    if (a.head_dim == 64) { // no mask form: decode_select sends masked steps to other kernels
         const dim3 grid((unsigned)a.ranges, (unsigned)((a.num_kv_heads + 2 * waves - 1) / (2 * waves)), 1);
         const bool paged = a.cache_mode == 1;
         switch (waves) {

@@ -14,7 +14,8 @@ constexpr float kNegBig = -1.0e30f; // finite "no token yet" running max (log2 u
 
 constexpr int kDecodeThreads = 256;
 constexpr int kDecodeWaves = kDecodeThreads / kWave;
-constexpr int kTB = 4; // tokens a slot handles per block (= lanes of a quad)
+constexpr int kTB = kDecodeSlotTokens; // tokens a slot handles per block (= lanes of a quad)
+static_assert(kDecodeWaves == kDecodeGeneralWaves, "decode_wg_tokens counts these waves");
 static_assert(kTB == 4, "the quad reduce-scatter and the explicit wait counts assume four tokens per block");
 
 // ---- hand-scheduled cache loads of the pipelined loop ---------------------------------------

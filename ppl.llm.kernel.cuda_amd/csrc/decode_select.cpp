@@ -142,9 +142,13 @@ double lane_offset_span(const DecodeChoice& c, int64_t head_dim, int64_t stride_
     return (double)tokens * (double)stride_s + (double)heads_apart * (double)stride_h + (double)head_dim;
 }
 
-} // namespace
-
-bool decode_fit_cache_strides(int64_t head_dim, int64_t num_heads, int64_t num_kv_heads, int32_t requested,
+// Makes the choice fit a cache layout: the kernels address a row as a 64-bit base per wave plus a 32-bit offset per
+// lane, and where the kv heads of a wave lie further apart than such an offset reaches (cache_stride_h of a layout
+// that keeps the heads outermost) the general kernel takes fewer kv heads per workgroup and, unless the quad kernel
+// was requested, a kernel with a wave per kv head takes its steps.  The number of ranges of a plan stays valid: it
+// does not depend on the grouping.  False: no kernel serves the strides (a block of tokens alone spans 2 GiB, or a
+// stride is negative).
+bool fit_cache_strides(int64_t head_dim, int64_t num_heads, int64_t num_kv_heads, int32_t requested,
                               int64_t stride_s, int64_t stride_h, DecodeChoice* c)
 {
     constexpr double kLimit = 2147483648.0;
@@ -168,10 +172,12 @@ bool decode_fit_cache_strides(int64_t head_dim, int64_t num_heads, int64_t num_k
                               : (head_dim == 128 || head_dim == 64 ? kDecodeKernelMfma32 : kDecodeKernelGeneral);
         if (!decode_choose(head_dim, num_heads, num_kv_heads, other, &alt)) return false;
         *c = alt;
-        return decode_fit_cache_strides(head_dim, num_heads, num_kv_heads, other, stride_s, stride_h, c);
+        return fit_cache_strides(head_dim, num_heads, num_kv_heads, other, stride_s, stride_h, c);
     }
     return false;
 }
+
+} // namespace
 
 bool decode_choose_columns(int64_t head_dim, int64_t columns, int64_t num_kv_heads, DecodeChoice* out)
 {
@@ -213,10 +219,14 @@ int decode_share(int64_t workgroups, int64_t head_dim, int compute_units)
 }
 
 // The quad kernel takes its shapes sequence by sequence where every one of its waves (two kv heads, eight to a CU) has a sequence to
-// begin with: 32 q / 8 kv heads of 128, 512 sequences of 100-300 tokens 57 us, 61 on the column kernel, 68 cut into ranges.
-bool quad_by_sequence(int64_t sequences, int64_t num_kv_heads, int64_t g, int compute_units)
+// begin with: 32 q / 8 kv heads of 128, 512 sequences of 100-300 tokens 57 us, 61 on the column kernel, 68 cut into ranges.  With a
+// mask, whose values the column kernel waits for together with its rows, from where that kernel's waves come in a second round: the
+// same heads, 300 sequences of 100-300 48.8 us, 56.9 on the column kernel; 16 / 4 heads, 512 of them 47.3 and 45.1.
+bool quad_by_sequence(int64_t sequences, int64_t num_kv_heads, int64_t g, bool mask, int compute_units)
 {
-    return g <= 4 && compute_units > 0 && sequences * num_kv_heads >= 16 * (int64_t)compute_units;
+    if (g > 4 || compute_units <= 0) return false;
+    const int64_t pairs = sequences * num_kv_heads;
+    return pairs >= 16 * (int64_t)compute_units || (mask && pairs > 8 * (int64_t)compute_units);
 }
 
 // What a batch costs (us) sequence by sequence, and cut into ranges with a combine launch behind it: fits to timings of 11
@@ -236,7 +246,7 @@ double sequence_cost(int64_t sequences, int64_t max_kvlen, int64_t head_dim, int
     if (share == 8) return 4.4 + shared * blocks * (wgs > cus ? 2 : 1);
     if (share == 4 && wgs <= cus) return 4.4 + alone * blocks;
     if (share == 4 && wgs <= 2 * cus) return 4.6 + shared * blocks;
-    if (quad > 0 && quad_by_sequence(sequences, num_kv_heads, 1, cus)) { // its waves have two kv heads, or one of 256 channels
+    if (quad > 0 && quad_by_sequence(sequences, num_kv_heads, 1, false, cus)) { // its waves have two kv heads, or one of 256 channels
         const double rounds = sequences * num_kv_heads / (16.0 * cus);
         return 1 + rounds * (4.5 + 0.7 * quad * 2 * blocks);
     }
@@ -272,18 +282,32 @@ bool few_sequences_on_columns(int64_t sequences, int64_t head_dim, int64_t g)
     return sequences <= kFewSequences && (head_dim == 64 || (head_dim == 128 && g >= 2));
 }
 
+// The quad kernel's form for whole sequences has one set of waves.
+bool quad_takes_whole(const DecodeLaunch& a) { return a.num_kv_repeats <= 4 && decode_quad_launch_ok(a); }
+
 } // namespace
 
-bool decode_choose_launch(int64_t sequences, int64_t ranges, int64_t head_dim, int64_t num_heads, int64_t num_kv_heads, int compute_units,
-                          DecodeChoice* c)
+// The kernel of a launch without a request, in place of the choice by shape.
+static void choose_launch(const DecodeLaunch& a, int compute_units, DecodeChoice* c)
 {
-    const int64_t g = num_heads / num_kv_heads;
-    if (ranges == 1) {
-        if (c->kernel == kDecodeKernelQuad && quad_by_sequence(sequences, num_kv_heads, g, compute_units)) return true;
-        return decode_choose_columns(head_dim, g, num_kv_heads, c);
+    const int64_t g = a.num_heads / a.num_kv_heads;
+    if (a.ranges == 1) {
+        // A single range is for kernels that take every sequence whole (a kernel over ranges would walk the batch with one
+        // workgroup), and the plan knows neither mask nor buffers.  What the quad kernel cannot take whole is the column kernels',
+        // except one query head per kv head at head_dim 64 where those have a wave per pair: 8 / 8 heads, 512 sequences of 100-300
+        // tokens with a mask 53.0 us on the column kernel, 37.9 on the general one, with rows of 8 bytes 46.9 and 36.2.
+        if (c->kernel == kDecodeKernelQuad) {
+            if (quad_takes_whole(a) && quad_by_sequence(a.decoding_batches, a.num_kv_heads, g, a.attn_mask != nullptr, compute_units)) return;
+            if (a.head_dim == 64 && g == 1 && a.num_kv_heads % 8 == 0 && !quad_takes_whole(a) &&
+                decode_share(a.decoding_batches * a.num_kv_heads, a.head_dim, compute_units) == 1 && compute_units > 0) {
+                decode_choose(a.head_dim, a.num_heads, a.num_kv_heads, kDecodeKernelGeneral, c);
+                return;
+            }
+        }
+        decode_choose_columns(a.head_dim, g, a.num_kv_heads, c);
+    } else if (c->kernel == kDecodeKernelQuad && few_sequences_on_columns(a.decoding_batches, a.head_dim, g)) {
+        decode_choose_columns(a.head_dim, g, a.num_kv_heads, c);
     }
-    if (c->kernel == kDecodeKernelQuad && few_sequences_on_columns(sequences, head_dim, g)) return decode_choose_columns(head_dim, g, num_kv_heads, c);
-    return true;
 }
 
 int64_t decode_choose_ranges(const DecodeChoice& by_shape, int64_t sequences, int64_t max_kvlen, int64_t head_dim, int64_t num_heads,
@@ -297,7 +321,7 @@ int64_t decode_choose_ranges(const DecodeChoice& by_shape, int64_t sequences, in
         if (sequence_cost(sequences, max_kvlen > 0 ? max_kvlen : 1, head_dim, g, num_kv_heads, compute_units, quad) <
             kSequenceMargin * ranges_cost(by_shape, sequences, max_kvlen > 0 ? max_kvlen : 1, head_dim, g, num_kv_heads, compute_units))
             return 1;
-        decode_choose_launch(sequences, 2, head_dim, num_heads, num_kv_heads, compute_units, &c);
+        if (c.kernel == kDecodeKernelQuad && few_sequences_on_columns(sequences, head_dim, g)) decode_choose_columns(head_dim, g, num_kv_heads, &c);
     }
     const bool columns = c.kernel == kDecodeKernelMfma16 || c.kernel == kDecodeKernelMfma32;
     const int min_tokens = decode_min_tokens_per_range(c.wg_tokens);
@@ -338,13 +362,13 @@ int64_t decode_choose_ranges(const DecodeChoice& by_shape, int64_t sequences, in
     return ranges > 1 ? ranges : 1;
 }
 
-void decode_choose_form(DecodeLaunch* a, int compute_units)
+// How the kernel takes the launch: by_sequence and shared_pieces.
+static void choose_form(DecodeLaunch* a, int compute_units)
 {
     a->by_sequence = 0;
     a->shared_pieces = 1;
     const bool columns = a->kernel == kDecodeKernelMfma16 || a->kernel == kDecodeKernelMfma32;
-    if (!columns && a->kernel != kDecodeKernelQuad) return;
-    a->by_sequence = a->ranges == 1 && (columns || (a->attn_mask == nullptr && a->num_kv_repeats <= 4));
+    a->by_sequence = a->ranges == 1 && (a->kernel != kDecodeKernelQuad || quad_takes_whole(*a));
     if (!columns) return;
     const int64_t wgs = (a->by_sequence ? a->decoding_batches : a->ranges) * a->num_kv_heads * a->num_passes;
     if (a->by_sequence) a->shared_pieces = decode_share(wgs, a->head_dim, compute_units);
@@ -360,6 +384,37 @@ bool decode_quad_launch_ok(const DecodeLaunch& a)
         if (((double)a.num_heads * (double)a.mask_stride_h + 64.0) * 2.0 >= 4294967296.0) return false;
     }
     return true;
+}
+
+DecodeSelect decode_select(DecodeLaunch* a, int32_t requested, bool columns, int compute_units, DecodeChoice* out)
+{
+    DecodeChoice c{};
+    *out = c;
+    if (columns ? !decode_choose_columns(a->head_dim, a->num_kv_repeats, a->num_kv_heads, &c)
+                : !decode_choose(a->head_dim, a->num_heads, a->num_kv_heads, requested, &c))
+        return DecodeSelect::kNoKernel;
+    if (!columns && requested == kDecodeKernelAuto) choose_launch(*a, compute_units, &c);
+    if (c.kernel == kDecodeKernelQuad && !decode_quad_launch_ok(*a)) {
+        if (requested == kDecodeKernelQuad) return DecodeSelect::kQuadBuffers;
+        decode_choose(a->head_dim, a->num_heads, a->num_kv_heads, kDecodeKernelGeneral, &c);
+    }
+    const bool fits = fit_cache_strides(a->head_dim, a->num_heads, a->num_kv_heads, requested, a->cache_stride_s, a->cache_stride_h, &c);
+    *out = c;
+    if (!fits) return DecodeSelect::kCacheStrides;
+    a->kernel = c.kernel;
+    a->kv_heads_per_group = c.kv_heads_per_group;
+    a->q_heads_per_pass = c.q_heads_per_pass;
+    a->num_passes = c.num_passes;
+    a->wg_tokens = c.wg_tokens;
+    a->min_tokens_per_range = decode_floor_tokens_per_range(c.wg_tokens);
+    choose_form(a, compute_units);
+    return DecodeSelect::kSelected;
+}
+
+int decode_wg_tokens(int head_dim, int kv_heads_per_group)
+{
+    const int lps = head_dim == 64 ? 4 : (head_dim == 256 ? 16 : 8); // lanes per slot
+    return kDecodeSlotTokens * (64 / lps / kv_heads_per_group) * kDecodeGeneralWaves;
 }
 
 // Short chunks (a few query tokens per sequence: speculative decoding's candidates, the tail of a chunked prefill)

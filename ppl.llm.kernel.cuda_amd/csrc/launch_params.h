@@ -67,7 +67,7 @@ struct DecodeLaunch {
     int32_t wg_tokens;            // tokens one workgroup iteration covers: the unit of the range cuts, a property
                                   // of the kernel named by `kernel` (the combine kernel derives the same cuts from it)
     int32_t min_tokens_per_range;
-    int32_t by_sequence;          // one range, quad and column kernels: workgroup x takes sequence x whole (and writes the rows of an empty one)
+    int32_t by_sequence;          // one range: workgroup x takes sequence x whole (quad and column kernels: and writes the rows of an empty one)
     int32_t shared_pieces;        // column kernels: waves per kv head that share the tokens of a piece (1, 4 or 8)
     int32_t kernel;               // DecodeKernel that runs the token ranges; never kDecodeKernelAuto at launch
     // Chunks of a few query tokens per sequence on the 32-column kernel (nullptr = one query token per sequence, row =
@@ -290,34 +290,27 @@ struct DecodeChoice {
 // The kernel that serves a shape, and the grouping it implies.  `requested` kDecodeKernelAuto picks by shape;
 // any other value insists on that kernel and the call fails (false) when it cannot serve the shape.
 bool decode_choose(int64_t head_dim, int64_t num_heads, int64_t num_kv_heads, int32_t requested, DecodeChoice* out);
-// Makes the choice fit a cache layout: the kernels address a row as a 64-bit base per wave plus a 32-bit offset per
-// lane, and where the kv heads of a wave lie further apart than such an offset reaches (cache_stride_h of a layout
-// that keeps the heads outermost) the general kernel takes fewer kv heads per workgroup and, unless the quad kernel
-// was requested, a kernel with a wave per kv head takes its steps.  The number of ranges of a plan stays valid: it
-// does not depend on the grouping.  False: no kernel serves the strides (a block of tokens alone spans 2 GiB, or a
-// stride is negative).
-bool decode_fit_cache_strides(int64_t head_dim, int64_t num_heads, int64_t num_kv_heads, int32_t requested,
-                              int64_t stride_s, int64_t stride_h, DecodeChoice* c);
 // What the quad kernel needs of a launch beyond the C ABI's own checks: 16-byte aligned output rows and,
 // with attn_mask, one set of waves and mask offsets within 32 bits.
 bool decode_quad_launch_ok(const DecodeLaunch& a);
 // The column kernels (decode_attn_columns.hip, decode_attn_mfma.hip) for any head_dim and number of columns per kv head: what short chunks and
 // batches taken sequence by sequence run on (as requests of the C ABI they serve fewer shapes, decode_choose).
 bool decode_choose_columns(int64_t head_dim, int64_t columns, int64_t num_kv_heads, DecodeChoice* out);
-// The kernel of a launch without a request, from the choice by shape (`c`, replaced) and the number of ranges: a single
-// range means that every sequence is taken whole by workgroups of its own.
-bool decode_choose_launch(int64_t sequences, int64_t ranges, int64_t head_dim, int64_t num_heads, int64_t num_kv_heads, int compute_units,
-                          DecodeChoice* c);
 // The number of ranges of a plan.  `automatic`: no kernel was requested.
 int64_t decode_choose_ranges(const DecodeChoice& by_shape, int64_t sequences, int64_t max_kvlen, int64_t head_dim, int64_t num_heads,
                              int64_t num_kv_heads, int compute_units, bool automatic);
 // A single sequence of more tokens is cut as any other stream.
 constexpr int64_t kSharedStreamTokens = 32768;
-// How the kernel takes the launch: by_sequence and shared_pieces.
-void decode_choose_form(DecodeLaunch* a, int compute_units);
+// The kernel of a launch whose shape, ranges, strides and buffers are filled in, and how it takes it: the fields from
+// kv_heads_per_group on.  A single range without a request means that every sequence is taken whole by workgroups of its own.
+// `columns`: the column kernels whatever the shape.  `out`: the choice, also where its strides were refused.
+enum class DecodeSelect { kSelected, kNoKernel, kQuadBuffers, kCacheStrides };
+DecodeSelect decode_select(DecodeLaunch* a, int32_t requested, bool columns, int compute_units, DecodeChoice* out);
 const char* decode_kernel_name(const DecodeLaunch& a);
 const char* decode_kernel_name(int32_t kernel); // over token ranges
-int decode_wg_tokens(int head_dim, int kv_heads_per_group); // of the general kernel
+int decode_wg_tokens(int head_dim, int kv_heads_per_group); // of the general kernel:
+constexpr int kDecodeSlotTokens = 4;   // tokens of a slot per iteration
+constexpr int kDecodeGeneralWaves = 4; // waves of a workgroup
 constexpr int kDecodeQuadTokens = 16;
 constexpr int kDecodeMfmaWavesPerCu = 8; // 20 KB of LDS per wave
 constexpr int kDecodeMfmaTokens = 32;

@@ -1,0 +1,67 @@
+"""Which kernel a decode call runs and whether it takes its sequences whole, on the CPU: csrc/decode_select.cpp compiled with
+g++ behind a small program that reads calls and prints the decision for a given number of compute units."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+GENERAL, QUAD, MFMA16, MFMA32, MFMA = ("decode_attention_kernel", "decode_attention_quad_kernel", "decode_attention_mfma16_kernel",
+                                       "decode_attention_mfma32_kernel", "decode_attention_mfma_kernel")
+
+
+@pytest.fixture(scope="module")
+def select(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("select") / "decode_select_check")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Wno-unused-function", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(ROOT, "ppl.llm.kernel.cuda_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "select", "decode_select_check.cpp"), "-o", exe], check=True, timeout=300)
+
+    def call(sequences, heads, kv_heads, head_dim, max_kvlen, ranges=0, mask=False, output_offset=0, output_stride=None, stride_s=None,
+             stride_h=None, scale=0.088, requested=0, cus=256):
+        """(kernel, ranges, whole sequences) of one call, or ("refused", ranges, reason)"""
+        d = head_dim
+        fields = (sequences, max_kvlen, ranges, heads, kv_heads, d, int(mask), output_offset,
+                  heads * d if output_stride is None else output_stride, 2 * kv_heads * d if stride_s is None else stride_s,
+                  d if stride_h is None else stride_h, scale, requested, cus)
+        out = subprocess.run([exe], input=" ".join(str(f) for f in fields) + "\n", capture_output=True, text=True, check=True, timeout=60).stdout.split()
+        if len(out) < 4:
+            return "refused", int(out[1]) if len(out) > 1 else 0, out[0]
+        return out[0], int(out[1]), out[2] == "1"
+    return call
+
+
+MANY_SHORT = [(512, 32, 8, 128, 300), (128, 32, 32, 128, 400), (512, 8, 8, 64, 300), (512, 16, 8, 256, 150), (600, 9, 9, 64, 100)]
+
+
+@pytest.mark.parametrize("shape", MANY_SHORT)
+def test_many_short_sequences_are_taken_whole_whatever_the_mask_and_the_buffers(select, shape):
+    """The plan of one range knows neither mask nor output: a kernel over ranges would walk the batch with one workgroup."""
+    assert select(*shape) == (QUAD, 1, True)
+    hq, d = shape[1], shape[3]
+    instead = GENERAL if shape[1:4] == (8, 8, 64) else MFMA16
+    assert select(*shape, mask=True) == (instead if d == 64 else QUAD, 1, True)  # the quad kernel has no mask form at head_dim 64
+    for form in (dict(output_offset=8), dict(output_stride=hq * d + 4), dict(mask=True, output_offset=8)):
+        assert select(*shape, **form) == (instead, 1, True), form
+
+
+@pytest.mark.parametrize("form", [dict(), dict(mask=True), dict(output_offset=8)])
+def test_a_single_range_without_a_request_is_never_one_workgroup(select, form):
+    for hq, hkv, d in [(8, 8, 64), (32, 8, 64), (14, 2, 64), (5, 1, 64), (32, 32, 96), (40, 1, 96), (32, 32, 128), (32, 8, 128), (64, 8, 128),
+                       (28, 4, 128), (8, 1, 128), (5, 5, 128), (48, 1, 128), (16, 16, 256), (16, 8, 256), (8, 1, 256), (24, 1, 256)]:
+        for n in (1, 4, 5, 60, 512, 3000):
+            kernel, ranges, whole = select(n, hq, hkv, d, 200, ranges=1, **form)
+            assert whole and ranges == 1, (n, hq, hkv, d, kernel)
+
+
+def test_ranges_and_requests_keep_their_kernels(select):
+    assert select(64, 32, 8, 128, 4096)[::2] == (QUAD, False)
+    assert select(64, 32, 8, 128, 4096, mask=True)[::2] == (QUAD, False)
+    assert select(64, 32, 8, 128, 4096, output_offset=8)[::2] == (GENERAL, False)
+    assert select(64, 8, 8, 64, 4096, mask=True)[::2] == (GENERAL, False)
+    assert select(64, 64, 8, 128, 4096, mask=True)[::2] == (MFMA16, False)
+    assert select(64, 48, 1, 128, 4096)[::2] == (MFMA, False)
+    assert select(2, 32, 8, 128, 8192, mask=True)[::2] == (MFMA16, False)
+    assert select(512, 32, 8, 128, 300, requested=2)[0] == QUAD
+    assert select(512, 32, 8, 128, 300, requested=2, output_offset=8)[::2] == ("refused", "quad-buffers")
+    assert select(512, 32, 8, 128, 300, requested=1)[0] == GENERAL

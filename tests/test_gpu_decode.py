@@ -361,3 +361,46 @@ def test_decode_of_a_few_sequences(pkg, oracle, shape, lens, cache_mode):
     for ranges in (0, 2, 9, 40):
         got, plan = run_decode(dev, ranges)
         assert_attention_close(got, ref, "%s %s ranges %d" % (shape, lens, plan.num_token_ranges))
+
+
+@pytest.mark.parametrize("cache_mode", [0, 1])
+@pytest.mark.parametrize("shape,sequences", [((8, 8, 64), 512), ((9, 9, 64), 456), ((12, 12, 128), 342), ((16, 8, 128), 512), ((18, 9, 256), 456)])
+def test_many_short_sequences_with_mask_and_unaligned_rows(pkg, oracle, shape, sequences, cache_mode):
+    """At least 16 (sequence, kv head) pairs per compute unit and a plan of one range, which the quad kernel takes where it can:
+    output rows that are only 8-byte aligned, and a mask at head_dim 64, go to the column or the general kernel, which take the
+    sequences whole as well."""
+    hq, hkv, d = shape
+    bt, dev, q, cache, scale = make_case(pkg, oracle, 640 + hq + d, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=cache_mode,
+                                         dec_kv_lens=[EDGES[i % 13] + 160 * (i % 7 == 3) for i in range(sequences)], outliers=True)
+    empty = [0, 6, sequences - 1]
+    bt.kv_lens[empty] = 0
+    bt.kvstarts = np.concatenate([[0], np.cumsum(bt.kv_lens)]).astype(np.int64)
+    dev.kvstarts.copy_(torch.from_numpy(bt.kvstarts))
+    assert dev.decode_only(1, name_only=True) == "decode_attention_quad_kernel"
+    instead = "decode_attention_kernel" if shape == (8, 8, 64) else "decode_attention_mfma16_kernel"
+    # a mask's rows may overlap: (head, sequence, token) is element 24 head + 8 sequence + token of one row of values
+    rng = np.random.default_rng(11)
+    mask = rng.standard_normal(24 * hq + 8 * sequences + int(bt.kvstarts[-1])).astype(np.float16)
+    mask[rng.random(mask.shape) < 0.05] = -np.inf
+    mask[rng.random(mask.shape) < 0.02] = np.float16(-65504)
+    strides = dict(mask_stride_s=8, mask_stride_h=24)
+    md = torch.from_numpy(mask).cuda()
+    assert dev.decode_only(1, attn_mask=md, name_only=True, **strides) == (instead if d == 64 else "decode_attention_quad_kernel")
+    ref = oracle_decode(oracle, bt, q, cache, scale, attn_mask=mask, **strides)
+    got, plan = run_decode(dev, 1, attn_mask=md, **strides)
+    seen = np.isfinite(ref)  # a row whose every token is masked with -inf has no softmax
+    assert seen.mean() > 0.9
+    assert_attention_close(np.where(seen, got, 0), np.where(seen, ref, 0), "mask %s" % (shape,))
+    assert (got[empty] == 0).all()
+
+    n, row = sequences, hq * d + 4
+    buf = torch.full((n * row + 8,), float("nan"), dtype=torch.float16, device="cuda")
+    out = buf[4:]
+    assert dev.decode_only(1, output=out, output_stride_s=row, name_only=True) == instead
+    dev.decode_only(1, output=out, output_stride_s=row)
+    torch.cuda.synchronize()
+    ref = oracle_decode(oracle, bt, q, cache, scale)
+    rows = buf[4:4 + n * row].view(n, row)
+    assert_attention_close(rows[:, :hq * d].float().cpu().numpy().reshape(n, hq, d), ref, "rows of 8 bytes %s" % (shape,))
+    assert (rows[empty, :hq * d] == 0).all()
+    assert torch.isnan(rows[:, hq * d:]).all() and torch.isnan(buf[:4]).all()
