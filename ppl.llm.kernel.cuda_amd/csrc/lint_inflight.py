@@ -12,8 +12,6 @@ statement.  Exit status 1 when it finds either: such a kernel must not run.
 
     hipcc ... --cuda-device-only -S file.hip -o file.s && python3 lint_inflight.py file.s
 """
-import contextlib
-import io
 import re
 import sys
 
@@ -91,74 +89,6 @@ def lint(name, lines):
     return problems, asm_loads, hazards
 
 
-def clean_on_every_path(lines):
-    """Whether no instruction touches a register with a hand-scheduled load in flight on any path through the kernel's branches
-    (taken or not, whatever their conditions).  The text order of lint() follows the compiler's block layout: a block that runs
-    before a load may stand behind it.  A state is the queue of outstanding operations from the oldest hand-scheduled
-    load with a destination on; False also where there are too many states to visit."""
-    blocks, label, cur = [], {}, []
-    in_asm = False
-    for raw in lines:
-        t = raw.strip()
-        if t.startswith(';;#ASMSTART') or t.startswith(';;#ASMEND'):
-            in_asm = t.startswith(';;#ASMSTART')
-            continue
-        m = re.match(r'^(\.LBB\w+):', t)
-        if m:
-            blocks.append(cur)
-            cur = []
-            label[m.group(1)] = len(blocks)
-            continue
-        if not t or t.startswith(';') or t.startswith('.') or t.endswith(':'):
-            continue
-        t = t.split(';')[0].strip()
-        cur.append((t, in_asm))
-        if t.split()[0].startswith(('s_branch', 's_cbranch')):
-            blocks.append(cur)
-            cur = []
-    blocks.append(cur)
-
-    def step(block, queue):
-        for t, from_asm in block:
-            op = t.split()[0]
-            if op == 's_waitcnt':
-                m = re.search(r'vmcnt\((\d+)\)', t)
-                if m:
-                    queue = queue[max(0, len(queue) - int(m.group(1))):]
-            else:
-                pending = set().union(*queue) if queue else set()
-                memory = op.startswith(LOADS) or op.startswith(STORES)
-                if pending & registers(t):
-                    return None
-                if memory:
-                    has_dst = op.startswith(LOADS) and '_load_lds_' not in op
-                    queue = queue + (frozenset(registers(t.split(',')[0])) if from_asm and has_dst else frozenset(),)
-            while queue and not queue[0]:
-                queue = queue[1:]
-        return queue
-
-    seen = [set() for _ in blocks]
-    todo = [(0, ())]
-    visits = 0
-    while todo:
-        i, queue = todo.pop()
-        if i >= len(blocks) or queue in seen[i]:
-            continue
-        seen[i].add(queue)
-        visits += 1
-        if visits > 20000:
-            return False
-        queue = step(blocks[i], queue)
-        if queue is None:
-            return False
-        last = blocks[i][-1][0].split() if blocks[i] else ['']
-        if last[0].startswith(('s_branch', 's_cbranch')):
-            todo.append((label[last[1]], queue))
-        if last[0] != 's_branch':
-            todo.append((i + 1, queue))
-    return True
-
-
 def main():
     total = 0
     checked = 0
@@ -169,19 +99,13 @@ def main():
             m = re.match(r'^(_Z\S+):', src[i])
             if m and '.' not in m.group(1):
                 j = i + 1
-                while j < len(src) and 's_endpgm' not in src[j]:
+                while j < len(src) and not src[j].startswith('.Lfunc_end') and not re.match(r'^_Z\S+:', src[j]):
                     j += 1
-                with io.StringIO() as said:
-                    with contextlib.redirect_stdout(said):
-                        problems, asm_loads, hazards = lint(m.group(1), src[i:j])
-                    if problems and clean_on_every_path(src[i:j]):
-                        problems = 0
-                    if problems or hazards:
-                        print(said.getvalue(), end='')
+                problems, asm_loads, hazards = lint(m.group(1), src[i:j])
                 if asm_loads:
                     checked += 1
                 total += (problems if asm_loads else 0) + hazards
-                i = j
+                i = j - 1
             i += 1
     print("lint_inflight: %d hand-scheduled kernels checked, %d problems" % (checked, total))
     return 1 if total or not checked else 0

@@ -24,6 +24,11 @@ def asm_load(dst, addr="v2", base="s[4:5]"):
     return [";;#ASMSTART", "global_load_dwordx4 %s, %s, %s nt" % (dst, addr, base), ";;#ASMEND"]
 
 
+def asm_load_lds(addr="v2", base="s[4:5]"):
+    """a load into LDS: no destination register, but a place in the queue"""
+    return [";;#ASMSTART", "s_mov_b32 m0, s8", "s_nop 0", "global_load_lds_dwordx4 %s, %s" % (addr, base), ";;#ASMEND"]
+
+
 def asm_wait(n):
     return [";;#ASMSTART", "s_waitcnt vmcnt(%d)" % n, ";;#ASMEND"]
 
@@ -36,6 +41,12 @@ CLEAN = (asm_load("v[10:13]") + asm_load("v[14:17]") + ["v_add_u32 v2, v2, v3", 
 def test_clean_schedule_is_accepted(lint):
     problems, asm_loads, hazards = lint.lint("clean", CLEAN)
     assert (problems, asm_loads, hazards) == (0, 2, 0)
+
+
+def test_loads_into_lds_are_counted_and_have_no_destination(lint):
+    lines = (asm_load("v[10:13]") + asm_load_lds("v2") + ["v_add_u32 v2, v2, v3"] + asm_load_lds("v2") + asm_wait(2)
+             + ["v_perm_b32 v30, v10, v11, s8", "s_endpgm"])
+    assert lint.lint("lds", lines) == (0, 3, 0)
 
 
 @pytest.mark.parametrize("what,lines", [
@@ -51,6 +62,12 @@ def test_clean_schedule_is_accepted(lint):
      asm_load("v[10:13]") + ["global_load_dword v11, v2, s[4:5]"] + asm_wait(0)),
     ("staging register used as an address",
      asm_load("v[10:13]") + ["global_load_dword v50, v10, s[4:5]"] + asm_wait(0)),
+    ("asm load into a register with a load of the compiler in flight",
+     ["global_load_dwordx4 v[10:13], v2, s[4:5]"] + asm_load("v[10:13]") + asm_wait(0)),
+    ("load into LDS from an address that is still in flight",
+     asm_load("v[10:13]") + asm_load_lds("v10") + asm_wait(0)),
+    ("wait that counts a load into LDS behind the load it is for",
+     asm_load("v[10:13]") + asm_load_lds("v2") + asm_wait(2) + ["v_perm_b32 v31, v10, v11, s8"]),
     ("staging register stored before its wait",
      asm_load("v[10:13]") + ["global_store_dword v2, v13, s[6:7]"] + asm_wait(0)),
 ])
@@ -66,6 +83,17 @@ def test_transcendental_result_read_by_the_next_asm_instruction(lint):
     assert lint.lint("trans", spaced)[2] == 0
     other_reg = ["v_exp_f32_e32 v5, v4", ";;#ASMSTART", "v_mul_f32 v6, v8, v7", ";;#ASMEND"]
     assert lint.lint("trans", other_reg)[2] == 0
+
+
+def test_the_command_waives_no_hazard_that_lint_reports(lint, tmp_path, monkeypatch):
+    """whatever the branches around it"""
+    hazards = [m.args[1] for m in test_register_hazards_are_rejected.pytestmark if m.name == "parametrize"][0]
+    for what, lines in hazards:
+        for body in (lines, ["s_cbranch_scc1 .LBB0_2"] + lines + [".LBB0_2:"], ["s_branch .LBB0_2", ".LBB0_1:", "s_endpgm", ".LBB0_2:"] + lines):
+            path = tmp_path / "k.s"
+            path.write_text("_Z6kernelv:\n" + "\n".join(body) + "\ns_endpgm\n.Lfunc_end0:\n")
+            monkeypatch.setattr("sys.argv", ["lint_inflight.py", str(path)])
+            assert lint.main() == 1, what
 
 
 def test_the_command_fails_on_a_hazard_and_on_nothing_to_check(lint, tmp_path, monkeypatch, capsys):
