@@ -227,6 +227,16 @@ int pmxhip_decode_plan_make_kernel(int64_t decoding_batches, int64_t num_heads, 
                                    int64_t max_kvlen, int32_t compute_units, int32_t num_token_ranges_hint,
                                    int32_t kernel_request, pmxhip_decode_plan* plan)
 {
+    return pmxhip::decode_plan_make(decoding_batches, num_heads, num_kv_heads, head_dim, max_kvlen, compute_units,
+                                    num_token_ranges_hint, kernel_request, false, plan);
+}
+
+} // extern "C"
+
+int pmxhip::decode_plan_make(int64_t decoding_batches, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim, int64_t max_kvlen,
+                             int32_t compute_units, int32_t num_token_ranges_hint, int32_t kernel_request, bool mask,
+                             pmxhip_decode_plan* plan)
+{
     if (!plan) return fail(PMXHIP_INVALID_VALUE, "decode_plan: null plan");
     memset(plan, 0, sizeof(*plan));
     if (!head_dim_supported(head_dim))
@@ -246,7 +256,7 @@ int pmxhip_decode_plan_make_kernel(int64_t decoding_batches, int64_t num_heads, 
         const int cus = compute_units > 0 ? compute_units : current_compute_units();
         if (cus <= 0) return fail(PMXHIP_INVALID_VALUE, "decode_plan: compute_units not given and no current device");
         ranges = pmxhip::decode_choose_ranges(c, decoding_batches, max_kvlen, head_dim, num_heads, num_kv_heads, cus,
-                                              kernel_request == PMXHIP_DECODE_KERNEL_AUTO);
+                                              kernel_request == PMXHIP_DECODE_KERNEL_AUTO, mask);
     }
     plan->num_token_ranges = (int32_t)ranges;
     plan->kv_heads_per_group = c.kv_heads_per_group;
@@ -261,6 +271,8 @@ int pmxhip_decode_plan_make_kernel(int64_t decoding_batches, int64_t num_heads, 
     plan->workspace_size = plan->partial_out_size + plan->partial_ml_size;
     return PMXHIP_SUCCESS;
 }
+
+extern "C" {
 
 namespace {
 

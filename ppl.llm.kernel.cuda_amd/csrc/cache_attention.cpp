@@ -197,8 +197,8 @@ ppl::common::RetCode dynamic_batching_multi_head_cache_attention::heuristic_prep
     memset(&plan, 0, sizeof(plan));
     if (decoding_batches > 0) {
         const int32_t hint = specify_decoding_multi_block == 0 ? 1 : 0;
-        const int rc = pmxhip_decode_plan_make(decoding_batches, num_heads, num_kv_heads, head_dim, max_kvlen,
-                                               device_prop.multiProcessorCount, hint, &plan);
+        const int rc = pmxhip::decode_plan_make(decoding_batches, num_heads, num_kv_heads, head_dim, max_kvlen,
+                                                device_prop.multiProcessorCount, hint, PMXHIP_DECODE_KERNEL_AUTO, attn_mask != nullptr, &plan);
         // an unsupported head_dim is reported by forward_decode, as in the reference (kernel.cu:1975-2006)
         if (rc != PMXHIP_SUCCESS) memset(&plan, 0, sizeof(plan));
     }

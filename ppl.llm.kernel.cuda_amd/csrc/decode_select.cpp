@@ -219,57 +219,16 @@ int decode_share(int64_t workgroups, int64_t head_dim, int compute_units)
 }
 
 // The quad kernel takes its shapes sequence by sequence where every one of its waves (two kv heads, eight to a CU) has a sequence to
-// begin with: 32 q / 8 kv heads of 128, 512 sequences of 100-300 tokens 57 us, 61 on the column kernel, 68 cut into ranges.  With a
-// mask, whose values the column kernel waits for together with its rows, from where that kernel's waves come in a second round: the
-// same heads, 300 sequences of 100-300 48.8 us, 56.9 on the column kernel; 16 / 4 heads, 512 of them 47.3 and 45.1.
+// begin with: 32 q / 8 kv heads of 128, 512 sequences of 100-300 tokens 57 us, 61 on the column kernel, 68 cut into ranges.  With
+// one query head per kv head, a quarter of the column kernel's work, from where that kernel has a wave per pair: 32 / 32 heads of
+// 128, 100 sequences of 43-128 23.5 us, 31.4 on the column kernel, 26.8 over ranges.  With a mask, whose values the column kernel
+// waits for together with its rows, from where that kernel's waves come in a second round: 32 / 8 heads, 300 sequences of 100-300
+// 48.8 us, 56.9 on the column kernel; 16 / 4 heads, 512 of them 47.3 and 45.1.
 bool quad_by_sequence(int64_t sequences, int64_t num_kv_heads, int64_t g, bool mask, int compute_units)
 {
     if (g > 4 || compute_units <= 0) return false;
     const int64_t pairs = sequences * num_kv_heads;
-    return pairs >= 16 * (int64_t)compute_units || (mask && pairs > 8 * (int64_t)compute_units);
-}
-
-// What a batch costs (us) sequence by sequence, and cut into ranges with a combine launch behind it: fits to timings of 11
-// head shapes x 1-256 sequences x 256-16384 tokens (lengths L/3 to L), within 20 % of nearly all of them.  Only their
-// order is used.
-constexpr double kSequenceMargin = 0.8; // (estimates: a batch goes sequence by sequence where that is clearly the cheaper one)
-// A wave's block of 32 tokens takes `alone` with a wave per SIMD and `shared` with two; a workgroup starts in 3.5.
-// `quad`: the rate of the quad kernel, where that is the one for the shape (0: the column kernels).
-double sequence_cost(int64_t sequences, int64_t max_kvlen, int64_t head_dim, int64_t columns, int64_t num_kv_heads, int cus, double quad = 0)
-{
-    const int64_t wgs = sequences * column_groups(head_dim, columns, num_kv_heads);
-    const double wide = columns > kDecodeMfma16Columns && head_dim != 256 ? 1.15 : 1.0;
-    const double shared = wide * (head_dim == 64 ? 1.6 : head_dim == 96 ? 2.6 : head_dim == 128 ? 3.0 : 4.6);
-    const double alone = wide * (head_dim == 64 ? 1.24 : head_dim == 96 ? 1.55 : head_dim == 128 ? 1.75 : 2.8);
-    const int share = decode_share(wgs, head_dim, cus);
-    const double blocks = (double)((max_kvlen + 32 * share - 1) / (32 * share));
-    if (share == 8) return 4.4 + shared * blocks * (wgs > cus ? 2 : 1);
-    if (share == 4 && wgs <= cus) return 4.4 + alone * blocks;
-    if (share == 4 && wgs <= 2 * cus) return 4.6 + shared * blocks;
-    if (quad > 0 && quad_by_sequence(sequences, num_kv_heads, 1, false, cus)) { // its waves have two kv heads, or one of 256 channels
-        const double rounds = sequences * num_kv_heads / (16.0 * cus);
-        return 1 + rounds * (4.5 + 0.7 * quad * 2 * blocks);
-    }
-    const double rounds = share == 4 ? wgs / (2.0 * cus) : wgs / (8.0 * cus);
-    if (rounds <= 1) return 4.5 + (wgs <= 4 * cus ? alone : shared) * blocks;
-    return 1 + rounds * (3.5 + 0.8 * shared * blocks);
-}
-double quad_rate(int64_t head_dim, int64_t g) { return head_dim == 64 ? 2.2 : (head_dim == 128 ? (g == 1 ? 2.4 : 3.5) : (g == 1 ? 4.8 : (g <= 4 ? 5.7 : 12.0))); }
-double ranges_cost(const DecodeChoice& c, int64_t sequences, int64_t max_kvlen, int64_t head_dim, int64_t g, int64_t num_kv_heads, int cus)
-{
-    // waves' blocks of 32 tokens and one kv head, two more for the start and the end of a sequence
-    const double blocks = (double)(sequences * num_kv_heads * (c.kernel == kDecodeKernelQuad ? 1 : c.num_passes)) *
-                          (0.67 * (double)max_kvlen / 32 + 2);
-    double each = 0; // us for eight of them on every CU
-    switch (c.kernel) {
-        case kDecodeKernelQuad:
-            each = quad_rate(head_dim, g);
-            break;
-        case kDecodeKernelMfma16: each = 3.6; break;
-        case kDecodeKernelMfma32: each = head_dim == 64 ? 2.3 : 4.7; break;
-        default: each = 2.7 * (double)head_dim / 96; break;
-    }
-    return 12 + each * blocks / (8.0 * cus);
+    return pairs >= 16 * (int64_t)compute_units || (g == 1 && pairs > 5 * (int64_t)compute_units) || (mask && pairs > 8 * (int64_t)compute_units);
 }
 
 // One to four sequences cut into ranges run on the column kernels where those are the faster ones: 32 q / 8 kv heads of 128, one
@@ -284,6 +243,88 @@ bool few_sequences_on_columns(int64_t sequences, int64_t head_dim, int64_t g)
 
 // The quad kernel's form for whole sequences has one set of waves.
 bool quad_takes_whole(const DecodeLaunch& a) { return a.num_kv_repeats <= 4 && decode_quad_launch_ok(a); }
+
+// How long the sequences of a batch may be (its longest) to be taken whole instead of cut into ranges with a combine launch
+// behind them, by the (sequence, kv head, pass) workgroups per CU: the crossing of the two times, measured over 30 head shapes x
+// 1-512 sequences x 64-16384 tokens and short chunks of 1-32 columns, lengths L / 3 to L, ten layers in turn.  Where shapes of
+// a row differ the shorter one stands, so that a batch next to the line is seldom slower than over ranges (of 1900 batches 3 by
+// more than 8 %).  Few workgroups leave the chip idle and ranges fill it; from one per CU on the waves are there either
+// way, and ranges even out the lengths.  Past eight per CU the waves come in a second round.
+struct WholeUpTo {
+    double masked;         // with a mask, times this: the column kernels wait for its values, the quad kernel streams them
+    int32_t tokens[15];    // workgroups per CU up to kWholeLoads[i], and beyond
+};
+constexpr double kWholeLoads[14] = {0.05, 0.1, 0.2, 0.4, 0.75, 1, 1.6, 2, 2.75, 3.5, 5, 8, 15.99, 32};
+constexpr WholeUpTo kWholeColumns16 = {0.6, {440, 470, 500, 660, 825, 1150, 765, 765, 595, 590, 520, 500, 400, 500, 500}};
+constexpr WholeUpTo kWholeColumns32 = {0.6, {280, 330, 390, 580, 1300, 1600, 1400, 1400, 1290, 1200, 1200, 900, 700, 600, 600}};
+constexpr WholeUpTo kWholeColumns64 = {0.9, {600, 710, 740, 1030, 1500, 1030, 800, 560, 700, 550, 650, 720, 400, 550, 550}}; // head_dim 64
+constexpr WholeUpTo kWholeQuad64 = {0.45, {850, 850, 850, 1600, 1600, 1300, 800, 600, 560, 560, 530, 380, 380, 900, 900}};
+constexpr WholeUpTo kWholeQuad128One = {1.0, {480, 480, 510, 610, 620, 700, 350, 295, 175, 175, 140, 500, 220, 200, 200}}; // one query head per kv head
+constexpr WholeUpTo kWholeQuad128 = {0.6, {500, 570, 600, 800, 970, 1000, 880, 680, 640, 340, 300, 300, 150, 400, 400}};
+constexpr WholeUpTo kWholeQuad256One = {1.0, {400, 400, 400, 410, 420, 430, 250, 185, 90, 90, 0, 190, 190, 190, 190}};
+constexpr WholeUpTo kWholeQuad256 = {0.55, {450, 450, 470, 600, 760, 780, 550, 500, 300, 260, 160, 160, 160, 200, 200}};
+constexpr WholeUpTo kWholeQuad256Two = {1.0, {450, 570, 590, 1140, 1600, 1600, 1600, 1600, 1600, 1600, 1600, 1600, 1600, 1600, 1600}}; // two sets of waves
+constexpr WholeUpTo kWholeGeneralOne = {0.75, {580, 580, 600, 800, 520, 560, 350, 285, 200, 170, 145, 145, 128, 100, 0}};
+constexpr WholeUpTo kWholeGeneralFour = {1.0, {930, 930, 1100, 1600, 1600, 1600, 980, 980, 700, 600, 560, 500, 370, 530, 530}};
+constexpr int32_t kAnyLength = INT32_MAX; // many query heads on the general kernel: several times the column kernels' time
+constexpr WholeUpTo kWholeGeneral = {1.0, {870, 1400, 1400, kAnyLength, kAnyLength, kAnyLength, kAnyLength, kAnyLength, kAnyLength, kAnyLength,
+                                           kAnyLength, kAnyLength, kAnyLength, kAnyLength, kAnyLength}};
+
+const WholeUpTo& whole_row(const DecodeChoice& by_shape, int64_t head_dim, int64_t g, int64_t num_kv_heads)
+{
+    switch (by_shape.kernel) {
+        case kDecodeKernelMfma16: return kWholeColumns16;
+        case kDecodeKernelMfma32: return head_dim == 64 ? kWholeColumns64 : kWholeColumns32;
+        case kDecodeKernelQuad:
+            if (head_dim == 64) return kWholeQuad64;
+            if (head_dim == 128) return g == 1 ? kWholeQuad128One : kWholeQuad128;
+            return g == 1 ? kWholeQuad256One : (g <= 4 ? kWholeQuad256 : kWholeQuad256Two);
+        default: return head_dim == 96 && num_kv_heads > 1 && g <= 4 ? (g == 1 ? kWholeGeneralOne : kWholeGeneralFour) : kWholeGeneral;
+    }
+}
+
+// `columns`: query heads per kv head, or the (position, head) columns of a short chunk
+int64_t whole_up_to(const DecodeChoice& by_shape, int64_t sequences, int64_t head_dim, int64_t columns, int64_t num_kv_heads, bool mask, int cus)
+{
+    const WholeUpTo& row = whole_row(by_shape, head_dim, columns, num_kv_heads);
+    const double load = (double)(sequences * column_groups(head_dim, columns, num_kv_heads)) / cus;
+    int i = 0;
+    while (i < 14 && load > kWholeLoads[i]) ++i;
+    int64_t tokens = row.tokens[i];
+    const bool other_kernel = by_shape.kernel == kDecodeKernelQuad && head_dim == 64 && columns > 1; // (no mask form there)
+    if (mask && tokens != kAnyLength && !other_kernel) tokens = (int64_t)(row.masked * (double)tokens);
+    // the pieces of few columns cost less, those of many more (32 / 8 heads of 128, 100 chunks of one row: level at 476 tokens, of two
+    // rows at 616, of four at 957)
+    if (by_shape.kernel != kDecodeKernelQuad && by_shape.kernel != kDecodeKernelGeneral && load > 1) {
+        if (columns < 5) tokens = tokens * 3 / 5;
+        else if (columns >= 12 && columns <= kDecodeMfma16Columns) tokens = tokens * 5 / 4;
+        else if (columns > kDecodeMfmaColumns && head_dim == 64) tokens *= 2; // (the range kernel's passes: 71 / 1 heads, 300 of 1600)
+    }
+    if (by_shape.kernel == kDecodeKernelMfma32 && head_dim == 64 && sequences <= kFewSequences && tokens > 590) tokens = 590;
+    // a step of a few sequences has ranges of the column kernels' own
+    if (by_shape.kernel == kDecodeKernelQuad && few_sequences_on_columns(sequences, head_dim, columns))
+        tokens = tokens < (head_dim == 64 ? 700 : 480) ? tokens : (head_dim == 64 ? 700 : 480);
+    return tokens;
+}
+
+// What short chunks cost (us) sequence by sequence, against the tile kernel.  A wave's block of 32 tokens takes `alone` with a wave
+// per SIMD and `shared` with two; a workgroup starts in 3.5.
+constexpr double kSequenceMargin = 0.8;
+double sequence_cost(int64_t sequences, int64_t max_kvlen, int64_t head_dim, int64_t columns, int64_t num_kv_heads, int cus)
+{
+    const int64_t wgs = sequences * column_groups(head_dim, columns, num_kv_heads);
+    const double wide = columns > kDecodeMfma16Columns && head_dim != 256 ? 1.15 : 1.0;
+    const double shared = wide * (head_dim == 64 ? 1.6 : head_dim == 96 ? 2.6 : head_dim == 128 ? 3.0 : 4.6);
+    const double alone = wide * (head_dim == 64 ? 1.24 : head_dim == 96 ? 1.55 : head_dim == 128 ? 1.75 : 2.8);
+    const int share = decode_share(wgs, head_dim, cus);
+    const double blocks = (double)((max_kvlen + 32 * share - 1) / (32 * share));
+    if (share == 8) return 4.4 + shared * blocks * (wgs > cus ? 2 : 1);
+    if (share == 4 && wgs <= cus) return 4.4 + alone * blocks;
+    if (share == 4 && wgs <= 2 * cus) return 4.6 + shared * blocks;
+    const double rounds = share == 4 ? wgs / (2.0 * cus) : wgs / (8.0 * cus);
+    if (rounds <= 1) return 4.5 + (wgs <= 4 * cus ? alone : shared) * blocks;
+    return 1 + rounds * (3.5 + 0.8 * shared * blocks);
+}
 
 } // namespace
 
@@ -311,16 +352,13 @@ static void choose_launch(const DecodeLaunch& a, int compute_units, DecodeChoice
 }
 
 int64_t decode_choose_ranges(const DecodeChoice& by_shape, int64_t sequences, int64_t max_kvlen, int64_t head_dim, int64_t num_heads,
-                             int64_t num_kv_heads, int compute_units, bool automatic)
+                             int64_t num_kv_heads, int compute_units, bool automatic, bool mask)
 {
     const int64_t g = num_heads / num_kv_heads;
     const int64_t max_tokens = sequences * (max_kvlen > 0 ? max_kvlen : 1);
     DecodeChoice c = by_shape;
     if (automatic && compute_units > 0) {
-        const double quad = by_shape.kernel == kDecodeKernelQuad && g <= 4 ? quad_rate(head_dim, g) : 0;
-        if (sequence_cost(sequences, max_kvlen > 0 ? max_kvlen : 1, head_dim, g, num_kv_heads, compute_units, quad) <
-            kSequenceMargin * ranges_cost(by_shape, sequences, max_kvlen > 0 ? max_kvlen : 1, head_dim, g, num_kv_heads, compute_units))
-            return 1;
+        if (max_kvlen <= whole_up_to(by_shape, sequences, head_dim, g, num_kv_heads, mask, compute_units)) return 1;
         if (c.kernel == kDecodeKernelQuad && few_sequences_on_columns(sequences, head_dim, g)) decode_choose_columns(head_dim, g, num_kv_heads, &c);
     }
     const bool columns = c.kernel == kDecodeKernelMfma16 || c.kernel == kDecodeKernelMfma32;
@@ -396,7 +434,9 @@ DecodeSelect decode_select(DecodeLaunch* a, int32_t requested, bool columns, int
     if (!columns && requested == kDecodeKernelAuto) choose_launch(*a, compute_units, &c);
     if (c.kernel == kDecodeKernelQuad && !decode_quad_launch_ok(*a)) {
         if (requested == kDecodeKernelQuad) return DecodeSelect::kQuadBuffers;
-        decode_choose(a->head_dim, a->num_heads, a->num_kv_heads, kDecodeKernelGeneral, &c);
+        // (with a mask at head_dim 64: 32 / 8 heads, 100 sequences of 233-700 51.0 us on the general kernel, 40 / 8 35.2 on this one)
+        const bool columns64 = a->head_dim == 64 && a->attn_mask != nullptr && a->num_kv_repeats > 1;
+        decode_choose(a->head_dim, a->num_heads, a->num_kv_heads, columns64 ? kDecodeKernelMfma32 : kDecodeKernelGeneral, &c);
     }
     const bool fits = fit_cache_strides(a->head_dim, a->num_heads, a->num_kv_heads, requested, a->cache_stride_s, a->cache_stride_h, &c);
     *out = c;
@@ -430,11 +470,11 @@ bool prefill_chunk_shape(int64_t max_seqlen, int64_t num_heads, int64_t num_kv_h
     return max_seqlen * (num_heads / num_kv_heads) <= kPrefillChunkColumns;
 }
 
-// Chunks of up to 32 columns go sequence by sequence where the estimates say so: against ranges (equal work, the estimates differ by
-// the combine launch and the pieces; 12 % is what they err by) 64 q / 8 kv heads of 128, 147 chunks of 2-4 rows over up to 391 tokens
-// 63 -> 52 us, 16 / 4 heads, 15 of 2 over 433 17.1 -> 14.0; against the tile kernel, whose workgroups have 256 columns for them and which
-// is what serves head_dim 96 and 256 and calls without a workspace: 16 / 16 heads of 256, 30 of 2-18 over 3208 429 -> 192 us, 8 / 1 heads
-// of 256, 178 of 1-2 over 591 59 -> 24, 32 / 32 heads of 96, four of 2 over 6971 114 -> 97.
+// Chunks of up to 32 columns go sequence by sequence where that is faster than ranges (whole_up_to) or, which is what serves head_dim 96
+// and 256 and calls without a workspace, than the tile kernel, whose workgroups have 256 columns for them: 64 q / 8 kv heads of 128, 147
+// chunks of 2-4 rows over up to 391 tokens 63 -> 52 us over ranges, 16 / 4 heads, 15 of 2 over 433 17.1 -> 14.0; against the tile kernel
+// 16 / 16 heads of 256, 30 of 2-18 over 3208 429 -> 192 us, 8 / 1 heads of 256, 178 of 1-2 over 591 59 -> 24, 32 / 32 heads of 96, four
+// of 2 over 6971 114 -> 97.
 bool prefill_by_sequence(int64_t sequences, int64_t max_seqlen, int64_t max_kvlen, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
                          bool ranges_served, int compute_units)
 {
@@ -443,8 +483,11 @@ bool prefill_by_sequence(int64_t sequences, int64_t max_seqlen, int64_t max_kvle
     const int64_t columns = max_seqlen * (num_heads / num_kv_heads);
     DecodeChoice c;
     if (columns > kMostColumns || !decode_choose_columns(head_dim, columns, num_kv_heads, &c)) return false;
+    if (ranges_served) { // (the kernel over ranges: prefill_chunk_kernel)
+        c.kernel = columns <= kDecodeMfma16Columns && head_dim == 128 ? kDecodeKernelMfma16 : kDecodeKernelMfma32;
+        return max_kvlen <= whole_up_to(c, sequences, head_dim, columns, num_kv_heads, false, compute_units);
+    }
     const double cost = sequence_cost(sequences, max_kvlen, head_dim, columns, num_kv_heads, compute_units);
-    if (ranges_served) return cost < 0.88 * ranges_cost(c, sequences, max_kvlen, head_dim, columns, num_kv_heads, compute_units);
     // the tile kernel: a workgroup per (sequence, kv head) and CU, 3.4 us for 64 kv tokens, or the tokens of few of them shared out
     const double tile = (head_dim == 256 ? 7.0 : head_dim == 64 ? 2.4 : 3.4) / 64 * (double)max_kvlen;
     const double rounds = (double)(sequences * num_kv_heads) / compute_units;

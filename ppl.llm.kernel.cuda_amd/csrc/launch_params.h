@@ -8,6 +8,8 @@
 
 #include <atomic>
 
+struct pmxhip_decode_plan;
+
 namespace pmxhip {
 
 struct QuantLaunch {
@@ -296,9 +298,12 @@ bool decode_quad_launch_ok(const DecodeLaunch& a);
 // The column kernels (decode_attn_columns.hip, decode_attn_mfma.hip) for any head_dim and number of columns per kv head: what short chunks and
 // batches taken sequence by sequence run on (as requests of the C ABI they serve fewer shapes, decode_choose).
 bool decode_choose_columns(int64_t head_dim, int64_t columns, int64_t num_kv_heads, DecodeChoice* out);
-// The number of ranges of a plan.  `automatic`: no kernel was requested.
+// The number of ranges of a plan.  `automatic`: no kernel was requested.  `mask`: the call will have one (false where the plan cannot know).
 int64_t decode_choose_ranges(const DecodeChoice& by_shape, int64_t sequences, int64_t max_kvlen, int64_t head_dim, int64_t num_heads,
-                             int64_t num_kv_heads, int compute_units, bool automatic);
+                             int64_t num_kv_heads, int compute_units, bool automatic, bool mask);
+// pmxhip_decode_plan_make_kernel for a caller that knows whether the step has a mask (c_api.cpp).
+int decode_plan_make(int64_t decoding_batches, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim, int64_t max_kvlen, int32_t compute_units,
+                     int32_t num_token_ranges_hint, int32_t kernel_request, bool mask, pmxhip_decode_plan* plan);
 // A single sequence of more tokens is cut as any other stream.
 constexpr int64_t kSharedStreamTokens = 32768;
 // The kernel of a launch whose shape, ranges, strides and buffers are filled in, and how it takes it: the fields from

@@ -18,7 +18,7 @@ int main()
             continue;
         }
         if (ranges == 0)
-            ranges = decode_choose_ranges(c, sequences, max_kvlen, head_dim, heads, kv_heads, (int)cus, requested == kDecodeKernelAuto);
+            ranges = decode_choose_ranges(c, sequences, max_kvlen, head_dim, heads, kv_heads, (int)cus, requested == kDecodeKernelAuto, mask == 2);
         DecodeLaunch a{};
         alignas(16) static char buffer[64];
         a.output = buffer + output_offset;

@@ -19,9 +19,9 @@ def select(tmp_path_factory):
 
     def call(sequences, heads, kv_heads, head_dim, max_kvlen, ranges=0, mask=False, output_offset=0, output_stride=None, stride_s=None,
              stride_h=None, scale=0.088, requested=0, cus=256):
-        """(kernel, ranges, whole sequences) of one call, or ("refused", ranges, reason)"""
+        """(kernel, ranges, whole sequences) of one call, or ("refused", ranges, reason).  mask: "planned" = the plan knows of it"""
         d = head_dim
-        fields = (sequences, max_kvlen, ranges, heads, kv_heads, d, int(mask), output_offset,
+        fields = (sequences, max_kvlen, ranges, heads, kv_heads, d, 2 if mask == "planned" else int(mask), output_offset,
                   heads * d if output_stride is None else output_stride, 2 * kv_heads * d if stride_s is None else stride_s,
                   d if stride_h is None else stride_h, scale, requested, cus)
         out = subprocess.run([exe], input=" ".join(str(f) for f in fields) + "\n", capture_output=True, text=True, check=True, timeout=60).stdout.split()
@@ -31,7 +31,7 @@ def select(tmp_path_factory):
     return call
 
 
-MANY_SHORT = [(512, 32, 8, 128, 300), (128, 32, 32, 128, 400), (512, 8, 8, 64, 300), (512, 16, 8, 256, 150), (600, 9, 9, 64, 100)]
+MANY_SHORT = [(512, 32, 8, 128, 300), (128, 32, 32, 128, 200), (512, 8, 8, 64, 300), (512, 16, 8, 256, 150), (600, 9, 9, 64, 100)]
 
 
 @pytest.mark.parametrize("shape", MANY_SHORT)
@@ -54,11 +54,35 @@ def test_a_single_range_without_a_request_is_never_one_workgroup(select, form):
             assert whole and ranges == 1, (n, hq, hkv, d, kernel)
 
 
+# (sequences, query heads, kv heads, head_dim, longest): measured per decode call, whole sequences / ranges + combine
+WHOLE = [(60, 8, 8, 64, 500), (100, 32, 8, 64, 300), (16, 14, 2, 64, 700), (32, 32, 8, 128, 256), (5, 32, 8, 128, 500), (60, 64, 8, 128, 500),
+         (300, 8, 1, 128, 500), (512, 8, 1, 128, 500), (100, 40, 1, 96, 8000), (300, 24, 2, 256, 8000), (30, 24, 1, 256, 8000), (300, 32, 32, 128, 128),
+         (512, 32, 8, 128, 300), (300, 8, 1, 256, 1600), (512, 16, 8, 256, 150)]
+CUT = [(300, 8, 8, 64, 1600), (100, 8, 8, 64, 2400), (300, 32, 8, 64, 1000), (100, 40, 8, 64, 4000), (300, 14, 2, 64, 8000), (300, 48, 1, 128, 2400),
+       (100, 32, 32, 96, 200), (300, 32, 32, 96, 128), (30, 8, 8, 96, 1000), (300, 16, 8, 128, 500), (160, 32, 32, 128, 300), (160, 16, 16, 256, 200),
+       (5, 8, 1, 128, 700), (160, 28, 4, 128, 1000), (300, 64, 8, 128, 500)]
+
+
+def test_sequences_are_taken_whole_where_that_was_measured_faster(select):
+    for shape in WHOLE:
+        assert select(*shape)[1:] == (1, True), shape
+    for shape in CUT:
+        kernel, ranges, whole = select(*shape)
+        assert ranges > 1 and not whole, shape
+    # longer sequences are never taken whole where shorter ones are cut, and a plan that knows of a mask takes no more of them whole
+    for n, hq, hkv, d, _ in WHOLE + CUT:
+        whole = [select(n, hq, hkv, d, kv)[2] for kv in (64, 200, 700, 2000, 6000, 60000)]
+        assert whole == sorted(whole, reverse=True), (n, hq, hkv, d, whole)
+        masked = [select(n, hq, hkv, d, kv, mask="planned")[2] for kv in (64, 200, 700, 2000, 6000, 60000)]
+        assert all(w or not m for w, m in zip(whole, masked)), (n, hq, hkv, d, whole, masked)
+
+
 def test_ranges_and_requests_keep_their_kernels(select):
     assert select(64, 32, 8, 128, 4096)[::2] == (QUAD, False)
     assert select(64, 32, 8, 128, 4096, mask=True)[::2] == (QUAD, False)
     assert select(64, 32, 8, 128, 4096, output_offset=8)[::2] == (GENERAL, False)
     assert select(64, 8, 8, 64, 4096, mask=True)[::2] == (GENERAL, False)
+    assert select(64, 32, 8, 64, 4096, mask=True)[::2] == (MFMA, False)
     assert select(64, 64, 8, 128, 4096, mask=True)[::2] == (MFMA16, False)
     assert select(64, 48, 1, 128, 4096)[::2] == (MFMA, False)
     assert select(2, 32, 8, 128, 8192, mask=True)[::2] == (MFMA16, False)
