@@ -278,9 +278,9 @@ namespace {
 
 // Checks of a decode call and the launch block it becomes.  `workspace` / `workspace_size` are the caller's
 // (pmxhip_decode_attention) or the library's static array (pmxhip_decode_attention_static).
-// `columns`: the column kernels whatever the shape (short chunks).
+// `columns`: the column kernels whatever the shape (short chunks).  `max_kvlen`: 0 = unknown.
 int decode_prepare(const char* who, const pmxhip_decode_params* p, void* workspace, int64_t workspace_size,
-                   pmxhip::DecodeLaunch* out, bool columns = false)
+                   pmxhip::DecodeLaunch* out, bool columns = false, int64_t max_kvlen = 0)
 {
     if (!head_dim_supported(p->head_dim))
         return fail(PMXHIP_UNSUPPORTED, "cache flash decoding attention do not support head dim %lld", (long long)p->head_dim);
@@ -333,7 +333,7 @@ int decode_prepare(const char* who, const pmxhip_decode_params* p, void* workspa
     // kernels need of the buffers and the cache layout beyond this entry point's own checks.  Everything that depends on
     // the kernel (the unit of the range cuts above all, which the combine kernel must share) follows from this one choice.
     pmxhip::DecodeChoice c;
-    switch (pmxhip::decode_select(&a, p->kernel_request, columns, current_compute_units(), &c)) {
+    switch (pmxhip::decode_select(&a, p->kernel_request, columns, current_compute_units(), max_kvlen, &c)) {
     case pmxhip::DecodeSelect::kSelected: break;
     case pmxhip::DecodeSelect::kNoKernel:
         return fail(PMXHIP_UNSUPPORTED, "%s: kernel %d (%s) does not serve this shape", who, p->kernel_request,
@@ -380,16 +380,30 @@ int pmxhip_decode_attention(const pmxhip_decode_params* p, pmxhip_stream_t strea
     return pmxhip_decode_attention_stage(p, 0, stream);
 }
 
-int pmxhip_decode_attention_stage(const pmxhip_decode_params* p, int32_t stage, pmxhip_stream_t stream)
+static int decode_stage(const pmxhip_decode_params* p, int64_t max_kvlen, int32_t stage, pmxhip_stream_t stream)
 {
     if (stage < 0 || stage > 2) return fail(PMXHIP_INVALID_VALUE, "decode_attention: stage must be 0, 1 or 2");
     if (!p) return fail(PMXHIP_INVALID_VALUE, "decode_attention: null params");
     if (p->decoding_batches < 0) return fail(PMXHIP_INVALID_VALUE, "decode_attention: negative decoding_batches");
     if (p->decoding_batches == 0) return PMXHIP_SUCCESS; // kernel.cu:2084
     pmxhip::DecodeLaunch a;
-    if (int rc = decode_prepare("decode_attention", p, p->workspace, p->workspace_size, &a)) return rc;
+    if (int rc = decode_prepare("decode_attention", p, p->workspace, p->workspace_size, &a, false, max_kvlen)) return rc;
     return launch_result("decode_attention", pmxhip::launch_decode(a, stage, stream));
 }
+
+int pmxhip_decode_attention_stage(const pmxhip_decode_params* p, int32_t stage, pmxhip_stream_t stream)
+{
+    return decode_stage(p, 0, stage, stream);
+}
+
+} // extern "C"
+
+int pmxhip::decode_attention_sized(const pmxhip_decode_params* p, int64_t max_kvlen, hipStream_t stream)
+{
+    return decode_stage(p, max_kvlen, 0, stream);
+}
+
+extern "C" {
 
 int pmxhip_decode_attention_static(const pmxhip_decode_params* p, pmxhip_stream_t stream)
 {
@@ -578,7 +592,10 @@ int pmxhip_prefill_attention_split(const pmxhip_prefill_params* p, void* split_w
             c.chunk_q_heads = (int32_t)g;
             c.chunk_causal = p->is_causal ? 1 : 0;
             c.by_sequence = by_sequence;
-            if (!by_sequence) c.shared_pieces = 1; // (the plan's ranges are a wave's)
+            if (!by_sequence) { // (the plan's ranges are a wave's)
+                c.shared_pieces = 1;
+                c.ring = pmxhip::decode_ring(c, p->max_kvlen);
+            }
             return launch_result("prefill_attention", pmxhip::launch_decode(c, 0, stream));
         }
     }

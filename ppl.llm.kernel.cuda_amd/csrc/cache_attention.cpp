@@ -342,7 +342,7 @@ ppl::common::RetCode dynamic_batching_multi_head_cache_attention::forward_decode
     p.num_token_ranges = (int32_t)cfg.decoding_multi_block_size;
     p.workspace = cfg.workspace;
     p.workspace_size = cfg.workspace_size;
-    const int rc = pmxhip_decode_attention(&p, stream);
+    const int rc = pmxhip::decode_attention_sized(&p, cfg.max_kvlen, stream);
     if (rc != PMXHIP_SUCCESS) {
         // the reference folds every decode dispatch failure into RC_UNSUPPORTED (kernel.cu:2118-2121); what is not a
         // matter of the configuration keeps its own code (a bad argument, a first launch under stream capture)

@@ -793,7 +793,9 @@ static int launch_decode_d(const DecodeLaunch& a, int stage, hipStream_t stream)
         switch (a.kernel) {
             case kDecodeKernelMfma16:
                 if (D != 64 && D != 128 && !a.by_sequence) return kLaunchNoKernel;
-                launch_decode_columns(a, stream);
+                if (a.by_sequence || a.ring) launch_decode_columns(a, stream);
+                else if (D != 128) return kLaunchNoKernel;
+                else launch_decode_mfma(a, stream);
                 break;
             case kDecodeKernelMfma32:
                 if (D == 256 || (D == 96 && !a.by_sequence)) return kLaunchNoKernel;

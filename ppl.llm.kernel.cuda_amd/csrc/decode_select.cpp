@@ -383,11 +383,18 @@ int64_t decode_choose_ranges(const DecodeChoice& by_shape, int64_t sequences, in
         ranges = useful;
         const int64_t half = slots / 2 / groups > 1 ? slots / 2 / groups : 1;
         if (ranges < half) {
-            // (the column kernels' smallest is a block: 64 q / 8 kv heads of 128, one sequence of 4096 tokens 15.1 us with ranges of 64
-            // tokens and 13.8 with 32, four of 1024 15.5 and 12.8; 14 / 2 heads of 64, 16 of 1024 13.0 and 10.5)
-            const int64_t smallest = automatic && columns ? kDecodeMfmaTokens : min_tokens;
-            const int64_t finer = (max_tokens + smallest - 1) / smallest;
+            const int64_t finer = (max_tokens + min_tokens - 1) / min_tokens;
             ranges = half < finer ? half : finer;
+            // The column kernels' smallest is a block: 64 q / 8 kv heads of 128, one sequence of 4096 tokens 15.1 us with ranges of 64
+            // tokens and 13.8 with 32, four of 1024 15.5 and 12.8; 14 / 2 heads of 64, 16 of 1024 13.0 and 10.5.  With 32 columns at
+            // head_dim 128 up to a wave per CU and pass: 48 / 1 heads, 16 sequences of 100-300 13.1 us with 69 ranges, 11.4 with
+            // 138, but 30 of 233-700 17.1 with 321 and 18.9 with 512.
+            if (automatic && columns) {
+                const int64_t most = c.kernel == kDecodeKernelMfma32 && head_dim == 128 ? slots / 4 / groups : half;
+                const int64_t finest = (max_tokens + kDecodeMfmaTokens - 1) / kDecodeMfmaTokens;
+                const int64_t blocks = most < finest ? most : finest;
+                if (blocks > ranges) ranges = blocks;
+            }
         }
         // a step of a few sequences: below a workgroup per two CUs the ranges go down to the kernel's floor
         const int64_t sparse = compute_units / 2 / groups > 1 ? compute_units / 2 / groups : 1;
@@ -400,17 +407,34 @@ int64_t decode_choose_ranges(const DecodeChoice& by_shape, int64_t sequences, in
     return ranges > 1 ? ranges : 1;
 }
 
-// How the kernel takes the launch: by_sequence and shared_pieces.
-static void choose_form(DecodeLaunch* a, int compute_units)
+// The two kernels of 16 columns over ranges (decode_attn_mfma.hip has the other's figures): the ring's where a single sequence's
+// pieces are shared by four waves, at head_dim 64, and where four waves of a workgroup walk 500 tokens and more per range (28 / 4
+// heads: 100 sequences of 1333-4000, 520 per range, 68.5 -> 67.9 us, 300 of them 196 -> 188; 64 / 8 heads, 30 of them, 310 per range,
+// 49.9 and 50.6).  One or two waves per workgroup gain nothing from it (10 / 2 heads, 100 sequences of 5333-16000 127 against 133 us), nor does a
+// mask, whose values are awaited together with the rows (28 / 4 heads, 300 of 1333-4000 219 against 221).  Without a length: as long
+// streams, but for a few sequences.
+bool decode_ring(const DecodeLaunch& a, int64_t max_kvlen)
+{
+    if (a.kernel != kDecodeKernelMfma16 || a.by_sequence) return false;
+    if (a.head_dim != 128 || a.shared_pieces > 1) return true;
+    if (a.kv_heads_per_group != 4 || a.attn_mask != nullptr) return false;
+    if (max_kvlen <= 0) return a.decoding_batches > kFewSequences;
+    return 0.67 * (double)max_kvlen * (double)a.decoding_batches >= 500.0 * (double)a.ranges;
+}
+
+// How the kernel takes the launch: by_sequence, shared_pieces and ring.
+static void choose_form(DecodeLaunch* a, int compute_units, int64_t max_kvlen)
 {
     a->by_sequence = 0;
     a->shared_pieces = 1;
     const bool columns = a->kernel == kDecodeKernelMfma16 || a->kernel == kDecodeKernelMfma32;
+    a->ring = 0;
     a->by_sequence = a->ranges == 1 && (a->kernel != kDecodeKernelQuad || quad_takes_whole(*a));
     if (!columns) return;
     const int64_t wgs = (a->by_sequence ? a->decoding_batches : a->ranges) * a->num_kv_heads * a->num_passes;
     if (a->by_sequence) a->shared_pieces = decode_share(wgs, a->head_dim, compute_units);
     else if (a->kernel == kDecodeKernelMfma16 && a->decoding_batches == 1 && wgs <= compute_units) a->shared_pieces = 4;
+    a->ring = decode_ring(*a, max_kvlen);
 }
 
 bool decode_quad_launch_ok(const DecodeLaunch& a)
@@ -424,7 +448,7 @@ bool decode_quad_launch_ok(const DecodeLaunch& a)
     return true;
 }
 
-DecodeSelect decode_select(DecodeLaunch* a, int32_t requested, bool columns, int compute_units, DecodeChoice* out)
+DecodeSelect decode_select(DecodeLaunch* a, int32_t requested, bool columns, int compute_units, int64_t max_kvlen, DecodeChoice* out)
 {
     DecodeChoice c{};
     *out = c;
@@ -447,7 +471,7 @@ DecodeSelect decode_select(DecodeLaunch* a, int32_t requested, bool columns, int
     a->num_passes = c.num_passes;
     a->wg_tokens = c.wg_tokens;
     a->min_tokens_per_range = decode_floor_tokens_per_range(c.wg_tokens);
-    choose_form(a, compute_units);
+    choose_form(a, compute_units, max_kvlen);
     return DecodeSelect::kSelected;
 }
 

@@ -9,6 +9,7 @@
 #include <atomic>
 
 struct pmxhip_decode_plan;
+struct pmxhip_decode_params;
 
 namespace pmxhip {
 
@@ -71,6 +72,7 @@ struct DecodeLaunch {
     int32_t min_tokens_per_range;
     int32_t by_sequence;          // one range: workgroup x takes sequence x whole (quad and column kernels: and writes the rows of an empty one)
     int32_t shared_pieces;        // column kernels: waves per kv head that share the tokens of a piece (1, 4 or 8)
+    int32_t ring;                 // 16 columns over ranges: on the kernel of decode_attn_columns.hip, not that of decode_attn_mfma.hip
     int32_t kernel;               // DecodeKernel that runs the token ranges; never kDecodeKernelAuto at launch
     // Chunks of a few query tokens per sequence on the 32-column kernel (nullptr = one query token per sequence, row =
     // sequence index): rows of sequence b are seqstarts[b] .. seqstarts[b + 1]; num_kv_repeats and num_heads then count
@@ -265,8 +267,8 @@ enum DecodeKernel : int32_t {
     kDecodeKernelAuto = 0,    // as a request: by shape
     kDecodeKernelGeneral = 1, // decode_attn.hip: VALU, every head_dim and head count, up to 8 query heads per pass
     kDecodeKernelQuad = 2,    // decode_attn_quad.hip: 4x4x4 MFMA per quad; head_dim 64 or 128 (two or more kv heads) or 256
-    kDecodeKernelMfma16 = 3,  // decode_attn_columns.hip: 16 query-head columns (as a request: head_dim 128)
-    kDecodeKernelMfma32 = 4,  // decode_attn_mfma.hip: 32 query-head columns per pass, head_dim 128 or 64
+    kDecodeKernelMfma16 = 3,  // decode_attn_mfma.hip, decode_attn_columns.hip: 16 query-head columns (as a request: head_dim 128)
+    kDecodeKernelMfma32 = 4,  // decode_attn_mfma.hip: 32 query-head columns per pass, head_dim 128 or 64 (whole sequences: decode_attn_columns.hip)
 };
 // Fewest tokens a range is given: with fewer, the start of a piece (lookups, query rows, first rows of the cache) and
 // its slot in the workspace cost more than the parallelism buys.  On batches far smaller than the chip 64 beats 128
@@ -304,13 +306,18 @@ int64_t decode_choose_ranges(const DecodeChoice& by_shape, int64_t sequences, in
 // pmxhip_decode_plan_make_kernel for a caller that knows whether the step has a mask (c_api.cpp).
 int decode_plan_make(int64_t decoding_batches, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim, int64_t max_kvlen, int32_t compute_units,
                      int32_t num_token_ranges_hint, int32_t kernel_request, bool mask, pmxhip_decode_plan* plan);
+// pmxhip_decode_attention for a caller that knows the longest sequence (c_api.cpp).
+int decode_attention_sized(const pmxhip_decode_params* p, int64_t max_kvlen, hipStream_t stream);
 // A single sequence of more tokens is cut as any other stream.
 constexpr int64_t kSharedStreamTokens = 32768;
 // The kernel of a launch whose shape, ranges, strides and buffers are filled in, and how it takes it: the fields from
 // kv_heads_per_group on.  A single range without a request means that every sequence is taken whole by workgroups of its own.
-// `columns`: the column kernels whatever the shape.  `out`: the choice, also where its strides were refused.
+// `columns`: the column kernels whatever the shape.  `max_kvlen`: the longest sequence, 0 = unknown (a long one).  `out`: the
+// choice, also where its strides were refused.
 enum class DecodeSelect { kSelected, kNoKernel, kQuadBuffers, kCacheStrides };
-DecodeSelect decode_select(DecodeLaunch* a, int32_t requested, bool columns, int compute_units, DecodeChoice* out);
+DecodeSelect decode_select(DecodeLaunch* a, int32_t requested, bool columns, int compute_units, int64_t max_kvlen, DecodeChoice* out);
+// DecodeLaunch::ring of a launch of the 16-column kernel over ranges.
+bool decode_ring(const DecodeLaunch& a, int64_t max_kvlen);
 const char* decode_kernel_name(const DecodeLaunch& a);
 const char* decode_kernel_name(int32_t kernel); // over token ranges
 int decode_wg_tokens(int head_dim, int kv_heads_per_group); // of the general kernel:
@@ -322,8 +329,8 @@ constexpr int kDecodeMfmaTokens = 32;
 constexpr int kDecodeMfma16Columns = 16;
 constexpr int kDecodeMfmaColumns = 32;
 void launch_decode_quad(const DecodeLaunch& a, hipStream_t stream);
-void launch_decode_mfma(const DecodeLaunch& a, hipStream_t stream);    // 32 columns over token ranges
-void launch_decode_columns(const DecodeLaunch& a, hipStream_t stream); // 16 columns, and 32 on whole sequences
+void launch_decode_mfma(const DecodeLaunch& a, hipStream_t stream);    // 16 or 32 columns over token ranges
+void launch_decode_columns(const DecodeLaunch& a, hipStream_t stream); // whole sequences, and 16 columns over long ranges
 // One-time attribute calls of the kernels whose dynamic LDS exceeds the default limit, all variants at once.
 int init_decode_kernels();
 int init_prefill_kernels();

@@ -8,10 +8,10 @@ using namespace pmxhip;
 
 int main()
 {
-    long long sequences, max_kvlen, ranges, heads, kv_heads, head_dim, mask, output_offset, output_stride, stride_s, stride_h, requested, cus;
+    long long sequences, max_kvlen, ranges, heads, kv_heads, head_dim, mask, output_offset, output_stride, stride_s, stride_h, requested, cus, sized;
     double scale;
-    while (scanf("%lld %lld %lld %lld %lld %lld %lld %lld %lld %lld %lld %lf %lld %lld", &sequences, &max_kvlen, &ranges, &heads, &kv_heads,
-                 &head_dim, &mask, &output_offset, &output_stride, &stride_s, &stride_h, &scale, &requested, &cus) == 14) {
+    while (scanf("%lld %lld %lld %lld %lld %lld %lld %lld %lld %lld %lld %lf %lld %lld %lld", &sequences, &max_kvlen, &ranges, &heads, &kv_heads,
+                 &head_dim, &mask, &output_offset, &output_stride, &stride_s, &stride_h, &scale, &requested, &cus, &sized) == 15) {
         DecodeChoice c;
         if (!decode_choose(head_dim, heads, kv_heads, (int32_t)requested, &c)) {
             printf("no-kernel\n");
@@ -34,12 +34,12 @@ int main()
         a.num_kv_heads = kv_heads;
         a.head_dim = (int32_t)head_dim;
         a.ranges = (int32_t)ranges;
-        const DecodeSelect rc = decode_select(&a, (int32_t)requested, false, (int)cus, &c);
+        const DecodeSelect rc = decode_select(&a, (int32_t)requested, false, (int)cus, sized ? max_kvlen : 0, &c);
         if (rc != DecodeSelect::kSelected) {
             printf("%s %lld\n", rc == DecodeSelect::kNoKernel ? "no-kernel" : rc == DecodeSelect::kQuadBuffers ? "quad-buffers" : "strides", ranges);
             continue;
         }
-        printf("%s %lld %d %d\n", decode_kernel_name(a), ranges, a.by_sequence, a.shared_pieces);
+        printf("%s %lld %d %d %d\n", decode_kernel_name(a), ranges, a.by_sequence, a.shared_pieces, a.ring);
     }
     return 0;
 }

@@ -18,16 +18,17 @@ def select(tmp_path_factory):
                     os.path.join(ROOT, "tests", "select", "decode_select_check.cpp"), "-o", exe], check=True, timeout=300)
 
     def call(sequences, heads, kv_heads, head_dim, max_kvlen, ranges=0, mask=False, output_offset=0, output_stride=None, stride_s=None,
-             stride_h=None, scale=0.088, requested=0, cus=256):
-        """(kernel, ranges, whole sequences) of one call, or ("refused", ranges, reason).  mask: "planned" = the plan knows of it"""
+             stride_h=None, scale=0.088, requested=0, cus=256, sized=False, ring=False):
+        """(kernel, ranges, whole sequences) of one call, or ("refused", ranges, reason).  mask: "planned" = the plan knows of it;
+        sized: the launch knows the longest sequence; ring: (waves that share a piece, the ring kernel) instead"""
         d = head_dim
         fields = (sequences, max_kvlen, ranges, heads, kv_heads, d, 2 if mask == "planned" else int(mask), output_offset,
                   heads * d if output_stride is None else output_stride, 2 * kv_heads * d if stride_s is None else stride_s,
-                  d if stride_h is None else stride_h, scale, requested, cus)
+                  d if stride_h is None else stride_h, scale, requested, cus, int(sized))
         out = subprocess.run([exe], input=" ".join(str(f) for f in fields) + "\n", capture_output=True, text=True, check=True, timeout=60).stdout.split()
-        if len(out) < 4:
+        if len(out) < 5:
             return "refused", int(out[1]) if len(out) > 1 else 0, out[0]
-        return out[0], int(out[1]), out[2] == "1"
+        return (int(out[3]), out[4] == "1") if ring else (out[0], int(out[1]), out[2] == "1")
     return call
 
 
@@ -75,6 +76,20 @@ def test_sequences_are_taken_whole_where_that_was_measured_faster(select):
         assert whole == sorted(whole, reverse=True), (n, hq, hkv, d, whole)
         masked = [select(n, hq, hkv, d, kv, mask="planned")[2] for kv in (64, 200, 700, 2000, 6000, 60000)]
         assert all(w or not m for w, m in zip(whole, masked)), (n, hq, hkv, d, whole, masked)
+
+
+def test_sixteen_columns_over_ranges_run_on_the_ring_kernel_over_long_streams_of_four_waves(select):
+    def ring(*shape, **kw):
+        return select(*shape, ring=True, **kw)
+    assert ring(32, 64, 8, 128, 32768, sized=True) == (1, True) and ring(300, 28, 4, 128, 4000, sized=True) == (1, True)
+    assert ring(30, 64, 8, 128, 2400, sized=True) == (1, False) and ring(100, 28, 4, 128, 1600, sized=True) == (1, False)
+    assert ring(32, 64, 8, 128, 32768, sized=True, mask=True) == (1, False)
+    for shape in ((100, 8, 1, 128, 16000), (100, 10, 2, 128, 16000)):  # one or two waves per workgroup
+        assert ring(*shape, sized=True) == (1, False) and ring(*shape) == (1, False)
+    assert ring(32, 64, 8, 128, 32768) == (1, True) and ring(3, 64, 8, 128, 32768) == (1, False)  # no length given
+    assert ring(1, 64, 8, 128, 8192) == (4, True) and ring(3, 8, 8, 64, 8192) == (1, True)
+    assert ring(32, 64, 8, 128, 200) == (8, False)  # whole sequences
+    assert select(30, 48, 1, 128, 700)[1] == 329 and select(16, 48, 1, 128, 1000)[1] == 256 and select(16, 48, 1, 128, 600)[1] == 256
 
 
 def test_ranges_and_requests_keep_their_kernels(select):
