@@ -124,6 +124,7 @@ bool decode_choose(int64_t head_dim, int64_t num_heads, int64_t num_kv_heads, in
 
 namespace {
 
+constexpr double kLaneOffsets = 2147483648.0; // what a 32-bit lane offset reaches
 // Bytes that the 32-bit lane offsets of a kernel span: the tokens of one wave block times the row stride, the kv
 // heads that share a wave's 64-bit base times the head stride, and a row.
 double lane_offset_span(const DecodeChoice& c, int64_t head_dim, int64_t stride_s, int64_t stride_h)
@@ -151,16 +152,15 @@ double lane_offset_span(const DecodeChoice& c, int64_t head_dim, int64_t stride_
 bool fit_cache_strides(int64_t head_dim, int64_t num_heads, int64_t num_kv_heads, int32_t requested,
                               int64_t stride_s, int64_t stride_h, DecodeChoice* c)
 {
-    constexpr double kLimit = 2147483648.0;
     if (stride_s < 0 || stride_h < 0) return false;
-    if (lane_offset_span(*c, head_dim, stride_s, stride_h) < kLimit) return true;
+    if (lane_offset_span(*c, head_dim, stride_s, stride_h) < kLaneOffsets) return true;
     if (c->kernel == kDecodeKernelGeneral) {
         // fewer kv heads per wave (more tokens instead) until the heads' distance fits; one kv head per workgroup
         // has no head term at all
         while (c->kv_heads_per_group > 1) {
             c->kv_heads_per_group /= 2;
             c->wg_tokens = decode_wg_tokens((int)head_dim, c->kv_heads_per_group);
-            if (lane_offset_span(*c, head_dim, stride_s, stride_h) < kLimit) return true;
+            if (lane_offset_span(*c, head_dim, stride_s, stride_h) < kLaneOffsets) return true;
         }
         return false;
     }
@@ -332,6 +332,10 @@ double sequence_cost(int64_t sequences, int64_t max_kvlen, int64_t head_dim, int
 static void choose_launch(const DecodeLaunch& a, int compute_units, DecodeChoice* c)
 {
     const int64_t g = a.num_heads / a.num_kv_heads;
+    // the column kernels' blocks are 32 tokens, the quad kernel's at head_dim 128 and 256 16: rows further apart stay where they fit
+    DecodeChoice columns{};
+    const bool fit = decode_choose_columns(a.head_dim, g, a.num_kv_heads, &columns) &&
+                     lane_offset_span(columns, a.head_dim, a.cache_stride_s, a.cache_stride_h) < kLaneOffsets;
     if (a.ranges == 1) {
         // A single range is for kernels that take every sequence whole (a kernel over ranges would walk the batch with one
         // workgroup), and the plan knows neither mask nor buffers.  What the quad kernel cannot take whole is the column kernels',
@@ -345,9 +349,10 @@ static void choose_launch(const DecodeLaunch& a, int compute_units, DecodeChoice
                 return;
             }
         }
-        decode_choose_columns(a.head_dim, g, a.num_kv_heads, c);
-    } else if (c->kernel == kDecodeKernelQuad && few_sequences_on_columns(a.decoding_batches, a.head_dim, g)) {
-        decode_choose_columns(a.head_dim, g, a.num_kv_heads, c);
+        if (fit) *c = columns;
+        else if (c->kernel == kDecodeKernelQuad && !quad_takes_whole(a)) decode_choose(a.head_dim, a.num_heads, a.num_kv_heads, kDecodeKernelGeneral, c);
+    } else if (fit && c->kernel == kDecodeKernelQuad && few_sequences_on_columns(a.decoding_batches, a.head_dim, g)) {
+        *c = columns;
     }
 }
 

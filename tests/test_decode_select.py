@@ -92,6 +92,23 @@ def test_sixteen_columns_over_ranges_run_on_the_ring_kernel_over_long_streams_of
     assert select(30, 48, 1, 128, 700)[1] == 329 and select(16, 48, 1, 128, 1000)[1] == 256 and select(16, 48, 1, 128, 600)[1] == 256
 
 
+def test_rows_too_far_apart_for_the_column_kernels_stay_where_they_fit(select):
+    """32 rows of a column kernel's block have to lie within 2 GiB, 16 of the quad kernel's."""
+    far = 100 << 20
+    for n, kv in ((1, 300), (4, 300), (4, 8192), (64, 8192), (64, 200), (2000, 200)):  # whatever the number of sequences and ranges
+        kernel, ranges, whole = select(n, 32, 8, 128, kv, stride_s=far)
+        assert kernel == QUAD and whole == (ranges == 1), (n, kv)
+        kernel, ranges, whole = select(n, 16, 8, 256, kv, stride_s=far, ranges=1)
+        assert kernel == QUAD and whole, (n, kv)
+        kernel, ranges, whole = select(n, 32, 8, 128, kv, stride_s=far, output_offset=8, ranges=1)
+        assert kernel == GENERAL and whole, (n, kv)
+        assert select(n, 12, 3, 96, kv, stride_s=30 << 20, ranges=1)[::2] == (MFMA16, True)
+        assert select(n, 4, 4, 96, kv, stride_s=far, ranges=1) == select(n, 4, 4, 96, kv, stride_s=far, ranges=1, requested=1)
+        # neither the kernel by shape nor another one takes them: refused, as for ever
+        assert select(n, 64, 8, 128, kv, stride_s=far)[::2] == ("refused", "strides")
+    assert select(4, 32, 8, 128, 8192, stride_s=60 << 20)[0] == MFMA16
+
+
 def test_ranges_and_requests_keep_their_kernels(select):
     assert select(64, 32, 8, 128, 4096)[::2] == (QUAD, False)
     assert select(64, 32, 8, 128, 4096, mask=True)[::2] == (QUAD, False)
