@@ -114,7 +114,7 @@ typedef struct pmxhip_decode_params {
     const void* scale;     /* half */
     const int64_t* cachestarts;
     const int64_t* kvstarts; /* (B_dec + 1) */
-    float attn_scale;
+    float attn_scale; /* any; below 1e-20 the MFMA kernels do not serve (their request is refused) and others do */
     int64_t layer_idx;
     int64_t num_kv_repeats; /* Hq / KVH */
     int64_t page_size;

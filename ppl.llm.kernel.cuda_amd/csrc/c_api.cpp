@@ -341,6 +341,9 @@ int decode_prepare(const char* who, const pmxhip_decode_params* p, void* workspa
     case pmxhip::DecodeSelect::kQuadBuffers:
         return fail(PMXHIP_UNSUPPORTED, "%s: the quad kernel needs 16-byte aligned output rows and, with attn_mask, at "
                                         "most four query heads per kv head", who);
+    case pmxhip::DecodeSelect::kScale:
+        return fail(PMXHIP_UNSUPPORTED, "%s: kernel %d (%s) needs a positive attn_scale", who, p->kernel_request,
+                    pmxhip::decode_kernel_name(p->kernel_request));
     case pmxhip::DecodeSelect::kCacheStrides: // 32-bit lane offsets against a 64-bit base per wave
         return fail(PMXHIP_UNSUPPORTED,
                     "%s: cache_stride_s %lld / cache_stride_h %lld: the rows of one block of %d tokens%s must lie within 2 GiB",

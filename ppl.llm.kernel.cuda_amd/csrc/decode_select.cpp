@@ -328,13 +328,17 @@ double sequence_cost(int64_t sequences, int64_t max_kvlen, int64_t head_dim, int
 
 } // namespace
 
+// The column and MFMA kernels take the maximum of the raw products and divide the mask by the scale: it has to be positive, and not so
+// small that a mask divided by it passes the maximum they begin with.  The quad and general kernels scale first.
+bool columns_scale(float attn_scale) { return attn_scale >= 1e-20f; }
+
 // The kernel of a launch without a request, in place of the choice by shape.
 static void choose_launch(const DecodeLaunch& a, int compute_units, DecodeChoice* c)
 {
     const int64_t g = a.num_heads / a.num_kv_heads;
     // the column kernels' blocks are 32 tokens, the quad kernel's at head_dim 128 and 256 16: rows further apart stay where they fit
     DecodeChoice columns{};
-    const bool fit = decode_choose_columns(a.head_dim, g, a.num_kv_heads, &columns) &&
+    const bool fit = columns_scale(a.attn_scale) && decode_choose_columns(a.head_dim, g, a.num_kv_heads, &columns) &&
                      lane_offset_span(columns, a.head_dim, a.cache_stride_s, a.cache_stride_h) < kLaneOffsets;
     if (a.ranges == 1) {
         // A single range is for kernels that take every sequence whole (a kernel over ranges would walk the batch with one
@@ -461,10 +465,14 @@ DecodeSelect decode_select(DecodeLaunch* a, int32_t requested, bool columns, int
                 : !decode_choose(a->head_dim, a->num_heads, a->num_kv_heads, requested, &c))
         return DecodeSelect::kNoKernel;
     if (!columns && requested == kDecodeKernelAuto) choose_launch(*a, compute_units, &c);
+    if ((c.kernel == kDecodeKernelMfma16 || c.kernel == kDecodeKernelMfma32) && !columns_scale(a->attn_scale)) {
+        if (columns || requested != kDecodeKernelAuto) return DecodeSelect::kScale;
+        decode_choose(a->head_dim, a->num_heads, a->num_kv_heads, kDecodeKernelGeneral, &c);
+    }
     if (c.kernel == kDecodeKernelQuad && !decode_quad_launch_ok(*a)) {
         if (requested == kDecodeKernelQuad) return DecodeSelect::kQuadBuffers;
         // (with a mask at head_dim 64: 32 / 8 heads, 100 sequences of 233-700 51.0 us on the general kernel, 40 / 8 35.2 on this one)
-        const bool columns64 = a->head_dim == 64 && a->attn_mask != nullptr && a->num_kv_repeats > 1;
+        const bool columns64 = a->head_dim == 64 && a->attn_mask != nullptr && a->num_kv_repeats > 1 && columns_scale(a->attn_scale);
         decode_choose(a->head_dim, a->num_heads, a->num_kv_heads, columns64 ? kDecodeKernelMfma32 : kDecodeKernelGeneral, &c);
     }
     const bool fits = fit_cache_strides(a->head_dim, a->num_heads, a->num_kv_heads, requested, a->cache_stride_s, a->cache_stride_h, &c);

@@ -314,8 +314,10 @@ constexpr int64_t kSharedStreamTokens = 32768;
 // kv_heads_per_group on.  A single range without a request means that every sequence is taken whole by workgroups of its own.
 // `columns`: the column kernels whatever the shape.  `max_kvlen`: the longest sequence, 0 = unknown (a long one).  `out`: the
 // choice, also where its strides were refused.
-enum class DecodeSelect { kSelected, kNoKernel, kQuadBuffers, kCacheStrides };
+enum class DecodeSelect { kSelected, kNoKernel, kQuadBuffers, kCacheStrides, kScale };
 DecodeSelect decode_select(DecodeLaunch* a, int32_t requested, bool columns, int compute_units, int64_t max_kvlen, DecodeChoice* out);
+// whether the column and MFMA kernels, and the tile kernel without its extra terms, take this attn_scale
+bool columns_scale(float attn_scale);
 // DecodeLaunch::ring of a launch of the 16-column kernel over ranges.
 bool decode_ring(const DecodeLaunch& a, int64_t max_kvlen);
 const char* decode_kernel_name(const DecodeLaunch& a);

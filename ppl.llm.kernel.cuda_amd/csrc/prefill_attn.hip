@@ -1415,7 +1415,8 @@ static int launch_prefill_variant(const PrefillLaunch& a, dim3 grid, hipStream_t
 template <int D>
 static int launch_prefill_src(const PrefillLaunch& a, dim3 grid, hipStream_t stream)
 {
-    const bool extra = a.attn_mask != nullptr || a.alibi_slopes != nullptr;
+    // (the form with extra terms scales the logits before it takes their maximum: any attn_scale)
+    const bool extra = a.attn_mask != nullptr || a.alibi_slopes != nullptr || !columns_scale(a.attn_scale);
     const int src = a.current_key ? 2 : (a.cache_mode == 1 ? 0 : 1);
     if (extra) {
         if (src == 0) return launch_prefill_variant<D, 0, true>(a, grid, stream);

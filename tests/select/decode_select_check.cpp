@@ -36,7 +36,7 @@ int main()
         a.ranges = (int32_t)ranges;
         const DecodeSelect rc = decode_select(&a, (int32_t)requested, false, (int)cus, sized ? max_kvlen : 0, &c);
         if (rc != DecodeSelect::kSelected) {
-            printf("%s %lld\n", rc == DecodeSelect::kNoKernel ? "no-kernel" : rc == DecodeSelect::kQuadBuffers ? "quad-buffers" : "strides", ranges);
+            printf("%s %lld\n", rc == DecodeSelect::kNoKernel ? "no-kernel" : rc == DecodeSelect::kQuadBuffers ? "quad-buffers" : rc == DecodeSelect::kScale ? "scale" : "strides", ranges);
             continue;
         }
         printf("%s %lld %d %d %d\n", decode_kernel_name(a), ranges, a.by_sequence, a.shared_pieces, a.ring);

@@ -109,6 +109,17 @@ def test_rows_too_far_apart_for_the_column_kernels_stay_where_they_fit(select):
     assert select(4, 32, 8, 128, 8192, stride_s=60 << 20)[0] == MFMA16
 
 
+def test_scales_that_are_not_positive_run_on_kernels_that_scale_first(select):
+    for scale in (-0.3, 0.0, 1e-30, float("nan")):
+        for n, hq, hkv, d, kv in [(2, 32, 8, 128, 300), (4, 32, 8, 128, 8192), (64, 32, 8, 128, 200), (2000, 8, 8, 64, 200), (64, 64, 8, 128, 8192),
+                                  (64, 64, 8, 128, 200), (3, 14, 2, 64, 900), (64, 48, 1, 128, 200), (30, 12, 3, 96, 200), (8, 24, 2, 256, 300)]:
+            for form in (dict(), dict(mask=True), dict(output_offset=8)):
+                kernel, ranges, whole = select(n, hq, hkv, d, kv, scale=scale, **form)
+                assert kernel in (QUAD, GENERAL) and whole == (ranges == 1), (scale, n, hq, hkv, d, kv, form)
+        assert select(64, 64, 8, 128, 8192, scale=scale, requested=3)[::2] == ("refused", "scale")
+    assert select(64, 64, 8, 128, 8192, scale=1e-6)[0] == MFMA16
+
+
 def test_ranges_and_requests_keep_their_kernels(select):
     assert select(64, 32, 8, 128, 4096)[::2] == (QUAD, False)
     assert select(64, 32, 8, 128, 4096, mask=True)[::2] == (QUAD, False)

@@ -404,3 +404,21 @@ def test_many_short_sequences_with_mask_and_unaligned_rows(pkg, oracle, shape, s
     assert_attention_close(rows[:, :hq * d].float().cpu().numpy().reshape(n, hq, d), ref, "rows of 8 bytes %s" % (shape,))
     assert (rows[empty, :hq * d] == 0).all()
     assert torch.isnan(rows[:, hq * d:]).all() and torch.isnan(buf[:4]).all()
+
+
+@pytest.mark.parametrize("attn_scale", [-0.3, 0.0, 1e-30])
+@pytest.mark.parametrize("shape", [(32, 8, 128), (8, 8, 64), (8, 1, 128), (48, 1, 128), (12, 3, 96), (16, 8, 256), (24, 2, 256)])
+def test_decode_with_a_scale_that_is_not_positive(pkg, oracle, monkeypatch, shape, attn_scale):
+    """A few sequences, ranges and whole sequences; the scale multiplies the logits, whatever its sign."""
+    hq, hkv, d = shape
+    bt, dev, q, cache, scale = make_case(pkg, oracle, 670 + hq + d, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=1,
+                                         dec_kv_lens=[70, 300, 33, 5], outliers=True)
+    monkeypatch.setattr(pkg.workloads.Batch, "attn_scale", attn_scale)
+    width = (int(bt.kvstarts[-1]) + 7) // 8 * 8
+    mask = np.random.default_rng(3).standard_normal((bt.batch, width)).astype(np.float16)
+    md = torch.from_numpy(mask).cuda()
+    for host, device in (({}, {}), (dict(attn_mask=mask, mask_stride_s=width), dict(attn_mask=md, mask_stride_s=width))):
+        ref = oracle_decode(oracle, bt, q, cache, scale, **host)
+        for ranges in (1, 0, 4):
+            got, plan = run_decode(dev, ranges, **device)
+            assert_attention_close(got, ref, "%s scale %g ranges %d %s" % (shape, attn_scale, plan.num_token_ranges, sorted(host)))

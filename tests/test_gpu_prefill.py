@@ -460,3 +460,19 @@ def test_prefill_short_chunks_sequence_by_sequence(pkg, oracle, shape, sequences
     got = run_prefill(pkg, dev, is_causal=is_causal)
     assert_attention_close(got[1:], ref[1:], "chunks by sequence %s" % (shape,))
     assert np.isnan(got[:1]).all()
+
+
+@pytest.mark.parametrize("attn_scale", [-0.3, 0.0])
+@pytest.mark.parametrize("shape", [(32, 8, 128), (8, 8, 64), (12, 3, 96), (8, 1, 256)])
+def test_prefill_with_a_scale_that_is_not_positive(pkg, oracle, monkeypatch, shape, attn_scale):
+    """Short chunks with and without a workspace, and prompts: the scale multiplies the logits, whatever its sign."""
+    hq, hkv, d = shape
+    for q_lens in ([2, 1, 4, 3], [130, 17]):
+        bt, dev, q, cache, scale = make_case(pkg, oracle, 390 + hq + d, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=1,
+                                             dec_kv_lens=[33], prefill_q_lens=q_lens, prefill_prior=[40, 200, 0, 129][:len(q_lens)], outliers=True)
+        monkeypatch.setattr(pkg.workloads.Batch, "attn_scale", attn_scale)
+        ref = oracle_prefill(oracle, bt, q, cache, scale)
+        nbytes = pkg.ops.prefill_workspace_size(bt.batch, bt.decoding_batches, bt.max_seqlen, bt.max_kvlen, hq, hkv, d)
+        for ws in (None, torch.empty(nbytes, dtype=torch.uint8, device="cuda") if nbytes else None):
+            got = run_prefill(pkg, dev, workspace=ws)
+            assert_attention_close(got[1:], ref[1:], "%s scale %g %s" % (shape, attn_scale, q_lens))
