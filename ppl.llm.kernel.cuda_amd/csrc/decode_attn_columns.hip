@@ -15,9 +15,12 @@
 // passes (blockIdx.z), each of which reads the cache again: the bytes of one kv head are few and stay in the L2.
 //
 // Exactness follows the prefill kernel: K^ = int8 * scale, V^ and p are kept as hi + lo pairs of halves
-// (2 MFMAs per QK step, 3 per PV step), so no fp16 rounding of the dequantised cache enters the result.
-// Against float64 the outputs' error is that of rounding them to half, as with the kernels that served these batches before (32 q /
-// 8 kv heads of 128, 16 sequences of 30-200: rms 7.43e-5, maximum 9.60e-4 for either, and for the rounding alone; ten shapes).
+// (2 MFMAs per QK step, 3 per PV step), so no fp16 rounding of the dequantised cache enters the result.  Those pairs hold 22 bits
+// where the quad and general kernels, which served some of these batches before, multiply p and V in float32, and the product of the two
+// low parts, 2^-22 of a term, is left out.  Against float64 the error is no larger than theirs: the float32 pieces of one sequence of
+// 512 tokens are off by 3.3e-7 (rms, of 8 / 8 heads of 64) to 4.8e-7 (32 / 8 of 128), on the quad kernel by 4.4e-7 (8 / 8 of 64), and the half
+// outputs of twelve shapes of decode batches and seven of short chunks by their rounding to half alone (2.06e-4 to 2.10e-4, to four
+// digits; 12 / 3 heads of 96, 20 chunks of 1-5 rows 2.064e-4, on the tile kernel, whose row sums run over p's high halves, 2.075e-4).
 //
 // The cache rows travel from memory into a wave-private LDS ring without registers (global_load_lds), two blocks
 // ahead of the arithmetic, and across sequences: the blocks of a range are one stream to the requests, so the first
@@ -48,6 +51,7 @@ namespace {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
@@ -626,8 +630,9 @@ __device__ __forceinline__ void decode_columns(const DecodeLaunch& a, char* cons
                     const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[t][e], sm_scale, bias));
                     const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[t][e + 1], sm_scale, bias));
                     lsum += p0 + p1;
-                    const half2_t h = bitcast<half2_t>(__builtin_amdgcn_cvt_pkrtz(p0, p1));
-                    const half2_t l = bitcast<half2_t>(__builtin_amdgcn_cvt_pkrtz(sub_half_lo(p0, h), sub_half_hi(p1, h)));
+                    // both parts rounded to nearest: p within 2^-23 of itself (up to three times that, and always below it, when they are cut off)
+                    const half2_t h = __builtin_convertvector(f32x2{p0, p1}, half2_t);
+                    const half2_t l = __builtin_convertvector(f32x2{sub_half_lo(p0, h), sub_half_hi(p1, h)}, half2_t);
                     const int k = 4 * t + e; // C = 16: tile t's four results follow each other
                     ph[k >> 3][k & 7] = h.x;
                     ph[k >> 3][(k & 7) + 1] = h.y;

@@ -75,3 +75,26 @@ def test_hi_lo_pairs_are_what_the_tolerance_costs(seed, prior, nq):
     assert _worst(*case, p_lo=False) > 3 * full
     assert _worst(*case, v_lo=False) > 3 * full
     assert _worst(*case, p_lo=False, v_lo=False) > 5 * full
+
+
+def test_both_parts_of_a_probability_are_rounded_to_nearest():
+    """p in (0, 2^14] as two halves: to nearest it is within 2^-23 of itself (2^-25 absolute where the low part is subnormal) and off
+    to either side; cut off, as v_cvt_pkrtz does, up to three times that and always below.  The column kernel has no cut-off conversion."""
+    import os
+    rng = np.random.default_rng(0)
+    p = (2.0 ** rng.uniform(-10, 14, 200000)).astype(np.float32)
+
+    def cut_off(x):
+        h = x.astype(np.float16)
+        return np.where(h.astype(np.float32) > x, np.nextafter(h, np.float16(0)), h).astype(np.float32)
+
+    def error(to_half):
+        hi = to_half(p)
+        lo = to_half(p - hi)  # exact difference
+        return (hi.astype(np.float64) + lo.astype(np.float64) - p) / np.maximum(p * 2.0 ** -23, 2.0 ** -25)
+
+    nearest, cut = error(_f16), error(cut_off)
+    assert np.abs(nearest).max() <= 1.0 and abs(nearest.mean()) < 0.01
+    assert cut.max() <= 0.0 and cut.min() < -2.9
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "ppl.llm.kernel.cuda_amd", "csrc")
+    assert "cvt_pkrtz" not in open(os.path.join(csrc, "decode_attn_columns.hip")).read()
