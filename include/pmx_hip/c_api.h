@@ -283,19 +283,25 @@ typedef struct pmxhip_prefill_params {
      * <= 32, head_dim 64 or 128, no attn_mask, alibi or current_key -- runs on the decode step's MFMA kernels over
      * token ranges, with (query position, query head) pairs as its columns and the split-KV pieces in this
      * workspace; without it, or for any other batch, the tile kernel runs.  Results are the same within the tolerance.
-     * (Chunks of that size over short histories run there sequence by sequence, at every head_dim, and use no workspace.)
-     * On that path max_seqlen must bound the query rows of every prefill sequence, as it does in the reference's
+     * Chunks of that size over short histories run there sequence by sequence, at every head_dim, and use no workspace.
+     * Over token ranges max_seqlen must bound the query rows of every prefill sequence, as it does in the reference's
      * call (kernel.cu:2143), because the step has max_seqlen query positions per sequence.  A max_seqlen that
-     * prefill_query_rows proves too small (more rows than prefill sequences * max_seqlen) keeps the batch on the tile
-     * kernel, which walks every row whatever the hint; otherwise the rows of a sequence beyond max_seqlen are not
-     * computed and are filled with NaN, so that an understated hint shows in the output.  A layout or alignment that
-     * the decode kernels refuse also keeps the batch on the tile kernel.  A batch that is not one of short chunks leaves
-     * the buffer alone (pmxhip_prefill_attention_split has one of its own). */
+     * prefill_query_rows proves too small (more rows than prefill sequences * max_seqlen) keeps the batch from that route;
+     * otherwise the rows of a sequence beyond max_seqlen are not computed and are filled with NaN, so that an
+     * understated hint shows in the output.  Sequence by sequence, and on the tile kernel, every row is computed whatever
+     * the hint.  A layout, an alignment or an attn_scale that the decode kernels refuse also keeps the batch on the tile
+     * kernel.  A batch that is not one of short chunks leaves the buffer alone (pmxhip_prefill_attention_split has one of
+     * its own).  pmxhip_prefill_kernel_name tells what a call runs. */
     void* workspace;
     int64_t workspace_size;
 } pmxhip_prefill_params;
 
 PMXHIP_API int pmxhip_prefill_attention(const pmxhip_prefill_params* p, pmxhip_stream_t stream);
+
+/* Name of the kernel that pmxhip_prefill_attention(p) launches ("" if nothing is launched or the call would be rejected):
+ * prefill_attention_kernel or prefill_attention16_kernel (head_dim 256), the tile kernels; for short chunks one of the names of
+ * pmxhip_decode_kernel_name.  Host only, launches nothing. */
+PMXHIP_API const char* pmxhip_prefill_kernel_name(const pmxhip_prefill_params* p);
 
 /* pmxhip_prefill_attention with a second workspace (16-byte aligned; NULL = none): where it has the bytes of
  * pmxhip_prefill_split_workspace_size(), a batch of few query tiles that does not run as short chunks shares the kv

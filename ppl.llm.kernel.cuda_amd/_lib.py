@@ -27,7 +27,7 @@ EXPORTED_SYMBOLS = (
     "pmxhip_decode_plan_make", "pmxhip_decode_plan_make_kernel", "pmxhip_decode_attention",
     "pmxhip_decode_attention_stage", "pmxhip_decode_attention_static", "pmxhip_decode_kernel_name",
     "pmxhip_splitkv_combine",
-    "pmxhip_prefill_attention", "pmxhip_prefill_attention_split", "pmxhip_prefill_workspace_size", "pmxhip_prefill_split_workspace_size",
+    "pmxhip_prefill_attention", "pmxhip_prefill_attention_split", "pmxhip_prefill_kernel_name", "pmxhip_prefill_workspace_size", "pmxhip_prefill_split_workspace_size",
     "pmxhip_mhca_create", "pmxhip_mhca_destroy", "pmxhip_mhca_heuristic_prepare", "pmxhip_mhca_heuristic_prepare_ex",
     "pmxhip_mhca_get_derived", "pmxhip_mhca_set_workspace",
     "pmxhip_mhca_forward_kvstore", "pmxhip_mhca_forward_decode", "pmxhip_mhca_forward_prefill",
@@ -253,6 +253,8 @@ def lib():
     L.pmxhip_prefill_workspace_size.argtypes = [c_i64] * 7 + [c_i32]
     L.pmxhip_prefill_split_workspace_size.restype = c_i64
     L.pmxhip_prefill_split_workspace_size.argtypes = [c_i64] * 8 + [c_i32] * 2
+    L.pmxhip_prefill_kernel_name.restype = ctypes.c_char_p
+    L.pmxhip_prefill_kernel_name.argtypes = [ctypes.POINTER(PrefillParams)]
     L.pmxhip_prefill_attention.restype = ctypes.c_int
     L.pmxhip_prefill_attention.argtypes = [ctypes.POINTER(PrefillParams), c_vp]
     L.pmxhip_prefill_attention_split.restype = ctypes.c_int

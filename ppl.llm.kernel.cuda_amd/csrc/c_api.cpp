@@ -370,9 +370,10 @@ int decode_prepare(const char* who, const pmxhip_decode_params* p, void* workspa
 int decode_prepare_quiet(const char* who, const pmxhip_decode_params* p, void* workspace, int64_t workspace_size,
                          pmxhip::DecodeLaunch* out, bool columns = false)
 {
+    const bool quiet = g_quiet;
     g_quiet = true;
     const int rc = decode_prepare(who, p, workspace, workspace_size, out, columns);
-    g_quiet = false;
+    g_quiet = quiet;
     return rc;
 }
 
@@ -499,8 +500,9 @@ int pmxhip_prefill_attention(const pmxhip_prefill_params* p, pmxhip_stream_t str
     return pmxhip_prefill_attention_split(p, nullptr, 0, stream);
 }
 
-int pmxhip_prefill_attention_split(const pmxhip_prefill_params* p, void* split_workspace, int64_t split_workspace_size,
-                                   pmxhip_stream_t stream)
+// `name`: NULL = launch; else nothing is launched and the name of the kernel that would be is written there.
+static int prefill_run(const pmxhip_prefill_params* p, void* split_workspace, int64_t split_workspace_size, pmxhip_stream_t stream,
+                       const char** name)
 {
     if (!p) return fail(PMXHIP_INVALID_VALUE, "prefill_attention: null params");
     const int64_t prefill_batches = p->batch - p->decoding_batches;
@@ -536,10 +538,10 @@ int pmxhip_prefill_attention_split(const pmxhip_prefill_params* p, void* split_w
     if ((reinterpret_cast<uintptr_t>(p->output) & 7u) || p->output_stride_s % 4 != 0)
         return fail(PMXHIP_UNSUPPORTED, "prefill_attention: output must be 8-byte aligned with a row stride that is a multiple of 4");
 
-    // short chunks on the decode step's kernels, where the shape, the inputs and the caller's workspace allow.  That
-    // route computes max_seqlen query positions per sequence, so a max_seqlen that the row count of the prefill
-    // sequences proves too small (more rows than sequences * max_seqlen) keeps the batch on the tile kernel, which
-    // walks every row whatever the hint.
+    // short chunks on the decode step's kernels, where the shape, the inputs and the caller's workspace allow.  Over
+    // ranges that route computes max_seqlen query positions per sequence, so a max_seqlen that the row count of the prefill
+    // sequences proves too small (more rows than sequences * max_seqlen) keeps the batch from it: sequence by sequence
+    // and on the tile kernel every row is walked whatever the hint.
     const bool hint_covers_rows = p->prefill_query_rows <= 0 || p->prefill_query_rows <= prefill_batches * p->max_seqlen;
     const bool short_chunks = !from_current && !p->attn_mask && !p->alibi_slopes &&
                               prefill_chunk_shape(p->max_seqlen, p->num_heads, p->num_kv_heads, p->head_dim);
@@ -599,6 +601,10 @@ int pmxhip_prefill_attention_split(const pmxhip_prefill_params* p, void* split_w
                 c.shared_pieces = 1;
                 c.ring = pmxhip::decode_ring(c, p->max_kvlen);
             }
+            if (name) {
+                *name = pmxhip::decode_kernel_name(c);
+                return PMXHIP_SUCCESS;
+            }
             return launch_result("prefill_attention", pmxhip::launch_decode(c, 0, stream));
         }
     }
@@ -654,8 +660,28 @@ int pmxhip_prefill_attention_split(const pmxhip_prefill_params* p, void* split_w
             a.split_ml = (float*)((char*)split_workspace + split.out_bytes);
         }
     }
+    if (name) {
+        *name = pmxhip::prefill_kernel_name(a);
+        return PMXHIP_SUCCESS;
+    }
     return launch_result("prefill_attention", pmxhip::launch_prefill(a, stream));
 }
+
+int pmxhip_prefill_attention_split(const pmxhip_prefill_params* p, void* split_workspace, int64_t split_workspace_size,
+                                   pmxhip_stream_t stream)
+{
+    return prefill_run(p, split_workspace, split_workspace_size, stream, nullptr);
+}
+
+const char* pmxhip_prefill_kernel_name(const pmxhip_prefill_params* p)
+{
+    const char* name = "";
+    g_quiet = true;
+    if (prefill_run(p, nullptr, 0, nullptr, &name) != PMXHIP_SUCCESS) name = "";
+    g_quiet = false;
+    return name;
+}
+
 
 static int reorder_common(const char* what, bool invert, pmxhip_stream_t stream, const void* cache, const void* scale,
                           const void* outer, const int64_t* page_ids, const pmxhip_reorder_stride* src,

@@ -340,6 +340,7 @@ void launch_splitkv_combine_rows(const float* partial_out, const float* partial_
                                  const int64_t* piece_end, int64_t rows, int64_t head_dim, void* output,
                                  hipStream_t stream);
 int launch_prefill(const PrefillLaunch& a, hipStream_t stream);
+const char* prefill_kernel_name(const PrefillLaunch& a); // "" where launch_prefill has none
 // decode_select.cpp: whether a prefill batch of this shape runs on the decode step's kernels when it has a workspace,
 bool prefill_chunk_shape(int64_t max_seqlen, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim);
 // and whether it runs there sequence by sequence, which takes no workspace (`ranges_served`: it could be cut into ranges)

@@ -1593,6 +1593,12 @@ int launch_prefill(const PrefillLaunch& in, hipStream_t stream)
     }
 }
 
+const char* prefill_kernel_name(const PrefillLaunch& a)
+{
+    if (a.head_dim == 256) return "prefill_attention16_kernel";
+    return a.num_heads / a.num_kv_heads > kCols ? "" : "prefill_attention_kernel";
+}
+
 template <int D, int SRC, bool EXTRA>
 static int init_prefill_variant()
 {

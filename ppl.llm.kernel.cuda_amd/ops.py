@@ -175,12 +175,13 @@ def prefill_attention(query, output, cache, scale, seqstarts, kvstarts, cachesta
                       head_dim, cache_mode, page_size, cache_stride_s, cache_stride_l, cache_stride_h,
                       cache_stride_kv, cachestarts_stride_b, attn_mask=None, mask_stride_s=0, mask_stride_h=0,
                       alibi_slopes=None, current_key=None, current_value=None, prefill_query_rows=None, workspace=None,
-                      stream=None, check=True):
+                      stream=None, check=True, name_only=False):
     """Multi-query-token attention of the prefill sequences.  Optional: additive half `attn_mask` with its
     strides, float32 `alibi_slopes` [Hq], `current_key`/`current_value` [rows, KVH, D] to attend over
     the step's own fp16 rows instead of the cache, and a `workspace` of prefill_workspace_size() bytes with which a
     batch of short chunks runs on the decode step's kernel, or of prefill_split_workspace_size() bytes with which a batch
-    of few query tiles is split over its kv tokens (no other call may use the workspace while this one runs)."""
+    of few query tiles is split over its kv tokens (no other call may use the workspace while this one runs).  `name_only`
+    launches nothing and returns the name of the kernel the call would run."""
     p = PrefillParams()
     p.query = _ptr(query)
     p.output = _ptr(output)
@@ -222,6 +223,8 @@ def prefill_attention(query, output, cache, scale, seqstarts, kvstarts, cachesta
     if workspace is not None:
         p.workspace = _ptr(workspace)
         p.workspace_size = int(workspace.numel() * workspace.element_size())
+    if name_only:
+        return _lib.lib().pmxhip_prefill_kernel_name(ctypes.byref(p)).decode()
     rc = _lib.lib().pmxhip_prefill_attention_split(ctypes.byref(p), p.workspace, p.workspace_size, _stream(stream))
     if check and rc != RC_SUCCESS:
         raise PmxError(rc, "prefill_attention")

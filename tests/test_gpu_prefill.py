@@ -476,3 +476,33 @@ def test_prefill_with_a_scale_that_is_not_positive(pkg, oracle, monkeypatch, sha
         for ws in (None, torch.empty(nbytes, dtype=torch.uint8, device="cuda") if nbytes else None):
             got = run_prefill(pkg, dev, workspace=ws)
             assert_attention_close(got[1:], ref[1:], "%s scale %g %s" % (shape, attn_scale, q_lens))
+
+
+@pytest.mark.parametrize("d,q_lens,prior,claimed,kernel", [
+    # rows that the hint denies: sequence by sequence over a short history, on the tile kernel where the columns are too many for that
+    (128, [4, 2, 8, 3], [200, 0, 90, 33], 4, "decode_attention_mfma16_kernel"),
+    (96, [6, 1, 3, 2], [64, 31, 0, 5], 2, "decode_attention_mfma16_kernel"),
+    (128, [40, 2, 60, 3], [200, 0, 90, 33], 20, "prefill_attention_kernel"),
+    (128, [40, 2, 60, 3], [1500, 0, 900, 33], 9, "prefill_attention_kernel"),
+    (256, [40, 2, 60, 3], [200, 0, 90, 33], 20, "prefill_attention16_kernel")])
+def test_prefill_understated_max_seqlen_by_the_kernel_that_runs(pkg, oracle, d, q_lens, prior, claimed, kernel):
+    """Sequence by sequence and on the tile kernel every row is computed, whatever max_seqlen says."""
+    hq, hkv = 32, 8
+    bt, dev, q, cache, scale = make_case(pkg, oracle, 397, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=1, dec_kv_lens=[33],
+                                         prefill_q_lens=q_lens, prefill_prior=prior, outliers=True)
+    ref = oracle_prefill(oracle, bt, q, cache, scale)
+    nbytes = pkg.ops.prefill_workspace_size(bt.batch, 1, claimed, bt.max_kvlen, hq, hkv, d)
+    ws = torch.full((nbytes // 4,), float("nan"), dtype=torch.float32, device="cuda") if nbytes else None
+
+    def call(**kw):
+        return pkg.ops.prefill_attention(dev.query, dev.output, dev.cache, dev.scale, dev.seqstarts, dev.kvstarts, dev.cachestarts,
+                                         attn_scale=bt.attn_scale, is_causal=True, batch=bt.batch, decoding_batches=1, max_seqlen=claimed,
+                                         max_kvlen=bt.max_kvlen, layer_idx=0, num_heads=hq, num_kv_heads=hkv, head_dim=d, workspace=ws,
+                                         **dev.layout_kwargs(), **kw)
+    assert call(name_only=True) == kernel
+    dev.output.fill_(3.0)
+    call()
+    torch.cuda.synchronize()
+    got = dev.output.float().cpu().numpy()
+    assert_attention_close(got[1:], ref[1:], "%s, max_seqlen %d of %d" % (kernel, claimed, max(q_lens)))
+    assert (got[0] == 3.0).all() and (ws is None or torch.isnan(ws).all())
