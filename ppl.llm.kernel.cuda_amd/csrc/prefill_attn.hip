@@ -1402,11 +1402,10 @@ static int launch_prefill_variant(const PrefillLaunch& a, dim3 grid, hipStream_t
         if constexpr (SRC == 2)
             hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, false, 2, 4>), grid, dim3(256), (prefill_lds_bytes<D, SRC, 4>()), stream, a);
     } else if (D == 64 && SRC == 2 && !EXTRA && grid.x > (unsigned)a.compute_units) {
-        // More workgroups than CUs: two per CU cover each other's waits although a few registers spill (32 q / 8 kv heads, 12
-        // prompts of 300-3000 rows: layer call 356 -> 287 us).  With a workgroup per CU or fewer only the spills are left
-        // (8 / 8 heads, six prompts of 300-1500 rows: 46.9 against 48.7 us).
-        if constexpr (D == 64 && SRC == 2 && !EXTRA)
-            hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, false, 4>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
+        // Eight waves of 256 columns, where the heads of a group fill 128 worse (prefill_columns): with more workgroups than CUs two per
+        // CU cover each other's waits although 13 registers spill (12 prompts of 300-3000 rows, 48 / 1 heads: 571 -> 460 us, four waves
+        // 515; 71 / 1 heads 931 -> 694, four waves 989).  With a workgroup per CU or fewer only the spills are left.
+        hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, false, 4>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
     } else
         hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, EXTRA, false>), grid, dim3(kPrefillThreads), lds_bytes, stream, a);
     return kLaunchOk;
@@ -1568,9 +1567,11 @@ PrefillSplit prefill_split_choose(int64_t sequences, int64_t max_seqlen, int64_t
 
 // Columns of a workgroup of the 32-column kernel.  Over half K/V rows (no dequantisation, so little shared work to lose) four waves
 // of 128 columns do better than eight of 256: two workgroups fit a CU (at most 68 KB of LDS each) and one computes while the other
-// waits at its tile's barriers, and the last tiles of a batch are half as long: 32 q / 8 kv heads of 128, 12 prompts
-// of 300-3000 rows 509 -> 497 us, 64 prompts of 30-150 rows 59 -> 54, with alibi slopes four prompts of
-// 300-2500 rows 239 -> 218; 32 / 32 heads, 26 prompts of 270-336 rows 158 -> 128; one prompt of 1000 rows is level.
+// waits at its tile's barriers, and the last tiles of a batch are half as long.  Against 256 columns, head_dim 128: 32 q / 8 kv heads,
+// 64 prompts of 30-150 rows 54.5 -> 49.5 us, 26 of 270-336 86.7 -> 79.7, 12 of 300-3000 level (502, 510), one of 1000 51.7 -> 41.6, with
+// alibi slopes the twelve 723 -> 671; 32 / 32 heads, the 26 127 -> 92.  head_dim 64, whose form of 256 columns has two workgroups per CU as
+// well: 32 / 8 heads, the 64 35.5 -> 33.2, the twelve level (305, 307), one of 1000 38.9 -> 32.3; 8 / 8 heads, six of 300-1500 49.0 -> 39.4;
+// 64 / 8 heads, those six the only batch that lost, 119.5 -> 122.6.
 // The int8 cache keeps 256: its tiles, dequantised once per workgroup, take all of a CU's LDS.  So does a group whose heads fill
 // 128 columns worse (48 heads per kv head: 96 of 128, 240 of 256).
 static int prefill_columns(const PrefillLaunch& a)

@@ -506,3 +506,22 @@ def test_prefill_understated_max_seqlen_by_the_kernel_that_runs(pkg, oracle, d, 
     got = dev.output.float().cpu().numpy()
     assert_attention_close(got[1:], ref[1:], "%s, max_seqlen %d of %d" % (kernel, claimed, max(q_lens)))
     assert (got[0] == 3.0).all() and (ws is None or torch.isnan(ws).all())
+
+
+@pytest.mark.parametrize("shape,prompts", [((48, 1, 64), 270), ((26, 2, 64), 150)])
+def test_prefill_from_current_key_value_of_groups_that_fill_256_columns_better(pkg, oracle, shape, prompts):
+    """Half K/V rows at head_dim 64 with more tiles of 256 columns than compute units, in group sizes that do not fill 128: eight
+    waves whose registers are cut for two workgroups per CU."""
+    hq, hkv, d = shape
+    assert 2 * (128 // (hq // hkv) * (hq // hkv)) * 25 < (256 // (hq // hkv) * (hq // hkv)) * 24
+    q_lens = [1 + (7 * i) % 11 for i in range(prompts)]
+    bt, rng = pkg.workloads.custom_batch(890 + hq, num_heads=hq, num_kv_heads=hkv, head_dim=d, cache_mode=0, dec_kv_lens=[5],
+                                         prefill_q_lens=q_lens, prefill_prior=[0] * prompts, outliers=True)
+    dev = pkg.harness.DeviceBatch(bt)
+    q, k, v = pkg.workloads.step_inputs(bt, rng)
+    dev.set_step_inputs(q, k, v)
+    cache, scale = host_cache(bt)
+    ref = oracle_prefill_ex(oracle, bt, q, cache, scale, current_key=k, current_value=v)
+    got = run_prefill(pkg, dev, current_key=dev.new_key, current_value=dev.new_value)
+    assert_attention_close(got[1:], ref[1:], "groups of %d" % (hq // hkv))
+    assert np.isnan(got[:1]).all()
