@@ -234,7 +234,8 @@ bool quad_by_sequence(int64_t sequences, int64_t num_kv_heads, int64_t g, bool m
 // One to four sequences cut into ranges run on the column kernels where those are the faster ones: 32 q / 8 kv heads of 128, one
 // sequence of 1024 / 4096 / 16384 tokens 14.1 / 15.3 / 21.4 us on the quad kernel, 11.3 / 12.8 / 19.5 here; four of 1024 / 2048 /
 // 4096 14.0 / 16.7 / 19.1 and 11.6 / 13.3 / 16.9.  Not with one query head per kv head at head_dim 128 (the quad kernel has a
-// quarter of the arithmetic to do there: one of 4096 15.5 against 18.8) and not at head_dim 256.  Sixteen are level.
+// quarter of the arithmetic to do there: one of 4096 15.5 against 18.8) and not at head_dim 256.  From five on the quad kernel is
+// the faster one (five of 333-1000 14.0 against 14.9, of 1333-4000 19.9 against 22.7; eight 16.0 / 15.1 and 24.1 / 25.1).
 constexpr int64_t kFewSequences = 4;
 bool few_sequences_on_columns(int64_t sequences, int64_t head_dim, int64_t g)
 {
@@ -373,9 +374,10 @@ int64_t decode_choose_ranges(const DecodeChoice& by_shape, int64_t sequences, in
     const bool columns = c.kernel == kDecodeKernelMfma16 || c.kernel == kDecodeKernelMfma32;
     const int min_tokens = decode_min_tokens_per_range(c.wg_tokens);
     const int64_t groups = ((num_kv_heads + c.kv_heads_per_group - 1) / c.kv_heads_per_group) * c.num_passes;
-    if (automatic && c.kernel == kDecodeKernelMfma16 && sequences == 1 && max_tokens <= kSharedStreamTokens) {
+    const int64_t shared_groups = column_groups(head_dim, g, num_kv_heads);
+    if (automatic && c.kernel == kDecodeKernelMfma16 && sequences == 1 && max_tokens * shared_groups <= kSharedStreamTokens) {
         // a single sequence: ranges of 128 tokens or more that four waves share, one workgroup per CU
-        const int64_t most = compute_units / column_groups(head_dim, g, num_kv_heads);
+        const int64_t most = compute_units / shared_groups;
         const int64_t useful = (max_tokens + 127) / 128;
         return useful < most ? useful : (most > 1 ? most : 2);
     }

@@ -308,8 +308,10 @@ int decode_plan_make(int64_t decoding_batches, int64_t num_heads, int64_t num_kv
                      int32_t num_token_ranges_hint, int32_t kernel_request, bool mask, pmxhip_decode_plan* plan);
 // pmxhip_decode_attention for a caller that knows the longest sequence (c_api.cpp).
 int decode_attention_sized(const pmxhip_decode_params* p, int64_t max_kvlen, hipStream_t stream);
-// A single sequence of more tokens is cut as any other stream.
-constexpr int64_t kSharedStreamTokens = 32768;
+// A single sequence of more tokens times kv heads (and passes) is cut as any other stream, whose waves then have a range each: with
+// eight kv heads of 128 that is level at 32768 tokens (28.4 us shared, 28.6 as 256 ranges) and the faster one at 65536 (43.1, 40.3); with four
+// shared pieces are at 65536 (28.2, 32.4), with one at 131072 (21.2, 38.9).
+constexpr int64_t kSharedStreamTokens = 262144;
 // The kernel of a launch whose shape, ranges, strides and buffers are filled in, and how it takes it: the fields from
 // kv_heads_per_group on.  A single range without a request means that every sequence is taken whole by workgroups of its own.
 // `columns`: the column kernels whatever the shape.  `max_kvlen`: the longest sequence, 0 = unknown (a long one).  `out`: the

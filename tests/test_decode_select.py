@@ -120,6 +120,13 @@ def test_scales_that_are_not_positive_run_on_kernels_that_scale_first(select):
     assert select(64, 64, 8, 128, 8192, scale=1e-6)[0] == MFMA16
 
 
+def test_a_single_sequence_is_shared_by_four_waves_up_to_a_length_that_its_kv_heads_set(select):
+    for shape, most in (((1, 32, 8, 128, 32768), 32), ((1, 28, 4, 128, 65536), 64), ((1, 8, 1, 128, 262144), 256), ((1, 8, 1, 128, 40000), 256)):
+        assert select(*shape)[1] == most and select(*shape, ring=True) == (4, True), shape
+    for shape in ((1, 32, 8, 128, 40000), (1, 28, 4, 128, 70000)):
+        assert select(*shape)[1] > 256 // shape[2] and select(*shape, ring=True)[0] == 1, shape
+
+
 def test_ranges_and_requests_keep_their_kernels(select):
     assert select(64, 32, 8, 128, 4096)[::2] == (QUAD, False)
     assert select(64, 32, 8, 128, 4096, mask=True)[::2] == (QUAD, False)
