@@ -252,7 +252,7 @@ bool quad_takes_whole(const DecodeLaunch& a) { return a.num_kv_repeats <= 4 && d
 // more than 8 %).  Few workgroups leave the chip idle and ranges fill it; from one per CU on the waves are there either
 // way, and ranges even out the lengths.  Past eight per CU the waves come in a second round.
 struct WholeUpTo {
-    double masked;         // with a mask, times this: the column kernels wait for its values, the quad kernel streams them
+    double masked;         // with a mask, times this where the column kernels run: they wait for its values, the quad kernel streams them
     int32_t tokens[15];    // workgroups per CU up to kWholeLoads[i], and beyond
 };
 constexpr double kWholeLoads[14] = {0.05, 0.1, 0.2, 0.4, 0.75, 1, 1.6, 2, 2.75, 3.5, 5, 8, 15.99, 32};
@@ -292,8 +292,10 @@ int64_t whole_up_to(const DecodeChoice& by_shape, int64_t sequences, int64_t hea
     int i = 0;
     while (i < 14 && load > kWholeLoads[i]) ++i;
     int64_t tokens = row.tokens[i];
-    const bool other_kernel = by_shape.kernel == kDecodeKernelQuad && head_dim == 64 && columns > 1; // (no mask form there)
-    if (mask && tokens != kAnyLength && !other_kernel) tokens = (int64_t)(row.masked * (double)tokens);
+    // (at head_dim 64 a masked step over ranges is another kernel's, and slower as well)
+    const bool quad = by_shape.kernel == kDecodeKernelQuad;
+    const bool streams_mask = quad && (head_dim == 64 ? columns > 1 : quad_by_sequence(sequences, num_kv_heads, columns, true, cus));
+    if (mask && tokens != kAnyLength && !streams_mask) tokens = (int64_t)(row.masked * (double)tokens);
     // the pieces of few columns cost less, those of many more (32 / 8 heads of 128, 100 chunks of one row: level at 476 tokens, of two
     // rows at 616, of four at 957)
     if (by_shape.kernel != kDecodeKernelQuad && by_shape.kernel != kDecodeKernelGeneral && load > 1) {
