@@ -73,7 +73,7 @@ def test_sequences_are_taken_whole_where_that_was_measured_faster(select):
     # a mask that the quad kernel streams changes nothing, one that the column kernels wait for takes whole sequences half as far
     for shape in ((512, 32, 8, 128, 300), (600, 16, 8, 256, 150), (300, 32, 32, 128, 128)):
         assert select(*shape, mask="planned") == (QUAD, 1, True), shape
-    assert select(60, 64, 8, 128, 700)[2] is False and select(60, 64, 8, 128, 500)[2] is True
+    assert select(60, 64, 8, 128, 800)[2] is False and select(60, 64, 8, 128, 700)[2] is True
     assert select(60, 64, 8, 128, 500, mask="planned")[2] is False and select(60, 64, 8, 128, 300, mask="planned")[2] is True
     # longer sequences are never taken whole where shorter ones are cut, and a plan that knows of a mask takes no more of them whole
     for n, hq, hkv, d, _ in WHOLE + CUT:
