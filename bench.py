@@ -203,8 +203,9 @@ def rope_sweep_bench(torch, pkg, steps, replays):
 
 def chunk_bench(torch, pkg, spec, steps, replays):
     """--chunks: the prefill stage on a batch of short chunks (a few query tokens per sequence over a long history, no
-    decode sequences), once on the tile kernel (no workspace) and once with the workspace that routes it to the decode
-    step's MFMA kernel.  A graph of `steps` stage calls replayed `replays` times back to back, median replay."""
+    decode sequences), on the tile kernel (a hint of more rows than short chunks have keeps the batch on it), without a
+    workspace, and with the workspace that lets the decode step's MFMA kernels run over token ranges.  A graph of `steps`
+    stage calls replayed `replays` times back to back, median replay."""
     wl, harness, ops = pkg.workloads, pkg.harness, pkg.ops
     c = dict(hq=32, hkv=8, d=128, seqs=64, qmin=2, qmax=8, prior=2048, mode=1)
     c.update({k: int(v) for k, v in (kv.split("=") for kv in spec.split(","))})
@@ -215,17 +216,19 @@ def chunk_bench(torch, pkg, spec, steps, replays):
     dev.fill_history(rng, max_rows=1 << 15)
     q, k, v = wl.step_inputs(bt, rng)
     dev.set_step_inputs(q, k, v)
-    kw = dict(attn_scale=bt.attn_scale, is_causal=True, batch=bt.batch, decoding_batches=0, max_seqlen=bt.max_seqlen,
+    kw = dict(attn_scale=bt.attn_scale, is_causal=True, batch=bt.batch, decoding_batches=0, prefill_query_rows=sum(q_lens),
               max_kvlen=bt.max_kvlen, layer_idx=bt.layer_idx, num_heads=c["hq"], num_kv_heads=c["hkv"], head_dim=c["d"],
               **dev.layout_kwargs())
+    more_rows = max(bt.max_seqlen, 32 * c["hkv"] // c["hq"] + 1)
     ws_bytes = ops.prefill_workspace_size(bt.batch, 0, bt.max_seqlen, bt.max_kvlen, c["hq"], c["hkv"], c["d"])
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev.device)
     stream, side = torch.cuda.current_stream(), torch.cuda.Stream()
 
-    def timed(workspace):
-        def call(st):
-            ops.prefill_attention(dev.query, dev.output, dev.cache, dev.scale, dev.seqstarts, dev.kvstarts, dev.cachestarts,
-                                  workspace=workspace, stream=st, **kw)
+    def timed(workspace, max_seqlen):
+        def call(st, **options):
+            return ops.prefill_attention(dev.query, dev.output, dev.cache, dev.scale, dev.seqstarts, dev.kvstarts, dev.cachestarts,
+                                         workspace=workspace, max_seqlen=max_seqlen, stream=st, **kw, **options)
+        kernel = call(stream, name_only=True)
         call(stream)
         torch.cuda.synchronize()
         with torch.cuda.stream(side):
@@ -241,11 +244,12 @@ def chunk_bench(torch, pkg, spec, steps, replays):
                 graph.replay()
                 evs[r + 1].record(side)
             side.synchronize()
-        return float(np.median([evs[r].elapsed_time(evs[r + 1]) * 1e3 / steps for r in range(replays)]))
+        return kernel, float(np.median([evs[r].elapsed_time(evs[r + 1]) * 1e3 / steps for r in range(replays)]))
 
-    tile_us = timed(None)
+    tile, tile_us = timed(None, more_rows)
     tile_out = dev.output.clone()
-    chunk_us = timed(ws) if ws_bytes else None
+    plain, plain_us = timed(None, bt.max_seqlen)
+    chunk, chunk_us = timed(ws, bt.max_seqlen) if ws_bytes else (None, None)
     diff = float((dev.output.float() - tile_out.float()).abs().max()) if ws_bytes else None
     cache_bytes = int(sum(int(x) for x in bt.kv_lens)) * c["hkv"] * (2 * c["d"] + c["d"] // 2)
     print(json.dumps({
@@ -254,7 +258,8 @@ def chunk_bench(torch, pkg, spec, steps, replays):
         "config": {"workload": "chunks(%s)" % spec, "sequences": c["seqs"], "query_tokens": [c["qmin"], c["qmax"]],
                    "prior_tokens": c["prior"], "columns_per_kv_head": int(bt.max_seqlen) * (c["hq"] // c["hkv"]),
                    "cache_bytes": cache_bytes},
-        "tile_kernel_us": tile_us, "decode_kernel_path_us": chunk_us, "value": chunk_us if chunk_us else tile_us,
+        "tile_kernel_us": tile_us, "decode_kernel_path_us": chunk_us, "value": chunk_us if chunk_us else plain_us,
+        "no_workspace_us": plain_us, "kernels": {"tile": tile, "no_workspace": plain, "workspace": chunk},
         "decode_kernel_path_gbs": cache_bytes / (chunk_us * 1e-6) / 1e9 if chunk_us else None,
         "workspace_bytes": ws_bytes, "max_abs_difference_between_the_two": diff}))
 
