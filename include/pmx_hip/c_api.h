@@ -165,9 +165,10 @@ typedef struct pmxhip_decode_plan {
     int64_t partial_ml_size;    /* bytes: float32 (running max, exp-sum) pairs */
     int64_t workspace_size;     /* total bytes */
     int32_t kernel;             /* pmxhip_decode_kernel_t the plan was made for: the shape's over long streams.  A launch without
-                                   a request takes a few, or whole, sequences to the column kernels, and falls back to the
-                                   general kernel when the quad kernel's needs of the buffers (16-byte aligned
-                                   output rows) are not met; pmxhip_decode_kernel_name tells what a call runs. */
+                                   a request takes a few, or whole, sequences to the column kernels (MFMA16 / MFMA32), and
+                                   runs another kernel where the mask, the scale, the strides or the buffers (16-byte aligned
+                                   output rows) are not what the plan's needs: a column kernel for whole sequences, else the
+                                   general one; pmxhip_decode_kernel_name tells what a call runs. */
 } pmxhip_decode_plan;
 
 /* Host-only.  `compute_units` is hipDeviceProp_t::multiProcessorCount (0 = ask the current device).
@@ -185,7 +186,9 @@ PMXHIP_API int pmxhip_decode_attention(const pmxhip_decode_params* p, pmxhip_str
 
 /* Name of the token-range kernel that pmxhip_decode_attention(p) launches ("" if the call would be rejected):
  * one of decode_attention_kernel, decode_attention_quad_kernel, decode_attention_mfma16_kernel,
- * decode_attention_mfma_kernel, decode_attention_mfma32_kernel (32 columns, whole sequences) -- the names a profiler's kernel trace shows.  Host only, launches nothing. */
+ * decode_attention_mfma_kernel (32 columns over token ranges), decode_attention_mfma32_kernel (32 columns, whole sequences) -- the names
+ * a profiler's kernel trace shows; decode_attention_mfma16_kernel is a name of two kernels, for long and for short token ranges.  Host
+ * only, launches nothing. */
 PMXHIP_API const char* pmxhip_decode_kernel_name(const pmxhip_decode_params* p);
 
 /* pmxhip_decode_attention for callers that cannot allocate: it has no counterpart in the reference, whose caller

@@ -1,5 +1,5 @@
-// Decode attention over the int8 group-8 KV cache, variant for five to sixteen query heads per kv head at
-// head_dim 128 and for whole sequences of every shape (reference: src/ppl/kernel/llm/cuda/pmx/multi_head_cache_attention/kernel.cu:1090-1891,
+// Decode attention over the int8 group-8 KV cache, variant for whole sequences of every shape, for five to sixteen query heads per
+// kv head at head_dim 128 over long token ranges, for the shared pieces of a single sequence and for a few sequences at head_dim 64 (reference: src/ppl/kernel/llm/cuda/pmx/multi_head_cache_attention/kernel.cu:1090-1891,
 // the GQCA kernel, which also puts the query heads of a kv head on tensor cores), and for short prefill chunks.
 //
 // With that many query heads the per-head arithmetic of the VALU kernels outweighs the cache stream.
@@ -36,10 +36,11 @@
 //
 // What bounds it: over long ranges the arithmetic beside the cache stream (a wave's requests alone stream at 7.1 TB/s; two waves
 // per SIMD have some 460 vector instructions and 40 products per block to issue), with short sequences the chain of look-ups,
-// first rows and results of every wave.  Against the form that transposed V through LDS and requested a block ahead into registers:
-// 64 q / 8 kv heads of 128, 32 sequences of 10923-32768 tokens 268 -> 256 us (layer call), four of 30000-32768 75 -> 68.  Whole
-// sequences in one launch, against ranges and a combine launch: 32 / 8 heads, four of 85-256 13.8 -> 9.5; 8 / 1 heads of 256, 448 of
-// 92-148 39.2 -> 18.2; 28 / 4 heads, 49 of 138-381 18.3 -> 14.1.
+// first rows and results of every wave.  Layer calls against the kernel of decode_attn_mfma.hip, which transposes V through LDS and requests
+// a block ahead into registers: 64 q / 8 kv heads of 128, 32 sequences of 10923-32768 tokens 338 -> 320 us, four of 30000-32768 72.1 -> 68.7
+// (over short ranges that one is the faster: decode_ring).  Whole sequences in one launch, against ranges and a combine launch: 32 / 8 heads,
+// four of 85-256 14.7 -> 9.3; 8 / 1 heads of 256, 448 of 92-148 38.6 -> 19.1; 28 / 4 heads, 49 of 138-381 18.7 -> 15.2.
+// The form of 32 columns holds 255-256 VGPRs at head_dim 128 and spills two to four (12-20 bytes of scratch a lane); no other form spills.
 //
 // Ranges, pieces and the workspace are those of decode_attn.hip: one workgroup (a wave per kv head: four, or two
 // or one when the kv heads do not come in fours) per token range, cuts on multiples of 32 tokens, float32 pieces merged by decode_combine_kernel.

@@ -403,7 +403,8 @@ def test_prefill_tiles_split_from_current_key_value(pkg, oracle, shape, decodes)
 
 @pytest.mark.parametrize("shape,q_lens", [((32, 8, 64), [1, 63, 64, 65, 200, 700, 333, 900]), ((8, 8, 64), [1100, 257] * 6)])
 def test_prefill_from_current_key_value_more_tiles_than_compute_units(pkg, oracle, shape, q_lens):
-    """head_dim 64 over the step's half K/V rows with more (tile, kv head) items than compute units: two workgroups per CU."""
+    """head_dim 64 over the step's half K/V rows with more (tile, kv head) items than compute units: workgroups of four
+    waves, two per CU."""
     hq, hkv, d = shape
     ppw = 256 * hkv // hq
     assert sum((n + ppw - 1) // ppw for n in q_lens) * hkv > pkg.ops.compute_units()
