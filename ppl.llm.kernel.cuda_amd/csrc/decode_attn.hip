@@ -43,8 +43,9 @@ constexpr size_t decode_lds_bytes(int head_dim, int gt)
     return (size_t)gt * nslot * (head_dim + 2) * sizeof(float);
 }
 
-// D: head dim (64, 96, 128, 256).  GT: query heads per kv head held in registers.
-template <int D, int GT, bool PAGED, bool MASK>
+// D: head dim (64, 96, 128, 256).  GT: query heads per kv head held in registers.  SEQ: workgroup x takes sequence x whole (a form
+// of its own: decided at run time it cost the ranges 2 %, 32 / 32 heads of 96, one sequence of 3770-17224 tokens 19.8 -> 20.2 us a step).
+template <int D, int GT, bool PAGED, bool MASK, bool SEQ>
 __global__ __launch_bounds__(kDecodeThreads, (GT <= 4 ? 2 : 1)) void decode_attention_kernel(const DecodeLaunch a)
 {
     constexpr int LPS = (D == 64) ? 4 : (D == 256 ? 16 : 8); // lanes per slot
@@ -95,13 +96,9 @@ __global__ __launch_bounds__(kDecodeThreads, (GT <= 4 ? 2 : 1)) void decode_atte
     const int64_t kv_base = kvstarts[0];
     const int64_t total = stream_length(kvstarts[a.decoding_batches] - kv_base, a.decoding_batches);
     const int64_t per = tokens_per_range(total, a.ranges, wg_tokens, a.min_tokens_per_range);
-    int64_t r0 = (int64_t)blockIdx.x * per;
-    int64_t r1 = (r0 + per < total) ? r0 + per : total;
-    if (a.by_sequence) { // the workgroup's range is sequence blockIdx.x
-        r0 = sequence_origin(kvstarts[blockIdx.x] - kv_base, blockIdx.x);
-        r1 = r0 + (kvstarts[blockIdx.x + 1] - kvstarts[blockIdx.x]);
-    }
+    const int64_t r0 = SEQ ? sequence_origin(kvstarts[blockIdx.x] - kv_base, blockIdx.x) : (int64_t)blockIdx.x * per;
     if (r0 >= total) return;
+    const int64_t r1 = SEQ ? r0 + (kvstarts[blockIdx.x + 1] - kvstarts[blockIdx.x]) : ((r0 + per < total) ? r0 + per : total);
 
     // Addressing: a wave-uniform 64-bit base per block (scalar registers) plus a 32-bit per-lane
     // offset: (token in block) * stride_s + (head in group) * stride_h + channel.
@@ -756,34 +753,40 @@ __global__ __launch_bounds__(64) void splitkv_combine_rows_kernel(
 
 // ---- host-side launchers (called from the C ABI) -------------------------------
 
-template <int D, int GT, bool PAGED, bool MASK>
+template <int D, int GT, bool PAGED, bool MASK, bool SEQ>
 static DeviceMask& decode_variant_ready()
 {
     static DeviceMask ready{0};
     return ready;
 }
 
-template <int D, int GT, bool PAGED, bool MASK>
+template <int D, int GT, bool PAGED, bool MASK, bool SEQ>
 static int launch_decode_variant(const DecodeLaunch& a, dim3 grid, hipStream_t stream)
 {
     constexpr size_t lds_bytes = decode_lds_bytes(D, GT);
     // above the default limit of dynamic LDS per workgroup for the wider variants
-    if (int rc = ensure_dynamic_lds((const void*)decode_attention_kernel<D, GT, PAGED, MASK>, (int)lds_bytes, stream,
-                                    decode_variant_ready<D, GT, PAGED, MASK>()))
+    if (int rc = ensure_dynamic_lds((const void*)decode_attention_kernel<D, GT, PAGED, MASK, SEQ>, (int)lds_bytes, stream,
+                                    decode_variant_ready<D, GT, PAGED, MASK, SEQ>()))
         return rc;
-    hipLaunchKernelGGL((decode_attention_kernel<D, GT, PAGED, MASK>), grid, dim3(kDecodeThreads), lds_bytes, stream, a);
+    hipLaunchKernelGGL((decode_attention_kernel<D, GT, PAGED, MASK, SEQ>), grid, dim3(kDecodeThreads), lds_bytes, stream, a);
     return kLaunchOk;
+}
+
+template <int D, int GT, bool SEQ>
+static int launch_decode_dgts(const DecodeLaunch& a, dim3 grid, hipStream_t stream)
+{
+    const bool paged = a.cache_mode == 1;
+    const bool mask = a.attn_mask != nullptr;
+    if (paged) return mask ? launch_decode_variant<D, GT, true, true, SEQ>(a, grid, stream)
+                           : launch_decode_variant<D, GT, true, false, SEQ>(a, grid, stream);
+    return mask ? launch_decode_variant<D, GT, false, true, SEQ>(a, grid, stream)
+                : launch_decode_variant<D, GT, false, false, SEQ>(a, grid, stream);
 }
 
 template <int D, int GT>
 static int launch_decode_dgt(const DecodeLaunch& a, dim3 grid, hipStream_t stream)
 {
-    const bool paged = a.cache_mode == 1;
-    const bool mask = a.attn_mask != nullptr;
-    if (paged) return mask ? launch_decode_variant<D, GT, true, true>(a, grid, stream)
-                           : launch_decode_variant<D, GT, true, false>(a, grid, stream);
-    return mask ? launch_decode_variant<D, GT, false, true>(a, grid, stream)
-                : launch_decode_variant<D, GT, false, false>(a, grid, stream);
+    return a.by_sequence ? launch_decode_dgts<D, GT, true>(a, grid, stream) : launch_decode_dgts<D, GT, false>(a, grid, stream);
 }
 
 template <int D>
@@ -841,18 +844,24 @@ static int launch_decode_d(const DecodeLaunch& a, int stage, hipStream_t stream)
 }
 
 // the one-time attribute call of every variant (pmxhip_init)
-template <int D, int GT>
-static int init_decode_dgt()
+template <int D, int GT, bool SEQ>
+static int init_decode_dgts()
 {
     int rc = kLaunchOk;
     auto one = [&](const void* k, DeviceMask& ready) {
         if (rc == kLaunchOk) rc = set_dynamic_lds_once(k, (int)decode_lds_bytes(D, GT), ready);
     };
-    one((const void*)decode_attention_kernel<D, GT, true, true>, decode_variant_ready<D, GT, true, true>());
-    one((const void*)decode_attention_kernel<D, GT, true, false>, decode_variant_ready<D, GT, true, false>());
-    one((const void*)decode_attention_kernel<D, GT, false, true>, decode_variant_ready<D, GT, false, true>());
-    one((const void*)decode_attention_kernel<D, GT, false, false>, decode_variant_ready<D, GT, false, false>());
+    one((const void*)decode_attention_kernel<D, GT, true, true, SEQ>, decode_variant_ready<D, GT, true, true, SEQ>());
+    one((const void*)decode_attention_kernel<D, GT, true, false, SEQ>, decode_variant_ready<D, GT, true, false, SEQ>());
+    one((const void*)decode_attention_kernel<D, GT, false, true, SEQ>, decode_variant_ready<D, GT, false, true, SEQ>());
+    one((const void*)decode_attention_kernel<D, GT, false, false, SEQ>, decode_variant_ready<D, GT, false, false, SEQ>());
     return rc;
+}
+template <int D, int GT>
+static int init_decode_dgt()
+{
+    if (int rc = init_decode_dgts<D, GT, false>()) return rc;
+    return init_decode_dgts<D, GT, true>();
 }
 template <int D>
 static int init_decode_d()
