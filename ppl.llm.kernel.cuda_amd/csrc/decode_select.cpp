@@ -250,22 +250,25 @@ bool quad_takes_whole(const DecodeLaunch& a) { return a.num_kv_repeats <= 4 && d
 // 1-512 sequences x 64-16384 tokens and short chunks of 1-32 columns, lengths L / 3 to L, ten layers in turn.  Where shapes of
 // a row differ the shorter one stands, so that a batch next to the line is seldom slower than over ranges (of 1900 batches 3 by
 // more than 8 %).  Few workgroups leave the chip idle and ranges fill it; from one per CU on the waves are there either
-// way, and ranges even out the lengths.  Past eight per CU the waves come in a second round.
+// way, and ranges even out the lengths.  Past eight per CU the waves come in a second round.  While workgroups are few, eight waves
+// share a sequence and another 256 tokens are another block for each: the step's time rises there at once (32 / 32 heads of 96, one
+// sequence: whole 0.93 of the time over ranges at 500 tokens, 1.18 at 600; 24 / 1 of 128, seven: 0.99 at 250, 1.20 at 320; 16 / 16 of
+// 256, four: 0.95 and 1.12), so those lines lie on multiples of 256.
 struct WholeUpTo {
     double masked;         // with a mask, times this where the column kernels run: they wait for its values, the quad kernel streams them
     int32_t tokens[15];    // workgroups per CU up to kWholeLoads[i], and beyond
 };
 constexpr double kWholeLoads[14] = {0.05, 0.1, 0.2, 0.4, 0.75, 1, 1.6, 2, 2.75, 3.5, 5, 8, 15.99, 32};
-constexpr WholeUpTo kWholeColumns16 = {0.6, {440, 470, 500, 660, 825, 1150, 765, 765, 595, 590, 520, 500, 400, 500, 500}};
-constexpr WholeUpTo kWholeColumns32 = {0.6, {280, 330, 390, 580, 1300, 1600, 1400, 1400, 1290, 1200, 1200, 900, 700, 600, 600}};
+constexpr WholeUpTo kWholeColumns16 = {0.6, {440, 470, 500, 512, 825, 1150, 765, 765, 595, 590, 520, 500, 400, 500, 500}};
+constexpr WholeUpTo kWholeColumns32 = {0.6, {256, 256, 256, 580, 1300, 1600, 1400, 1400, 1290, 1200, 1200, 900, 700, 600, 600}};
 constexpr WholeUpTo kWholeColumns64 = {0.9, {600, 710, 740, 1030, 1500, 1030, 800, 560, 700, 550, 650, 720, 400, 550, 550}}; // head_dim 64
-constexpr WholeUpTo kWholeQuad64 = {0.45, {850, 850, 850, 1600, 1600, 1300, 800, 600, 560, 560, 530, 380, 380, 900, 900}};
-constexpr WholeUpTo kWholeQuad128One = {1.0, {480, 480, 510, 610, 620, 700, 350, 295, 175, 175, 140, 500, 220, 200, 200}}; // one query head per kv head
-constexpr WholeUpTo kWholeQuad128 = {0.6, {500, 570, 600, 800, 970, 1000, 880, 680, 640, 340, 300, 300, 150, 400, 400}};
-constexpr WholeUpTo kWholeQuad256One = {1.0, {400, 400, 400, 410, 420, 430, 250, 185, 90, 90, 0, 190, 190, 190, 190}};
-constexpr WholeUpTo kWholeQuad256 = {0.55, {450, 450, 470, 600, 760, 780, 550, 500, 300, 260, 160, 160, 160, 200, 200}};
-constexpr WholeUpTo kWholeQuad256Two = {1.0, {450, 570, 590, 1140, 1600, 1600, 1600, 1600, 1600, 1600, 1600, 1600, 1600, 1600, 1600}}; // two sets of waves
-constexpr WholeUpTo kWholeGeneralOne = {0.75, {580, 580, 600, 800, 520, 560, 350, 285, 200, 170, 145, 145, 128, 100, 0}};
+constexpr WholeUpTo kWholeQuad64 = {0.45, {850, 850, 850, 1600, 1600, 1000, 800, 600, 560, 560, 530, 380, 380, 900, 900}};
+constexpr WholeUpTo kWholeQuad128One = {1.0, {480, 480, 510, 512, 512, 512, 350, 295, 175, 175, 140, 500, 220, 200, 200}}; // one query head per kv head
+constexpr WholeUpTo kWholeQuad128 = {0.6, {500, 512, 512, 512, 970, 1000, 880, 680, 640, 340, 300, 300, 150, 400, 400}};
+constexpr WholeUpTo kWholeQuad256One = {1.0, {256, 256, 256, 256, 420, 430, 250, 185, 90, 90, 0, 190, 190, 190, 190}};
+constexpr WholeUpTo kWholeQuad256 = {0.55, {450, 450, 470, 512, 760, 780, 550, 500, 300, 260, 160, 160, 160, 200, 200}};
+constexpr WholeUpTo kWholeQuad256Two = {1.0, {256, 512, 512, 1140, 1600, 1600, 1600, 1600, 1600, 1600, 1600, 1600, 1600, 1600, 1600}}; // two sets of waves
+constexpr WholeUpTo kWholeGeneralOne = {0.75, {512, 512, 512, 512, 512, 512, 350, 285, 200, 170, 145, 145, 128, 100, 0}};
 constexpr WholeUpTo kWholeGeneralFour = {1.0, {930, 930, 1100, 1600, 1600, 1600, 980, 980, 700, 600, 560, 500, 370, 530, 530}};
 constexpr int32_t kAnyLength = INT32_MAX; // many query heads on the general kernel: several times the column kernels' time
 constexpr WholeUpTo kWholeGeneral = {1.0, {870, 1400, 1400, kAnyLength, kAnyLength, kAnyLength, kAnyLength, kAnyLength, kAnyLength, kAnyLength,
@@ -305,8 +308,10 @@ int64_t whole_up_to(const DecodeChoice& by_shape, int64_t sequences, int64_t hea
     }
     if (by_shape.kernel == kDecodeKernelMfma32 && head_dim == 64 && sequences <= kFewSequences && tokens > 590) tokens = 590;
     // a step of a few sequences has ranges of the column kernels' own
-    if (by_shape.kernel == kDecodeKernelQuad && few_sequences_on_columns(sequences, head_dim, columns))
-        tokens = tokens < (head_dim == 64 ? 700 : 480) ? tokens : (head_dim == 64 ? 700 : 480);
+    if (by_shape.kernel == kDecodeKernelQuad && few_sequences_on_columns(sequences, head_dim, columns)) {
+        const int64_t most = head_dim != 64 ? 480 : (sequences == 1 ? 512 : 700);
+        if (tokens > most) tokens = most;
+    }
     return tokens;
 }
 

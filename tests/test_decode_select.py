@@ -58,10 +58,13 @@ def test_a_single_range_without_a_request_is_never_one_workgroup(select, form):
 # (sequences, query heads, kv heads, head_dim, longest): measured per decode call, whole sequences / ranges + combine
 WHOLE = [(60, 8, 8, 64, 500), (100, 32, 8, 64, 300), (16, 14, 2, 64, 700), (32, 32, 8, 128, 256), (5, 32, 8, 128, 500), (60, 64, 8, 128, 500),
          (300, 8, 1, 128, 500), (512, 8, 1, 128, 500), (100, 40, 1, 96, 8000), (300, 24, 2, 256, 8000), (30, 24, 1, 256, 8000), (300, 32, 32, 128, 128),
-         (512, 32, 8, 128, 300), (300, 8, 1, 256, 1600), (512, 16, 8, 256, 150)]
+         (512, 32, 8, 128, 300), (300, 8, 1, 256, 1600), (512, 16, 8, 256, 150), (1, 32, 32, 96, 500), (7, 16, 4, 128, 500), (7, 24, 1, 128, 250),
+         (4, 16, 16, 256, 250), (16, 8, 1, 256, 510), (4, 32, 8, 64, 600)]
 CUT = [(300, 8, 8, 64, 1600), (100, 8, 8, 64, 2400), (300, 32, 8, 64, 1000), (100, 40, 8, 64, 4000), (300, 14, 2, 64, 8000), (300, 48, 1, 128, 2400),
        (100, 32, 32, 96, 200), (300, 32, 32, 96, 128), (30, 8, 8, 96, 1000), (300, 16, 8, 128, 500), (160, 32, 32, 128, 300), (160, 16, 16, 256, 200),
-       (5, 8, 1, 128, 700), (160, 28, 4, 128, 1000), (300, 64, 8, 128, 500)]
+       (5, 8, 1, 128, 700), (160, 28, 4, 128, 1000), (300, 64, 8, 128, 500), (1, 32, 32, 96, 600), (2, 32, 32, 96, 600), (7, 8, 8, 96, 600),
+       (2, 32, 32, 128, 600), (7, 16, 4, 128, 600), (7, 64, 8, 128, 600), (7, 24, 1, 128, 320), (4, 16, 16, 256, 320), (7, 8, 8, 256, 320),
+       (1, 8, 1, 256, 320), (7, 32, 32, 64, 1030), (1, 32, 8, 64, 600)]
 
 
 def test_sequences_are_taken_whole_where_that_was_measured_faster(select):
